@@ -1,0 +1,305 @@
+"""Performance cases of the quantized matrix path and of the layers around it.
+
+What users have the library do, over the range they do it in: one product, the packed products of a
+model's step at every run length of a serving schedule (one token up to a chunk of 512), whole layers and
+whole models with every small op, and the packing of a model's matrices at load time.  Four kinds of case:
+
+  product  one `Matrix.matmul_op` call, issued eagerly (a host program that calls op by op)
+  step     the eight packed products of `layers` v6 layers for `tokens` tokens: {k, v, r, g} in one grouped
+           call, att.output, {ffn.key, ffn.receptance} in one grouped call, ffn.value; the step is captured
+           once into a HIP graph per run length and replayed, as a serving loop keeps it
+  model    every op of `layers` v5, v6 or v7 layers (with `vocab` > 0 also embedding, head and softmax) for a
+           run of `tokens` tokens of `requests` requests, from a HIP graph as well; the recurrent state is kept
+           from pass to pass as generation keeps it
+  pack     Int8 or NF4 packing of the eight matrices of a layer, eager, outputs allocated as the loader does
+
+Model shapes are the repository's own (d_model, FFN): the 0.1B shape of the end-to-end test and the v6
+sizes of the benchmark; v7 layers take FFN = 4 x d_model.
+"""
+import importlib
+import math
+
+import numpy as np
+import torch
+
+wrq = importlib.import_module("web-rwkv_amd")
+
+SHAPES = {"0b1": (768, 2688), "0b4": (1024, 3584), "1b6": (2048, 7168), "3b": (2560, 8960), "7b": (4096, 14336), "14b": (5120, 17920)}
+HEAD = 64  # channels per head
+MAX_BYTES, MAX_FLOPS = 0.9e9, 3.3e11  # a drawn case stays below the listed ones: 4 layers of 7B Int8, 3 layers x 256 tokens of 7B
+
+
+def listed():
+    return [
+        # the smallest call: one attention-sized product of a 1.6B model at one token, from an eager program
+        dict(name="product_1b6_int8_t1", kind="product", quant="int8", K=2048, R=2048, tokens=1, x="f16", out="f16", act=0),
+        # one user generating: batch-1 decode of the 7B shape, both formats
+        dict(name="step_7b_int8_t1", kind="step", model="7b", quant="int8", tokens=1, layers=4),
+        dict(name="step_7b_nf4_t1", kind="step", model="7b", quant="nf4", tokens=1, layers=4),
+        # a handful of slots decoding together, the tail of a schedule: small matrices, many launches
+        dict(name="step_1b6_nf4_t5", kind="step", model="1b6", quant="nf4", tokens=5, layers=12),
+        # a ragged mixture of decoding slots and a short prompt on a width that is no power of two
+        dict(name="step_3b_int8_t19", kind="step", model="3b", quant="int8", tokens=19, layers=6),
+        # all 32 slots of a server decoding
+        dict(name="step_7b_nf4_t32", kind="step", model="7b", quant="nf4", tokens=32, layers=3),
+        # prompt chunks: 128 tokens for one user, 256 in the multi-slot server
+        dict(name="step_7b_int8_t128", kind="step", model="7b", quant="int8", tokens=128, layers=2),
+        dict(name="step_7b_nf4_t256", kind="step", model="7b", quant="nf4", tokens=256, layers=3),
+        # whole models with every op: a token of one user and the last, odd chunk of a prompt on v6, 32 decoding slots on v7
+        dict(name="model_v6_7b_int8_t1", kind="model", version=6, model="7b", quant="int8", tokens=1, requests=1, layers=2, vocab=65536),
+        dict(name="model_v6_1b6_int8_t100", kind="model", version=6, model="1b6", quant="int8", tokens=100, requests=1, layers=4, vocab=0),
+        dict(name="model_v7_1b6_nf4_32x1", kind="model", version=7, model="1b6", quant="nf4", tokens=32, requests=32, layers=4, vocab=0),
+        # loading: the eight matrices of a 7B layer packed
+        dict(name="pack_7b_int8", kind="pack", model="7b", quant="int8"),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return min(hi, max(lo, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+
+def draw(rng):
+    kind = rng.choice(["product", "step", "step", "step", "model", "model", "pack"])
+    quant = rng.choice(["int8", "nf4"])
+    if kind == "product":
+        quant = rng.choice(["int8", "nf4", "fp16"])
+        # K in whole 64-element blocks and R in quads, as the reference wants them; odd multiples among both
+        K, R = 64 * _log_int(rng, 5, 224), 4 * _log_int(rng, 32, 4608)
+        while quant == "int8" and K * R % 128:
+            R += 4
+        tokens = _log_int(rng, 1, 512)
+        while 2.0 * K * R * tokens > MAX_FLOPS:
+            tokens //= 2
+        return dict(kind=kind, quant=quant, K=K, R=R, tokens=tokens, x=rng.choice(["f16", "f16", "f32"]), out=rng.choice(["f16", "f32"]), act=rng.randrange(8))
+    if kind == "pack":
+        return dict(kind=kind, model=rng.choice(list(SHAPES)[:5]), quant=quant)
+    model = rng.choice(list(SHAPES))
+    case = dict(kind=kind, model=model, quant=quant, tokens=_log_int(rng, 1, 512), layers=1)
+    if kind == "model":
+        case["version"] = rng.choice([5, 6, 7])
+        case["tokens"] = _log_int(rng, 1, 128)
+        case["requests"] = rng.choice([1, 1, min(case["tokens"], rng.randint(2, 8)), case["tokens"]])
+        case["vocab"] = 65536 if case["tokens"] <= 32 and rng.random() < 0.5 else 0
+    one = work(case)
+    most = int(min(MAX_BYTES / one["bytes"], MAX_FLOPS / one["flops"], 4 if kind == "model" else 12))
+    case["layers"] = max(1, rng.randint(max(1, most // 2), max(1, most)))
+    return case
+
+
+def _generator(seed):
+    return torch.Generator(device="cuda").manual_seed(int(seed))
+
+
+def _pack(quant, w):
+    return wrq.Matrix.fp16(w) if quant == "fp16" else wrq.Matrix.quant_u8(w) if quant == "int8" else wrq.Matrix.quant_nf4(w)
+
+
+def _dtype(name):
+    return torch.float16 if name == "f16" else torch.float32
+
+
+def _weights(g, R, K, scale=0.02):
+    # N(0, 0.02), the initialisation the repository's models use
+    return (torch.randn((R, K), generator=g, device="cuda") * scale).half()
+
+
+def _capture(step):
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    return graph
+
+
+def _prepare_product(case, g):
+    m = _pack(case["quant"], _weights(g, case["R"], case["K"]))
+    x = torch.randn((case["tokens"], case["K"]), generator=g, device="cuda").to(_dtype(case["x"]))
+    out = torch.empty((case["tokens"], case["R"]), dtype=_dtype(case["out"]), device="cuda")
+    return dict(kind="product", m=m, x=x, out=out, act=case["act"], turbo=wrq.turbo(case["tokens"]))
+
+
+def _prepare_step(case, g):
+    C, H = SHAPES[case["model"]]
+    T, quant = case["tokens"], case["quant"]
+    f16, f32 = torch.float16, torch.float32
+    turbo = wrq.turbo(T)
+    new = lambda n, dt: torch.empty((T, n), dtype=dt, device="cuda")
+    sx = torch.randn((5, T, C), generator=g, device="cuda").to(f16)
+    ax, kx, rx = (torch.randn((T, C), generator=g, device="cuda").to(f16) for _ in range(3))
+    layers = []
+    for i in range(case["layers"]):
+        mats = [_pack(quant, _weights(g, C, C)) for _ in range(6)] + [_pack(quant, _weights(g, H, C)), _pack(quant, _weights(g, C, H))]
+        # key, value and receptance are f32 for the recurrence, the rest f16 (the runtime buffers of a v6 layer)
+        outs = [new(C, f32), new(C, f32), new(C, f32), new(C, f16), new(C, f16), new(C, f16), new(H, f16), new(C, f16)]
+        layers.append((mats, outs))
+
+    def step():
+        for (k, v, r, g_, o, fr, fk, fv), (ok, ov, orr, og, oo, ofr, ofk, ofv) in layers:
+            wrq.matmul_vec_group([(m, sx, out, wrq.ACT_NONE, False, dict(input_view=((C, T, 1), (C, T, 5), (0, 0, j))))
+                                  for j, (m, out) in enumerate(((k, ok), (v, ov), (r, orr), (g_, og)), 1)])
+            o.matmul_op(ax, oo, turbo=turbo)
+            wrq.matmul_vec_group([(fk, kx, ofk, wrq.ACT_SQUARED_RELU, False, {}), (fr, rx, ofr, wrq.ACT_NONE, False, {})])
+            fv.matmul_op_sparse(ofk, ofv, turbo=turbo)
+
+    return dict(kind="step", graph=_capture(step), outs=[o for _, outs in layers for o in outs][:64], keep=(layers, sx, ax, kx, rx))
+
+
+def _random_layer(version, g, C, H, layer):
+    """The weights of one layer in the form `Layer` takes (numpy, made on the GPU): matrices N(0, 0.02),
+    vectors in the ranges the layer modules' own random weights have."""
+    heads = C // HEAD
+    n = lambda *s, std=0.02, mean=0.0, dt=torch.float16: (torch.randn(s, generator=g, device="cuda") * std + mean).to(dt).cpu().numpy()
+    u = lambda *s: torch.rand(s, generator=g, device="cuda").half().cpu().numpy()
+    disc = 2.0 ** -(layer // 6)
+    w = {"att_ln_w": n(C, std=0.1, mean=1.0), "att_ln_b": n(C, std=0.1), "ffn_ln_w": n(C, std=0.1, mean=1.0), "ffn_ln_b": n(C, std=0.1),
+         "gn_w": n(heads, HEAD, std=0.1, mean=1.0), "gn_b": n(heads, HEAD, std=0.1)}
+    if version == 7:
+        w.update(w0=n(C, std=0.5, mean=-1.0), a0=n(C, std=0.5), v0=n(C, std=0.5), r_k=n(heads, HEAD, std=0.3), k_k=n(C, std=0.3, mean=0.5), k_a=u(C))
+        for name, rank in (("w", 64), ("a", 64), ("g", 128), ("v", 32)):
+            w[name + "1"], w[name + "2"] = n(rank, C, std=0.05), n(C, rank, std=0.1)
+        for name in ("x_r", "x_w", "x_k", "x_v", "x_a", "x_g", "ffn_x_k"):
+            w[name] = u(C)
+        mats = {"att_w_r": (C, C), "att_w_k": (C, C), "att_w_v": (C, C), "att_w_o": (C, C), "ffn_w_k": (H, C), "ffn_w_v": (C, H)}
+    else:
+        w["time_first"] = n(heads, HEAD, std=0.3, dt=torch.float32)
+        decay = n(heads, HEAD, std=0.5, mean=-1.0, dt=torch.float32)
+        if version == 5:
+            w["time_decay"] = np.exp(-np.exp(decay)).astype(np.float32)
+            shifts = ("time_mix_k", "time_mix_v", "time_mix_r", "time_mix_g")
+        else:
+            w["time_decay"] = decay.reshape(-1).astype(np.float16)
+            w.update(time_mix=u(5, 1, C), time_mix_w1=n(5 * 32, C), time_mix_w2=n(5, C, 32, std=0.1), time_decay_w1=n(64, C), time_decay_w2=n(C, 64, std=0.1))
+            shifts = ("time_mix_x",)
+        for name in shifts + ("ffn_time_mix_k", "ffn_time_mix_r"):
+            w[name] = u(C)
+        mats = {"att_w_k": (C, C), "att_w_v": (C, C), "att_w_r": (C, C), "att_w_g": (C, C), "att_w_o": (C, C), "ffn_w_k": (H, C), "ffn_w_v": (C, H), "ffn_w_r": (C, C)}
+    for name, (R, K) in mats.items():
+        scale = 0.02 * (disc if version != 7 and name in ("att_w_o", "ffn_w_v") else 1.0)
+        w[name] = _weights(g, R, K, scale).cpu().numpy()
+    return w
+
+
+def _split(tokens, requests):
+    """Lengths of `requests` consecutive requests that fill a stack of `tokens` tokens."""
+    return [tokens // requests + (i < tokens % requests) for i in range(requests)]
+
+
+def _prepare_model(case, g):
+    version, A, n = case["version"], case["tokens"], case["requests"]
+    C, H = SHAPES[case["model"]]
+    H = 4 * C if version == 7 else H
+    heads = C // HEAD
+    mod = importlib.import_module("web-rwkv_amd.v%d" % version)
+    layers = [mod.Layer(torch, _random_layer(version, g, C, H, i), case["quant"]) for i in range(case["layers"])]
+    # the slots hold a conversation already: a state of the size the recurrence keeps
+    states = [torch.randn((n, HEAD + 2, C), generator=g, device="cuda") * 0.3 for _ in layers]
+    cursors, at = [], 0
+    for slot, length in enumerate(_split(A, n)):
+        cursors += [slot | at << 8 | length << 24] * length
+        at += length
+    cursors = torch.from_numpy(np.array(cursors, dtype=np.uint32).view(np.int32)).cuda()
+    buf = mod.Runtime(torch, C, H, A)
+    ln_w, ln_b = (1.0 + 0.1 * torch.randn(C, generator=g, device="cuda")).half(), (0.1 * torch.randn(C, generator=g, device="cuda")).half()
+    V = case["vocab"]
+    x0 = torch.randn((1, A, C), generator=g, device="cuda").half()
+    if V:
+        embed, head = _weights(g, V, C, 0.5), wrq.Matrix.fp16(_weights(g, V, C))
+        ids = torch.randint(0, V, (1, A), generator=g, device="cuda", dtype=torch.int32)
+        last = np.cumsum(_split(A, n)) - 1
+        head_x = torch.zeros((1, n, C), dtype=torch.float16, device="cuda")
+        logits = torch.zeros((1, n, V), dtype=torch.float32, device="cuda")
+        probs = torch.zeros((1, n, V), dtype=torch.float32, device="cuda")
+
+    def step():
+        if V:
+            wrq.LayerOp.embed(ids, embed, x0)
+            wrq.LayerOp.layer_norm(ln_w, ln_b, x0, mod.LN_EPS)
+        wrq.LayerOp.blit(x0, buf.x)
+        for i, (layer, state) in enumerate(zip(layers, states)):
+            rescale = (i + 1) % 6 == 0
+            if version == 6:
+                mod.dispatch_layer_auto(layer, buf, state, cursors, A, heads, HEAD, rescale)
+            elif version == 5:
+                mod.dispatch_layer(layer, buf, state, cursors, A, heads, HEAD, rescale)
+            else:
+                mod.dispatch_layer(layer, buf, state, cursors, A, heads, HEAD, i)
+        if V:
+            for i, t in enumerate(last):
+                wrq.LayerOp.blit(buf.x, head_x, input_view=((C, 1, 1), (C, A, 1), (0, int(t), 0)), output_view=((C, 1, 1), (C, n, 1), (0, i, 0)))
+            wrq.LayerOp.layer_norm(ln_w, ln_b, head_x, mod.LN_EPS)
+            head.matmul_op(head_x, logits, turbo=wrq.turbo(n))
+            wrq.LayerOp.blit(logits, probs)
+            wrq.LayerOp.softmax(probs)
+
+    start = [s.clone() for s in states]
+    graph = _capture(step)
+    for s, s0 in zip(states, start):
+        s.copy_(s0)  # the warm-up pass of the capture leaves no trace
+    outs = [buf.x] + states + ([logits, probs] if V else [])
+    return dict(kind="model", graph=graph, outs=outs, keep=(layers, states, cursors, buf, ln_w, ln_b, x0, (embed, head, ids, head_x) if V else None))
+
+
+def _prepare_pack(case, g):
+    C, H = SHAPES[case["model"]]
+    return dict(kind="pack", quant=case["quant"], ws=[_weights(g, C, C) for _ in range(6)] + [_weights(g, H, C), _weights(g, C, H)])
+
+
+def prepare(case, seed):
+    g = _generator(seed)
+    return dict(product=_prepare_product, step=_prepare_step, model=_prepare_model, pack=_prepare_pack)[case["kind"]](case, g)
+
+
+def run(state):
+    kind = state["kind"]
+    if kind == "product":
+        state["m"].matmul_op(state["x"], state["out"], state["act"], state["turbo"])
+        return state["out"]
+    if kind == "pack":
+        packed = [_pack(state["quant"], w) for w in state["ws"]]
+        return [t for m in packed for t in (m.w, m.m)]
+    state["graph"].replay()
+    return state["outs"]
+
+
+def _weight_bytes(quant, n):
+    return 2 * n if quant == "fp16" else n + 4 * n / 128 if quant == "int8" else n / 2 + 2 * n / 64
+
+
+def work(case):
+    if case["kind"] == "product":
+        K, R, T = case["K"], case["R"], case["tokens"]
+        xs, os_ = (2 if case["x"] == "f16" else 4), (2 if case["out"] == "f16" else 4)
+        return {"bytes": _weight_bytes(case["quant"], K * R) + xs * K * T + os_ * R * T, "flops": 2.0 * K * R * T}
+    C, H = SHAPES[case["model"]]
+    if case["kind"] == "pack":
+        n = 6 * C * C + 2 * C * H
+        return {"bytes": 2 * n + _weight_bytes(case["quant"], n), "flops": 0}
+    T, L, quant = case["tokens"], case["layers"], case["quant"]
+    if case["kind"] == "step":
+        n = 6 * C * C + 2 * C * H
+        io = T * (2 * (7 * C) + 4 * 3 * C + 2 * (3 * C + H) + 2 * H)  # inputs, f32 outputs, f16 outputs, ffn.value's input
+        return {"bytes": L * (_weight_bytes(quant, n) + io), "flops": 2.0 * n * T * L}
+    version, n_req, V = case["version"], case["requests"], case["vocab"]
+    if version == 7:
+        n, small = 4 * C * C + 8 * C * C, 2 * C * (64 + 64 + 128 + 32)
+    else:
+        n, small = 6 * C * C + 2 * C * H, 0 if version == 5 else C * (2 * 5 * 32 + 2 * 64)
+    state = 2 * 4 * n_req * (HEAD + 2) * C
+    layer = _weight_bytes(quant, n) + 2 * small + 2 * 30 * C + state
+    flops = 2.0 * T * (n + small) + T * C * HEAD * (10.0 if version == 7 else 5.0)
+    ends = 2 * 2 * T * C + (V * C * 2 + 2 * T * C + 8 * n_req * V if V else 0)
+    return {"bytes": L * layer + ends, "flops": L * flops + (2.0 * n_req * V * C if V else 0)}
+
+
+def tolerance(case):
+    if case["kind"] == "pack":
+        return "exact"  # packed bytes and scale blocks are fixed bit for bit
+    # Four times what the same kernels differ by when tiles, splits and kernel choice (and with them the order of
+    # the f32 sums) are changed: 3e-7 with f32 outputs, 1.8e-4 and one f16 ulp (9.8e-4 of the value) where outputs
+    # are rounded to f16, 1.7e-3 and 1.2e-2 of the rms where such roundings pass through up to four layers.
+    if case["kind"] == "product" and case["out"] == "f32":
+        return {"rel": 1e-5}
+    if case["kind"] in ("product", "step"):
+        return {"rel": 8e-4, "max": 4e-3}
+    return {"rel": 7e-3, "max": 5e-2}
