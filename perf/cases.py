@@ -303,3 +303,58 @@ def tolerance(case):
     if case["kind"] in ("product", "step"):
         return {"rel": 8e-4, "max": 4e-3}
     return {"rel": 7e-3, "max": 5e-2}
+
+
+NF4 = (-1.0, -0.6961928009986877, -0.5250730514526367, -0.39491748809814453, -0.28444138169288635, -0.18477343022823334, -0.09105003625154495, 0.0,
+       0.07958029955625534, 0.16093020141124725, 0.24611230194568634, 0.33791524171829224, 0.44070982933044434, 0.5626170039176941, 0.7229568362236023, 1.0)
+
+
+def _dequantized(quant, w):
+    """The matrix that the packed form of `w` stands for, in 64 bits: the packing rules are fixed bit for bit."""
+    if quant == "fp16":
+        return w.double()
+    if quant == "int8":
+        block = w.float().view(-1, 128)
+        lo, hi = block.amin(1, keepdim=True), block.amax(1, keepdim=True)
+        code = torch.round(((block - lo) / (hi - lo)).nan_to_num(0.0).clamp(0.0, 1.0) * 255.0)
+        return (lo.double() + (hi - lo).double() * (code.double() / 255.0)).view(w.shape)
+    block = w.float().view(-1, 64)
+    absmax = block.abs().amax(1, keepdim=True)
+    scaled = block * (1.0 / absmax)
+    best, code = torch.ones_like(scaled), torch.zeros_like(scaled, dtype=torch.int64)
+    for i, q in enumerate(NF4):  # the nearest entry, the later one on a tie
+        err = (torch.full_like(scaled, q) - scaled).abs()
+        take = err <= best
+        best, code = torch.where(take, err, best), torch.where(take, torch.full_like(code, i), code)
+    table = torch.tensor(NF4, dtype=torch.float32, device=w.device).double()
+    return (absmax.double() * table[code]).view(w.shape)
+
+
+def _activation(act, x):
+    return (lambda v: v, lambda v: v.clamp(min=0.0) ** 2, torch.tanh, lambda v: torch.exp(-torch.exp(v)), lambda v: -torch.exp(v),
+            lambda v: torch.log1p(torch.exp(v)), torch.sigmoid, lambda v: v * torch.sigmoid(v))[act](x)
+
+
+def exact(case, seed):
+    """`run` in 64 bits on the dequantized matrices.  A step's ffn.value takes its input rounded to f16, the type
+    of the buffer between the two products.  None for packing, whose bytes are compared as they are, and for whole
+    models: between any two of their ops lie buffers that are f16 by definition."""
+    g = _generator(seed)
+    if case["kind"] == "product":
+        w = _dequantized(case["quant"], _weights(g, case["R"], case["K"]))
+        x = torch.randn((case["tokens"], case["K"]), generator=g, device="cuda").to(_dtype(case["x"]))
+        return _activation(case["act"], x.double() @ w.t())
+    if case["kind"] != "step":
+        return None
+    C, H = SHAPES[case["model"]]
+    T, quant = case["tokens"], case["quant"]
+    sx = torch.randn((5, T, C), generator=g, device="cuda").half().double()
+    ax, kx, rx = (torch.randn((T, C), generator=g, device="cuda").half().double() for _ in range(3))
+    outs = []
+    for _ in range(case["layers"]):
+        weights = [_weights(g, C, C) for _ in range(6)] + [_weights(g, H, C), _weights(g, C, H)]
+        product = lambda i, x: x @ _dequantized(quant, weights[i]).t()
+        outs += [product(i, sx[i + 1]) for i in range(4)] + [product(4, ax), product(5, rx)]
+        key = product(6, kx).clamp(min=0.0) ** 2
+        outs += [key, product(7, key.half().double())]
+    return outs[:64]
