@@ -1,0 +1,45 @@
+"""The state recurrences where a workgroup walks one slot's tokens: more tokens than one scan of the cursors (256),
+a slot that comes twice in the stack, slots without a token, a view of one slot only."""
+import importlib
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from helpers import assert_close
+from test_layer_ops import wkv6_float64, wkv6_inputs, wkv7_float64, wkv7_inputs
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("version,S", [(5, 16), (5, 256), (6, 16), (6, 32), (6, 64), (6, 256), (7, 32), (7, 64), (7, 128)])
+@pytest.mark.parametrize("B,runs", [(6, [(4, 15), (1, 241), (4, 17), (0, 3), (5, 1)]), (1, [(0, 255), (0, 18)]), (6, [(b, 1) for b in range(6)])])
+def test_gpu_slots(gpu, version, S, B, runs):
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("recurrence over slots on the GPU", version, S, B, runs, flush=True)
+    rng = np.random.default_rng(0x57525400 + S + B)
+    H = 2
+    cur = lop.pack_cursors(runs)
+    A = len(cur)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    curd = dev(cur.view(np.int32))
+    if version == 7:
+        r, w, n, x, state = wkv7_inputs(rng, A, H, S, B, np.float32)
+        sd, xd = dev(state), dev(x)
+        gpu.LayerOp.time_mix_v7(curd, sd, dev(r), dev(w), dev(n), xd)
+        want, want_state = wkv7_float64(cur, state, r, w, n, x)
+    else:
+        k, v, r, x, w, u, state = wkv6_inputs(rng, A, H, S, B, np.float32)
+        if version == 5:
+            w = np.broadcast_to(w[0], w.shape)
+        sd, xd = dev(state), dev(x)
+        (gpu.LayerOp.time_mix_v5 if version == 5 else gpu.LayerOp.time_mix_v6)(curd, dev(w[0] if version == 5 else w), dev(u), sd, dev(k), dev(v), dev(r), xd)
+        want, want_state = wkv6_float64(cur, w, u, state, k, v, r, x)
+    # f32 sums of S terms, the state's rounding accumulated over up to 273 tokens with a decay below 1
+    assert_close(xd.cpu().numpy(), want, 5e-5, "y vs float64")
+    assert_close(sd.cpu().numpy(), want_state, 5e-5, "state vs float64")

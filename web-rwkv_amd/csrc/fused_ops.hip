@@ -10,7 +10,7 @@
 //   wrq_v6_post_ffn     channel_mix + add (+ affine 0.5)                   v6.rs:942-955
 // They have no counterpart among the reference's constructors; buffers are the f16 / f32 tensors of
 // `Runtime<f16>` (v6.rs:270-303), contiguous, [C, A, 1, 1].
-#include "layer_device.h"
+#include "recurrence.h"
 
 namespace wrq {
 
@@ -18,8 +18,6 @@ namespace {
 
 constexpr int kPreThreads = 256;
 constexpr int kPreCache = 8; // 4-element vectors a thread keeps of a row: rows up to 8192 elements
-
-__device__ __forceinline__ float round_h(float v) { return h2f(f2h(v)); }
 
 // One workgroup per token.  row = x[t] (+ add[t]), written to x_out when given; ln = f16(LN(row)) -> ln_out;
 // shift_out[s][t] = f16(mix(ln, prev, factor[s])) with prev = the request's state row for its first
@@ -186,75 +184,6 @@ __global__ __launch_bounds__(256) void v6_decay_kernel(const uint16_t *lora, con
     out[(uint64_t)t * C + c] = act_one<WRQ_ACT_STABLE_EXP>(bias + acc);
 }
 
-// One wave per head of 64: lane i keeps the whole column S[.][i] of the request's state in registers;
-// k, r, w of a token go round the wave through LDS.  After the recurrence of a token: group norm over
-// the head (wave reduction), rounded to f16, times silu(g).
-__global__ __launch_bounds__(64) void v6_wkv_gate_kernel(const uint32_t *cursors, const float *decay, const float *time_first, float *state, ViewArgs vs,
-                                                         const float *k, const float *v, const float *r, const uint16_t *g, const uint16_t *gn_w,
-                                                         const uint16_t *gn_b, float eps, uint16_t *att_x, uint32_t H, uint32_t A) {
-    constexpr int S = 64;
-    __shared__ __align__(16) float ks[S], rs[S], ws[S], us[S];
-    const uint32_t head = blockIdx.x, i = threadIdx.x;
-    const uint32_t C = S * H, chan = head * S + i;
-    us[i] = time_first[chan];
-    const float gw = h2f(gn_w[chan]), gb = h2f(gn_b[chan]);
-    float s[S];
-    uint32_t held = 0xffffffffu;
-    // the operands of the next token are fetched while this one is worked on (clamped at the end)
-    float nk = k[chan], nr = r[chan], nw = decay[chan], nv = v[chan];
-    uint16_t ng = g[chan], nx = att_x[chan];
-    uint32_t ncur = cursors[0];
-    for (uint32_t t = 0; t < A; t++) {
-        const float ck = nk, cr = nr, cw = nw, vv = nv;
-        const uint16_t cg = ng, cx = nx;
-        Cursor cur = unpack_cursor(ncur);
-        cur.batch = min(cur.batch, vs.shape[2] - 1); // as read_cursor
-        cur.token = min(cur.token, t);
-        const uint64_t ti = (uint64_t)t * C + chan;
-        {
-            const uint64_t tn = (uint64_t)min(t + 1, A - 1) * C + chan;
-            nk = k[tn], nr = r[tn], nw = decay[tn], nv = v[tn], ng = g[tn], nx = att_x[tn];
-            ncur = cursors[min(t + 1, A - 1)];
-        }
-        __syncthreads(); // the previous token's reads of ks / rs / ws are done
-        ks[i] = ck, rs[i] = cr, ws[i] = cw;
-        if (cur.batch != held) {
-            if (held != 0xffffffffu) {
-#pragma unroll
-                for (int j = 0; j < S; j++) state[view_elem(vs, held, j + 1, chan)] = s[j];
-            }
-            held = cur.batch;
-#pragma unroll
-            for (int j = 0; j < S; j++) s[j] = state[view_elem(vs, held, j + 1, chan)];
-        }
-        // row 0 of the request's state keeps the layer's normalised input at its last token
-        if (t - cur.token + 1 == cur.len) state[view_elem(vs, cur.batch, 0, chan)] = h2f(cx);
-        __syncthreads();
-        float y4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int j4 = 0; j4 < S / 4; j4++) {
-            const float4 k4 = *reinterpret_cast<const float4 *>(&ks[4 * j4]), r4 = *reinterpret_cast<const float4 *>(&rs[4 * j4]),
-                         w4 = *reinterpret_cast<const float4 *>(&ws[4 * j4]), u4 = *reinterpret_cast<const float4 *>(&us[4 * j4]);
-            const float kk[4] = {k4.x, k4.y, k4.z, k4.w}, rr[4] = {r4.x, r4.y, r4.z, r4.w}, ww[4] = {w4.x, w4.y, w4.z, w4.w}, uu[4] = {u4.x, u4.y, u4.z, u4.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float kv = kk[e] * vv;
-                y4[e] += rr[e] * fmaf(uu[e], kv, s[4 * j4 + e]);
-                s[4 * j4 + e] = fmaf(ww[e], s[4 * j4 + e], kv);
-            }
-        }
-        const float y = (y4[0] + y4[1]) + (y4[2] + y4[3]);
-        const float mean = wave_sum(y) * (1.0f / S);
-        const float dev = rsqrtf(wave_sum((y - mean) * (y - mean)) * (1.0f / S) + eps);
-        const float gn = round_h(fmaf((y - mean) * dev, gw, gb));
-        att_x[ti] = f2h(act_one<WRQ_ACT_SILU>(h2f(cg)) * gn);
-    }
-    if (held != 0xffffffffu) {
-#pragma unroll
-        for (int j = 0; j < S; j++) state[view_elem(vs, held, j + 1, chan)] = s[j];
-    }
-}
-
 // state[request] <- ffn_x at its last token; x_out = f16(f16(sigmoid(r) v) + x_in) (halved when `rescale`)
 __global__ __launch_bounds__(256) void v6_post_ffn_kernel(const uint32_t *cursors, float *state, ViewArgs vs, const uint16_t *r, const uint16_t *v,
                                                           const uint16_t *ffn_x, const uint16_t *x_in, uint16_t *x_out, uint32_t C, int rescale) {
@@ -384,9 +313,9 @@ int wrq_v6_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const
     const ViewArgs vs = view_args(state->view);
     auto f32 = [](const void *p) { return static_cast<const float *>(p); };
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
-    hipLaunchKernelGGL(v6_wkv_gate_kernel, dim3(H), dim3(64), 0, static_cast<hipStream_t>(stream), static_cast<const uint32_t *>(cursors), f32(time_decay),
-                       f32(time_first), static_cast<float *>(state->data), vs, f32(k), f32(v), f32(r), u16(g), u16(gn_w), u16(gn_b), eps,
-                       static_cast<uint16_t *>(att_x), H, A);
+    hipLaunchKernelGGL((time_mix_kernel<float, 64, true, true>), dim3(H, slot_grid(vs)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint32_t *>(cursors), f32(time_decay), f32(time_first), static_cast<float *>(state->data), f32(k), f32(v), f32(r),
+                       static_cast<float *>(nullptr), vs, H, A, GateArgs{u16(g), u16(gn_w), u16(gn_b), static_cast<uint16_t *>(att_x), eps});
     return check_launch(what);
 }
 

@@ -1,0 +1,404 @@
+// The state recurrences of the v5 / v6 / v7 layers (recurrent_ops.hip, v7_ops.hip, fused_ops.hip).
+//
+// A run is a stack of A tokens from several requests; the state of a request is one 64 x 64 matrix S per head (or
+// SZ x SZ).  Requests do not depend on each other, so a workgroup takes one head of ONE state slot and walks that
+// slot's tokens only: 32 requests of one token each are 32 workgroups per head instead of a chain of 32 state
+// reloads in one.  S stays in registers over the slot's tokens: L = 8 lanes share two columns of S and hold SZ / 8
+// of their rows each (SZ = 16: four lanes, one column).  What bounds a long run is the vector ALU of the one CU a
+// head's state lives on: per element of S three fmas in v5 / v6 (k v, the decay, y) and five in v7; the bonus term
+// of v5 / v6, sum_j r[j] u[j] k[j] v[i], does not depend on S and is one number per token, formed while the operands
+// are staged.  Sharing two columns halves the LDS reads per token against one column per quad, which came out as
+// the second bound.
+#pragma once
+
+#include "layer_device.h"
+
+namespace wrq {
+
+constexpr uint32_t kSlotScan = 256; // cursors scanned at a time: one per thread
+
+// The tokens of `slot` among cursors[base .. base + 256): their offsets from `base` in stack order, and their number.
+// With a single slot every token is its own (a slot beyond the view counts as the last one) and `list` stays unused.
+__device__ __forceinline__ uint32_t slot_tokens(const uint32_t *cursors, uint32_t base, uint32_t A, uint32_t slot, uint32_t slots, uint8_t *list, uint32_t *count) {
+    if (slots == 1) return min(kSlotScan, A - base);
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const bool mine = base + tid < A && min(cursors[min(base + tid, A - 1)] & 0xffu, slots - 1) == slot;
+    const uint64_t mask = __ballot(mine);
+    if (lane == 0) count[wave] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kSlotScan / 64; w++) {
+        before += w < wave ? count[w] : 0u;
+        total += count[w];
+    }
+    if (mine) list[before + (uint32_t)__popcll(mask & ((1ull << lane) - 1))] = (uint8_t)tid;
+    __syncthreads();
+    return total;
+}
+
+// Sum over groups of LANES adjacent lanes (a power of two), the same value in each of them.
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float v) {
+    if constexpr (LANES >= 2) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
+    if constexpr (LANES >= 4) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
+    if constexpr (LANES >= 8) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, true)); // row_half_mirror
+    if constexpr (LANES >= 16) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, true)); // row_mirror
+    if constexpr (LANES >= 32) v += __shfl_xor(v, 16, 64);
+    if constexpr (LANES >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
+__device__ __forceinline__ float round_h(float v) { return h2f(f2h(v)); }
+
+template <int SZ>
+struct RecurrenceTile {
+    static constexpr int L = SZ >= 32 ? 8 : 4;  // lanes that share CPT columns of S
+    static constexpr int CPT = L / 4;           // columns of a lane
+    static constexpr int JL = SZ / L;           // rows of S a lane holds
+    static constexpr int TB = 1024 / SZ;        // tokens per chunk: a 4-element vector of each operand per thread
+    static constexpr int TL = SZ / 4;           // threads per token of a chunk
+};
+
+template <int N>
+__device__ __forceinline__ void load_cols(float (&d)[N], const float *p) {
+    if constexpr (N == 2) {
+        const float2 v = *reinterpret_cast<const float2 *>(p);
+        d[0] = v.x, d[1] = v.y;
+    } else {
+        d[0] = *p;
+    }
+}
+template <int N>
+__device__ __forceinline__ void store_cols(float *p, const float (&d)[N]) {
+    if constexpr (N == 2) *reinterpret_cast<float2 *>(p) = make_float2(d[0], d[1]);
+    else *p = d[0];
+}
+
+// What follows the recurrence in the fused forms of a layer (head size 64): the group norm over the head and the gate.
+// att_x holds the layer's normalised input before and the gated output after.
+struct GateArgs {
+    const uint16_t *g, *gn_w, *gn_b;
+    uint16_t *att_x;
+    float eps;
+};
+
+// y4[e] (f32) of 4 elements per thread, 16 threads per token -> group norm over the 64 elements of the head, in f32
+__device__ __forceinline__ float4 head_norm(float4 y, uint2 wq, uint2 bq, float eps) {
+    const float mean = lanes_sum<16>((y.x + y.y) + (y.z + y.w)) * (1.0f / 64);
+    const float4 d = make_float4(y.x - mean, y.y - mean, y.z - mean, y.w - mean);
+    const float dev = rsqrtf(lanes_sum<16>((d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w)) * (1.0f / 64) + eps);
+    auto w = [](uint2 v, int i) { return h2f((uint16_t)((i < 2 ? v.x : v.y) >> (16 * (i & 1)))); };
+    return make_float4(fmaf(d.x * dev, w(wq, 0), w(bq, 0)), fmaf(d.y * dev, w(wq, 1), w(bq, 1)), fmaf(d.z * dev, w(wq, 2), w(bq, 2)),
+                       fmaf(d.w * dev, w(wq, 3), w(bq, 3)));
+}
+
+// v5 (a decay per channel) and v6 (TOKEN_DECAY: a decay per token):
+//   y[i] = sum_j r[j] (u[j] k[j] v[i] + S[j][i]),  S[j][i] <- w[j] S[j][i] + k[j] v[i]
+// GATE: the fused form, y then goes through the group norm (rounded to f16) and silu(g) into att_x; otherwise into x.
+// grid (heads, slots).  The operands come in chunks of TB tokens of the slot: every thread fetches one 4-element
+// vector of each while the previous chunk is worked on and passes it round through LDS (two buffers).
+template <typename XT, int SZ, bool TOKEN_DECAY, bool GATE>
+__global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
+                                                       const XT *v, const XT *r, XT *x, ViewArgs vs, uint32_t H, uint32_t A, GateArgs ga) {
+    using G = RecurrenceTile<SZ>;
+    constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL;
+    static_assert(!GATE || (SZ == 64 && sizeof(XT) == 4), "the fused form: head size 64, f32 operands");
+    __shared__ __align__(16) float ks[2][1024], rs[2][1024], ws[TOKEN_DECAY ? 2 : 1][TOKEN_DECAY ? 1024 : 4], vsh[2][1024], ysh[GATE ? 1024 : 4];
+    __shared__ float bonus[2][TB];
+    __shared__ uint32_t csh[2][TB], tsh[2][TB]; // cursors and numbers of the chunk's tokens
+    __shared__ uint8_t list[kSlotScan];
+    __shared__ uint32_t count[kSlotScan / 64];
+    const uint32_t head = blockIdx.x, slot = blockIdx.y, slots = vs.shape[2], tid = threadIdx.x;
+    const uint32_t l = tid % L;
+    const uint32_t C = SZ * H;
+    // this thread's vector of a chunk: token tid / TL of the chunk, elements 4 (tid % TL) ..
+    const uint32_t lt = tid / TL, le = 4 * (tid % TL);
+    const float4 u4 = *reinterpret_cast<const float4 *>(time_first + head * SZ + le);
+    uint2 gw = make_uint2(0, 0), gb = make_uint2(0, 0);
+    if constexpr (GATE) gw = *reinterpret_cast<const uint2 *>(ga.gn_w + head * SZ + le), gb = *reinterpret_cast<const uint2 *>(ga.gn_b + head * SZ + le);
+    float4 fk, fr, fw, fv;
+    uint2 fg = make_uint2(0, 0), fx = make_uint2(0, 0);
+    uint32_t fc = 0, ft = 0, fct = 0;
+    uint32_t base = 0, n = 0;
+    auto fetch = [&](uint32_t chunk) {
+        auto token = [&](uint32_t j) { return base + (slots == 1 ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
+        ft = token(chunk * TB + lt);
+        const uint64_t g = (uint64_t)ft * C + head * SZ + le;
+        fk = load_vec4(k + g), fr = load_vec4(r + g), fv = load_vec4(v + g);
+        if constexpr (TOKEN_DECAY) fw = load_vec4(time_decay + g);
+        if constexpr (GATE) fg = *reinterpret_cast<const uint2 *>(ga.g + g), fx = *reinterpret_cast<const uint2 *>(ga.att_x + g);
+        if (GATE) fc = cursors[ft];
+        else if (tid < (uint32_t)TB) fct = token(chunk * TB + tid), fc = cursors[fct];
+    };
+    auto stage = [&](int buf) {
+        *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
+        *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
+        if constexpr (TOKEN_DECAY) *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = fw;
+        *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
+        const float b = lanes_sum<TL>(fmaf(fr.x, u4.x * fk.x, fr.y * (u4.y * fk.y)) + fmaf(fr.z, u4.z * fk.z, fr.w * (u4.w * fk.w)));
+        if (tid % TL == 0) bonus[buf][lt] = b;
+        if (!GATE && tid < (uint32_t)TB) csh[buf][tid] = fc, tsh[buf][tid] = fct;
+    };
+    for (uint32_t i0 = 0; i0 < SZ; i0 += 64) {
+        const uint32_t i = i0 + CPT * (tid / L);
+        const bool live = i < SZ; // head sizes below 64 leave waves without a column
+        const uint32_t chan = head * SZ + min(i, (uint32_t)(SZ - CPT));
+        float s[JL][CPT], wc[TOKEN_DECAY ? 1 : JL]; // wc: the constant decay of this lane's rows
+        if constexpr (!TOKEN_DECAY) {
+#pragma unroll
+            for (int jj = 0; jj < JL; jj++) wc[jj] = time_decay[head * SZ + l * JL + jj];
+        }
+        bool held = false;
+        for (base = 0; base < A; base += kSlotScan) {
+            n = slot_tokens(cursors, base, A, slot, slots, list, count);
+            if (n == 0) continue;
+            fetch(0);
+            if (!held) {
+#pragma unroll
+                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], state + view_elem(vs, slot, l * JL + jj + 1, chan));
+                held = true;
+            }
+            const uint32_t nchunk = (n + TB - 1) / TB;
+            __syncthreads(); // the buffers may still be read
+            stage(0);
+            for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
+                const int buf = chunk & 1;
+                const uint2 cg = fg, cx = fx;
+                const uint32_t cc = fc, ct = ft;
+                if (chunk + 1 < nchunk) fetch(chunk + 1);
+                __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
+                const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
+                if (live) {
+                    for (uint32_t tt = 0; tt < tend; tt++) {
+                        float vv[CPT], y[CPT];
+                        load_cols(vv, &vsh[buf][tt * SZ + i]);
+                        const float *kp = &ks[buf][tt * SZ + l * JL], *rp = &rs[buf][tt * SZ + l * JL], *wp = &ws[TOKEN_DECAY ? buf : 0][TOKEN_DECAY ? tt * SZ + l * JL : 0];
+                        float y2[CPT][2];
+#pragma unroll
+                        for (int c = 0; c < CPT; c++) y2[c][0] = y2[c][1] = 0.0f;
+#pragma unroll
+                        for (int q = 0; q < JL / 4; q++) {
+                            const float4 k4 = *reinterpret_cast<const float4 *>(kp + 4 * q), r4 = *reinterpret_cast<const float4 *>(rp + 4 * q);
+                            const float kk[4] = {k4.x, k4.y, k4.z, k4.w}, rr[4] = {r4.x, r4.y, r4.z, r4.w};
+                            float ww[4];
+                            if constexpr (TOKEN_DECAY) {
+                                const float4 w4 = *reinterpret_cast<const float4 *>(wp + 4 * q);
+                                ww[0] = w4.x, ww[1] = w4.y, ww[2] = w4.z, ww[3] = w4.w;
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < 4; e++) ww[e] = wc[4 * q + e];
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; e++)
+#pragma unroll
+                                for (int c = 0; c < CPT; c++) {
+                                    float &sv = s[4 * q + e][c];
+                                    y2[c][e & 1] = fmaf(rr[e], sv, y2[c][e & 1]);
+                                    sv = fmaf(ww[e], sv, kk[e] * vv[c]);
+                                }
+                        }
+#pragma unroll
+                        for (int c = 0; c < CPT; c++) y[c] = lanes_sum<L>(y2[c][0] + y2[c][1]);
+                        if (l == 0) {
+                            if constexpr (GATE) {
+                                store_cols(&ysh[tt * SZ + i], y);
+                            } else {
+                                const uint32_t t = tsh[buf][tt];
+                                Cursor cur = unpack_cursor(csh[buf][tt]);
+                                cur.token = min(cur.token, t); // as read_cursor
+                                const uint64_t ti = (uint64_t)t * C + chan;
+#pragma unroll
+                                for (int c = 0; c < CPT; c++) {
+                                    // row 0 of the request's state keeps the layer's input at its last token (read before x is overwritten)
+                                    if (t - cur.token + 1 == cur.len) state[view_elem(vs, slot, 0, chan + c)] = load_one(x + ti + c);
+                                    const float o = fmaf(bonus[buf][tt], vv[c], y[c]);
+                                    if constexpr (sizeof(XT) == 2) x[ti + c] = f2h(o);
+                                    else x[ti + c] = o;
+                                }
+                            }
+                        }
+                    }
+                }
+                if constexpr (GATE) {
+                    __syncthreads(); // the chunk's y are in LDS
+                    if (lt < tend) {
+                        Cursor cur = unpack_cursor(cc);
+                        cur.token = min(cur.token, ct); // as read_cursor
+                        if (ct - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
+                        const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
+                        const float b = bonus[buf][lt];
+                        const float4 o = head_norm(make_float4(fmaf(b, v4.x, y0.x), fmaf(b, v4.y, y0.y), fmaf(b, v4.z, y0.z), fmaf(b, v4.w, y0.w)), gw, gb, ga.eps);
+                        const float4 g4 = load_vec4(reinterpret_cast<const uint16_t *>(&cg));
+                        auto gate = [](float gv, float ov) { return act_one<WRQ_ACT_SILU>(gv) * round_h(ov); };
+                        store_vec4(ga.att_x + ((uint64_t)ct * C + head * SZ + le), make_float4(gate(g4.x, o.x), gate(g4.y, o.y), gate(g4.z, o.z), gate(g4.w, o.w)));
+                    }
+                }
+                if (chunk + 1 < nchunk) stage(buf ^ 1); // read two chunks ago, before the barrier above
+            }
+        }
+        if (live && held) {
+#pragma unroll
+            for (int jj = 0; jj < JL; jj++) store_cols(state + view_elem(vs, slot, l * JL + jj + 1, chan), s[jj]);
+        }
+    }
+}
+
+// v7, with a = -kk, b = kk * a_in and w = exp(-exp(-0.5) sigmoid(w_in)):
+//   sa[i] = sum_j S[j][i] a[j];   S[j][i] <- S[j][i] w[j] + k[j] v[i] + sa[i] b[j];   y[i] = sum_j r[j] S[j][i]
+// GATE: the fused form; y (rounded to f16) then goes through the group norm, the bonus (sum_j u[j] k[j] r[j]) v[i]
+// (u = `first`) and the gate g into att_x, rounded to f16 after each as the op list stores it.
+template <typename XT, int SZ, bool GATE>
+__global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursors, float *state, const XT *r, const XT *w, const XT *n_, XT *x, ViewArgs vs,
+                                                          uint32_t H, uint32_t A, const uint16_t *first, GateArgs ga) {
+    using G = RecurrenceTile<SZ>;
+    constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL;
+    static_assert(!GATE || (SZ == 64 && sizeof(XT) == 2), "the fused form: head size 64, f16 operands");
+    __shared__ __align__(16) float rs[2][1024], ws[2][1024], ks[2][1024], as[2][1024], bs[2][1024], vsh[2][1024], ysh[GATE ? 1024 : 4];
+    __shared__ uint32_t csh[2][TB], tsh[2][TB]; // cursors and numbers of the chunk's tokens
+    __shared__ uint8_t list[kSlotScan];
+    __shared__ uint32_t count[kSlotScan / 64];
+    const uint32_t head = blockIdx.x, slot = blockIdx.y, slots = vs.shape[2], tid = threadIdx.x;
+    const uint32_t l = tid % L;
+    const uint32_t C = SZ * H;
+    const uint64_t plane = (uint64_t)A * C; // n_ holds k, v, a, kk one after the other
+    const uint32_t lt = tid / TL, le = 4 * (tid % TL);
+    uint2 gw = make_uint2(0, 0), gb = make_uint2(0, 0);
+    float4 u4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (GATE) {
+        gw = *reinterpret_cast<const uint2 *>(ga.gn_w + head * SZ + le), gb = *reinterpret_cast<const uint2 *>(ga.gn_b + head * SZ + le);
+        u4 = load_vec4(first + head * SZ + le);
+    }
+    float4 fr, fw, fk, fv, fa, fkk;
+    uint2 fg = make_uint2(0, 0), fx = make_uint2(0, 0);
+    uint32_t fc = 0, ft = 0, fct = 0;
+    uint32_t base = 0, n = 0;
+    auto fetch = [&](uint32_t chunk) {
+        auto token = [&](uint32_t j) { return base + (slots == 1 ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
+        ft = token(chunk * TB + lt);
+        const uint64_t g = (uint64_t)ft * C + head * SZ + le;
+        fr = load_vec4(r + g), fw = load_vec4(w + g), fk = load_vec4(n_ + g), fv = load_vec4(n_ + plane + g);
+        fa = load_vec4(n_ + 2 * plane + g), fkk = load_vec4(n_ + 3 * plane + g);
+        if constexpr (GATE) fg = *reinterpret_cast<const uint2 *>(ga.g + g), fx = *reinterpret_cast<const uint2 *>(ga.att_x + g);
+        if (GATE) fc = cursors[ft];
+        else if (tid < (uint32_t)TB) fct = token(chunk * TB + tid), fc = cursors[fct];
+    };
+    auto decay = [](float v) { return expf(-0.606531f / (1.0f + expf(-v))); }; // exp(-exp(-0.5) sigmoid(w))
+    auto stage = [&](int buf) {
+        *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
+        *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = make_float4(decay(fw.x), decay(fw.y), decay(fw.z), decay(fw.w));
+        *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
+        *reinterpret_cast<float4 *>(&as[buf][4 * tid]) = make_float4(-fkk.x, -fkk.y, -fkk.z, -fkk.w);
+        *reinterpret_cast<float4 *>(&bs[buf][4 * tid]) = make_float4(fkk.x * fa.x, fkk.y * fa.y, fkk.z * fa.z, fkk.w * fa.w);
+        *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
+        if (!GATE && tid < (uint32_t)TB) csh[buf][tid] = fc, tsh[buf][tid] = fct;
+    };
+    for (uint32_t i0 = 0; i0 < SZ; i0 += 64) {
+        const uint32_t i = i0 + CPT * (tid / L);
+        const bool live = i < SZ; // head sizes below 64 leave waves without a column
+        const uint32_t chan = head * SZ + min(i, (uint32_t)(SZ - CPT));
+        float s[JL][CPT];
+        bool held = false;
+        for (base = 0; base < A; base += kSlotScan) {
+            n = slot_tokens(cursors, base, A, slot, slots, list, count);
+            if (n == 0) continue;
+            fetch(0);
+            if (!held) {
+#pragma unroll
+                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], state + view_elem(vs, slot, l * JL + jj + 1, chan));
+                held = true;
+            }
+            const uint32_t nchunk = (n + TB - 1) / TB;
+            __syncthreads(); // the buffers may still be read
+            stage(0);
+            for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
+                const int buf = chunk & 1;
+                const uint2 cg = fg, cx = fx;
+                const uint32_t cc = fc, ct = ft;
+                if (chunk + 1 < nchunk) fetch(chunk + 1);
+                __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
+                const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
+                if (live) {
+                    for (uint32_t tt = 0; tt < tend; tt++) {
+                        float vv[CPT], sa[CPT], y[CPT], acc[CPT][2];
+                        load_cols(vv, &vsh[buf][tt * SZ + i]);
+                        const uint32_t at = tt * SZ + l * JL;
+#pragma unroll
+                        for (int c = 0; c < CPT; c++) acc[c][0] = acc[c][1] = 0.0f;
+#pragma unroll
+                        for (int q = 0; q < JL / 4; q++) {
+                            const float4 a4 = *reinterpret_cast<const float4 *>(&as[buf][at + 4 * q]);
+                            const float aa[4] = {a4.x, a4.y, a4.z, a4.w};
+#pragma unroll
+                            for (int e = 0; e < 4; e++)
+#pragma unroll
+                                for (int c = 0; c < CPT; c++) acc[c][e & 1] = fmaf(s[4 * q + e][c], aa[e], acc[c][e & 1]);
+                        }
+#pragma unroll
+                        for (int c = 0; c < CPT; c++) sa[c] = lanes_sum<L>(acc[c][0] + acc[c][1]), acc[c][0] = acc[c][1] = 0.0f;
+#pragma unroll
+                        for (int q = 0; q < JL / 4; q++) {
+                            const float4 w4 = *reinterpret_cast<const float4 *>(&ws[buf][at + 4 * q]), k4 = *reinterpret_cast<const float4 *>(&ks[buf][at + 4 * q]),
+                                         b4 = *reinterpret_cast<const float4 *>(&bs[buf][at + 4 * q]), r4 = *reinterpret_cast<const float4 *>(&rs[buf][at + 4 * q]);
+                            const float ww[4] = {w4.x, w4.y, w4.z, w4.w}, kk[4] = {k4.x, k4.y, k4.z, k4.w}, bb[4] = {b4.x, b4.y, b4.z, b4.w},
+                                        rr[4] = {r4.x, r4.y, r4.z, r4.w};
+#pragma unroll
+                            for (int e = 0; e < 4; e++)
+#pragma unroll
+                                for (int c = 0; c < CPT; c++) {
+                                    float &sv = s[4 * q + e][c];
+                                    sv = fmaf(sa[c], bb[e], fmaf(sv, ww[e], kk[e] * vv[c]));
+                                    acc[c][e & 1] = fmaf(rr[e], sv, acc[c][e & 1]);
+                                }
+                        }
+#pragma unroll
+                        for (int c = 0; c < CPT; c++) y[c] = lanes_sum<L>(acc[c][0] + acc[c][1]);
+                        if (l == 0) {
+                            if constexpr (GATE) {
+                                store_cols(&ysh[tt * SZ + i], y);
+                            } else {
+                                const uint32_t t = tsh[buf][tt];
+                                Cursor cur = unpack_cursor(csh[buf][tt]);
+                                cur.token = min(cur.token, t); // as read_cursor
+                                const uint64_t ti = (uint64_t)t * C + chan;
+#pragma unroll
+                                for (int c = 0; c < CPT; c++) {
+                                    // row 0 of the request's state keeps the layer's input at its last token (read before x is overwritten)
+                                    if (t - cur.token + 1 == cur.len) state[view_elem(vs, slot, 0, chan + c)] = load_one(x + ti + c);
+                                    if constexpr (sizeof(XT) == 2) x[ti + c] = f2h(y[c]);
+                                    else x[ti + c] = y[c];
+                                }
+                            }
+                        }
+                    }
+                }
+                if constexpr (GATE) {
+                    __syncthreads(); // the chunk's y are in LDS
+                    if (lt < tend) {
+                        Cursor cur = unpack_cursor(cc);
+                        cur.token = min(cur.token, ct); // as read_cursor
+                        if (ct - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
+                        const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
+                        const float4 k4 = *reinterpret_cast<const float4 *>(&ks[buf][4 * tid]), r4 = *reinterpret_cast<const float4 *>(&rs[buf][4 * tid]);
+                        const float b = lanes_sum<16>((u4.x * k4.x * r4.x + u4.y * k4.y * r4.y) + (u4.z * k4.z * r4.z + u4.w * k4.w * r4.w));
+                        const float4 o = head_norm(make_float4(round_h(y0.x), round_h(y0.y), round_h(y0.z), round_h(y0.w)), gw, gb, ga.eps);
+                        const float4 g4 = load_vec4(reinterpret_cast<const uint16_t *>(&cg));
+                        auto gate = [&](float gv, float ov, float vv) { return gv * round_h(round_h(ov) + b * vv); };
+                        store_vec4(ga.att_x + ((uint64_t)ct * C + head * SZ + le),
+                                   make_float4(gate(g4.x, o.x, v4.x), gate(g4.y, o.y, v4.y), gate(g4.z, o.z, v4.z), gate(g4.w, o.w, v4.w)));
+                    }
+                }
+                if (chunk + 1 < nchunk) stage(buf ^ 1); // read two chunks ago, before the barrier above
+            }
+        }
+        if (live && held) {
+#pragma unroll
+            for (int jj = 0; jj < JL; jj++) store_cols(state + view_elem(vs, slot, l * JL + jj + 1, chan), s[jj]);
+        }
+    }
+}
+
+// State slots a cursor can name: 8 bits, the last slot of the view for what lies beyond it.
+inline uint32_t slot_grid(const ViewArgs &vs) { return vs.shape[2] < 256u ? vs.shape[2] : 256u; }
+
+} // namespace wrq

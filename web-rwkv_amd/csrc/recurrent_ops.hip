@@ -11,12 +11,9 @@
 //
 // time_mix_v6 is the recurrence  y[i] = sum_j r[j] (u[j] k[j] v[i] + S[j][i]),  S[j][i] <- w[j] S[j][i] + k[j] v[i]
 // per head, token after token; time_mix_v5 is the same recurrence with a decay w that is a constant of
-// the channel instead of a value per token (one kernel, TOKEN_DECAY tells them apart).  The shader re-reads and re-writes the head's S (64 x 64 f32) in memory
-// for every token; here a request's S stays in registers for all its tokens of the run: four lanes
-// share an output element i and hold a quarter of j each (16 values of S), one DPP quad reduction
-// per token; S is read when a request's tokens begin and written when they end.  The sum over j is
-// therefore taken in interleaved partial sums instead of one chain (a difference of rounding order only).
-#include "layer_device.h"
+// the channel instead of a value per token.  The shader re-reads and re-writes the head's S (64 x 64 f32)
+// in memory for every token; recurrence.h keeps it in registers over all tokens of a request in the run.
+#include "recurrence.h"
 
 namespace wrq {
 
@@ -50,124 +47,6 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const uint32_t *cursor
     if (stack - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = xx;
     auto g = [](float a, float b) { return 1.0f / (1.0f + expf(-a)) * b; };
     store_vec4(x + bti, make_float4(g(rr.x, vv.x), g(rr.y, vv.y), g(rr.z, vv.z), g(rr.w, vv.w)));
-}
-
-__device__ __forceinline__ float quad_sum(float v) {
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true)); // quad_perm [1,0,3,2]
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true)); // quad_perm [2,3,0,1]
-    return v;
-}
-
-// One workgroup per head: thread = (output element i of the head, quarter q of the j range), four
-// waves of 16 i x 4 q; JQ = S / 4 values of S[.][i] per lane.  The operands of the head (k, r, w, v:
-// S values each per token) come in chunks of 1024 / S tokens: every thread fetches one 4-element
-// vector of each while the previous chunk is worked on, and the chunk is passed round through LDS
-// (two buffers), from where the lanes of a quarter read their j range as broadcasts.
-template <typename XT, int JQ, bool TOKEN_DECAY>
-__global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
-                                                          const XT *v, const XT *r, XT *x, ViewArgs vs, uint32_t S, uint32_t H, uint32_t A) {
-    constexpr int SZ = 4 * JQ;      // head size
-    constexpr int TB = 1024 / SZ;   // tokens per chunk
-    __shared__ __align__(16) float ks[2][1024], rs[2][1024], ws[2][1024], vsh[2][1024];
-    __shared__ uint32_t csh[2][TB]; // the chunk's cursors
-    const uint32_t head = blockIdx.x, tid = threadIdx.x;
-    const uint32_t q = tid & 3;
-    const uint32_t C = S * H;
-    const uint32_t nchunk = (A + TB - 1) / TB;
-    // this thread's vector of a chunk: token tid / (SZ / 4) of the chunk, elements 4 (tid % (SZ / 4)) ..
-    const uint32_t lt = tid / (SZ / 4), le = 4 * (tid % (SZ / 4));
-    float4 fk, fr, fw, fv;
-    uint32_t fc = 0;
-    auto fetch = [&](uint32_t chunk) {
-        const uint32_t t = min(chunk * TB + lt, A - 1); // clamped: tokens past the run are never used
-        const uint64_t g = (uint64_t)t * C + head * SZ + le;
-        fk = load_vec4(k + g), fr = load_vec4(r + g), fv = load_vec4(v + g);
-        if constexpr (TOKEN_DECAY) fw = load_vec4(time_decay + g);
-        if (tid < (uint32_t)TB) fc = cursors[min(chunk * TB + tid, A - 1)];
-    };
-    auto stage = [&](int buf) {
-        *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
-        *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
-        if constexpr (TOKEN_DECAY) *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = fw;
-        *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
-        if (tid < (uint32_t)TB) csh[buf][tid] = fc;
-    };
-    for (uint32_t i0 = 0; i0 < SZ; i0 += 64) {
-        const uint32_t i = i0 + (tid >> 2);
-        const bool live = i < SZ; // head sizes below 64 leave waves without an output element
-        const uint32_t chan = head * SZ + min(i, (uint32_t)SZ - 1);
-        float u[JQ], s[JQ], wc[TOKEN_DECAY ? 1 : JQ]; // wc: the constant decay of this lane's j range
-#pragma unroll
-        for (int c = 0; c < JQ / 4; c++) {
-            const float4 t4 = *reinterpret_cast<const float4 *>(time_first + head * SZ + q * JQ + 4 * c);
-            u[4 * c] = t4.x, u[4 * c + 1] = t4.y, u[4 * c + 2] = t4.z, u[4 * c + 3] = t4.w;
-            if constexpr (!TOKEN_DECAY) {
-                const float4 d4 = *reinterpret_cast<const float4 *>(time_decay + head * SZ + q * JQ + 4 * c);
-                wc[4 * c] = d4.x, wc[4 * c + 1] = d4.y, wc[4 * c + 2] = d4.z, wc[4 * c + 3] = d4.w;
-            }
-        }
-        uint32_t held = 0xffffffffu; // request whose S is in registers
-        fetch(0);
-        __syncthreads(); // the buffers may still be read by the previous pass over i
-        stage(0);
-        for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
-            const int buf = chunk & 1;
-            if (chunk + 1 < nchunk) fetch(chunk + 1);
-            __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
-            const uint32_t tend = min((uint32_t)TB, A - chunk * TB);
-            if (live) {
-                for (uint32_t tt = 0; tt < tend; tt++) {
-                    const uint32_t t = chunk * TB + tt;
-                    Cursor cur = unpack_cursor(csh[buf][tt]);
-                    cur.batch = min(cur.batch, vs.shape[2] - 1); // as read_cursor
-                    cur.token = min(cur.token, t);
-                    if (cur.batch != held) {
-                        if (held != 0xffffffffu) {
-#pragma unroll
-                            for (int jj = 0; jj < JQ; jj++) state[view_elem(vs, held, q * JQ + jj + 1, chan)] = s[jj];
-                        }
-                        held = cur.batch;
-#pragma unroll
-                        for (int jj = 0; jj < JQ; jj++) s[jj] = state[view_elem(vs, held, q * JQ + jj + 1, chan)];
-                    }
-                    const uint64_t ti = (uint64_t)t * C + chan;
-                    // row 0 of the request's state keeps the layer's input at its last token (read before x is overwritten)
-                    if (q == 0 && t - cur.token + 1 == cur.len) state[view_elem(vs, cur.batch, 0, chan)] = load_one(x + ti);
-                    const float vv = vsh[buf][tt * SZ + i];
-                    const float *kp = &ks[buf][tt * SZ + q * JQ], *rp = &rs[buf][tt * SZ + q * JQ], *wp = &ws[buf][tt * SZ + q * JQ];
-                    float y4[4] = {0.0f, 0.0f, 0.0f, 0.0f}; // four chains instead of one of JQ dependent adds
-#pragma unroll
-                    for (int c = 0; c < JQ / 4; c++) {
-                        const float4 k4 = *reinterpret_cast<const float4 *>(kp + 4 * c), r4 = *reinterpret_cast<const float4 *>(rp + 4 * c);
-                        const float kk[4] = {k4.x, k4.y, k4.z, k4.w}, rr[4] = {r4.x, r4.y, r4.z, r4.w};
-                        float ww[4];
-                        if constexpr (TOKEN_DECAY) {
-                            const float4 w4 = *reinterpret_cast<const float4 *>(wp + 4 * c);
-                            ww[0] = w4.x, ww[1] = w4.y, ww[2] = w4.z, ww[3] = w4.w;
-                        } else {
-                            ww[0] = wc[4 * c], ww[1] = wc[4 * c + 1], ww[2] = wc[4 * c + 2], ww[3] = wc[4 * c + 3];
-                        }
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const float kv = kk[e] * vv;
-                            y4[e] += rr[e] * fmaf(u[4 * c + e], kv, s[4 * c + e]);
-                            s[4 * c + e] = fmaf(ww[e], s[4 * c + e], kv);
-                        }
-                    }
-                    const float y = quad_sum((y4[0] + y4[1]) + (y4[2] + y4[3]));
-                    if (q == 0) {
-                        if constexpr (sizeof(XT) == 2) x[ti] = f2h(y);
-                        else x[ti] = y;
-                    }
-                }
-            }
-            if (chunk + 1 < nchunk) stage(buf ^ 1); // read two chunks ago, before the barrier above
-        }
-        if (live && held != 0xffffffffu) {
-#pragma unroll
-            for (int jj = 0; jj < JQ; jj++) state[view_elem(vs, held, q * JQ + jj + 1, chan)] = s[jj];
-        }
-    }
 }
 
 // The v4 recurrence, per channel: a numerator aa, a denominator bb and their common exponent pp,
@@ -326,21 +205,22 @@ int time_mix(const char *name, bool token_decay, wrq_stream stream, const wrq_te
     const uint32_t *cur = static_cast<const uint32_t *>(cursors->data);
     const float *td = static_cast<const float *>(time_decay->data), *tfp = static_cast<const float *>(time_first->data);
     float *sp = static_cast<float *>(state->data);
-#define WRQ_TM_LAUNCH(XT, JQ, TD)                                                                                                                \
-    hipLaunchKernelGGL((time_mix_kernel<XT, JQ, TD>), dim3(H), dim3(256), 0, hs, cur, td, tfp, sp, static_cast<const XT *>(k->data),               \
-                       static_cast<const XT *>(v->data), static_cast<const XT *>(r->data), static_cast<XT *>(x->data), vs, S, H, A)
-#define WRQ_TM(JQ)                                                                                                                               \
-    if (S == 4 * JQ) {                                                                                                                           \
+    const dim3 grid(H, slot_grid(vs));
+#define WRQ_TM_LAUNCH(XT, SZ, TD)                                                                                                                \
+    hipLaunchKernelGGL((time_mix_kernel<XT, SZ, TD, false>), grid, dim3(256), 0, hs, cur, td, tfp, sp, static_cast<const XT *>(k->data),           \
+                       static_cast<const XT *>(v->data), static_cast<const XT *>(r->data), static_cast<XT *>(x->data), vs, H, A, GateArgs{})
+#define WRQ_TM(SZ)                                                                                                                               \
+    if (S == SZ) {                                                                                                                               \
         if (dtype == WRQ_F16) {                                                                                                                  \
-            if (token_decay) WRQ_TM_LAUNCH(uint16_t, JQ, true);                                                                                  \
-            else WRQ_TM_LAUNCH(uint16_t, JQ, false);                                                                                             \
+            if (token_decay) WRQ_TM_LAUNCH(uint16_t, SZ, true);                                                                                  \
+            else WRQ_TM_LAUNCH(uint16_t, SZ, false);                                                                                             \
         } else {                                                                                                                                 \
-            if (token_decay) WRQ_TM_LAUNCH(float, JQ, true);                                                                                     \
-            else WRQ_TM_LAUNCH(float, JQ, false);                                                                                                \
+            if (token_decay) WRQ_TM_LAUNCH(float, SZ, true);                                                                                     \
+            else WRQ_TM_LAUNCH(float, SZ, false);                                                                                                \
         }                                                                                                                                        \
         return check_launch(name);                                                                                                               \
     }
-    WRQ_TM(4) WRQ_TM(8) WRQ_TM(16) WRQ_TM(32) WRQ_TM(64)
+    WRQ_TM(16) WRQ_TM(32) WRQ_TM(64) WRQ_TM(128) WRQ_TM(256)
 #undef WRQ_TM
 #undef WRQ_TM_LAUNCH
     return fail(WRQ_ERR_UNSUPPORTED, "%s: head size %u (16, 32, 64, 128 or 256 is built)", name, S);
