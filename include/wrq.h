@@ -440,6 +440,31 @@ int wrq_v6_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const
 int wrq_v6_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const wrq_tensor_view *state,
                     const void *r, const void *v, const void *ffn_x, const void *x_in, void *x_out, int rescale);
 
+/*
+ * wrq_fused_pre: wrq_v6_pre with 1, 2 or 6 token shifts; factors and outs are host arrays of `shifts` device pointers.
+ * wrq_adapters_in: the first halves of up to 4 low-rank adapters, out[i] f16 [ranks[i], A] <- act(w[i] x[i]), w[i] f16
+ *   [C, ranks[i]], x[i] f16 [C, A]; ranks in multiples of 16, C of 32.
+ * Fused forms of the small ops of an RWKV-v7 layer (src/runtime/v7.rs:704-1006), under the same rules:
+ * wrq_v7_mid: the second halves of the adapters w, a, g, v (ranks 64, 64, 128, 32; aux, w2: 4 device pointers each) + add /
+ *   sigmoid + lerp with the first layer's values + mul(k_k) + l2_norm + control_k_v7 + the blits into n [C, A, 4];
+ *   vectors: w0, a0, v0, k_k, k_a; `first`: the layer whose values att_v0 keeps (no adapter v).  k and v are not written.
+ * wrq_v7_wkv_gate: time_mix_v7 + group_norm + time_first_v7 + mul(g); att_x f16 in (the normalised layer input) and out.
+ * wrq_v7_post_ffn: channel_mix_v7 + add (+ affine(0.5) when `rescale`); x_in, ffn_x and v are not written.
+ */
+int wrq_fused_pre(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const void *x, const void *add,
+                  void *x_out, const void *ln_w, const void *ln_b, float eps, const wrq_tensor_view *state, int shifts,
+                  const void *const *factors, void *ln_out, void *const *outs);
+int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void *const *w, const uint32_t *ranks,
+                    const int *acts, const void *const *x, void *const *out);
+int wrq_v7_mid(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first, const uint32_t *ranks,
+               const void *const *aux, const void *const *w2, const void *const *vectors, float eps, const void *k,
+               const void *v, void *att_v0, void *att_w, void *att_g, void *n);
+int wrq_v7_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const void *cursors,
+                    const wrq_tensor_view *state, const void *r, const void *w, const void *n, const void *r_k,
+                    const void *g, const void *gn_w, const void *gn_b, float eps, void *att_x);
+int wrq_v7_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const wrq_tensor_view *state,
+                    const void *v, const void *ffn_x, const void *x_in, void *x_out, int rescale);
+
 #ifdef __cplusplus
 }
 #endif

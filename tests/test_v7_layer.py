@@ -130,3 +130,41 @@ def test_v7_layer_packed_token_shifts_equal_the_op_list(gpu, runs):
         torch.cuda.synchronize()
         outs.append((buf.x.cpu().numpy(), sd.cpu().numpy()))
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 17, 33, 65], ids=lambda h: f"{64 * h} channels")
+@pytest.mark.parametrize("runs", [[(4, 1)], [(2, 3), (0, 12), (5, 1)], [(1, 15), (3, 2)], [(i, 1) for i in range(5)] + [(5, 251)]],
+                         ids=["1 token", "16 tokens", "17 tokens", "256 tokens"])
+def test_v7_layer_fused_equals_op_list(gpu, runs, H):
+    # edges of the fused kernels: one row vector per thread up to eight (channels), whole and ragged tiles of 16 tokens,
+    # the first layer (no adapter v) and a later one.  The bound is the v6 layer's: both sides round the same f16
+    # buffers, sums in another order move single values by an ulp (2^-11) and the products behind carry a few of them on
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    v7 = importlib.import_module(gpu.__name__ + ".v7")
+    print("v7 layer, fused", runs, H, flush=True)
+    S, hidden, B = 64, 256, 6
+    C = H * S
+    rng = np.random.default_rng(SEED + 90 + len(runs) + H)
+    cursors = lop.pack_cursors(runs)
+    A = len(cursors)
+    curd = torch.from_numpy(cursors.view(np.int32)).cuda()
+    layer = v7.Layer(torch, v7.random_layer_weights(rng, C, H, S, hidden), "int8" if C % 128 == 0 or H > 1 else "nf4")
+    assert v7.fused_is_built(layer, H, S)
+    x, v0 = (rng.standard_normal((1, A, C)).astype(np.float16) for _ in range(2))
+    state = (0.1 * rng.standard_normal((B, S + 2, C))).astype(np.float32)
+    for index, rescale in ((0, False), (1, True)):
+        outs = []
+        for dispatch in (v7.dispatch_layer_ops, v7.dispatch_layer_fused):
+            buf = v7.Runtime(torch, C, hidden, A)
+            buf.x.copy_(torch.from_numpy(x).cuda())
+            buf.att_v0.copy_(torch.from_numpy(v0).cuda())
+            sd = torch.from_numpy(state.copy()).cuda()
+            dispatch(layer, buf, sd, curd, A, H, S, index, rescale)
+            torch.cuda.synchronize()
+            outs.append((buf.x.cpu().numpy(), sd.cpu().numpy(), buf.att_v0.cpu().numpy()))
+        for i, what in enumerate(("layer output", "state", "first layer's values")):
+            assert_close(outs[1][i], outs[0][i], 4e-3, f"{what}, fused vs op list")

@@ -49,6 +49,7 @@ EXPORTS = [
     "wrq_l2_norm", "wrq_control_k_v7", "wrq_time_mix_v7", "wrq_time_first_v7", "wrq_channel_mix_v7",
     "wrq_recenter", "wrq_rms_norm", "wrq_broadcast", "wrq_blend", "wrq_blend_lora",
     "wrq_v6_pre", "wrq_v6_time_mix", "wrq_v6_decay", "wrq_v6_wkv_gate", "wrq_v6_post_ffn",
+    "wrq_fused_pre", "wrq_adapters_in", "wrq_v7_mid", "wrq_v7_wkv_gate", "wrq_v7_post_ffn",
 ]
 MAX_GROUP = 8
 
@@ -224,6 +225,12 @@ def lib():
         L.wrq_v6_decay.argtypes = [vp, u, u, u, vp, vp, vp, vp]
         L.wrq_v6_wkv_gate.argtypes = [vp, u, u, u, vp, vp, vp, V, vp, vp, vp, vp, vp, vp, C.c_float, vp]
         L.wrq_v6_post_ffn.argtypes = [vp, u, u, vp, V, vp, vp, vp, vp, vp, i]
+        P = C.POINTER(vp)
+        L.wrq_fused_pre.argtypes = [vp, u, u, vp, vp, vp, vp, vp, vp, C.c_float, V, i, P, vp, P]
+        L.wrq_adapters_in.argtypes = [vp, u, u, i, P, C.POINTER(u), C.POINTER(i), P, P]
+        L.wrq_v7_mid.argtypes = [vp, u, u, u, i, C.POINTER(u), P, P, P, C.c_float, vp, vp, vp, vp, vp, vp]
+        L.wrq_v7_wkv_gate.argtypes = [vp, u, u, u, vp, V, vp, vp, vp, vp, vp, vp, vp, C.c_float, vp]
+        L.wrq_v7_post_ffn.argtypes = [vp, u, u, vp, V, vp, vp, vp, vp, i]
         for name in EXPORTS:
             if name not in ("wrq_status_string", "wrq_last_error"):
                 getattr(L, name).restype = i
@@ -488,6 +495,45 @@ class FusedV6:
     def post_ffn(Cn, A, cursors, state, state_view, r, v, ffn_x, x_in, x_out, rescale):
         p = FusedV6._p
         _check(lib().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
+
+
+class FusedV7:
+    """The fused forms of a v7 layer's small ops (`wrq_fused_pre`, `wrq_adapters_in`, `wrq_v7_*`); arguments are contiguous
+    torch tensors.  `adapters_in` serves any layer with low-rank adapters."""
+
+    @staticmethod
+    def _a(ts):
+        return (C.c_void_p * len(ts))(*(None if t is None else t.data_ptr() for t in ts))
+
+    @staticmethod
+    def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts):
+        p, a = FusedV6._p, FusedV7._a
+        _check(lib().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
+                                   a(factors), p(ln_out), a(shifts)))
+
+    @staticmethod
+    def adapters_in(Cn, A, ops):
+        """`ops`: list of `(w, x, out, act)`, w [rank, C]."""
+        a, n = FusedV7._a, len(ops)
+        w, x, out, act = zip(*ops)
+        _check(lib().wrq_adapters_in(_stream(), Cn, A, n, a(w), (C.c_uint32 * n)(*(t.shape[0] for t in w)), (C.c_int * n)(*act), a(x), a(out)))
+
+    @staticmethod
+    def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n):
+        p, a = FusedV6._p, FusedV7._a
+        ranks = (C.c_uint32 * 4)(*(t.shape[1] for t in w2))
+        _check(lib().wrq_v7_mid(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n)))
+
+    @staticmethod
+    def wkv_gate(S, H, A, cursors, state, state_view, r, w, n, r_k, g, gn_w, gn_b, eps, att_x):
+        p = FusedV6._p
+        _check(lib().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
+                                     p(att_x)))
+
+    @staticmethod
+    def post_ffn(Cn, A, cursors, state, state_view, v, ffn_x, x_in, x_out, rescale):
+        p = FusedV6._p
+        _check(lib().wrq_v7_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
 
 
 def matmul_vec_group(ops):

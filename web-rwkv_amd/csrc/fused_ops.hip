@@ -4,6 +4,7 @@
 // reference's list in one launch each and bring a layer from 35 launches to 12.  Each computes what the
 // op list computes, with the same roundings where the list stores an f16 buffer in between:
 //   wrq_v6_pre          (add) + blit + layer_norm + token_shift x 1..2     v6.rs:759-777, :906-933
+//   (wrq_fused_pre: the same with up to 6 shifts, for the layers of v7, src/runtime/v7.rs:705-760)
 //   wrq_v6_time_mix     transpose + time_mix_w2 + add + token_shift(5)     v6.rs:785-805
 //   wrq_v6_decay        time_decay_w2 + add + activate(StableExp)          v6.rs:839-848
 //   wrq_v6_wkv_gate     blit + time_mix_v6 + group_norm + blit + mul(Silu) v6.rs:851-887
@@ -17,30 +18,36 @@ namespace wrq {
 namespace {
 
 constexpr int kPreThreads = 256;
-constexpr int kPreCache = 8; // 4-element vectors a thread keeps of a row: rows up to 8192 elements
+constexpr int kPreCache = 8; // 4-element vectors a thread keeps of a row at most: rows up to 8192 elements
+constexpr int kPreShifts = 6;
+
+struct ShiftArgs {
+    const uint16_t *factor[kPreShifts];
+    uint16_t *out[kPreShifts];
+};
 
 // One workgroup per token.  row = x[t] (+ add[t]), written to x_out when given; ln = f16(LN(row)) -> ln_out;
-// shift_out[s][t] = f16(mix(ln, prev, factor[s])) with prev = the request's state row for its first
-// token of the stack, else f16(LN(row t-1)) recomputed here.
-template <int NS>
-__global__ __launch_bounds__(kPreThreads) void v6_pre_kernel(const uint32_t *cursors, const uint16_t *x, const uint16_t *add, uint16_t *x_out,
-                                                             const uint16_t *ln_w, const uint16_t *ln_b, float eps, const float *state, ViewArgs vs,
-                                                             const uint16_t *factor0, const uint16_t *factor1, uint16_t *ln_out, uint16_t *shift0,
-                                                             uint16_t *shift1, uint32_t C) {
+// out[s][t] = f16(mix(ln, prev, factor[s])) with prev = the request's state row for its first
+// token of the stack, else f16(LN(row t-1)) recomputed here.  NC vectors of a row per thread (the smallest of 1, 2, 4, 8
+// that holds it): the six factors of a v7 layer then cost no registers for vectors that a row does not have.
+template <int NS, int NC>
+__global__ __launch_bounds__(kPreThreads) void pre_kernel(const uint32_t *cursors, const uint16_t *x, const uint16_t *add, uint16_t *x_out,
+                                                          const uint16_t *ln_w, const uint16_t *ln_b, float eps, uint32_t C, const float *state, ViewArgs vs,
+                                                          uint16_t *ln_out, ShiftArgs sh) {
     __shared__ float red[kPreThreads / 64];
     const uint32_t t = blockIdx.x, nv = C / 4;
     // Everything that does not depend on the row statistics is requested first: a workgroup is a chain of
     // dependent memory round trips otherwise (cursor, row, weights after the reductions, state, factors),
     // and at one token per launch that chain is the kernel's whole time.
-    uint2 wq[kPreCache], bq[kPreCache], fq[NS][kPreCache];
+    uint2 wq[NC], bq[NC], fq[NS][NC];
 #pragma unroll
-    for (int c = 0; c < kPreCache; c++) {
+    for (int c = 0; c < NC; c++) {
         const uint32_t i = threadIdx.x + c * kPreThreads;
         if (i < nv) {
             wq[c] = *reinterpret_cast<const uint2 *>(ln_w + 4 * i);
             bq[c] = *reinterpret_cast<const uint2 *>(ln_b + 4 * i);
 #pragma unroll
-            for (int s = 0; s < NS; s++) fq[s][c] = *reinterpret_cast<const uint2 *>((s == 0 ? factor0 : factor1) + 4 * i);
+            for (int s = 0; s < NS; s++) fq[s][c] = *reinterpret_cast<const uint2 *>(sh.factor[s] + 4 * i);
         }
     }
     auto unpack = [](uint2 v) {
@@ -48,24 +55,24 @@ __global__ __launch_bounds__(kPreThreads) void v6_pre_kernel(const uint32_t *cur
     };
     const Cursor cur = read_cursor(cursors, t, vs);
     const bool first = t == cur.token;
-    float4 pst[kPreCache]; // the request's state row, for its first token of the stack
+    float4 pst[NC]; // the request's state row, for its first token of the stack
     if (first) {
 #pragma unroll
-        for (int c = 0; c < kPreCache; c++) {
+        for (int c = 0; c < NC; c++) {
             const uint32_t i = threadIdx.x + c * kPreThreads;
             if (i < nv) pst[c] = load_vec4(state + view_elem(vs, cur.batch, 0, 4 * i));
         }
     }
     // rows t (which = 0) and t - 1 (which = 1): normalised, rounded to f16 as the op list stores them
-    float4 ln[2][kPreCache];
+    float4 ln[2][NC];
 #pragma unroll
     for (int which = 0; which < 2; which++) {
         if (which == 1 && first) break;
         const uint64_t base = (uint64_t)(t - which) * C;
-        float4 row[kPreCache];
+        float4 row[NC];
         float part = 0.0f;
 #pragma unroll
-        for (int c = 0; c < kPreCache; c++) {
+        for (int c = 0; c < NC; c++) {
             const uint32_t i = threadIdx.x + c * kPreThreads;
             if (i < nv) {
                 float4 v = load_vec4(x + base + 4 * i);
@@ -81,14 +88,14 @@ __global__ __launch_bounds__(kPreThreads) void v6_pre_kernel(const uint32_t *cur
         const float mean = block_reduce<false, kPreThreads>(part, red) / (float)C;
         float acc = 0.0f;
 #pragma unroll
-        for (int c = 0; c < kPreCache; c++)
+        for (int c = 0; c < NC; c++)
             if (threadIdx.x + c * kPreThreads < nv) {
                 const float4 v = row[c];
                 acc += ((v.x - mean) * (v.x - mean) + (v.y - mean) * (v.y - mean)) + ((v.z - mean) * (v.z - mean) + (v.w - mean) * (v.w - mean));
             }
         const float dev = rsqrtf(block_reduce<false, kPreThreads>(acc, red) / (float)C + eps);
 #pragma unroll
-        for (int c = 0; c < kPreCache; c++) {
+        for (int c = 0; c < NC; c++) {
             const uint32_t i = threadIdx.x + c * kPreThreads;
             if (i < nv) {
                 const float4 v = row[c], w = unpack(wq[c]), b = unpack(bq[c]);
@@ -99,7 +106,7 @@ __global__ __launch_bounds__(kPreThreads) void v6_pre_kernel(const uint32_t *cur
         }
     }
 #pragma unroll
-    for (int c = 0; c < kPreCache; c++) {
+    for (int c = 0; c < NC; c++) {
         const uint32_t i = threadIdx.x + c * kPreThreads;
         if (i >= nv) continue;
         const float4 p = first ? pst[c] : ln[1][c];
@@ -108,7 +115,7 @@ __global__ __launch_bounds__(kPreThreads) void v6_pre_kernel(const uint32_t *cur
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             const float4 f = unpack(fq[s][c]);
-            store_vec4((s == 0 ? shift0 : shift1) + (uint64_t)t * C + 4 * i, make_float4(mix(a.x, p.x, f.x), mix(a.y, p.y, f.y), mix(a.z, p.z, f.z), mix(a.w, p.w, f.w)));
+            store_vec4(sh.out[s] + (uint64_t)t * C + 4 * i, make_float4(mix(a.x, p.x, f.x), mix(a.y, p.y, f.y), mix(a.z, p.z, f.z), mix(a.w, p.w, f.w)));
         }
     }
 }
@@ -200,42 +207,23 @@ __global__ __launch_bounds__(256) void v6_post_ffn_kernel(const uint32_t *cursor
     store_vec4(x_out + bti, make_float4(f(rr.x, vv.x, xx.x), f(rr.y, vv.y, xx.y), f(rr.z, vv.z, xx.z), f(rr.w, vv.w, xx.w)));
 }
 
-int check_ptr(const void *p, const char *what) {
-    if (!p) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
-    if ((uintptr_t)p % 16) return fail(WRQ_ERR_ALIGNMENT, "%s: device pointers must be 16-byte aligned", what);
-    return WRQ_OK;
-}
-
-int check_state(const wrq_tensor_view *state, uint32_t C, uint32_t rows, const char *what) {
-    const int s = check_state_view(state, what);
-    if (s != WRQ_OK) return s;
-    if (state->dtype != WRQ_F32) return fail(WRQ_ERR_TYPE, "%s: the state is f32", what);
-    if (state->view.shape[0] != C || state->view.shape[1] != rows || state->view.shape[2] == 0 || state->view.shape[3] != 1)
-        return fail(WRQ_ERR_SHAPE, "%s: state shape [%u, %u, %u, %u] not match [%u, %u, _, 1]", what, state->view.shape[0], state->view.shape[1],
-                    state->view.shape[2], state->view.shape[3], C, rows);
-    return WRQ_OK;
-}
-
-} // namespace
-
-} // namespace wrq
-
-using namespace wrq;
-
-extern "C" {
-
-int wrq_v6_pre(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const void *x, const void *add, void *x_out, const void *ln_w,
-               const void *ln_b, float eps, const wrq_tensor_view *state, int shifts, const void *factor0, const void *factor1, void *ln_out,
-               void *shift0, void *shift1) {
-    const char *what = "v6_pre";
+// `most`: shifts of the entry point
+int launch_pre(const char *what, int most, wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const void *x, const void *add, void *x_out, const void *ln_w,
+                  const void *ln_b, float eps, const wrq_tensor_view *state, int shifts, const void *const *factors, void *ln_out, void *const *outs) {
     if (C == 0 || A == 0) return WRQ_OK;
     if (C % 4 || C > 4u * kPreThreads * kPreCache) return fail(WRQ_ERR_UNSUPPORTED, "%s: %u channels (a multiple of 4 up to %d is built)", what, C, 4 * kPreThreads * kPreCache);
-    if (shifts != 1 && shifts != 2) return fail(WRQ_ERR_UNSUPPORTED, "%s: %d token shifts (1 or 2)", what, shifts);
+    if ((shifts != 1 && shifts != 2 && shifts != 6) || shifts > most)
+        return fail(WRQ_ERR_UNSUPPORTED, "%s: %d token shifts (%s)", what, shifts, most > 2 ? "1, 2 or 6" : "1 or 2");
+    if (!factors || !outs) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
     int s = check_state(state, C, state ? state->view.shape[1] : 0, what);
-    for (const void *p : {cursors, x, ln_w, ln_b, factor0, (const void *)ln_out, (const void *)shift0})
+    for (const void *p : {cursors, x, ln_w, ln_b, (const void *)ln_out})
         if (s == WRQ_OK) s = check_ptr(p, what);
-    if (s == WRQ_OK && shifts == 2) s = check_ptr(factor1, what);
-    if (s == WRQ_OK && shifts == 2) s = check_ptr(shift1, what);
+    ShiftArgs sh{};
+    for (int i = 0; i < shifts && s == WRQ_OK; i++) {
+        sh.factor[i] = static_cast<const uint16_t *>(factors[i]), sh.out[i] = static_cast<uint16_t *>(outs[i]);
+        s = check_ptr(factors[i], what);
+        if (s == WRQ_OK) s = check_ptr(outs[i], what);
+    }
     if (s == WRQ_OK && add) s = check_ptr(x_out, what);
     if (s != WRQ_OK) return s;
     if (add) {
@@ -248,16 +236,38 @@ int wrq_v6_pre(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, c
         }
     }
     const ViewArgs vs = view_args(state->view);
-    hipStream_t hs = static_cast<hipStream_t>(stream);
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     auto o16 = [](void *p) { return static_cast<uint16_t *>(p); };
-    if (shifts == 1)
-        hipLaunchKernelGGL((v6_pre_kernel<1>), dim3(A), dim3(kPreThreads), 0, hs, static_cast<const uint32_t *>(cursors), u16(x), u16(add), o16(x_out), u16(ln_w),
-                           u16(ln_b), eps, static_cast<const float *>(state->data), vs, u16(factor0), u16(factor1), o16(ln_out), o16(shift0), o16(shift1), C);
-    else
-        hipLaunchKernelGGL((v6_pre_kernel<2>), dim3(A), dim3(kPreThreads), 0, hs, static_cast<const uint32_t *>(cursors), u16(x), u16(add), o16(x_out), u16(ln_w),
-                           u16(ln_b), eps, static_cast<const float *>(state->data), vs, u16(factor0), u16(factor1), o16(ln_out), o16(shift0), o16(shift1), C);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(A), dim3(kPreThreads), 0, static_cast<hipStream_t>(stream), static_cast<const uint32_t *>(cursors), u16(x), u16(add),
+                           o16(x_out), u16(ln_w), u16(ln_b), eps, C, static_cast<const float *>(state->data), vs, o16(ln_out), sh);
+    };
+    const uint32_t nc = (C / 4 + kPreThreads - 1) / kPreThreads;
+#define WRQ_PRE(NS) (nc <= 1 ? go(pre_kernel<NS, 1>) : nc <= 2 ? go(pre_kernel<NS, 2>) : nc <= 4 ? go(pre_kernel<NS, 4>) : go(pre_kernel<NS, 8>))
+    shifts == 1 ? WRQ_PRE(1) : shifts == 2 ? WRQ_PRE(2) : WRQ_PRE(6);
+#undef WRQ_PRE
     return check_launch(what);
+}
+
+} // namespace
+
+} // namespace wrq
+
+using namespace wrq;
+
+extern "C" {
+
+int wrq_fused_pre(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const void *x, const void *add, void *x_out, const void *ln_w,
+                  const void *ln_b, float eps, const wrq_tensor_view *state, int shifts, const void *const *factors, void *ln_out, void *const *outs) {
+    return launch_pre("fused_pre", kPreShifts, stream, C, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, shifts, factors, ln_out, outs);
+}
+
+int wrq_v6_pre(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const void *x, const void *add, void *x_out, const void *ln_w,
+               const void *ln_b, float eps, const wrq_tensor_view *state, int shifts, const void *factor0, const void *factor1, void *ln_out,
+               void *shift0, void *shift1) {
+    const void *const factors[2] = {factor0, factor1};
+    void *const outs[2] = {shift0, shift1};
+    return launch_pre("v6_pre", 2, stream, C, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, shifts, factors, ln_out, outs);
 }
 
 int wrq_v6_time_mix(wrq_stream stream, uint32_t C, uint32_t A, uint32_t lora_size, const void *cursors, const void *lora, const void *w2, const void *time_mix,

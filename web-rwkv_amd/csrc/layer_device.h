@@ -115,6 +115,23 @@ inline int check_layer_tensor(const wrq_tensor *t, const char *what) {
     return WRQ_OK;
 }
 
+// operands of the fused ops: contiguous device buffers, and the rows of a state
+inline int check_ptr(const void *p, const char *what) {
+    if (!p) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
+    if ((uintptr_t)p % 16) return fail(WRQ_ERR_ALIGNMENT, "%s: device pointers must be 16-byte aligned", what);
+    return WRQ_OK;
+}
+
+inline int check_state(const wrq_tensor_view *state, uint32_t C, uint32_t rows, const char *what) {
+    const int s = check_state_view(state, what);
+    if (s != WRQ_OK) return s;
+    if (state->dtype != WRQ_F32) return fail(WRQ_ERR_TYPE, "%s: the state is f32", what);
+    if (state->view.shape[0] != C || state->view.shape[1] != rows || state->view.shape[2] == 0 || state->view.shape[3] != 1)
+        return fail(WRQ_ERR_SHAPE, "%s: state shape [%u, %u, %u, %u] not match [%u, %u, _, 1]", what, state->view.shape[0], state->view.shape[1],
+                    state->view.shape[2], state->view.shape[3], C, rows);
+    return WRQ_OK;
+}
+
 inline bool same_shape(const uint32_t *a, const uint32_t *b) { return a[0] == b[0] && a[1] == b[1] && a[2] == b[2] && a[3] == b[3]; }
 
 } // namespace wrq

@@ -10,11 +10,158 @@
 //   sa[i] = sum_j S[j][i] a[j];   S[j][i] <- S[j][i] w[j] + k[j] v[i] + sa[i] b[j];   y[i] = sum_j r[j] S[j][i]
 // The shader walks the state in memory twice per token; recurrence.h keeps it in registers over all tokens of
 // a request in the run.
+//
+// Fused forms of the layer's small ops (src/runtime/v7.rs:704-1006), which are bound by their launches at the run
+// lengths of a serving schedule: wrq_adapters_in, wrq_v7_mid, wrq_v7_wkv_gate, wrq_v7_post_ffn (with wrq_fused_pre of
+// fused_ops.hip).  A layer takes 10 launches beside the second ones of split products instead of 45.
 #include "recurrence.h"
 
 namespace wrq {
 
 namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxAdapters = 4;
+constexpr int kAdapterWaves = 8;
+struct AdapterArgs {
+    const uint16_t *w[kMaxAdapters], *x[kMaxAdapters];
+    uint16_t *out[kMaxAdapters];
+    uint32_t rank[kMaxAdapters], tile_begin[kMaxAdapters + 1]; // 16-row tiles of all adapters, one adapter after the other
+    int act[kMaxAdapters];
+};
+
+// First halves of a layer's low-rank adapters, out[t][r] = f16(act(sum_k w[r][k] x[t][k])): a few dozen rows over K = C
+// per adapter, so the product is one short pass over weights that fit in the caches and its time is latency.  One workgroup
+// per 16 rows x 16 tokens of any adapter of the layer; its eight waves take every eighth 32-element step of K, straight from
+// memory in the operand layout of the 16x16x32 MFMA, eight steps in flight, and add up through LDS.  2048 channels, 32 tokens, four adapters: 7 us
+// in one launch, against 4 x (5 + 3) us for products split over K and summed by a second launch each.
+__global__ __launch_bounds__(64 * kAdapterWaves) void adapters_in_kernel(uint32_t K, uint32_t T, AdapterArgs aa) {
+    __shared__ float4 red[kAdapterWaves - 1][64];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+    uint32_t p = 0;
+#pragma unroll
+    for (uint32_t i = 1; i < kMaxAdapters; i++)
+        if (blockIdx.x >= aa.tile_begin[i]) p = i;
+    const uint32_t row0 = 16 * (blockIdx.x - aa.tile_begin[p]), t0 = 16 * blockIdx.y;
+    const uint32_t steps = K / 32;
+    const uint16_t *wp = aa.w[p] + (uint64_t)(row0 + r16) * K + 8 * g;
+    const uint16_t *xp = aa.x[p] + (uint64_t)min(t0 + r16, T - 1) * K + 8 * g; // columns past the run repeat its last token, never stored
+    float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t s0 = wave; s0 < steps; s0 += 8 * kAdapterWaves) {
+        uint4 a[8], b[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const uint32_t at = 32 * min(s0 + q * kAdapterWaves, steps - 1);
+            a[q] = load128(wp + at), b[q] = load128(xp + at);
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            if (s0 + q * kAdapterWaves < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[q]), __builtin_bit_cast(half8, b[q]), acc, 0, 0, 0);
+    }
+    if (wave) red[wave - 1][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    __syncthreads();
+    if (wave) return;
+#pragma unroll
+    for (int w = 0; w < kAdapterWaves - 1; w++) {
+        const float4 v = red[w][lane];
+        acc[0] += v.x, acc[1] += v.y, acc[2] += v.z, acc[3] += v.w;
+    }
+    // lane: token r16 of the tile, rows 4 g .. 4 g + 3
+    if (t0 + r16 < T) {
+        const int act = aa.act[p];
+        store_vec4(aa.out[p] + (uint64_t)(t0 + r16) * aa.rank[p] + row0 + 4 * g,
+                   make_float4(act_apply(act, acc[0]), act_apply(act, acc[1]), act_apply(act, acc[2]), act_apply(act, acc[3])));
+    }
+}
+
+struct MidArgs {
+    const uint16_t *aux_w, *aux_a, *aux_g, *aux_v;                 // [T, rank]
+    const uint16_t *w2, *a2, *g2, *v2;                             // [C, rank]
+    const uint16_t *w0, *a0, *v0, *k_k, *k_a;                      // [C]
+    const uint16_t *k, *v;                                         // [T, C]
+    uint16_t *att_v0, *att_w, *att_g, *n;                          // [T, C], n: [4, T, C]
+};
+
+// Second halves of the four adapters and what a v7 layer makes of them before the recurrence.  A workgroup takes one head
+// (64 channels, 16 per wave) and 16 tokens: nine MFMAs of 32 inner elements per wave, then every lane holds 4 channels of
+// one token and finishes them in registers with the roundings to f16 the op list has:
+//   w = w0 + w2 aux_w;   a = sigmoid(a0 + a2 aux_a);   g = g2 aux_g;   v <- mix(v, v0, sigmoid(v_0 + v2 aux_v)) (FIRST: v0 <- v);
+//   kk = l2_norm(k k_k) over the head;   k <- k (1 + (a - 1) k_a);   n = (k, v, a, kk)
+// (src/runtime/v7.rs:780-880).  2048 channels, 32 tokens: 5.8 us against about 60 us for the 17 launches of the list; bound by one
+// round trip to memory, which is why every operand is requested before the first use.
+template <int RW, int RA, int RG, int RV, bool FIRST>
+__global__ __launch_bounds__(256) void v7_mid_kernel(uint32_t C, uint32_t T, float eps, MidArgs m) {
+    __shared__ float part[4][16];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
+    const uint32_t t0 = 16 * blockIdx.y, t = min(t0 + r16, T - 1);
+    const uint32_t c0 = 64 * blockIdx.x + 16 * wave; // the wave's 16 channels; this lane finishes c0 + 4 g ..
+    constexpr int NW = RW / 32, NA = RA / 32, NG = RG / 32, NV = FIRST ? 0 : RV / 32;
+    uint4 wa[NW + NA + NG + NV + 1], xb[NW + NA + NG + NV + 1];
+    auto fetch = [&](auto rank, const uint16_t *w, const uint16_t *x, int at) {
+        constexpr int R = decltype(rank)::value;
+#pragma unroll
+        for (int s = 0; s < R / 32; s++) {
+            wa[at + s] = load128(w + (uint64_t)(c0 + r16) * R + 32 * s + 8 * g);
+            xb[at + s] = load128(x + (uint64_t)t * R + 32 * s + 8 * g);
+        }
+    };
+    fetch(std::integral_constant<int, RW>{}, m.w2, m.aux_w, 0);
+    fetch(std::integral_constant<int, RA>{}, m.a2, m.aux_a, NW);
+    fetch(std::integral_constant<int, RG>{}, m.g2, m.aux_g, NW + NA);
+    if constexpr (!FIRST) fetch(std::integral_constant<int, RV>{}, m.v2, m.aux_v, NW + NA + NG);
+    const uint32_t ch = c0 + 4 * g;
+    const uint64_t at = (uint64_t)t * C + ch, plane = (uint64_t)T * C;
+    const float4 w0 = load_vec4(m.w0 + ch), a0 = load_vec4(m.a0 + ch), v0 = load_vec4(m.v0 + ch), k_k = load_vec4(m.k_k + ch), k_a = load_vec4(m.k_a + ch);
+    const float4 k = load_vec4(m.k + at), v = load_vec4(m.v + at);
+    const float4 first = FIRST ? v : load_vec4(m.att_v0 + at);
+    auto product = [&](int from, int count) {
+        float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < count; s++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, wa[from + s]), __builtin_bit_cast(half8, xb[from + s]), acc, 0, 0, 0);
+        return make_float4(round_h(acc[0]), round_h(acc[1]), round_h(acc[2]), round_h(acc[3]));
+    };
+    auto each = [](auto f, float4 a, float4 b, float4 c) { return make_float4(f(a.x, b.x, c.x), f(a.y, b.y, c.y), f(a.z, b.z, c.z), f(a.w, b.w, c.w)); };
+    auto sigmoid_sum = [](float bias, float y, float) { return round_h(act_one<WRQ_ACT_SIGMOID>(bias + y)); };
+    const float4 w = each([](float bias, float y, float) { return bias + y; }, w0, product(0, NW), w0);
+    const float4 a = each(sigmoid_sum, a0, product(NW, NA), a0);
+    const float4 gate = product(NW + NA, NG);
+    float4 vm = v;
+    if constexpr (!FIRST) {
+        const float4 f = each(sigmoid_sum, v0, product(NW + NA + NG, NV), v0);
+        vm = each([](float vv, float ff, float va) { return vv * (1.0f - ff) + va * ff; }, v, f, first);
+    }
+    const float4 kk = each([](float p, float kv, float) { return round_h(p * kv); }, k_k, k, k);
+    float sum = kk.x * kk.x + kk.y * kk.y + kk.z * kk.z + kk.w * kk.w;
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (lane < 16) part[wave][lane] = sum;
+    __syncthreads();
+    const float norm = 1.0f / sqrtf((part[0][r16] + part[1][r16]) + (part[2][r16] + part[3][r16]) + eps);
+    if (t0 + r16 >= T) return;
+    store_vec4(m.att_w + at, w);
+    store_vec4(m.att_g + at, gate);
+    if constexpr (FIRST) store_vec4(m.att_v0 + at, v);
+    store_vec4(m.n + at, each([](float kv, float av, float p) { return kv * (1.0f + (av - 1.0f) * p); }, k, a, k_a));
+    store_vec4(m.n + plane + at, vm);
+    store_vec4(m.n + 2 * plane + at, a);
+    store_vec4(m.n + 3 * plane + at, make_float4(kk.x * norm, kk.y * norm, kk.z * norm, kk.w * norm));
+}
+
+// state[request] <- ffn_x at its last token; x_out = f16(v + x_in) (halved when `rescale`)
+__global__ __launch_bounds__(256) void v7_post_ffn_kernel(const uint32_t *cursors, float *state, const uint16_t *v, const uint16_t *ffn_x, const uint16_t *x_in,
+                                                          uint16_t *x_out, uint32_t C, int rescale, ViewArgs vs) {
+    const uint32_t index = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
+    if (index >= C / 4) return;
+    const uint64_t bti = (uint64_t)t * C + 4 * index;
+    const float4 vv = load_vec4(v + bti), xx = load_vec4(x_in + bti), fx = load_vec4(ffn_x + bti); // before the cursor's round trip and the store into the state
+    const Cursor cur = read_cursor(cursors, t, vs);
+    if (t - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = fx;
+    const float sc = rescale ? 0.5f : 1.0f;
+    auto f = [&](float a, float b) { return round_h(a + b) * sc; };
+    store_vec4(x_out + bti, make_float4(f(vv.x, xx.x), f(vv.y, xx.y), f(vv.z, xx.z), f(vv.w, xx.w)));
+}
 
 template <typename XT>
 __global__ __launch_bounds__(64) void l2_norm_kernel(XT *x, uint32_t C, float eps) {
@@ -212,6 +359,97 @@ int wrq_channel_mix_v7(wrq_stream stream, const wrq_tensor *cursors, const wrq_t
         hipLaunchKernelGGL((channel_mix_v7_kernel<float>), grid, dim3(256), 0, hs, cur, static_cast<float *>(state->data), static_cast<const float *>(v->data),
                            static_cast<float *>(x->data), vs, sh[0]);
     return check_launch("channel_mix_v7");
+}
+
+int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void *const *w, const uint32_t *ranks, const int *acts, const void *const *x,
+                    void *const *out) {
+    const char *what = "adapters_in";
+    if (n < 0 || n > kMaxAdapters) return fail(WRQ_ERR_UNSUPPORTED, "%s: %d adapters (up to %d)", what, n, kMaxAdapters);
+    if (n == 0 || C == 0 || A == 0) return WRQ_OK;
+    if (!w || !ranks || !acts || !x || !out) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
+    if (C % 32) return fail(WRQ_ERR_ALIGNMENT, "%s: row length %u not a multiple of 32", what, C);
+    if (A > 65535u * 16u) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
+    AdapterArgs aa{};
+    uint32_t tiles = 0;
+    for (int i = 0; i < kMaxAdapters; i++) {
+        aa.tile_begin[i] = i < n ? tiles : ~0u;
+        if (i >= n) continue;
+        if (ranks[i] == 0 || ranks[i] % 16 || ranks[i] > 65536u) return fail(WRQ_ERR_UNSUPPORTED, "%s: adapter size %u (a multiple of 16 up to 65536 is built)", what, ranks[i]);
+        if (acts[i] < 0 || acts[i] > WRQ_ACT_SILU) return fail(WRQ_ERR_UNSUPPORTED, "%s: activation %d", what, acts[i]);
+        for (const void *p : {w[i], x[i], (const void *)out[i]}) {
+            const int s = check_ptr(p, what);
+            if (s != WRQ_OK) return s;
+        }
+        aa.w[i] = static_cast<const uint16_t *>(w[i]), aa.x[i] = static_cast<const uint16_t *>(x[i]), aa.out[i] = static_cast<uint16_t *>(out[i]);
+        aa.rank[i] = ranks[i], aa.act[i] = acts[i];
+        tiles += ranks[i] / 16;
+    }
+    hipLaunchKernelGGL(adapters_in_kernel, dim3(tiles, (A + 15) / 16), dim3(64 * kAdapterWaves), 0, static_cast<hipStream_t>(stream), C, A, aa);
+    return check_launch(what);
+}
+
+int wrq_v7_mid(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first, const uint32_t *ranks, const void *const *aux, const void *const *w2,
+               const void *const *vectors, float eps, const void *k, const void *v, void *att_v0, void *att_w, void *att_g, void *n) {
+    const char *what = "v7_mid";
+    if (H == 0 || A == 0) return WRQ_OK;
+    if (S != 64) return fail(WRQ_ERR_UNSUPPORTED, "%s: head size %u (64 is built)", what, S);
+    if (!ranks || !aux || !w2 || !vectors) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
+    if (ranks[0] != 64 || ranks[1] != 64 || ranks[2] != 128 || ranks[3] != 32)
+        return fail(WRQ_ERR_UNSUPPORTED, "%s: adapter sizes %u, %u, %u, %u (64, 64, 128, 32 are built)", what, ranks[0], ranks[1], ranks[2], ranks[3]);
+    if (A > 65535u * 16u) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
+    int s = WRQ_OK;
+    for (int i = 0; i < (first ? 3 : 4) && s == WRQ_OK; i++) {
+        s = check_ptr(aux[i], what);
+        if (s == WRQ_OK) s = check_ptr(w2[i], what);
+    }
+    for (int i = 0; i < 5 && s == WRQ_OK; i++) s = check_ptr(vectors[i], what);
+    for (const void *p : {k, v, (const void *)att_v0, (const void *)att_w, (const void *)att_g, (const void *)n})
+        if (s == WRQ_OK) s = check_ptr(p, what);
+    if (s != WRQ_OK) return s;
+    auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
+    auto o16 = [](void *p) { return static_cast<uint16_t *>(p); };
+    const MidArgs m{u16(aux[0]),     u16(aux[1]),     u16(aux[2]),     u16(aux[3]),     u16(w2[0]), u16(w2[1]), u16(w2[2]),  u16(w2[3]),  u16(vectors[0]),
+                    u16(vectors[1]), u16(vectors[2]), u16(vectors[3]), u16(vectors[4]), u16(k),     u16(v),     o16(att_v0), o16(att_w), o16(att_g),
+                    o16(n)};
+    const dim3 grid(H, (A + 15) / 16);
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    if (first) hipLaunchKernelGGL((v7_mid_kernel<64, 64, 128, 32, true>), grid, dim3(256), 0, hs, S * H, A, eps, m);
+    else hipLaunchKernelGGL((v7_mid_kernel<64, 64, 128, 32, false>), grid, dim3(256), 0, hs, S * H, A, eps, m);
+    return check_launch(what);
+}
+
+int wrq_v7_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const void *cursors, const wrq_tensor_view *state, const void *r, const void *w,
+                    const void *n, const void *r_k, const void *g, const void *gn_w, const void *gn_b, float eps, void *att_x) {
+    const char *what = "v7_wkv_gate";
+    if (H == 0 || A == 0) return WRQ_OK;
+    if (S != 64) return fail(WRQ_ERR_UNSUPPORTED, "%s: head size %u (64 is built)", what, S);
+    int s = check_state(state, S * H, S + 1, what);
+    for (const void *p : {cursors, r, w, n, r_k, g, gn_w, gn_b, (const void *)att_x})
+        if (s == WRQ_OK) s = check_ptr(p, what);
+    if (s != WRQ_OK) return s;
+    const ViewArgs vs = view_args(state->view);
+    auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
+    hipLaunchKernelGGL((time_mix_v7_kernel<uint16_t, 64, true>), dim3(H, slot_grid(vs)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint32_t *>(cursors), static_cast<float *>(state->data), u16(r), u16(w), u16(n), static_cast<uint16_t *>(nullptr), vs, H, A,
+                       u16(r_k), GateArgs{u16(g), u16(gn_w), u16(gn_b), static_cast<uint16_t *>(att_x), eps});
+    return check_launch(what);
+}
+
+int wrq_v7_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const wrq_tensor_view *state, const void *v, const void *ffn_x,
+                    const void *x_in, void *x_out, int rescale) {
+    const char *what = "v7_post_ffn";
+    if (C == 0 || A == 0) return WRQ_OK;
+    if (C % 4) return fail(WRQ_ERR_ALIGNMENT, "%s: row length %u not a multiple of 4", what, C);
+    if (A > 65535u) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
+    int s = check_state(state, C, 1, what);
+    for (const void *p : {cursors, v, ffn_x, x_in, (const void *)x_out})
+        if (s == WRQ_OK) s = check_ptr(p, what);
+    if (s != WRQ_OK) return s;
+    const ViewArgs vs = view_args(state->view);
+    auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
+    hipLaunchKernelGGL(v7_post_ffn_kernel, dim3((C / 4 + 255) / 256, A), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint32_t *>(cursors),
+                       static_cast<float *>(state->data), u16(v), u16(ffn_x), u16(x_in), static_cast<uint16_t *>(x_out), C, rescale, vs);
+    return check_launch(what);
 }
 
 } // extern "C"

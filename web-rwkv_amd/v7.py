@@ -7,7 +7,7 @@ import importlib
 import numpy as np
 
 _pkg = importlib.import_module(__name__.rsplit(".", 1)[0])
-LayerOp, Matrix, turbo, matmul_vec_group = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group
+LayerOp, FusedV7, Matrix, turbo, matmul_vec_group = _pkg.LayerOp, _pkg.FusedV7, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group
 ACT_NONE, ACT_SQUARED_RELU, ACT_TANH, ACT_SIGMOID = _pkg.ACT_NONE, _pkg.ACT_SQUARED_RELU, _pkg.ACT_TANH, _pkg.ACT_SIGMOID
 
 L2_EPS = 1.0e-12  # Model::L2_EPS, src/runtime/v7.rs:46
@@ -64,6 +64,7 @@ class Runtime:
         self.att_n = z(4, A, C)
         self.aux_w, self.aux_a, self.aux_g, self.aux_v = z(1, A, RANK_W), z(1, A, RANK_A), z(1, A, RANK_G), z(1, A, RANK_V)
         self.ffn_k = z(1, A, hidden)
+        self.x2 = z(1, A, C)  # the residual between the two halves of a layer on the fused path
 
 
 class PackedShifts:
@@ -83,7 +84,53 @@ class PackedShifts:
 def dispatch_layer(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
     """src/runtime/v7.rs:704-1006.  `state`: this layer's f32 tensor (B, S + 2, C): rows 0..S the
     attention state, row S + 1 the feed-forward one; `index`: the layer's number (layer 0 keeps its
-    values as `att_v0`, the later ones mix theirs with it)."""
+    values as `att_v0`, the later ones mix theirs with it).  The fused form where it is built (every v7 model has
+    heads of 64; adapters of the sizes above and up to 8192 channels), the op list otherwise."""
+    if fused_is_built(layer, H, S):
+        dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts)
+    else:
+        dispatch_layer_ops(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts)
+
+
+def fused_is_built(layer, H, S):
+    t = layer.t
+    ranks = tuple(t[n].shape[0] for n in ("w1", "a1", "g1", "v1"))
+    return S == 64 and H * S <= 8192 and ranks == (64, 64, 128, 32)
+
+
+def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
+    """The layer in 10 launches (beside the second ones of split products): the six quantized products in four and six
+    fused launches for the 40 small ops.  Same results as `dispatch_layer_ops` up to f32 summation order; the buffers
+    between the fused ops (`att_kk`, `att_vv`, `att_a`) stay unwritten, and `att_k`, `att_v` keep the projections.
+    Four layers of 2048 channels, 32 requests of one token: 195 -> 84 us per layer."""
+    t, m, C = layer.t, layer.m, H * S
+    B = state.shape[0]
+    fast = turbo(A)
+    att_state = ((C, S + 1, B), (C, S + 2, B), (0, 0, 0))
+    ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
+    if shifts is None:
+        rx, wx, kx, vx, ax, gx = buf.att_rx, buf.att_wx, buf.att_kx, buf.att_vx, buf.att_ax, buf.att_gx
+    else:
+        rx, wx, kx, vx, ax, gx = (shifts.sx[i].view(1, A, C) for i in range(6))
+
+    FusedV7.pre(C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state,
+                [t[n] for n in PackedShifts.NAMES], buf.att_x, [rx, wx, kx, vx, ax, gx])
+    matmul_vec_group([(m["att_w_r"], rx, buf.att_r, ACT_NONE, False, {}), (m["att_w_k"], kx, buf.att_k, ACT_NONE, False, {}),
+                      (m["att_w_v"], vx, buf.att_v, ACT_NONE, False, {})])
+    adapters = [(t["w1"], wx, buf.aux_w, ACT_TANH), (t["a1"], ax, buf.aux_a, ACT_NONE), (t["g1"], gx, buf.aux_g, ACT_SIGMOID), (t["v1"], vx, buf.aux_v, ACT_NONE)]
+    FusedV7.adapters_in(C, A, adapters[:3] if index == 0 else adapters)
+    FusedV7.mid(S, H, A, index == 0, [buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v], [t["w2"], t["a2"], t["g2"], t["v2"]],
+                [t["w0"], t["a0"], t["v0"], t["k_k"], t["k_a"]], L2_EPS, buf.att_k, buf.att_v, buf.att_v0, buf.att_w, buf.att_g, buf.att_n)
+    FusedV7.wkv_gate(S, H, A, cursors, state, att_state, buf.att_r, buf.att_w, buf.att_n, t["r_k"], buf.att_g, t["gn_w"], t["gn_b"], GN_EPS, buf.att_x)
+    m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)
+    FusedV7.pre(C, A, cursors, buf.x, buf.att_o, buf.x2, t["ffn_ln_w"], t["ffn_ln_b"], LN_EPS, state, ffn_state, [t["ffn_x_k"]], buf.ffn_x, [buf.ffn_kx])
+    m["ffn_w_k"].matmul_op(buf.ffn_kx, buf.ffn_k, ACT_SQUARED_RELU, fast)
+    m["ffn_w_v"].matmul_op_sparse(buf.ffn_k, buf.ffn_v, ACT_NONE, fast)
+    FusedV7.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now)
+
+
+def dispatch_layer_ops(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
+    """The layer op by op, as the reference lists it."""
     t, m, C = layer.t, layer.m, H * S
     B = state.shape[0]
     fast = turbo(A)
