@@ -43,3 +43,33 @@ def test_gpu_slots(gpu, version, S, B, runs):
     # f32 sums of S terms, the state's rounding accumulated over up to 273 tokens with a decay below 1
     assert_close(xd.cpu().numpy(), want, 5e-5, "y vs float64")
     assert_close(sd.cpu().numpy(), want_state, 5e-5, "state vs float64")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("version", [6, 7])
+@pytest.mark.parametrize("runs", [[(0, 1), (1, 2), (0, 1), (0, 3), (1, 1)], [(0, 3), (0, 9), (0, 2)], [(0, 1)] * 16 + [(0, 5)]])
+def test_gpu_fused_keeps_the_last_input(gpu, version, runs):
+    """Requests of one slot that end close together: row 0 of the state is the layer's input at the last of them."""
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("fused recurrence, slots that come again", version, runs, flush=True)
+    H, S, B = 2, 64, 2
+    C = H * S
+    cur = lop.pack_cursors(runs)
+    A = len(cur)
+    g = torch.Generator().manual_seed(0x5753 + A)
+    f32 = lambda *s: (torch.randn(s, generator=g) * 0.3).cuda()
+    f16 = lambda *s: f32(*s).half()
+    curd, state, att_x = torch.from_numpy(cur.view(np.int32)).cuda(), f32(B, S + 2, C), f16(A, C)
+    view, before = ((C, S + 1, B), (C, S + 2, B), (0, 0, 0)), att_x.clone()
+    if version == 6:
+        gpu.FusedV6.wkv_gate(S, H, A, curd, torch.sigmoid(f32(A, C)), f32(H, S), state, view, f32(A, C), f32(A, C), f32(A, C), f16(A, C), f16(H, S), f16(H, S),
+                             64e-5, att_x)
+    else:
+        gpu.FusedV7.wkv_gate(S, H, A, curd, state, view, f16(A, C), f16(A, C), f16(4, A, C), f16(H, S), f16(A, C), f16(H, S), f16(H, S), 64e-5, att_x)
+    slots = cur & 0xff
+    for slot in set(slots.tolist()):
+        last = int(np.flatnonzero(slots == slot)[-1])
+        assert torch.equal(state[slot, 0], before[last].float()), slot

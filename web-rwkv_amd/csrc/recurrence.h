@@ -75,6 +75,19 @@ __device__ __forceinline__ void store_cols(float *p, const float (&d)[N]) {
     else *p = d[0];
 }
 
+// Row 0 of a slot's state keeps the layer's input at the last token of a request; the tokens of a chunk are finished side by
+// side, so where several requests of the slot end among its `count` tokens the latest one's input is the one kept.
+__device__ __forceinline__ bool keeps_input(const uint32_t *tokens, const uint32_t *cursors, uint32_t at, uint32_t count) {
+    auto ends = [&](uint32_t j) {
+        const Cursor cur = unpack_cursor(cursors[j]);
+        return tokens[j] - min(cur.token, tokens[j]) + 1 == cur.len; // the first token clamped as in read_cursor
+    };
+    if (!ends(at)) return false;
+    for (uint32_t j = at + 1; j < count; j++)
+        if (ends(j)) return false;
+    return true;
+}
+
 // What follows the recurrence in the fused forms of a layer (head size 64): the group norm over the head and the gate.
 // att_x holds the layer's normalised input before and the gated output after.
 struct GateArgs {
@@ -138,6 +151,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
         *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
         const float b = lanes_sum<TL>(fmaf(fr.x, u4.x * fk.x, fr.y * (u4.y * fk.y)) + fmaf(fr.z, u4.z * fk.z, fr.w * (u4.w * fk.w)));
         if (tid % TL == 0) bonus[buf][lt] = b;
+        if (GATE && tid % TL == 0) csh[buf][lt] = fc, tsh[buf][lt] = ft;
         if (!GATE && tid < (uint32_t)TB) csh[buf][tid] = fc, tsh[buf][tid] = fct;
     };
     for (uint32_t i0 = 0; i0 < SZ; i0 += 64) {
@@ -165,7 +179,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
             for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
                 const int buf = chunk & 1;
                 const uint2 cg = fg, cx = fx;
-                const uint32_t cc = fc, ct = ft;
+                const uint32_t ct = ft;
                 if (chunk + 1 < nchunk) fetch(chunk + 1);
                 __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
                 const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
@@ -223,9 +237,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
                 if constexpr (GATE) {
                     __syncthreads(); // the chunk's y are in LDS
                     if (lt < tend) {
-                        Cursor cur = unpack_cursor(cc);
-                        cur.token = min(cur.token, ct); // as read_cursor
-                        if (ct - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
+                        if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
                         const float b = bonus[buf][lt];
                         const float4 o = head_norm(make_float4(fmaf(b, v4.x, y0.x), fmaf(b, v4.y, y0.y), fmaf(b, v4.z, y0.z), fmaf(b, v4.w, y0.w)), gw, gb, ga.eps);
@@ -291,6 +303,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
         *reinterpret_cast<float4 *>(&as[buf][4 * tid]) = make_float4(-fkk.x, -fkk.y, -fkk.z, -fkk.w);
         *reinterpret_cast<float4 *>(&bs[buf][4 * tid]) = make_float4(fkk.x * fa.x, fkk.y * fa.y, fkk.z * fa.z, fkk.w * fa.w);
         *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
+        if (GATE && tid % TL == 0) csh[buf][lt] = fc, tsh[buf][lt] = ft;
         if (!GATE && tid < (uint32_t)TB) csh[buf][tid] = fc, tsh[buf][tid] = fct;
     };
     for (uint32_t i0 = 0; i0 < SZ; i0 += 64) {
@@ -314,7 +327,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
             for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
                 const int buf = chunk & 1;
                 const uint2 cg = fg, cx = fx;
-                const uint32_t cc = fc, ct = ft;
+                const uint32_t ct = ft;
                 if (chunk + 1 < nchunk) fetch(chunk + 1);
                 __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
                 const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
@@ -375,9 +388,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
                 if constexpr (GATE) {
                     __syncthreads(); // the chunk's y are in LDS
                     if (lt < tend) {
-                        Cursor cur = unpack_cursor(cc);
-                        cur.token = min(cur.token, ct); // as read_cursor
-                        if (ct - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
+                        if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
                         const float4 k4 = *reinterpret_cast<const float4 *>(&ks[buf][4 * tid]), r4 = *reinterpret_cast<const float4 *>(&rs[buf][4 * tid]);
                         const float b = lanes_sum<16>((u4.x * k4.x * r4.x + u4.y * k4.y * r4.y) + (u4.z * k4.z * r4.z + u4.w * k4.w * r4.w));
