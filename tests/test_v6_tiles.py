@@ -1,0 +1,48 @@
+"""The second halves of a v6 layer's adapters in both forms: a token at a time and in tiles of 16 channels x 16 tokens, at the
+edges of the tiles and of the rule between them, against float64."""
+import importlib
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from helpers import assert_close
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C", [16, 80, 100, 256])
+@pytest.mark.parametrize("runs", [[(1, 7)], [(0, 3), (2, 5)], [(2, 1)] + [(1, 15)], [(0, 17)], [(2, 20), (0, 1), (1, 16)]], ids=lambda r: str(sum(n for _, n in r)))
+@pytest.mark.parametrize("mix_lora,decay_lora", [(32, 64), (64, 128)])
+def test_gpu_v6_tiles(gpu, C, runs, mix_lora, decay_lora):
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("v6 adapter tiles on the GPU", C, runs, mix_lora, decay_lora, flush=True)
+    B = 3
+    cur = lop.pack_cursors(runs)
+    A = len(cur)
+    g = torch.Generator().manual_seed(0x5754 + C + A)
+    h = lambda *s, std=0.3: (torch.randn(s, generator=g) * std).half()
+    lora, w2, mix, x = h(A, 5, mix_lora, std=0.5), h(5, C, mix_lora, std=0.1), torch.rand((5, C), generator=g).half(), h(A, C, std=1.0)
+    state = torch.randn((B, 66, C), generator=g)
+    dl, dw2, bias = h(A, decay_lora, std=0.5), h(C, decay_lora, std=0.1), h(C, std=0.5)
+    curd = torch.from_numpy(cur.view(np.int32)).cuda()
+    out, decay = torch.empty((5, A, C), dtype=torch.float16, device="cuda"), torch.empty((A, C), dtype=torch.float32, device="cuda")
+    gpu.FusedV6.time_mix(C, A, mix_lora, curd, lora.cuda(), w2.cuda(), mix.cuda(), state.cuda(), ((C, 65, B), (C, 66, B), (0, 0, 0)), x.cuda(), out)
+    gpu.FusedV6.decay(C, A, decay_lora, dl.cuda(), dw2.cuda(), bias.cuda(), decay)
+    prev = torch.cat([x[:1], x[:-1]]).double()
+    at = 0
+    for slot, n in runs:
+        prev[at] = state[slot, 0].double()
+        at += n
+    f = torch.einsum("ask,sck->sac", lora.double(), w2.double()) + mix.double()[:, None]
+    want = x.double() * (1 - f) + prev * f
+    # f passes through two f16 roundings (2^-11 of values up to 4 each) and meets |x| + |prev| up to 8; the output is rounded once more
+    assert_close(out.cpu().numpy(), want.numpy(), 1.6e-2, "time_mix vs float64")
+    assert float((out.cpu().double() - want).norm() / want.norm()) < 1e-3  # 2^-11 per rounding, three of them
+    want = torch.exp(-torch.exp(dl.double() @ dw2.double().t() + bias.double()))
+    assert_close(decay.cpu().numpy(), want.numpy(), 2e-6, "decay vs float64")  # sums of 128 terms in f32, two exponentials

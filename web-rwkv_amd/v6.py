@@ -7,7 +7,7 @@ import importlib
 import numpy as np
 
 _pkg = importlib.import_module(__name__.rsplit(".", 1)[0])
-LayerOp, Matrix, turbo, matmul_vec_group, FusedV6 = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group, _pkg.FusedV6
+LayerOp, Matrix, turbo, matmul_vec_group, FusedV6, FusedV7 = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group, _pkg.FusedV6, _pkg.FusedV7
 ACT_NONE, ACT_SQUARED_RELU, ACT_TANH, ACT_STABLE_EXP, ACT_SILU = _pkg.ACT_NONE, _pkg.ACT_SQUARED_RELU, _pkg.ACT_TANH, _pkg.ACT_STABLE_EXP, _pkg.ACT_SILU
 
 LN_EPS = 1.0e-5   # Model::LN_EPS, src/runtime/v6.rs:46
@@ -130,12 +130,23 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
     ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
     slice_of = lambda i: ((C, A, 1), (C, A, 5), (0, 0, i))
 
+    # First half of an adapter: the launch of small tiles where it beats the f16 product, which is a one-shot kernel up to 4
+    # tokens and splits K beyond (160 rows: 2048 channels 5.2 against 6.9 us at 5 tokens, 6.2 against 8.3 at 100; 768 channels
+    # 6.1 against 5.0 at 16, 6.2 against 8.5 at 32; 5120 channels 9.8 against 7.9 at 8, 11.4 against 10.5 at 100).
+    tiles = C <= 2560 and A > (16 if C <= 1024 else 4)
+
+    def adapter_in(name, x, out):
+        if tiles:
+            FusedV7.adapters_in(C, A, [(t[name], x, out, ACT_TANH)])
+        else:
+            m[name].matmul_op(x, out, ACT_TANH, fast)
+
     FusedV6.pre(C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state, [t["time_mix_x"]], buf.att_x, [buf.att_xx])
-    m["time_mix_w1"].matmul_op(buf.att_xx, buf.time_mix_x.view(1, A, 5 * TIME_MIX_LORA), ACT_TANH, fast)
+    adapter_in("time_mix_w1", buf.att_xx, buf.time_mix_x.view(1, A, 5 * TIME_MIX_LORA))
     FusedV6.time_mix(C, A, TIME_MIX_LORA, cursors, buf.time_mix_x, t["time_mix_w2"], t["time_mix"], state, att_state, buf.att_x, buf.att_sx)
     matmul_vec_group([(m[n], buf.att_sx, out, ACT_NONE, False, dict(input_view=slice_of(i)))
                       for n, out, i in (("att_w_k", buf.att_k, 1), ("att_w_v", buf.att_v, 2), ("att_w_r", buf.att_r, 3), ("att_w_g", buf.att_g, 4))])
-    m["time_decay_w1"].matmul_op(buf.att_sx, buf.att_w, ACT_TANH, fast, input_view=slice_of(0))
+    adapter_in("time_decay_w1", buf.att_sx[:1], buf.att_w)
     FusedV6.decay(C, A, TIME_DECAY_LORA, buf.att_w, t["time_decay_w2"], t["time_decay"], buf.time_decay)
     FusedV6.wkv_gate(S, H, A, cursors, buf.time_decay, t["time_first"], state, att_state, buf.att_k, buf.att_v, buf.att_r, buf.att_g, t["gn_w"], t["gn_b"],
                      GN_EPS, buf.att_x)
@@ -147,12 +158,12 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
     FusedV6.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_r, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now)
 
 
-FUSED_MAX_TOKENS = 16  # measured: beyond this the op list's chunked kernels win (the fused ones walk tokens one by one)
+FUSED_MAX_TOKENS = 65535  # what the fused ops take
 
 
 def dispatch_layer_auto(layer, buf, state, cursors, A, H, S, rescale_now=False):
-    """The fused form for short runs (decode and the tail of a schedule), the op list beyond."""
-    if A <= FUSED_MAX_TOKENS and S == 64:
+    """The fused form where it is built (heads of 64, up to 8192 channels), the op list otherwise."""
+    if A <= FUSED_MAX_TOKENS and S == 64 and H * S <= 8192:
         dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now)
     else:
         dispatch_layer(layer, buf, state, cursors, A, H, S, rescale_now)
