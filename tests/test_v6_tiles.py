@@ -46,3 +46,23 @@ def test_gpu_v6_tiles(gpu, C, runs, mix_lora, decay_lora):
     assert float((out.cpu().double() - want).norm() / want.norm()) < 1e-3  # 2^-11 per rounding, three of them
     want = torch.exp(-torch.exp(dl.double() @ dw2.double().t() + bias.double()))
     assert_close(decay.cpu().numpy(), want.numpy(), 2e-6, "decay vs float64")  # sums of 128 terms in f32, two exponentials
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C", [32, 2080, 2592, 4128, 8192])
+@pytest.mark.parametrize("A", [1, 17])
+def test_gpu_adapters_in_long_rows(gpu, C, A):
+    """First halves of adapters either side of the sizes where waves and steps in flight change."""
+    import torch
+
+    print("adapters_in on the GPU", C, A, flush=True)
+    g = torch.Generator().manual_seed(0x5755 + C + A)
+    h = lambda *s: (torch.randn(s, generator=g) * 0.05).half()
+    ops = [(h(16, C), h(A, C), torch.empty((A, 16), dtype=torch.float16, device="cuda"), gpu.ACT_NONE),
+           (h(48, C), h(A, C), torch.empty((A, 48), dtype=torch.float16, device="cuda"), gpu.ACT_TANH)]
+    gpu.FusedV7.adapters_in(C, A, [(w.cuda(), x.cuda(), out, act) for w, x, out, act in ops])
+    for w, x, out, act in ops:
+        want = x.double() @ w.double().t()
+        want = torch.tanh(want) if act == gpu.ACT_TANH else want
+        # f32 sums of up to 8192 products of 2.5e-3 each, one rounding to f16 (2^-11) of values below 1
+        assert_close(out.cpu().numpy(), want.numpy(), 1e-3, "adapters_in vs float64")

@@ -24,7 +24,6 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxAdapters = 4;
-constexpr int kAdapterWaves = 8;
 struct AdapterArgs {
     const uint16_t *w[kMaxAdapters], *x[kMaxAdapters];
     uint16_t *out[kMaxAdapters];
@@ -34,11 +33,12 @@ struct AdapterArgs {
 
 // First halves of a layer's low-rank adapters, out[t][r] = f16(act(sum_k w[r][k] x[t][k])): a few dozen rows over K = C
 // per adapter, so the product is one short pass over weights that fit in the caches and its time is latency.  One workgroup
-// per 16 rows x 16 tokens of any adapter of the layer; its eight waves take every eighth 32-element step of K, straight from
-// memory in the operand layout of the 16x16x32 MFMA, eight steps in flight, and add up through LDS.  2048 channels, 32 tokens, four adapters: 7 us
+// per 16 rows x 16 tokens of any adapter of the layer; its WAVES waves take every WAVES-th 32-element step of K, straight from
+// memory in the operand layout of the 16x16x32 MFMA, Q steps in flight, and add up through LDS.  2048 channels, 32 tokens, four adapters: 7 us
 // in one launch, against 4 x (5 + 3) us for products split over K and summed by a second launch each.
-__global__ __launch_bounds__(64 * kAdapterWaves) void adapters_in_kernel(uint32_t K, uint32_t T, AdapterArgs aa) {
-    __shared__ float4 red[kAdapterWaves - 1][64];
+template <int WAVES, int Q>
+__global__ __launch_bounds__(64 * WAVES) void adapters_in_kernel(uint32_t K, uint32_t T, AdapterArgs aa) {
+    __shared__ float4 red[WAVES - 1][64];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
     uint32_t p = 0;
 #pragma unroll
@@ -49,22 +49,22 @@ __global__ __launch_bounds__(64 * kAdapterWaves) void adapters_in_kernel(uint32_
     const uint16_t *wp = aa.w[p] + (uint64_t)(row0 + r16) * K + 8 * g;
     const uint16_t *xp = aa.x[p] + (uint64_t)min(t0 + r16, T - 1) * K + 8 * g; // columns past the run repeat its last token, never stored
     float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s0 = wave; s0 < steps; s0 += 8 * kAdapterWaves) {
-        uint4 a[8], b[8];
+    for (uint32_t s0 = wave; s0 < steps; s0 += Q * WAVES) {
+        uint4 a[Q], b[Q];
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const uint32_t at = 32 * min(s0 + q * kAdapterWaves, steps - 1);
+        for (int q = 0; q < Q; q++) {
+            const uint32_t at = 32 * min(s0 + q * WAVES, steps - 1);
             a[q] = load128(wp + at), b[q] = load128(xp + at);
         }
 #pragma unroll
-        for (int q = 0; q < 8; q++)
-            if (s0 + q * kAdapterWaves < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[q]), __builtin_bit_cast(half8, b[q]), acc, 0, 0, 0);
+        for (int q = 0; q < Q; q++)
+            if (s0 + q * WAVES < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[q]), __builtin_bit_cast(half8, b[q]), acc, 0, 0, 0);
     }
     if (wave) red[wave - 1][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
     __syncthreads();
     if (wave) return;
 #pragma unroll
-    for (int w = 0; w < kAdapterWaves - 1; w++) {
+    for (int w = 0; w < WAVES - 1; w++) {
         const float4 v = red[w][lane];
         acc[0] += v.x, acc[1] += v.y, acc[2] += v.z, acc[3] += v.w;
     }
@@ -384,7 +384,10 @@ int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void
         aa.rank[i] = ranks[i], aa.act[i] = acts[i];
         tiles += ranks[i] / 16;
     }
-    hipLaunchKernelGGL(adapters_in_kernel, dim3(tiles, (A + 15) / 16), dim3(64 * kAdapterWaves), 0, static_cast<hipStream_t>(stream), C, A, aa);
+    // Ten steps in flight where eight waves then take K in one go (2560 channels, 160 rows, 100 tokens: 9.7 -> 7.1 us), and
+    // sixteen waves of ten beyond 4096 channels (5120: 13.1 -> 11.5 us; at 4096 sixteen waves of eight steps gained nothing: 9.7 us).
+    auto go = [&](auto kern, int waves) { hipLaunchKernelGGL(kern, dim3(tiles, (A + 15) / 16), dim3(64 * waves), 0, static_cast<hipStream_t>(stream), C, A, aa); };
+    C > 4096 ? go(adapters_in_kernel<16, 10>, 16) : C > 2048 && C <= 2560 ? go(adapters_in_kernel<8, 10>, 8) : go(adapters_in_kernel<8, 8>, 8);
     return check_launch(what);
 }
 
