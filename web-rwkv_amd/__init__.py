@@ -462,44 +462,75 @@ class LayerOp:
                               C.byref(as_view(factor, factor_view)), int(reversed)))
 
 
+def _operands(what, A, cursors, f16=(), f32=()):
+    """What the C entry points of the fused ops cannot see behind a bare pointer: a cursor per token, and of every
+    `(tensor, elements)` the element type and that the tensor holds that many."""
+    import torch
+
+    if cursors is not None:
+        assert cursors.is_contiguous()
+        if cursors.numel() * cursors.element_size() < 4 * A:
+            raise TensorError(ERR_SHAPE, f"{what}: {cursors.numel()} cursors for {A} tokens")
+    for dtype, operands in ((torch.float16, f16), (torch.float32, f32)):
+        for t, n in operands:
+            if t is None:
+                continue  # refused by the library where it is needed
+            assert t.is_contiguous()
+            if t.dtype != dtype:
+                raise TensorError(ERR_TYPE, f"{what}: an operand of {t.dtype}, {dtype} is built")
+            if t.numel() < n:
+                raise TensorError(ERR_SHAPE, f"{what}: an operand of {t.numel()} elements, {n} are needed")
+
+
 class FusedV6:
-    """The fused forms of a v6 layer's small ops (`wrq_v6_*`); arguments are contiguous torch tensors."""
+    """The fused forms of a v6 layer's small ops (`wrq_v6_*`); arguments are contiguous torch tensors of the types and
+    sizes in `include/wrq.h`."""
 
     @staticmethod
     def _p(t):
         return None if t is None else C.c_void_p(t.data_ptr())
 
     @staticmethod
+    def _check_pre(what, Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts):
+        rows = [x, ln_out, *shifts] + ([add, x_out] if add is not None else [])
+        _operands(what, A, cursors, [(t, A * Cn) for t in rows] + [(t, Cn) for t in (ln_w, ln_b, *factors)])
+
+    @staticmethod
     def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts):
         p = FusedV6._p
+        FusedV6._check_pre("v6_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
         _check(lib().wrq_v6_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
                                 p(factors[0]), p(factors[1] if len(factors) > 1 else None), p(ln_out), p(shifts[0]), p(shifts[1] if len(shifts) > 1 else None)))
 
     @staticmethod
     def time_mix(Cn, A, lora_size, cursors, lora, w2, time_mix, state, state_view, att_x, att_sx):
-        p = FusedV6._p
+        p, r, n = FusedV6._p, lora_size, A * Cn
+        _operands("v6_time_mix", A, cursors, ((lora, 5 * A * r), (w2, 5 * Cn * r), (time_mix, 5 * Cn), (att_x, n), (att_sx, 5 * n)))
         _check(lib().wrq_v6_time_mix(_stream(), Cn, A, lora_size, p(cursors), p(lora), p(w2), p(time_mix), C.byref(as_view(state, state_view)), p(att_x), p(att_sx)))
 
     @staticmethod
     def decay(Cn, A, lora_size, lora, w2, time_decay, out):
-        p = FusedV6._p
+        p, r = FusedV6._p, lora_size
+        _operands("v6_decay", A, None, ((lora, A * r), (w2, Cn * r), (time_decay, Cn)), ((out, A * Cn),))
         _check(lib().wrq_v6_decay(_stream(), Cn, A, lora_size, p(lora), p(w2), p(time_decay), p(out)))
 
     @staticmethod
     def wkv_gate(S, H, A, cursors, time_decay, time_first, state, state_view, k, v, r, g, gn_w, gn_b, eps, att_x):
-        p = FusedV6._p
+        p, n = FusedV6._p, A * S * H
+        _operands("v6_wkv_gate", A, cursors, ((g, n), (gn_w, S * H), (gn_b, S * H), (att_x, n)), ((time_decay, n), (time_first, S * H), (k, n), (v, n), (r, n)))
         _check(lib().wrq_v6_wkv_gate(_stream(), S, H, A, p(cursors), p(time_decay), p(time_first), C.byref(as_view(state, state_view)), p(k), p(v), p(r), p(g),
                                      p(gn_w), p(gn_b), eps, p(att_x)))
 
     @staticmethod
     def post_ffn(Cn, A, cursors, state, state_view, r, v, ffn_x, x_in, x_out, rescale):
-        p = FusedV6._p
+        p, n = FusedV6._p, A * Cn
+        _operands("v6_post_ffn", A, cursors, ((r, n), (v, n), (ffn_x, n), (x_in, n), (x_out, n)))
         _check(lib().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
 
 
 class FusedV7:
     """The fused forms of a v7 layer's small ops (`wrq_fused_pre`, `wrq_adapters_in`, `wrq_v7_*`); arguments are contiguous
-    torch tensors.  `adapters_in` serves any layer with low-rank adapters."""
+    torch tensors of the types and sizes in `include/wrq.h`.  `adapters_in` serves any layer with low-rank adapters."""
 
     @staticmethod
     def _a(ts):
@@ -508,6 +539,9 @@ class FusedV7:
     @staticmethod
     def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts):
         p, a = FusedV6._p, FusedV7._a
+        FusedV6._check_pre("fused_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
+        if len(shifts) < len(factors):
+            raise TensorError(ERR_SHAPE, f"fused_pre: {len(shifts)} outputs for {len(factors)} token shifts")
         _check(lib().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
                                    a(factors), p(ln_out), a(shifts)))
 
@@ -516,23 +550,30 @@ class FusedV7:
         """`ops`: list of `(w, x, out, act)`, w [rank, C]."""
         a, n = FusedV7._a, len(ops)
         w, x, out, act = zip(*ops)
+        _operands("adapters_in", A, None, [(t, A * Cn) for t in x] + [(t, t.shape[0] * Cn) for t in w] + [(o, A * t.shape[0]) for o, t in zip(out, w)])
         _check(lib().wrq_adapters_in(_stream(), Cn, A, n, a(w), (C.c_uint32 * n)(*(t.shape[0] for t in w)), (C.c_int * n)(*act), a(x), a(out)))
 
     @staticmethod
     def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n):
-        p, a = FusedV6._p, FusedV7._a
+        p, a, Cn = FusedV6._p, FusedV7._a, S * H
+        if len(aux) != 4 or len(w2) != 4 or len(vectors) != 5:
+            raise TensorError(ERR_SHAPE, f"v7_mid: {len(aux)}, {len(w2)} and {len(vectors)} operands, 4, 4 and 5 are needed")
+        _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2)] + [(w, Cn * w.shape[1]) for w in w2] + [(t, Cn) for t in vectors]
+                  + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g)] + [(n, 4 * A * Cn)])
         ranks = (C.c_uint32 * 4)(*(t.shape[1] for t in w2))
         _check(lib().wrq_v7_mid(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n)))
 
     @staticmethod
     def wkv_gate(S, H, A, cursors, state, state_view, r, w, n, r_k, g, gn_w, gn_b, eps, att_x):
-        p = FusedV6._p
+        p, m = FusedV6._p, A * S * H
+        _operands("v7_wkv_gate", A, cursors, ((r, m), (w, m), (n, 4 * m), (r_k, S * H), (g, m), (gn_w, S * H), (gn_b, S * H), (att_x, m)))
         _check(lib().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
                                      p(att_x)))
 
     @staticmethod
     def post_ffn(Cn, A, cursors, state, state_view, v, ffn_x, x_in, x_out, rescale):
-        p = FusedV6._p
+        p, n = FusedV6._p, A * Cn
+        _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n)))
         _check(lib().wrq_v7_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
 
 
