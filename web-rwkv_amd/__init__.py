@@ -482,6 +482,25 @@ def _operands(what, A, cursors, f16=(), f32=()):
                 raise TensorError(ERR_SHAPE, f"{what}: an operand of {t.numel()} elements, {n} are needed")
 
 
+def fused_operands(f16, f32=(), adapters=()):
+    """Whether a layer's operands have the types and sizes its fused form is built for: lists of `(tensor, elements)` and of
+    `(matrix, rows, columns)` of low-rank adapters.  The op list takes more (f32 vectors and buffers, packed adapters) and
+    refuses the rest op by op, so what is not built goes there."""
+    import torch
+
+    for dtype, operands in ((torch.float16, f16), (torch.float32, f32)):
+        for t, n in operands:
+            if t is None or t.dtype != dtype or t.numel() != n or not t.is_contiguous():
+                return False
+    return all(m.kind == "Fp16" and m.w.dtype == torch.float16 and m.w.numel() == rows * columns and m.w.shape[-1] == columns and m.w.is_contiguous()
+               for m, rows, columns in adapters)
+
+
+def fused_run(cursors, A):
+    """Whether the fused forms take a run of `A` tokens with these cursors."""
+    return A <= 65535 and cursors.is_contiguous() and shape_of(cursors)[0] >= A
+
+
 class FusedV6:
     """The fused forms of a v6 layer's small ops (`wrq_v6_*`); arguments are contiguous torch tensors of the types and
     sizes in `include/wrq.h`."""

@@ -7,7 +7,7 @@ import importlib
 import numpy as np
 
 _pkg = importlib.import_module(__name__.rsplit(".", 1)[0])
-LayerOp, Matrix, turbo, matmul_vec_group, FusedV6, FusedV7 = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group, _pkg.FusedV6, _pkg.FusedV7
+LayerOp, Matrix, turbo, matmul_vec_group, FusedV6, FusedV7, fused_operands, fused_run = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group, _pkg.FusedV6, _pkg.FusedV7, _pkg.fused_operands, _pkg.fused_run
 ACT_NONE, ACT_SQUARED_RELU, ACT_TANH, ACT_STABLE_EXP, ACT_SILU = _pkg.ACT_NONE, _pkg.ACT_SQUARED_RELU, _pkg.ACT_TANH, _pkg.ACT_STABLE_EXP, _pkg.ACT_SILU
 
 LN_EPS = 1.0e-5   # Model::LN_EPS, src/runtime/v6.rs:46
@@ -159,11 +159,27 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
 
 
 FUSED_MAX_TOKENS = 65535  # what the fused ops take
+VECTORS = ("att_ln_w", "att_ln_b", "ffn_ln_w", "ffn_ln_b", "time_mix_x", "time_decay", "gn_w", "gn_b", "ffn_time_mix_k", "ffn_time_mix_r")
+FUSED_ROWS = ("x", "x2", "att_x", "att_xx", "att_g", "att_o", "ffn_x", "ffn_kx", "ffn_rx", "ffn_v", "ffn_r")
+
+
+def fused_is_built(layer, buf, cursors, A, H, S):
+    """Whether the fused form takes this run of this layer: heads of 64, up to 8192 channels, adapters of the sizes above,
+    vectors and buffers of the types `Layer` and `Runtime` give them."""
+    t, m, C = layer.t, layer.m, H * S
+    if S != 64 or C > 8192 or not fused_run(cursors, A):
+        return False
+    n, mix, decay = A * C, TIME_MIX_LORA, TIME_DECAY_LORA
+    rows = lambda names, size: [(getattr(buf, name, None), size) for name in names]  # None: buffers made for the op list alone have no x2
+    f16 = [(t[name], C) for name in VECTORS] + [(t["time_mix"], 5 * C)]
+    f16 += rows(FUSED_ROWS, n) + rows(("att_sx",), 5 * n) + rows(("time_mix_x",), 5 * mix * A) + rows(("att_w",), decay * A)
+    f32 = [(t["time_first"], C)] + rows(("att_k", "att_v", "att_r", "time_decay"), n)
+    return fused_operands(f16, f32, [(m["time_mix_w1"], 5 * mix, C), (m["time_mix_w2"], 5 * C, mix), (m["time_decay_w1"], decay, C), (m["time_decay_w2"], C, decay)])
 
 
 def dispatch_layer_auto(layer, buf, state, cursors, A, H, S, rescale_now=False):
-    """The fused form where it is built (heads of 64, up to 8192 channels), the op list otherwise."""
-    if A <= FUSED_MAX_TOKENS and S == 64 and H * S <= 8192:
+    """The fused form where it is built (`fused_is_built`), the op list otherwise."""
+    if A <= FUSED_MAX_TOKENS and fused_is_built(layer, buf, cursors, A, H, S):
         dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now)
     else:
         dispatch_layer(layer, buf, state, cursors, A, H, S, rescale_now)

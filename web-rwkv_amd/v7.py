@@ -7,7 +7,7 @@ import importlib
 import numpy as np
 
 _pkg = importlib.import_module(__name__.rsplit(".", 1)[0])
-LayerOp, FusedV7, Matrix, turbo, matmul_vec_group = _pkg.LayerOp, _pkg.FusedV7, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group
+LayerOp, FusedV7, fused_operands, fused_run, Matrix, turbo, matmul_vec_group = _pkg.LayerOp, _pkg.FusedV7, _pkg.fused_operands, _pkg.fused_run, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group
 ACT_NONE, ACT_SQUARED_RELU, ACT_TANH, ACT_SIGMOID = _pkg.ACT_NONE, _pkg.ACT_SQUARED_RELU, _pkg.ACT_TANH, _pkg.ACT_SIGMOID
 
 L2_EPS = 1.0e-12  # Model::L2_EPS, src/runtime/v7.rs:46
@@ -17,6 +17,9 @@ RANK_W, RANK_A, RANK_G, RANK_V = 64, 64, 128, 32  # inner sizes of the four adap
 
 QUANTIZED = ("att_w_r", "att_w_k", "att_w_v", "att_w_o", "ffn_w_k", "ffn_w_v")
 ADAPTERS = ("w1", "w2", "a1", "a2", "g1", "g2", "v1", "v2")
+VECTORS = ("att_ln_w", "att_ln_b", "ffn_ln_w", "ffn_ln_b", "x_r", "x_w", "x_k", "x_v", "x_a", "x_g", "ffn_x_k", "w0", "a0", "v0", "k_k", "k_a", "r_k", "gn_w", "gn_b")
+SHIFTED = ("att_rx", "att_wx", "att_kx", "att_vx", "att_ax", "att_gx")
+FUSED_ROWS = ("x", "x2", "att_x", "att_v0", "att_r", "att_w", "att_k", "att_v", "att_g", "att_o", "ffn_x", "ffn_kx", "ffn_v")
 
 
 def random_layer_weights(rng, C, H, S, hidden):
@@ -84,18 +87,30 @@ class PackedShifts:
 def dispatch_layer(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
     """src/runtime/v7.rs:704-1006.  `state`: this layer's f32 tensor (B, S + 2, C): rows 0..S the
     attention state, row S + 1 the feed-forward one; `index`: the layer's number (layer 0 keeps its
-    values as `att_v0`, the later ones mix theirs with it).  The fused form where it is built (every v7 model has
-    heads of 64; adapters of the sizes above and up to 8192 channels), the op list otherwise."""
-    if fused_is_built(layer, H, S):
+    values as `att_v0`, the later ones mix theirs with it).  The fused form where it is built (`fused_is_built`:
+    heads of 64, up to 8192 channels, adapters of the sizes above, f16 vectors and buffers), the op list otherwise."""
+    if fused_is_built(layer, H, S, buf, cursors, A, shifts):
         dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts)
     else:
         dispatch_layer_ops(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts)
 
 
-def fused_is_built(layer, H, S):
-    t = layer.t
-    ranks = tuple(t[n].shape[0] for n in ("w1", "a1", "g1", "v1"))
-    return S == 64 and H * S <= 8192 and ranks == (64, 64, 128, 32)
+def fused_is_built(layer, H, S, buf=None, cursors=None, A=None, shifts=None):
+    """Whether the fused form takes this layer, and with `buf`, `cursors` and `A` whether it takes this run."""
+    t, m, C = layer.t, layer.m, H * S
+    if S != 64 or C > 8192:
+        return False
+    ranks = (("w", RANK_W), ("a", RANK_A), ("g", RANK_G), ("v", RANK_V))
+    adapters = [(m[n + "1"], r, C) for n, r in ranks] + [(m[n + "2"], C, r) for n, r in ranks]
+    vectors = [(t.get(n), C) for n in VECTORS]
+    if buf is None:
+        return fused_operands(vectors, adapters=adapters)
+    n = A * C
+    rows = [(name, n) for name in FUSED_ROWS + (SHIFTED if shifts is None else ())] + [("aux_" + name, A * r) for name, r in ranks] + [("att_n", 4 * n)]
+    rows = [(getattr(buf, name, None), size) for name, size in rows]  # None: buffers made for the op list alone have no x2
+    if shifts is not None:
+        rows += [(shifts.mix, 6 * n), (shifts.sx, 6 * n)]
+    return fused_operands(vectors + rows, adapters=adapters) and fused_run(cursors, A)
 
 
 def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
