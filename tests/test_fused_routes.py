@@ -107,6 +107,36 @@ def test_other_heads_take_the_op_list(wrq, monkeypatch, version):
     assert route(monkeypatch, mod, version, layer, buf, cursors, heads=129)[-1] == "list"
 
 
+@pytest.mark.parametrize("version,names", [(6, ("time_mix_w1", "time_mix_w2", "time_decay_w1", "time_decay_w2")), (7, ("w1", "w2", "a1", "a2", "g1", "g2", "v1", "v2"))])
+def test_fused_form_takes_the_adapters_of_the_matrices(wrq, monkeypatch, version, names):
+    # an adapter replaced in `layer.m`, as the op list reads it, and not the tensor it was made from
+    A = 20
+    mod, layer, buf, cursors = setup(wrq, version, A)
+    fresh = {}
+    for n in names:
+        fresh[n] = layer.m[n] = wrq.Matrix.fp16(torch.ones_like(layer.t[n]))
+    seen = []
+    for cls in ("FusedV6", "FusedV7"):
+        if hasattr(mod, cls):
+            recorder = type("R", (), {n: staticmethod(lambda *a: seen.append(a)) for n in ("pre", "time_mix", "decay", "wkv_gate", "post_ffn", "adapters_in", "mid")})
+            monkeypatch.setattr(mod, cls, recorder)
+    monkeypatch.setattr(mod, "matmul_vec_group", lambda ops: None)
+    monkeypatch.setattr(wrq.Matrix, "matmul_op", lambda self, *a, **k: seen.append((self.w, a)))
+    monkeypatch.setattr(wrq.Matrix, "matmul_op_sparse", lambda self, *a, **k: None)
+    mod.dispatch_layer_fused(layer, buf, torch.zeros((1, 66, 64)), cursors, A, 1, 64, *([1] if version == 7 else []))
+
+    def tensors(a):
+        if torch.is_tensor(a):
+            yield a.data_ptr()
+        elif isinstance(a, (list, tuple)):
+            for e in a:
+                yield from tensors(e)
+
+    used = set(tensors(seen))
+    for n in names:
+        assert fresh[n].w.data_ptr() in used and layer.t[n].data_ptr() not in used, n
+
+
 def test_wrappers_refuse_what_the_library_cannot_see(wrq):
     h = lambda *s: torch.zeros(s, dtype=torch.float16)
     A, C, S = 4, 64, 64

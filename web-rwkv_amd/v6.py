@@ -137,17 +137,17 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
 
     def adapter_in(name, x, out):
         if tiles:
-            FusedV7.adapters_in(C, A, [(t[name], x, out, ACT_TANH)])
+            FusedV7.adapters_in(C, A, [(m[name].w, x, out, ACT_TANH)])
         else:
             m[name].matmul_op(x, out, ACT_TANH, fast)
 
     FusedV6.pre(C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state, [t["time_mix_x"]], buf.att_x, [buf.att_xx])
     adapter_in("time_mix_w1", buf.att_xx, buf.time_mix_x.view(1, A, 5 * TIME_MIX_LORA))
-    FusedV6.time_mix(C, A, TIME_MIX_LORA, cursors, buf.time_mix_x, t["time_mix_w2"], t["time_mix"], state, att_state, buf.att_x, buf.att_sx)
+    FusedV6.time_mix(C, A, TIME_MIX_LORA, cursors, buf.time_mix_x, m["time_mix_w2"].w, t["time_mix"], state, att_state, buf.att_x, buf.att_sx)
     matmul_vec_group([(m[n], buf.att_sx, out, ACT_NONE, False, dict(input_view=slice_of(i)))
                       for n, out, i in (("att_w_k", buf.att_k, 1), ("att_w_v", buf.att_v, 2), ("att_w_r", buf.att_r, 3), ("att_w_g", buf.att_g, 4))])
     adapter_in("time_decay_w1", buf.att_sx[:1], buf.att_w)
-    FusedV6.decay(C, A, TIME_DECAY_LORA, buf.att_w, t["time_decay_w2"], t["time_decay"], buf.time_decay)
+    FusedV6.decay(C, A, TIME_DECAY_LORA, buf.att_w, m["time_decay_w2"].w, t["time_decay"], buf.time_decay)
     FusedV6.wkv_gate(S, H, A, cursors, buf.time_decay, t["time_first"], state, att_state, buf.att_k, buf.att_v, buf.att_r, buf.att_g, t["gn_w"], t["gn_b"],
                      GN_EPS, buf.att_x)
     m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)

@@ -132,9 +132,10 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now
                 [t[n] for n in PackedShifts.NAMES], buf.att_x, [rx, wx, kx, vx, ax, gx])
     matmul_vec_group([(m["att_w_r"], rx, buf.att_r, ACT_NONE, False, {}), (m["att_w_k"], kx, buf.att_k, ACT_NONE, False, {}),
                       (m["att_w_v"], vx, buf.att_v, ACT_NONE, False, {})])
-    adapters = [(t["w1"], wx, buf.aux_w, ACT_TANH), (t["a1"], ax, buf.aux_a, ACT_NONE), (t["g1"], gx, buf.aux_g, ACT_SIGMOID), (t["v1"], vx, buf.aux_v, ACT_NONE)]
+    w = {n: m[n].w for n in ADAPTERS}
+    adapters = [(w["w1"], wx, buf.aux_w, ACT_TANH), (w["a1"], ax, buf.aux_a, ACT_NONE), (w["g1"], gx, buf.aux_g, ACT_SIGMOID), (w["v1"], vx, buf.aux_v, ACT_NONE)]
     FusedV7.adapters_in(C, A, adapters[:3] if index == 0 else adapters)
-    FusedV7.mid(S, H, A, index == 0, [buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v], [t["w2"], t["a2"], t["g2"], t["v2"]],
+    FusedV7.mid(S, H, A, index == 0, [buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v], [w["w2"], w["a2"], w["g2"], w["v2"]],
                 [t["w0"], t["a0"], t["v0"], t["k_k"], t["k_a"]], L2_EPS, buf.att_k, buf.att_v, buf.att_v0, buf.att_w, buf.att_g, buf.att_n)
     FusedV7.wkv_gate(S, H, A, cursors, state, att_state, buf.att_r, buf.att_w, buf.att_n, t["r_k"], buf.att_g, t["gn_w"], t["gn_b"], GN_EPS, buf.att_x)
     m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)
