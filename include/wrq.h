@@ -450,6 +450,9 @@ int wrq_v6_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *curso
  *   vectors: w0, a0, v0, k_k, k_a; `first`: the layer whose values att_v0 keeps (no adapter v).  k and v are not written.
  * wrq_v7_wkv_gate: time_mix_v7 + group_norm + time_first_v7 + mul(g); att_x f16 in (the normalised layer input) and out.
  * wrq_v7_post_ffn: channel_mix_v7 + add (+ affine(0.5) when `rescale`); x_in, ffn_x and v are not written.
+ * wrq_v7_mid_buffers, wrq_v7_post_ffn_buffers: the same, also filling what the op list leaves in its own buffers: `buffers`
+ *   is a host array of att_k (after control_k_v7), att_v (mixed), att_a, att_kk and att_vv (the mix factor; not with `first`),
+ *   f16 [C, A] each or null, of which att_k may be k and att_v may be v; ffn_out f16 [C, A] or null <- v, may be ffn_x.
  */
 int wrq_fused_pre(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const void *x, const void *add,
                   void *x_out, const void *ln_w, const void *ln_b, float eps, const wrq_tensor_view *state, int shifts,
@@ -459,11 +462,18 @@ int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void
 int wrq_v7_mid(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first, const uint32_t *ranks,
                const void *const *aux, const void *const *w2, const void *const *vectors, float eps, const void *k,
                const void *v, void *att_v0, void *att_w, void *att_g, void *n);
+int wrq_v7_mid_buffers(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first, const uint32_t *ranks,
+                       const void *const *aux, const void *const *w2, const void *const *vectors, float eps,
+                       const void *k, const void *v, void *att_v0, void *att_w, void *att_g, void *n,
+                       void *const *buffers);
 int wrq_v7_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const void *cursors,
                     const wrq_tensor_view *state, const void *r, const void *w, const void *n, const void *r_k,
                     const void *g, const void *gn_w, const void *gn_b, float eps, void *att_x);
 int wrq_v7_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const wrq_tensor_view *state,
                     const void *v, const void *ffn_x, const void *x_in, void *x_out, int rescale);
+int wrq_v7_post_ffn_buffers(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors,
+                            const wrq_tensor_view *state, const void *v, const void *ffn_x, const void *x_in,
+                            void *x_out, int rescale, void *ffn_out);
 
 #ifdef __cplusplus
 }

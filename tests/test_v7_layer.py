@@ -168,3 +168,42 @@ def test_v7_layer_fused_equals_op_list(gpu, runs, H):
             outs.append((buf.x.cpu().numpy(), sd.cpu().numpy(), buf.att_v0.cpu().numpy()))
         for i, what in enumerate(("layer output", "state", "first layer's values")):
             assert_close(outs[1][i], outs[0][i], 4e-3, f"{what}, fused vs op list")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True], ids=["six shifts", "packed shifts"])
+@pytest.mark.parametrize("runs", [[(4, 1)], [(2, 3), (0, 13), (5, 1)], [(1, 20), (3, 13)]], ids=["1 token", "17 tokens", "33 tokens"])
+def test_v7_dispatch_leaves_the_buffers_of_the_op_list(gpu, runs, packed):
+    # every buffer of the run, not the layer's output alone: a caller may read any of them behind `dispatch_layer`.
+    # The bound is that of the fused layer against the op list above
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    v7 = importlib.import_module(gpu.__name__ + ".v7")
+    print("v7 layer, buffers", runs, packed, flush=True)
+    H, S, hidden, B = 3, 64, 256, 6
+    C = H * S
+    rng = np.random.default_rng(SEED + 130 + len(runs))
+    cursors = lop.pack_cursors(runs)
+    A = len(cursors)
+    curd = torch.from_numpy(cursors.view(np.int32)).cuda()
+    layer = v7.Layer(torch, v7.random_layer_weights(rng, C, H, S, hidden), "int8")
+    x, v0 = (rng.standard_normal((1, A, C)).astype(np.float16) for _ in range(2))
+    state = (0.1 * rng.standard_normal((B, S + 2, C))).astype(np.float32)
+    for index in (0, 1):
+        outs = []
+        for dispatch in (v7.dispatch_layer_ops, v7.dispatch_layer):
+            buf = v7.Runtime(torch, C, hidden, A)
+            assert v7.fused_is_built(layer, H, S, buf, curd, A)
+            buf.x.copy_(torch.from_numpy(x).cuda())
+            buf.att_v0.copy_(torch.from_numpy(v0).cuda())
+            shifts = v7.PackedShifts(torch, layer, A) if packed else None
+            dispatch(layer, buf, torch.from_numpy(state.copy()).cuda(), curd, A, H, S, index, shifts=shifts)
+            torch.cuda.synchronize()
+            named = {name: t for name, t in vars(buf).items() if name != "x2"}
+            if packed:
+                named["sx"] = shifts.sx
+            outs.append({name: t.cpu().numpy() for name, t in named.items()})
+        for name in outs[0]:
+            assert_close(outs[1][name], outs[0][name], 4e-3, f"{name} of layer {index}")

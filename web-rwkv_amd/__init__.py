@@ -49,7 +49,8 @@ EXPORTS = [
     "wrq_l2_norm", "wrq_control_k_v7", "wrq_time_mix_v7", "wrq_time_first_v7", "wrq_channel_mix_v7",
     "wrq_recenter", "wrq_rms_norm", "wrq_broadcast", "wrq_blend", "wrq_blend_lora",
     "wrq_v6_pre", "wrq_v6_time_mix", "wrq_v6_decay", "wrq_v6_wkv_gate", "wrq_v6_post_ffn",
-    "wrq_fused_pre", "wrq_adapters_in", "wrq_v7_mid", "wrq_v7_wkv_gate", "wrq_v7_post_ffn",
+    "wrq_fused_pre", "wrq_adapters_in", "wrq_v7_mid", "wrq_v7_wkv_gate", "wrq_v7_post_ffn", "wrq_v7_mid_buffers",
+    "wrq_v7_post_ffn_buffers",
 ]
 MAX_GROUP = 8
 
@@ -229,8 +230,10 @@ def lib():
         L.wrq_fused_pre.argtypes = [vp, u, u, vp, vp, vp, vp, vp, vp, C.c_float, V, i, P, vp, P]
         L.wrq_adapters_in.argtypes = [vp, u, u, i, P, C.POINTER(u), C.POINTER(i), P, P]
         L.wrq_v7_mid.argtypes = [vp, u, u, u, i, C.POINTER(u), P, P, P, C.c_float, vp, vp, vp, vp, vp, vp]
+        L.wrq_v7_mid_buffers.argtypes = L.wrq_v7_mid.argtypes + [P]
         L.wrq_v7_wkv_gate.argtypes = [vp, u, u, u, vp, V, vp, vp, vp, vp, vp, vp, vp, C.c_float, vp]
         L.wrq_v7_post_ffn.argtypes = [vp, u, u, vp, V, vp, vp, vp, vp, i]
+        L.wrq_v7_post_ffn_buffers.argtypes = L.wrq_v7_post_ffn.argtypes + [vp]
         for name in EXPORTS:
             if name not in ("wrq_status_string", "wrq_last_error"):
                 getattr(L, name).restype = i
@@ -573,14 +576,15 @@ class FusedV7:
         _check(lib().wrq_adapters_in(_stream(), Cn, A, n, a(w), (C.c_uint32 * n)(*(t.shape[0] for t in w)), (C.c_int * n)(*act), a(x), a(out)))
 
     @staticmethod
-    def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n):
+    def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n, buffers=(None,) * 5):
         p, a, Cn = FusedV6._p, FusedV7._a, S * H
-        if len(aux) != 4 or len(w2) != 4 or len(vectors) != 5:
-            raise TensorError(ERR_SHAPE, f"v7_mid: {len(aux)}, {len(w2)} and {len(vectors)} operands, 4, 4 and 5 are needed")
+        if len(aux) != 4 or len(w2) != 4 or len(vectors) != 5 or len(buffers) != 5:
+            raise TensorError(ERR_SHAPE, f"v7_mid: {len(aux)}, {len(w2)}, {len(vectors)} and {len(buffers)} operands, 4, 4, 5 and 5 are needed")
         _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2)] + [(w, Cn * w.shape[1]) for w in w2] + [(t, Cn) for t in vectors]
-                  + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g)] + [(n, 4 * A * Cn)])
+                  + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g, *buffers)] + [(n, 4 * A * Cn)])
         ranks = (C.c_uint32 * 4)(*(t.shape[1] for t in w2))
-        _check(lib().wrq_v7_mid(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n)))
+        _check(lib().wrq_v7_mid_buffers(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n),
+                                        a(buffers)))
 
     @staticmethod
     def wkv_gate(S, H, A, cursors, state, state_view, r, w, n, r_k, g, gn_w, gn_b, eps, att_x):
@@ -590,10 +594,11 @@ class FusedV7:
                                      p(att_x)))
 
     @staticmethod
-    def post_ffn(Cn, A, cursors, state, state_view, v, ffn_x, x_in, x_out, rescale):
+    def post_ffn(Cn, A, cursors, state, state_view, v, ffn_x, x_in, x_out, rescale, ffn_out=None):
         p, n = FusedV6._p, A * Cn
-        _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n)))
-        _check(lib().wrq_v7_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
+        _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n), (ffn_out, n)))
+        _check(lib().wrq_v7_post_ffn_buffers(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale),
+                                             p(ffn_out)))
 
 
 def matmul_vec_group(ops):

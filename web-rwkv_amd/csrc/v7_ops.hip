@@ -82,6 +82,7 @@ struct MidArgs {
     const uint16_t *w0, *a0, *v0, *k_k, *k_a;                      // [C]
     const uint16_t *k, *v;                                         // [T, C]
     uint16_t *att_v0, *att_w, *att_g, *n;                          // [T, C], n: [4, T, C]
+    uint16_t *att_k, *att_v, *att_a, *att_kk, *att_vv;             // [T, C] or null: the list's buffers; att_k and att_v may be k and v
 };
 
 // Second halves of the four adapters and what a v7 layer makes of them before the recurrence.  A workgroup takes one head
@@ -127,9 +128,9 @@ __global__ __launch_bounds__(256) void v7_mid_kernel(uint32_t C, uint32_t T, flo
     const float4 w = each([](float bias, float y, float) { return bias + y; }, w0, product(0, NW), w0);
     const float4 a = each(sigmoid_sum, a0, product(NW, NA), a0);
     const float4 gate = product(NW + NA, NG);
-    float4 vm = v;
+    float4 vm = v, f = v;
     if constexpr (!FIRST) {
-        const float4 f = each(sigmoid_sum, v0, product(NW + NA + NG, NV), v0);
+        f = each(sigmoid_sum, v0, product(NW + NA + NG, NV), v0);
         vm = each([](float vv, float ff, float va) { return vv * (1.0f - ff) + va * ff; }, v, f, first);
     }
     const float4 kk = each([](float p, float kv, float) { return round_h(p * kv); }, k_k, k, k);
@@ -143,15 +144,22 @@ __global__ __launch_bounds__(256) void v7_mid_kernel(uint32_t C, uint32_t T, flo
     store_vec4(m.att_w + at, w);
     store_vec4(m.att_g + at, gate);
     if constexpr (FIRST) store_vec4(m.att_v0 + at, v);
-    store_vec4(m.n + at, each([](float kv, float av, float p) { return kv * (1.0f + (av - 1.0f) * p); }, k, a, k_a));
-    store_vec4(m.n + plane + at, vm);
-    store_vec4(m.n + 2 * plane + at, a);
-    store_vec4(m.n + 3 * plane + at, make_float4(kk.x * norm, kk.y * norm, kk.z * norm, kk.w * norm));
+    auto keep = [&](uint16_t *buffer, int i, float4 value) {
+        store_vec4(m.n + i * plane + at, value);
+        if (buffer) store_vec4(buffer + at, value);
+    };
+    keep(m.att_k, 0, each([](float kv, float av, float p) { return kv * (1.0f + (av - 1.0f) * p); }, k, a, k_a));
+    keep(m.att_v, 1, vm);
+    keep(m.att_a, 2, a);
+    keep(m.att_kk, 3, make_float4(kk.x * norm, kk.y * norm, kk.z * norm, kk.w * norm));
+    if constexpr (!FIRST) {
+        if (m.att_vv) store_vec4(m.att_vv + at, f);
+    }
 }
 
-// state[request] <- ffn_x at its last token; x_out = f16(v + x_in) (halved when `rescale`)
+// state[request] <- ffn_x at its last token; x_out = f16(v + x_in) (halved when `rescale`); ffn_out, where given, <- v
 __global__ __launch_bounds__(256) void v7_post_ffn_kernel(const uint32_t *cursors, float *state, const uint16_t *v, const uint16_t *ffn_x, const uint16_t *x_in,
-                                                          uint16_t *x_out, uint32_t C, int rescale, ViewArgs vs) {
+                                                          uint16_t *x_out, uint32_t C, int rescale, uint16_t *ffn_out, ViewArgs vs) {
     const uint32_t index = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
     if (index >= C / 4) return;
     const uint64_t bti = (uint64_t)t * C + 4 * index;
@@ -161,6 +169,7 @@ __global__ __launch_bounds__(256) void v7_post_ffn_kernel(const uint32_t *cursor
     const float sc = rescale ? 0.5f : 1.0f;
     auto f = [&](float a, float b) { return round_h(a + b) * sc; };
     store_vec4(x_out + bti, make_float4(f(vv.x, xx.x), f(vv.y, xx.y), f(vv.z, xx.z), f(vv.w, xx.w)));
+    if (ffn_out) store_vec4(ffn_out + bti, vv);
 }
 
 template <typename XT>
@@ -393,10 +402,17 @@ int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void
 
 int wrq_v7_mid(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first, const uint32_t *ranks, const void *const *aux, const void *const *w2,
                const void *const *vectors, float eps, const void *k, const void *v, void *att_v0, void *att_w, void *att_g, void *n) {
+    void *const none[5] = {};
+    return wrq_v7_mid_buffers(stream, S, H, A, first, ranks, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n, none);
+}
+
+int wrq_v7_mid_buffers(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first, const uint32_t *ranks, const void *const *aux, const void *const *w2,
+                       const void *const *vectors, float eps, const void *k, const void *v, void *att_v0, void *att_w, void *att_g, void *n,
+                       void *const *buffers) {
     const char *what = "v7_mid";
     if (H == 0 || A == 0) return WRQ_OK;
     if (S != 64) return fail(WRQ_ERR_UNSUPPORTED, "%s: head size %u (64 is built)", what, S);
-    if (!ranks || !aux || !w2 || !vectors) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
+    if (!ranks || !aux || !w2 || !vectors || !buffers) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
     if (ranks[0] != 64 || ranks[1] != 64 || ranks[2] != 128 || ranks[3] != 32)
         return fail(WRQ_ERR_UNSUPPORTED, "%s: adapter sizes %u, %u, %u, %u (64, 64, 128, 32 are built)", what, ranks[0], ranks[1], ranks[2], ranks[3]);
     if (A > 65535u * 16u) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
@@ -408,12 +424,14 @@ int wrq_v7_mid(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, int first,
     for (int i = 0; i < 5 && s == WRQ_OK; i++) s = check_ptr(vectors[i], what);
     for (const void *p : {k, v, (const void *)att_v0, (const void *)att_w, (const void *)att_g, (const void *)n})
         if (s == WRQ_OK) s = check_ptr(p, what);
+    for (int i = 0; i < 5 && s == WRQ_OK; i++)
+        if (buffers[i]) s = check_ptr(buffers[i], what);
     if (s != WRQ_OK) return s;
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     auto o16 = [](void *p) { return static_cast<uint16_t *>(p); };
     const MidArgs m{u16(aux[0]),     u16(aux[1]),     u16(aux[2]),     u16(aux[3]),     u16(w2[0]), u16(w2[1]), u16(w2[2]),  u16(w2[3]),  u16(vectors[0]),
                     u16(vectors[1]), u16(vectors[2]), u16(vectors[3]), u16(vectors[4]), u16(k),     u16(v),     o16(att_v0), o16(att_w), o16(att_g),
-                    o16(n)};
+                    o16(n),          o16(buffers[0]), o16(buffers[1]), o16(buffers[2]), o16(buffers[3]), o16(buffers[4])};
     const dim3 grid(H, (A + 15) / 16);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     if (first) hipLaunchKernelGGL((v7_mid_kernel<64, 64, 128, 32, true>), grid, dim3(256), 0, hs, S * H, A, eps, m);
@@ -440,6 +458,11 @@ int wrq_v7_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const
 
 int wrq_v7_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const wrq_tensor_view *state, const void *v, const void *ffn_x,
                     const void *x_in, void *x_out, int rescale) {
+    return wrq_v7_post_ffn_buffers(stream, C, A, cursors, state, v, ffn_x, x_in, x_out, rescale, nullptr);
+}
+
+int wrq_v7_post_ffn_buffers(wrq_stream stream, uint32_t C, uint32_t A, const void *cursors, const wrq_tensor_view *state, const void *v, const void *ffn_x,
+                            const void *x_in, void *x_out, int rescale, void *ffn_out) {
     const char *what = "v7_post_ffn";
     if (C == 0 || A == 0) return WRQ_OK;
     if (C % 4) return fail(WRQ_ERR_ALIGNMENT, "%s: row length %u not a multiple of 4", what, C);
@@ -447,11 +470,12 @@ int wrq_v7_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *curso
     int s = check_state(state, C, 1, what);
     for (const void *p : {cursors, v, ffn_x, x_in, (const void *)x_out})
         if (s == WRQ_OK) s = check_ptr(p, what);
+    if (s == WRQ_OK && ffn_out) s = check_ptr(ffn_out, what);
     if (s != WRQ_OK) return s;
     const ViewArgs vs = view_args(state->view);
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     hipLaunchKernelGGL(v7_post_ffn_kernel, dim3((C / 4 + 255) / 256, A), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint32_t *>(cursors),
-                       static_cast<float *>(state->data), u16(v), u16(ffn_x), u16(x_in), static_cast<uint16_t *>(x_out), C, rescale, vs);
+                       static_cast<float *>(state->data), u16(v), u16(ffn_x), u16(x_in), static_cast<uint16_t *>(x_out), C, rescale, static_cast<uint16_t *>(ffn_out), vs);
     return check_launch(what);
 }
 

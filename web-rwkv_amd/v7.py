@@ -19,7 +19,8 @@ QUANTIZED = ("att_w_r", "att_w_k", "att_w_v", "att_w_o", "ffn_w_k", "ffn_w_v")
 ADAPTERS = ("w1", "w2", "a1", "a2", "g1", "g2", "v1", "v2")
 VECTORS = ("att_ln_w", "att_ln_b", "ffn_ln_w", "ffn_ln_b", "x_r", "x_w", "x_k", "x_v", "x_a", "x_g", "ffn_x_k", "w0", "a0", "v0", "k_k", "k_a", "r_k", "gn_w", "gn_b")
 SHIFTED = ("att_rx", "att_wx", "att_kx", "att_vx", "att_ax", "att_gx")
-FUSED_ROWS = ("x", "x2", "att_x", "att_v0", "att_r", "att_w", "att_k", "att_v", "att_g", "att_o", "ffn_x", "ffn_kx", "ffn_v")
+FUSED_ROWS = ("x", "x2", "att_x", "att_v0", "att_r", "att_w", "att_k", "att_v", "att_a", "att_g", "att_kk", "att_vv", "att_o", "ffn_x", "ffn_kx",
+              "ffn_v")
 
 
 def random_layer_weights(rng, C, H, S, hidden):
@@ -115,8 +116,7 @@ def fused_is_built(layer, H, S, buf=None, cursors=None, A=None, shifts=None):
 
 def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
     """The layer in 10 launches (beside the second ones of split products): the six quantized products in four and six
-    fused launches for the 40 small ops.  Same results as `dispatch_layer_ops` up to f32 summation order; the buffers
-    between the fused ops (`att_kk`, `att_vv`, `att_a`) stay unwritten, and `att_k`, `att_v` keep the projections.
+    fused launches for the small ops.  Same results as `dispatch_layer_ops` up to f32 summation order, in `buf`'s buffers too.
     Four layers of 2048 channels, 32 requests of one token: 195 -> 84 us per layer."""
     t, m, C = layer.t, layer.m, H * S
     B = state.shape[0]
@@ -136,13 +136,14 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now
     adapters = [(w["w1"], wx, buf.aux_w, ACT_TANH), (w["a1"], ax, buf.aux_a, ACT_NONE), (w["g1"], gx, buf.aux_g, ACT_SIGMOID), (w["v1"], vx, buf.aux_v, ACT_NONE)]
     FusedV7.adapters_in(C, A, adapters[:3] if index == 0 else adapters)
     FusedV7.mid(S, H, A, index == 0, [buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v], [w["w2"], w["a2"], w["g2"], w["v2"]],
-                [t["w0"], t["a0"], t["v0"], t["k_k"], t["k_a"]], L2_EPS, buf.att_k, buf.att_v, buf.att_v0, buf.att_w, buf.att_g, buf.att_n)
+                [t["w0"], t["a0"], t["v0"], t["k_k"], t["k_a"]], L2_EPS, buf.att_k, buf.att_v, buf.att_v0, buf.att_w, buf.att_g, buf.att_n,
+                [buf.att_k, buf.att_v, buf.att_a, buf.att_kk, buf.att_vv])
     FusedV7.wkv_gate(S, H, A, cursors, state, att_state, buf.att_r, buf.att_w, buf.att_n, t["r_k"], buf.att_g, t["gn_w"], t["gn_b"], GN_EPS, buf.att_x)
     m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)
     FusedV7.pre(C, A, cursors, buf.x, buf.att_o, buf.x2, t["ffn_ln_w"], t["ffn_ln_b"], LN_EPS, state, ffn_state, [t["ffn_x_k"]], buf.ffn_x, [buf.ffn_kx])
     m["ffn_w_k"].matmul_op(buf.ffn_kx, buf.ffn_k, ACT_SQUARED_RELU, fast)
     m["ffn_w_v"].matmul_op_sparse(buf.ffn_k, buf.ffn_v, ACT_NONE, fast)
-    FusedV7.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now)
+    FusedV7.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now, buf.ffn_x)
 
 
 def dispatch_layer_ops(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
