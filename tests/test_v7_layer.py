@@ -207,3 +207,34 @@ def test_v7_dispatch_leaves_the_buffers_of_the_op_list(gpu, runs, packed):
             outs.append({name: t.cpu().numpy() for name, t in named.items()})
         for name in outs[0]:
             assert_close(outs[1][name], outs[0][name], 4e-3, f"{name} of layer {index}")
+
+
+@pytest.mark.gpu
+def test_v7_dispatch_takes_the_factors_of_packed_shifts(gpu):
+    # factors of its own in `PackedShifts.mix`, another for every token, as the op list takes them; the bound as above
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    v7 = importlib.import_module(gpu.__name__ + ".v7")
+    H, S, hidden, B = 2, 64, 256, 4
+    C = H * S
+    rng = np.random.default_rng(SEED + 140)
+    cursors = lop.pack_cursors([(1, 5), (3, 1), (0, 12)])
+    A = len(cursors)
+    curd = torch.from_numpy(cursors.view(np.int32)).cuda()
+    layer = v7.Layer(torch, v7.random_layer_weights(rng, C, H, S, hidden), "int8")
+    x, mix = rng.standard_normal((1, A, C)).astype(np.float16), rng.random((6, A, C)).astype(np.float16)
+    state = (0.1 * rng.standard_normal((B, S + 2, C))).astype(np.float32)
+    outs = []
+    for dispatch in (v7.dispatch_layer_ops, v7.dispatch_layer):
+        buf, shifts = v7.Runtime(torch, C, hidden, A), v7.PackedShifts(torch, layer, A)
+        shifts.mix.copy_(torch.from_numpy(mix).cuda())
+        assert v7.fused_is_built(layer, H, S, buf, curd, A, shifts)
+        buf.x.copy_(torch.from_numpy(x).cuda())
+        sd = torch.from_numpy(state.copy()).cuda()
+        dispatch(layer, buf, sd, curd, A, H, S, 0, shifts=shifts)
+        torch.cuda.synchronize()
+        outs.append([t.cpu().numpy() for t in (shifts.sx, buf.x, sd)])
+    for i, what in enumerate(("shifted rows", "layer output", "state")):
+        assert_close(outs[1][i], outs[0][i], 4e-3, what)

@@ -123,13 +123,15 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now
     fast = turbo(A)
     att_state = ((C, S + 1, B), (C, S + 2, B), (0, 0, 0))
     ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
+    att_ln = (C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state)
     if shifts is None:
-        rx, wx, kx, vx, ax, gx = buf.att_rx, buf.att_wx, buf.att_kx, buf.att_vx, buf.att_ax, buf.att_gx
+        rx, wx, kx, vx, ax, gx = shifted = [getattr(buf, name) for name in SHIFTED]
+        FusedV7.pre(*att_ln, [t[n] for n in PackedShifts.NAMES], buf.att_x, shifted)
     else:
-        rx, wx, kx, vx, ax, gx = (shifts.sx[i].view(1, A, C) for i in range(6))
-
-    FusedV7.pre(C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state,
-                [t[n] for n in PackedShifts.NAMES], buf.att_x, [rx, wx, kx, vx, ax, gx])
+        # the caller's factors may differ from token to token: the first shift is a layer norm's companion, the six are token_shift's
+        rx, wx, kx, vx, ax, gx = shifted = [shifts.sx[i].view(1, A, C) for i in range(6)]
+        FusedV7.pre(*att_ln, [t[PackedShifts.NAMES[0]]], buf.att_x, shifted[:1])
+        LayerOp.token_shift(cursors, shifts.mix, state, buf.att_x, shifts.sx, True, state_view=att_state)
     matmul_vec_group([(m["att_w_r"], rx, buf.att_r, ACT_NONE, False, {}), (m["att_w_k"], kx, buf.att_k, ACT_NONE, False, {}),
                       (m["att_w_v"], vx, buf.att_v, ACT_NONE, False, {})])
     w = {n: m[n].w for n in ADAPTERS}
