@@ -315,7 +315,8 @@ int wrq_lerp(wrq_stream stream, const wrq_tensor_view *input, const wrq_tensor_v
 /*
  * The ops that carry state from token to token.  A run is a stack of A tokens of several requests;
  * cursors u32 [A, 1, 1, 1]: for the request of token a, its state slot | first token in the stack << 8
- * | number of its tokens in the stack << 24 (compute_cursor of the shaders).  States are f32 views.
+ * | number of its tokens in the stack << 24 (compute_cursor of the shaders).  States are f32 views.  Where several
+ * requests of the stack name one slot, "every request's last token" below is the last one in stack order.
  *
  * TensorOp::token_shift(cursors, time_mix, state, input, output, reversed)
  *                                           src/tensor/ops.rs:1393-1462, src/shaders/token_shift.wgsl

@@ -73,3 +73,38 @@ def test_gpu_fused_keeps_the_last_input(gpu, version, runs):
     for slot in set(slots.tolist()):
         last = int(np.flatnonzero(slots == slot)[-1])
         assert torch.equal(state[slot, 0], before[last].float()), slot
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["channel_mix", "channel_mix_v7", "v6_post_ffn", "v7_post_ffn"])
+@pytest.mark.parametrize("C", [64, 1028, 4096])
+@pytest.mark.parametrize("runs", [[(0, 1)], [(0, 1), (1, 2), (0, 1), (0, 3), (1, 1)], [(1, 1)] + [(0, 1)] * 63 + [(1, 1)], [(1, 1)] * 70 + [(0, 2), (3, 1)], [(2, 255), (2, 9), (7, 3)]],
+                         ids=lambda r: f"{len(r)} requests")
+def test_gpu_channel_mixes_keep_the_last_input(gpu, op, C, runs):
+    """The feed-forward half under the same stacks: one row of the state per slot, written from one workgroup per token."""
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("channel mix, slots that come again", op, C, runs[:6], flush=True)
+    B = 4  # a slot beyond the state counts as the last one
+    cur = lop.pack_cursors(runs)
+    A = len(cur)
+    g = torch.Generator().manual_seed(0x5758 + A + C)
+    f16 = lambda *s: torch.randn(s, generator=g).half().cuda()
+    curd, state, view = torch.from_numpy(cur.view(np.int32)).cuda(), torch.randn((B, 1, C), generator=g).cuda(), ((C, 1, B), (C, 1, B), (0, 0, 0))
+    r, v, x, x_in, out = (f16(1, A, C) for _ in range(5))
+    want, rows = state.clone(), x.clone()
+    for t in range(A):
+        slot, first, n = int(cur[t]) & 0xff, int(cur[t]) >> 8 & 0xffff, int(cur[t]) >> 24
+        if t - first + 1 == n:
+            want[min(slot, B - 1), 0] = rows[0, t].float()
+    if op == "channel_mix":
+        gpu.LayerOp.channel_mix(curd, state, r, v, x)
+    elif op == "channel_mix_v7":
+        gpu.LayerOp.channel_mix_v7(curd, state, v, x)
+    elif op == "v6_post_ffn":
+        gpu.FusedV6.post_ffn(C, A, curd, state, view, r, v, x, x_in, out, False)
+    else:
+        gpu.FusedV7.post_ffn(C, A, curd, state, view, v, x, x_in, out, False)
+    assert torch.equal(state, want)

@@ -265,14 +265,16 @@ __global__ __launch_bounds__(256) void v6_decay_tile_kernel(const uint16_t *lora
 // state[request] <- ffn_x at its last token; x_out = f16(f16(sigmoid(r) v) + x_in) (halved when `rescale`)
 __global__ __launch_bounds__(256) void v6_post_ffn_kernel(const uint32_t *cursors, float *state, ViewArgs vs, const uint16_t *r, const uint16_t *v,
                                                           const uint16_t *ffn_x, const uint16_t *x_in, uint16_t *x_out, uint32_t C, int rescale) {
-    const uint32_t index = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
-    if (index >= C / 4) return;
+    const uint32_t at = blockIdx.x * 256 + threadIdx.x, index = min(at, C / 4 - 1), t = blockIdx.y;
     const uint64_t bti = (uint64_t)t * C + 4 * index;
     // all loads before the store into the state: the compiler cannot move them across it (the pointers may
     // alias), and behind it they would wait for the cursor's round trip first
     const float4 rr = load_vec4(r + bti), vv = load_vec4(v + bti), xx = load_vec4(x_in + bti), fx = load_vec4(ffn_x + bti);
+    const uint32_t ahead = cursor_ahead(cursors, t, gridDim.y);
     const Cursor cur = read_cursor(cursors, t, vs);
-    if (t - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = fx;
+    const bool keeps = keeps_row(cursors, t, gridDim.y, cur, vs, ahead);
+    if (at >= C / 4) return; // lanes past the row took part in the search
+    if (keeps) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = fx;
     const float sc = rescale ? 0.5f : 1.0f;
     auto f = [&](float a, float b, float c) { return round_h(round_h(1.0f / (1.0f + expf(-a)) * b) + c) * sc; };
     store_vec4(x_out + bti, make_float4(f(rr.x, vv.x, xx.x), f(rr.y, vv.y, xx.y), f(rr.z, vv.z, xx.z), f(rr.w, vv.w, xx.w)));

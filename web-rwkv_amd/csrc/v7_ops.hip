@@ -160,12 +160,14 @@ __global__ __launch_bounds__(256) void v7_mid_kernel(uint32_t C, uint32_t T, flo
 // state[request] <- ffn_x at its last token; x_out = f16(v + x_in) (halved when `rescale`); ffn_out, where given, <- v
 __global__ __launch_bounds__(256) void v7_post_ffn_kernel(const uint32_t *cursors, float *state, const uint16_t *v, const uint16_t *ffn_x, const uint16_t *x_in,
                                                           uint16_t *x_out, uint32_t C, int rescale, uint16_t *ffn_out, ViewArgs vs) {
-    const uint32_t index = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
-    if (index >= C / 4) return;
+    const uint32_t at = blockIdx.x * 256 + threadIdx.x, index = min(at, C / 4 - 1), t = blockIdx.y;
     const uint64_t bti = (uint64_t)t * C + 4 * index;
     const float4 vv = load_vec4(v + bti), xx = load_vec4(x_in + bti), fx = load_vec4(ffn_x + bti); // before the cursor's round trip and the store into the state
+    const uint32_t ahead = cursor_ahead(cursors, t, gridDim.y);
     const Cursor cur = read_cursor(cursors, t, vs);
-    if (t - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = fx;
+    const bool keeps = keeps_row(cursors, t, gridDim.y, cur, vs, ahead);
+    if (at >= C / 4) return; // lanes past the row took part in the search
+    if (keeps) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = fx;
     const float sc = rescale ? 0.5f : 1.0f;
     auto f = [&](float a, float b) { return round_h(a + b) * sc; };
     store_vec4(x_out + bti, make_float4(f(vv.x, xx.x), f(vv.y, xx.y), f(vv.z, xx.z), f(vv.w, xx.w)));
@@ -218,12 +220,14 @@ __global__ __launch_bounds__(64) void time_first_v7_kernel(const uint16_t *u, co
 // state[request] <- x at the request's last token of the stack; x <- v
 template <typename XT>
 __global__ __launch_bounds__(256) void channel_mix_v7_kernel(const uint32_t *cursors, float *state, const XT *v, XT *x, ViewArgs vs, uint32_t C) {
-    const uint32_t index = blockIdx.x * 256 + threadIdx.x, stack = blockIdx.y;
-    if (index >= C / 4) return;
+    const uint32_t at = blockIdx.x * 256 + threadIdx.x, index = min(at, C / 4 - 1), stack = blockIdx.y;
     const uint64_t bti = (uint64_t)stack * C + 4 * index;
     const float4 vv = load_vec4(v + bti), xx = load_vec4(x + bti); // both before the cursor's round trip and the store into the state
+    const uint32_t ahead = cursor_ahead(cursors, stack, gridDim.y);
     const Cursor cur = read_cursor(cursors, stack, vs);
-    if (stack - cur.token + 1 == cur.len) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = xx;
+    const bool keeps = keeps_row(cursors, stack, gridDim.y, cur, vs, ahead);
+    if (at >= C / 4) return; // lanes past the row took part in the search
+    if (keeps) *reinterpret_cast<float4 *>(state + view_elem(vs, cur.batch, 0, 4 * index)) = xx;
     store_vec4(x + bti, vv);
 }
 
