@@ -417,7 +417,8 @@ int wrq_blend_lora(wrq_stream stream, const wrq_tensor *factor, const wrq_tensor
  * Buffers are contiguous device arrays of `Runtime<f16>` (v6.rs:270-303): C channels x A tokens.
  *
  * wrq_v6_pre: [add(add, x) ->] blit + layer_norm + token_shift x `shifts` (reversed)   v6.rs:759-777, :906-933
- *   x_out (f16, only with `add`; its A * C elements may overlap neither x nor add) <- add + x;  ln_out <- LN(row);  shift_s <- mix(ln, previous, factor_s).
+ *   x_out (f16, only with `add`) <- add + x;  ln_out <- LN(row);  shift_s <- mix(ln, previous, factor_s).
+ *   The A * C elements of x_out and, with more than one token, of ln_out and shift_s may overlap neither x nor add.
  * wrq_v6_time_mix: transpose + time_mix_w2 + add(time_mix) + token_shift(5)           v6.rs:785-805
  *   lora f16 [lora_size, 5, A]; w2 f16 [lora_size, C, 5]; time_mix f16 [C, 1, 5]; att_sx f16 [C, A, 5].
  * wrq_v6_decay: time_decay_w2 + add(time_decay) + activate(StableExp)                 v6.rs:839-848

@@ -148,3 +148,20 @@ def test_sf4_table_matches_student_quantiles():
         assert q.shape == (16,) and q[0] == -1.0 and q[7] == 0.0 and q[15] == 1.0
         assert (np.diff(q) > 0).all()
         assert np.abs(q.astype(np.float64) - ref.astype(np.float64)).max() <= 1.2e-7
+
+
+def test_fused_pre_refuses_outputs_over_its_inputs(wrq):
+    # a token's workgroup reads its neighbour's row of x and add again while the neighbour stores
+    L = wrq.lib()
+    Cn, A, row = 64, 3, 64 * 2
+    state = C.byref(V(wrq, (Cn, 1, 2, 1), dtype=1))
+    far = lambda i: FAKE + 0x1000 * i
+    for x, add, ln_out, outs in [(far(1), None, far(1), [far(3)]), (far(1), None, far(2), [far(1) + row]), (far(1), far(2), far(4), [far(2) - 2 * row]),
+                                 (far(1), far(2), far(2), [far(5)]), (far(1), None, far(2), [far(3), far(1) + 2 * row])]:
+        factors = (C.c_void_p * 2)(far(8), far(8))
+        s = L.wrq_fused_pre(None, Cn, A, far(9), x, add, far(6) if add else None, far(7), far(7), 1e-5, state, len(outs), factors, ln_out, (C.c_void_p * 2)(*outs))
+        assert s == wrq.ERR_UNSUPPORTED and "overlap no input" in err(wrq), (x, add, ln_out, outs)
+        s = L.wrq_v6_pre(None, Cn, A, far(9), x, add, far(6) if add else None, far(7), far(7), 1e-5, state, len(outs), far(8), far(8), ln_out, *(outs + [None])[:2])
+        assert s == wrq.ERR_UNSUPPORTED and "overlap no input" in err(wrq)
+    s = L.wrq_fused_pre(None, Cn, A, far(9), far(1), far(2), far(1) + row, far(7), far(7), 1e-5, state, 1, (C.c_void_p * 1)(far(8)), far(3), (C.c_void_p * 1)(far(4)))
+    assert s == wrq.ERR_UNSUPPORTED and "the sum" in err(wrq)

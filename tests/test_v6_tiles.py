@@ -66,3 +66,20 @@ def test_gpu_adapters_in_long_rows(gpu, C, A):
         want = torch.tanh(want) if act == gpu.ACT_TANH else want
         # f32 sums of up to 8192 products of 2.5e-3 each, one rounding to f16 (2^-11) of values below 1
         assert_close(out.cpu().numpy(), want.numpy(), 1e-3, "adapters_in vs float64")
+
+
+@pytest.mark.gpu
+def test_gpu_pre_of_one_token_in_place(gpu):
+    """A single token has no neighbour that reads its row: normalised in place as into a buffer of its own."""
+    import torch
+
+    C = 4100
+    g = torch.Generator().manual_seed(0x5759)
+    h = lambda *s: torch.randn(s, generator=g).half().cuda()
+    cur, state, view = torch.tensor([1 << 24], dtype=torch.int32).cuda(), torch.randn((1, 1, C), generator=g).cuda(), ((C, 1, 1), (C, 1, 1), (0, 0, 0))
+    x, w, b, f, ln, out = (h(C) for _ in range(6))
+    args = lambda x, ln, out: (C, 1, cur, x, None, None, w, b, 1e-5, state, view, [f], ln, [out])
+    gpu.FusedV7.pre(*args(x, ln, out))
+    again, shifted = x.clone(), torch.empty_like(out)
+    gpu.FusedV7.pre(*args(again, again, shifted))
+    assert torch.equal(again, ln) and torch.equal(shifted, out)

@@ -299,15 +299,20 @@ int launch_pre(const char *what, int most, wrq_stream stream, uint32_t C, uint32
     }
     if (s == WRQ_OK && add) s = check_ptr(x_out, what);
     if (s != WRQ_OK) return s;
-    if (add) {
-        // workgroup t rebuilds row t - 1 from x and add while workgroup t - 1 stores x_out: the sum may overlap neither
-        const uintptr_t lo = (uintptr_t)x_out, hi = lo + (size_t)A * C * 2;
-        for (const void *src : {x, add}) {
-            const uintptr_t a0 = (uintptr_t)src, a1 = a0 + (size_t)A * C * 2;
-            if (lo < a1 && a0 < hi)
-                return fail(WRQ_ERR_UNSUPPORTED, "%s: the sum must go to a buffer that overlaps neither input (a token's workgroup reads its neighbour's row)", what);
-        }
-    }
+    // workgroup t rebuilds row t - 1 from x and add while workgroup t - 1 stores its rows: what is stored may overlap neither
+    // (a single token has no neighbour: it may be normalised in place)
+    auto overlaps_input = [&](const void *out) {
+        const uintptr_t lo = (uintptr_t)out, bytes = (uintptr_t)A * C * 2;
+        for (const void *src : {x, add})
+            if (src && lo < (uintptr_t)src + bytes && (uintptr_t)src < lo + bytes) return true;
+        return false;
+    };
+    if (add && overlaps_input(x_out))
+        return fail(WRQ_ERR_UNSUPPORTED, "%s: the sum must go to a buffer that overlaps neither input (a token's workgroup reads its neighbour's row)", what);
+    bool overlap = overlaps_input(ln_out);
+    for (int i = 0; i < shifts; i++) overlap = overlap || overlaps_input(outs[i]);
+    if (A > 1 && overlap)
+        return fail(WRQ_ERR_UNSUPPORTED, "%s: the outputs must go to buffers that overlap no input (a token's workgroup reads its neighbour's row)", what);
     const ViewArgs vs = view_args(state->view);
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     auto o16 = [](void *p) { return static_cast<uint16_t *>(p); };
