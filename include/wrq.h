@@ -449,7 +449,8 @@ int wrq_v6_post_ffn(wrq_stream stream, uint32_t C, uint32_t A, const void *curso
  * Fused forms of the small ops of an RWKV-v7 layer (src/runtime/v7.rs:704-1006), under the same rules:
  * wrq_v7_mid: the second halves of the adapters w, a, g, v (ranks 64, 64, 128, 32; aux, w2: 4 device pointers each) + add /
  *   sigmoid + lerp with the first layer's values + mul(k_k) + l2_norm + control_k_v7 + the blits into n [C, A, 4];
- *   vectors: w0, a0, v0, k_k, k_a; `first`: the layer whose values att_v0 keeps (no adapter v).  k and v are not written.
+ *   vectors: w0, a0, v0, k_k, k_a; `first`: the layer whose values att_v0 keeps (no adapter v: ranks, aux, w2 and v0 of it
+ *   are not looked at).  k and v are not written.
  * wrq_v7_wkv_gate: time_mix_v7 + group_norm + time_first_v7 + mul(g); att_x f16 in (the normalised layer input) and out.
  * wrq_v7_post_ffn: channel_mix_v7 + add (+ affine(0.5) when `rescale`); x_in, ffn_x and v are not written.
  * wrq_v7_mid_buffers, wrq_v7_post_ffn_buffers: the same, also filling what the op list leaves in its own buffers: `buffers`

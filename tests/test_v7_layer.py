@@ -238,3 +238,26 @@ def test_v7_dispatch_takes_the_factors_of_packed_shifts(gpu):
         outs.append([t.cpu().numpy() for t in (shifts.sx, buf.x, sd)])
     for i, what in enumerate(("shifted rows", "layer output", "state")):
         assert_close(outs[1][i], outs[0][i], 4e-3, what)
+
+
+@pytest.mark.gpu
+def test_v7_mid_of_the_first_layer_needs_no_adapter_v(gpu):
+    import torch
+
+    S, H, A = 64, 2, 17
+    C = S * H
+    g = torch.Generator().manual_seed(SEED + 150)
+    h = lambda *s: (0.3 * torch.randn(s, generator=g)).half().cuda()
+    aux, w2, vectors = [h(A, r) for r in (64, 64, 128, 32)], [h(C, r) for r in (64, 64, 128, 32)], [h(C) for _ in range(5)]
+    k, v = h(A, C), h(A, C)
+    outs = []
+    for last in (None, 0):
+        x, w, b = (list(a) for a in (aux, w2, vectors))
+        if last is None:
+            x[3], w[3], b[2] = None, None, None
+        out = [torch.empty((A, C), dtype=torch.float16, device="cuda") for _ in range(3)] + [torch.empty((4, A, C), dtype=torch.float16, device="cuda")]
+        gpu.FusedV7.mid(S, H, A, True, x, w, b, 1e-12, k, v, *out)
+        outs.append(out)
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    assert torch.equal(outs[0][0], v) and torch.equal(outs[0][3][1], v)

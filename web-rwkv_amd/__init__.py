@@ -580,9 +580,12 @@ class FusedV7:
         p, a, Cn = FusedV6._p, FusedV7._a, S * H
         if len(aux) != 4 or len(w2) != 4 or len(vectors) != 5 or len(buffers) != 5:
             raise TensorError(ERR_SHAPE, f"v7_mid: {len(aux)}, {len(w2)}, {len(vectors)} and {len(buffers)} operands, 4, 4, 5 and 5 are needed")
-        _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2)] + [(w, Cn * w.shape[1]) for w in w2] + [(t, Cn) for t in vectors]
+        if first:  # without the adapter v
+            aux, w2, vectors = [*aux[:3], None], [*w2[:3], None], [*vectors[:2], None, *vectors[3:]]
+        _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2) if w is not None] + [(w, Cn * w.shape[1]) for w in w2 if w is not None]
+                  + [(t, Cn) for t in vectors]
                   + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g, *buffers)] + [(n, 4 * A * Cn)])
-        ranks = (C.c_uint32 * 4)(*(t.shape[1] for t in w2))
+        ranks = (C.c_uint32 * 4)(*(0 if t is None else t.shape[1] for t in w2))
         _check(lib().wrq_v7_mid_buffers(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n),
                                         a(buffers)))
 

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void v7_mid_kernel(uint32_t C, uint32_t T, flo
     if constexpr (!FIRST) fetch(std::integral_constant<int, RV>{}, m.v2, m.aux_v, NW + NA + NG);
     const uint32_t ch = c0 + 4 * g;
     const uint64_t at = (uint64_t)t * C + ch, plane = (uint64_t)T * C;
-    const float4 w0 = load_vec4(m.w0 + ch), a0 = load_vec4(m.a0 + ch), v0 = load_vec4(m.v0 + ch), k_k = load_vec4(m.k_k + ch), k_a = load_vec4(m.k_a + ch);
+    const float4 w0 = load_vec4(m.w0 + ch), a0 = load_vec4(m.a0 + ch), v0 = FIRST ? make_float4(0.f, 0.f, 0.f, 0.f) : load_vec4(m.v0 + ch), k_k = load_vec4(m.k_k + ch), k_a = load_vec4(m.k_a + ch);
     const float4 k = load_vec4(m.k + at), v = load_vec4(m.v + at);
     const float4 first = FIRST ? v : load_vec4(m.att_v0 + at);
     auto product = [&](int from, int count) {
@@ -417,7 +417,7 @@ int wrq_v7_mid_buffers(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, in
     if (H == 0 || A == 0) return WRQ_OK;
     if (S != 64) return fail(WRQ_ERR_UNSUPPORTED, "%s: head size %u (64 is built)", what, S);
     if (!ranks || !aux || !w2 || !vectors || !buffers) return fail(WRQ_ERR_NULL, "%s: null pointer", what);
-    if (ranks[0] != 64 || ranks[1] != 64 || ranks[2] != 128 || ranks[3] != 32)
+    if (ranks[0] != 64 || ranks[1] != 64 || ranks[2] != 128 || (!first && ranks[3] != 32))
         return fail(WRQ_ERR_UNSUPPORTED, "%s: adapter sizes %u, %u, %u, %u (64, 64, 128, 32 are built)", what, ranks[0], ranks[1], ranks[2], ranks[3]);
     if (A > 65535u * 16u) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
     int s = WRQ_OK;
@@ -425,7 +425,8 @@ int wrq_v7_mid_buffers(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, in
         s = check_ptr(aux[i], what);
         if (s == WRQ_OK) s = check_ptr(w2[i], what);
     }
-    for (int i = 0; i < 5 && s == WRQ_OK; i++) s = check_ptr(vectors[i], what);
+    for (int i = 0; i < 5 && s == WRQ_OK; i++)
+        if (!first || i != 2) s = check_ptr(vectors[i], what); // the first layer has no adapter v and so no v0
     for (const void *p : {k, v, (const void *)att_v0, (const void *)att_w, (const void *)att_g, (const void *)n})
         if (s == WRQ_OK) s = check_ptr(p, what);
     for (int i = 0; i < 5 && s == WRQ_OK; i++)
