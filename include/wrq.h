@@ -44,7 +44,7 @@ extern "C" {
 #define WRQ_ABI_VERSION 1
 /* Counts additions that leave every existing signature as it is (new entry points, new override keys);
  * a binding built against minor m runs on any library of the same WRQ_ABI_VERSION with minor >= m. */
-#define WRQ_ABI_MINOR 3
+#define WRQ_ABI_MINOR 4
 #define WRQ_INT8_BLOCK_SIZE 128u /* TensorOp::INT8_BLOCK_SIZE, src/tensor/ops.rs:292 */
 #define WRQ_NF4_BLOCK_SIZE 64u   /* TensorOp::NF4_BLOCK_SIZE, src/tensor/ops.rs:291 */
 

@@ -165,3 +165,9 @@ def test_fused_pre_refuses_outputs_over_its_inputs(wrq):
         assert s == wrq.ERR_UNSUPPORTED and "overlap no input" in err(wrq)
     s = L.wrq_fused_pre(None, Cn, A, far(9), far(1), far(2), far(1) + row, far(7), far(7), 1e-5, state, 1, (C.c_void_p * 1)(far(8)), far(3), (C.c_void_p * 1)(far(4)))
     assert s == wrq.ERR_UNSUPPORTED and "the sum" in err(wrq)
+
+
+def test_minor_counts_the_fused_v7_forms(wrq):
+    # a binding that calls them asks for this minor: a library of minor 3 may have none of them
+    names = [n for n in declared_functions() if n.startswith("wrq_v7_") or n in ("wrq_fused_pre", "wrq_adapters_in")]
+    assert len(names) == 7 and wrq.lib().wrq_abi_minor() >= 4
