@@ -108,3 +108,45 @@ def test_gpu_channel_mixes_keep_the_last_input(gpu, op, C, runs):
     else:
         gpu.FusedV7.post_ffn(C, A, curd, state, view, v, x, x_in, out, False)
     assert torch.equal(state, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,runs", [(2, [(1, 1)]), (300, [(255, 1)]), (9, [(3, 2), (0, 1), (3, 1)]), (9, [(9, 1), (2, 3), (8, 2)]), (300, [(255, 2), (0, 1), (254, 9), (255, 1)]),
+                                    (256, [(i, 1) for i in range(200, 0, -1)] + [(77, 54)]), (256, [(5, 255)])], ids=lambda v: str(v if isinstance(v, int) else len(v)))
+@pytest.mark.parametrize("form", ["time_mix_v5", "time_mix_v6", "time_mix_v7", "v6 gate", "v7 gate"])
+def test_gpu_more_slots_than_tokens(gpu, form, B, runs):
+    """A state of more slots than the run has tokens gives what a state of the named slots alone gives, bit for bit, and
+    leaves the other slots as they are."""
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("more slots than tokens", form, B, runs[:4], flush=True)
+    H, S = 2, 64
+    C = H * S
+    named = sorted({min(slot, B - 1) for slot, _ in runs})
+    few = [(named.index(min(slot, B - 1)), n) for slot, n in runs]
+    A = sum(n for _, n in runs)
+    g = torch.Generator().manual_seed(0x575A + A)
+    f32 = lambda *s: (torch.randn(s, generator=g) * 0.3).cuda()
+    f16 = lambda *s: f32(*s).half()
+    state, x0 = f32(B, S + 2, C), (f16 if "gate" in form else f32)(A, H, S)
+    k, v, r, u, decay, kvak = f32(A, H, S), f32(A, H, S), f32(A, H, S), f32(H, S), torch.sigmoid(f32(A, H, S)), f32(4, A, H, S)
+    gates, gw, gb = f16(A, C), f16(H, S), f16(H, S)
+    outs = []
+    for stack, rows in ((runs, state.clone()), (few, state[named].contiguous())):
+        n = rows.shape[0]
+        cur, x, view = torch.from_numpy(lop.pack_cursors(stack).view(np.int32)).cuda(), x0.clone(), ((C, S + 1, n), (C, S + 2, n), (0, 0, 0))
+        if form == "time_mix_v7":
+            gpu.LayerOp.time_mix_v7(cur, rows, r, k, kvak, x, state_view=view)
+        elif form == "v6 gate":
+            gpu.FusedV6.wkv_gate(S, H, A, cur, decay, u, rows, view, k, v, r, gates, gw, gb, 64e-5, x)
+        elif form == "v7 gate":
+            gpu.FusedV7.wkv_gate(S, H, A, cur, rows, view, r.half(), k.half(), kvak.half(), gw, gates, gw, gb, 64e-5, x)
+        else:
+            getattr(gpu.LayerOp, form)(cur, decay[0].contiguous() if form == "time_mix_v5" else decay, u, rows, k, v, r, x, state_view=view)
+        outs.append((x, rows))
+    assert torch.equal(outs[0][0], outs[1][0])
+    want = state.clone()
+    want[named] = outs[1][1]
+    assert torch.equal(outs[0][1], want)

@@ -17,10 +17,24 @@ namespace wrq {
 
 constexpr uint32_t kSlotScan = 256; // cursors scanned at a time: one per thread
 
+// The slot a workgroup takes; false: none.  A grid of less than the slots has a workgroup per token (slot_grid): it takes its
+// token's slot, unless an earlier token has it.
+__device__ __forceinline__ bool own_slot(const uint32_t *cursors, uint32_t A, uint32_t slots, uint32_t *slot) {
+    *slot = blockIdx.y;
+    if (gridDim.y == A && A < slots) {
+        *slot = min(cursors[blockIdx.y] & 0xffu, slots - 1);
+        if (blockIdx.y) {
+            const bool taken = threadIdx.x < blockIdx.y && min(cursors[min(threadIdx.x, A - 1)] & 0xffu, slots - 1) == *slot;
+            return !__syncthreads_or(taken);
+        }
+    }
+    return true;
+}
+
 // The tokens of `slot` among cursors[base .. base + 256): their offsets from `base` in stack order, and their number.
-// With a single slot every token is its own (a slot beyond the view counts as the last one) and `list` stays unused.
-__device__ __forceinline__ uint32_t slot_tokens(const uint32_t *cursors, uint32_t base, uint32_t A, uint32_t slot, uint32_t slots, uint8_t *list, uint32_t *count) {
-    if (slots == 1) return min(kSlotScan, A - base);
+// With a single slot (a slot beyond the view counts as the last one) or a single token, `every` token is its own and `list` stays unused.
+__device__ __forceinline__ uint32_t slot_tokens(const uint32_t *cursors, uint32_t base, uint32_t A, uint32_t slot, uint32_t slots, bool every, uint8_t *list, uint32_t *count) {
+    if (every) return min(kSlotScan, A - base);
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const bool mine = base + tid < A && min(cursors[min(base + tid, A - 1)] & 0xffu, slots - 1) == slot;
     const uint64_t mask = __ballot(mine);
@@ -146,7 +160,7 @@ __device__ __forceinline__ float4 head_norm(float4 y, uint2 wq, uint2 bq, float 
 // v5 (a decay per channel) and v6 (TOKEN_DECAY: a decay per token):
 //   y[i] = sum_j r[j] (u[j] k[j] v[i] + S[j][i]),  S[j][i] <- w[j] S[j][i] + k[j] v[i]
 // GATE: the fused form, y then goes through the group norm (rounded to f16) and silu(g) into att_x; otherwise into x.
-// grid (heads, slots).  The operands come in chunks of TB tokens of the slot: every thread fetches one 4-element
+// grid (heads, slot_grid).  The operands come in chunks of TB tokens of the slot: every thread fetches one 4-element
 // vector of each while the previous chunk is worked on and passes it round through LDS (two buffers).
 template <typename XT, int SZ, bool TOKEN_DECAY, bool GATE>
 __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
@@ -159,7 +173,10 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
     __shared__ uint32_t csh[2][TB], tsh[2][TB]; // cursors and numbers of the chunk's tokens
     __shared__ uint8_t list[kSlotScan];
     __shared__ uint32_t count[kSlotScan / 64];
-    const uint32_t head = blockIdx.x, slot = blockIdx.y, slots = vs.shape[2], tid = threadIdx.x;
+    const uint32_t head = blockIdx.x, slots = vs.shape[2], tid = threadIdx.x;
+    const bool every = slots == 1 || A == 1;
+    uint32_t slot;
+    if (!own_slot(cursors, A, slots, &slot)) return;
     const uint32_t l = tid % L;
     const uint32_t C = SZ * H;
     // this thread's vector of a chunk: token tid / TL of the chunk, elements 4 (tid % TL) ..
@@ -172,7 +189,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
     uint32_t fc = 0, ft = 0, fct = 0;
     uint32_t base = 0, n = 0;
     auto fetch = [&](uint32_t chunk) {
-        auto token = [&](uint32_t j) { return base + (slots == 1 ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
+        auto token = [&](uint32_t j) { return base + (every ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
         ft = token(chunk * TB + lt);
         const uint64_t g = (uint64_t)ft * C + head * SZ + le;
         fk = load_vec4(k + g), fr = load_vec4(r + g), fv = load_vec4(v + g);
@@ -202,7 +219,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
         }
         bool held = false;
         for (base = 0; base < A; base += kSlotScan) {
-            n = slot_tokens(cursors, base, A, slot, slots, list, count);
+            n = slot_tokens(cursors, base, A, slot, slots, every, list, count);
             if (n == 0) continue;
             fetch(0);
             if (!held) {
@@ -301,7 +318,10 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
     __shared__ uint32_t csh[2][TB], tsh[2][TB]; // cursors and numbers of the chunk's tokens
     __shared__ uint8_t list[kSlotScan];
     __shared__ uint32_t count[kSlotScan / 64];
-    const uint32_t head = blockIdx.x, slot = blockIdx.y, slots = vs.shape[2], tid = threadIdx.x;
+    const uint32_t head = blockIdx.x, slots = vs.shape[2], tid = threadIdx.x;
+    const bool every = slots == 1 || A == 1;
+    uint32_t slot;
+    if (!own_slot(cursors, A, slots, &slot)) return;
     const uint32_t l = tid % L;
     const uint32_t C = SZ * H;
     const uint64_t plane = (uint64_t)A * C; // n_ holds k, v, a, kk one after the other
@@ -317,7 +337,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
     uint32_t fc = 0, ft = 0, fct = 0;
     uint32_t base = 0, n = 0;
     auto fetch = [&](uint32_t chunk) {
-        auto token = [&](uint32_t j) { return base + (slots == 1 ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
+        auto token = [&](uint32_t j) { return base + (every ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
         ft = token(chunk * TB + lt);
         const uint64_t g = (uint64_t)ft * C + head * SZ + le;
         fr = load_vec4(r + g), fw = load_vec4(w + g), fk = load_vec4(n_ + g), fv = load_vec4(n_ + plane + g);
@@ -344,7 +364,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
         float s[JL][CPT];
         bool held = false;
         for (base = 0; base < A; base += kSlotScan) {
-            n = slot_tokens(cursors, base, A, slot, slots, list, count);
+            n = slot_tokens(cursors, base, A, slot, slots, every, list, count);
             if (n == 0) continue;
             fetch(0);
             if (!held) {
@@ -434,7 +454,12 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
     }
 }
 
-// State slots a cursor can name: 8 bits, the last slot of the view for what lies beyond it.
-inline uint32_t slot_grid(const ViewArgs &vs) { return vs.shape[2] < 256u ? vs.shape[2] : 256u; }
+// Workgroups per head: one per state slot a cursor can name (8 bits, the last slot of the view for what lies beyond it), and no
+// more than tokens: idle slots are workgroups that look at the cursors and end, and a state holds more slots than a short run
+// names (64 heads, one request of one token, v6 gate form: 7.1 -> 4.9 us with 32 slots, 22.9 -> 4.9 with 256; one slot 4.9).
+inline uint32_t slot_grid(const ViewArgs &vs, uint32_t A) {
+    const uint32_t slots = vs.shape[2] < 256u ? vs.shape[2] : 256u;
+    return A < slots ? A : slots;
+}
 
 } // namespace wrq

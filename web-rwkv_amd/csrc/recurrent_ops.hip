@@ -207,7 +207,7 @@ int time_mix(const char *name, bool token_decay, wrq_stream stream, const wrq_te
     const uint32_t *cur = static_cast<const uint32_t *>(cursors->data);
     const float *td = static_cast<const float *>(time_decay->data), *tfp = static_cast<const float *>(time_first->data);
     float *sp = static_cast<float *>(state->data);
-    const dim3 grid(H, slot_grid(vs));
+    const dim3 grid(H, slot_grid(vs, A));
 #define WRQ_TM_LAUNCH(XT, SZ, TD)                                                                                                                \
     hipLaunchKernelGGL((time_mix_kernel<XT, SZ, TD, false>), grid, dim3(256), 0, hs, cur, td, tfp, sp, static_cast<const XT *>(k->data),           \
                        static_cast<const XT *>(v->data), static_cast<const XT *>(r->data), static_cast<XT *>(x->data), vs, H, A, GateArgs{})
