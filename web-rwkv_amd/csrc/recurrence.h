@@ -107,13 +107,18 @@ __device__ __forceinline__ bool keeps_input(const uint32_t *tokens, const uint32
 // reduction over the lanes and a branch for the store at each of them.  `token(tt, u)` leaves its result in lane u of the L
 // that share the columns, `flush(from, count)` then stores the group at once.
 // 32 heads of 64, one request: v6 gate form 100 tokens 31.0 -> 27.2 us, 255 tokens 72.5 -> 62.1; v7, whose tokens are a chain through
-// sa, 45.4 -> 44.4 and 109.0 -> 106.1; one token unchanged (4.5 and 5.0 us).
-template <int L, typename Token, typename Flush>
+// sa, 45.4 -> 44.4 and 109.0 -> 106.1.  Reads ahead stop at every second token where a lane holds up to eight rows: over the
+// whole group they took up to 250 registers, two waves per SIMD instead of three, and were slower in the end (v6 gate form 27.7 -> 25.6 us, v7
+// 45.2 -> 39.1 at 100 tokens; 32 requests of one token 15.7 -> 15.0).  With 16 rows and more per lane they are left as they fall.
+template <int L, int JL, typename Token, typename Flush>
 __device__ __forceinline__ void walk_tokens(uint32_t tend, Token token, Flush flush) {
     uint32_t tt = 0;
     for (; tt + L <= tend; tt += L) {
 #pragma unroll
-        for (int u = 0; u < L; u++) token(tt + u, u);
+        for (int u = 0; u < L; u++) {
+            token(tt + u, u);
+            if (JL <= 8 && u % 2) __builtin_amdgcn_sched_barrier(0);
+        }
         flush(tt, (uint32_t)L);
     }
     if (tt == tend) return;
@@ -121,17 +126,11 @@ __device__ __forceinline__ void walk_tokens(uint32_t tend, Token token, Flush fl
     flush(tt, tend - tt);
 }
 
-// Outputs of a group of tokens of one slot, token l in lane l; the layer's input is read before x is overwritten.
+// Outputs of a group of tokens of one slot, token l in lane l.
 template <int N, typename XT>
-__device__ __forceinline__ void store_tokens(uint32_t count, uint32_t l, const uint32_t *tokens, const uint32_t *cursors, const float (&y)[N], XT *x, float *state,
-                                             const ViewArgs &vs, uint32_t slot, uint32_t C, uint32_t chan) {
-    const uint32_t t = tokens[min(l, count - 1)];
-    const uint64_t ti = (uint64_t)t * C + chan;
+__device__ __forceinline__ void store_tokens(uint32_t count, uint32_t l, const uint32_t *tokens, const float (&y)[N], XT *x, uint32_t C, uint32_t chan) {
     if (l >= count) return;
-    if (keeps_input(tokens, cursors, l, count)) {
-#pragma unroll
-        for (int c = 0; c < N; c++) state[view_elem(vs, slot, 0, chan + c)] = load_one(x + ti + c);
-    }
+    const uint64_t ti = (uint64_t)tokens[l] * C + chan;
 #pragma unroll
     for (int c = 0; c < N; c++) {
         if constexpr (sizeof(XT) == 2) x[ti + c] = f2h(y[c]);
@@ -185,7 +184,16 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
     uint2 gw = make_uint2(0, 0), gb = make_uint2(0, 0);
     if constexpr (GATE) gw = *reinterpret_cast<const uint2 *>(ga.gn_w + head * SZ + le), gb = *reinterpret_cast<const uint2 *>(ga.gn_b + head * SZ + le);
     float4 fk, fr, fw, fv;
-    uint2 fg = make_uint2(0, 0), fx = make_uint2(0, 0);
+    // the layer's input, which row 0 of the slot's state keeps, comes with the operands of its chunk: read where it is stored it
+    // is a round trip to memory at the end of every run (32 heads of 64, one token: v6 5.06 -> 4.72 us, v7 5.49 -> 5.10)
+    using IT = std::conditional_t<GATE, uint16_t, XT>;
+    using IV = std::conditional_t<sizeof(IT) == 2, uint2, float4>;
+    const IT *in;
+    if constexpr (GATE) in = ga.att_x;
+    else in = x;
+    uint2 fg = make_uint2(0, 0);
+    IV fx = {};
+    bool first_pass = true; // over the columns: the later ones find x overwritten
     uint32_t fc = 0, ft = 0, fct = 0;
     uint32_t base = 0, n = 0;
     auto fetch = [&](uint32_t chunk) {
@@ -194,7 +202,8 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
         const uint64_t g = (uint64_t)ft * C + head * SZ + le;
         fk = load_vec4(k + g), fr = load_vec4(r + g), fv = load_vec4(v + g);
         if constexpr (TOKEN_DECAY) fw = load_vec4(time_decay + g);
-        if constexpr (GATE) fg = *reinterpret_cast<const uint2 *>(ga.g + g), fx = *reinterpret_cast<const uint2 *>(ga.att_x + g);
+        if constexpr (GATE) fg = *reinterpret_cast<const uint2 *>(ga.g + g);
+        if (SZ <= 64 || first_pass) fx = *reinterpret_cast<const IV *>(in + g);
         if (GATE) fc = cursors[ft];
         else if (tid < (uint32_t)TB) fct = token(chunk * TB + tid), fc = cursors[fct];
     };
@@ -212,6 +221,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
         const uint32_t i = i0 + CPT * (tid / L);
         const bool live = i < SZ; // head sizes below 64 leave waves without a column
         const uint32_t chan = head * SZ + min(i, (uint32_t)(SZ - CPT));
+        float *const rows = state + view_elem(vs, slot, l * JL + 1, chan); // the lane's rows of S, one row of the state apart
         float s[JL][CPT], wc[TOKEN_DECAY ? 1 : JL]; // wc: the constant decay of this lane's rows
         if constexpr (!TOKEN_DECAY) {
 #pragma unroll
@@ -224,7 +234,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
             fetch(0);
             if (!held) {
 #pragma unroll
-                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], state + view_elem(vs, slot, l * JL + jj + 1, chan));
+                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], rows + (uint64_t)jj * vs.stride[0]);
                 held = true;
             }
             const uint32_t nchunk = (n + TB - 1) / TB;
@@ -232,11 +242,14 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
             stage(0);
             for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
                 const int buf = chunk & 1;
-                const uint2 cg = fg, cx = fx;
+                const uint2 cg = fg;
+                const IV cx = fx;
                 const uint32_t ct = ft;
                 if (chunk + 1 < nchunk) fetch(chunk + 1);
                 __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
                 const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
+                if (!GATE && first_pass && lt < tend && keeps_input(tsh[buf], csh[buf], lt, tend))
+                    *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                 if (live) {
                     float yo[CPT] = {}; // y of token u of a group of L in lane u of the L that share the columns
                     auto token = [&](uint32_t tt, int u) {
@@ -274,18 +287,18 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
                             yo[c] = l == (uint32_t)u ? y[c] : yo[c];
                         }
                     };
-                    walk_tokens<L>(tend, token, [&](uint32_t from, uint32_t count) {
+                    walk_tokens<L, JL>(tend, token, [&](uint32_t from, uint32_t count) {
                         if constexpr (GATE) {
                             if (l < count) store_cols(&ysh[(from + l) * SZ + i], yo);
                         } else {
-                            store_tokens(count, l, tsh[buf] + from, csh[buf] + from, yo, x, state, vs, slot, C, chan);
+                            store_tokens(count, l, tsh[buf] + from, yo, x, C, chan);
                         }
                     });
                 }
                 if constexpr (GATE) {
                     __syncthreads(); // the chunk's y are in LDS
                     if (lt < tend) {
-                        if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
+                        if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
                         const float b = bonus[buf][lt];
                         const float4 o = head_norm(make_float4(fmaf(b, v4.x, y0.x), fmaf(b, v4.y, y0.y), fmaf(b, v4.z, y0.z), fmaf(b, v4.w, y0.w)), gw, gb, ga.eps);
@@ -299,8 +312,9 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
         }
         if (live && held) {
 #pragma unroll
-            for (int jj = 0; jj < JL; jj++) store_cols(state + view_elem(vs, slot, l * JL + jj + 1, chan), s[jj]);
+            for (int jj = 0; jj < JL; jj++) store_cols(rows + (uint64_t)jj * vs.stride[0], s[jj]);
         }
+        first_pass = false;
     }
 }
 
@@ -333,7 +347,14 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
         u4 = load_vec4(first + head * SZ + le);
     }
     float4 fr, fw, fk, fv, fa, fkk;
-    uint2 fg = make_uint2(0, 0), fx = make_uint2(0, 0);
+    using IT = std::conditional_t<GATE, uint16_t, XT>;
+    using IV = std::conditional_t<sizeof(IT) == 2, uint2, float4>;
+    const IT *in;
+    if constexpr (GATE) in = ga.att_x;
+    else in = x;
+    uint2 fg = make_uint2(0, 0);
+    IV fx = {};
+    bool first_pass = true; // over the columns: the later ones find x overwritten
     uint32_t fc = 0, ft = 0, fct = 0;
     uint32_t base = 0, n = 0;
     auto fetch = [&](uint32_t chunk) {
@@ -342,7 +363,8 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
         const uint64_t g = (uint64_t)ft * C + head * SZ + le;
         fr = load_vec4(r + g), fw = load_vec4(w + g), fk = load_vec4(n_ + g), fv = load_vec4(n_ + plane + g);
         fa = load_vec4(n_ + 2 * plane + g), fkk = load_vec4(n_ + 3 * plane + g);
-        if constexpr (GATE) fg = *reinterpret_cast<const uint2 *>(ga.g + g), fx = *reinterpret_cast<const uint2 *>(ga.att_x + g);
+        if constexpr (GATE) fg = *reinterpret_cast<const uint2 *>(ga.g + g);
+        if (SZ <= 64 || first_pass) fx = *reinterpret_cast<const IV *>(in + g);
         if (GATE) fc = cursors[ft];
         else if (tid < (uint32_t)TB) fct = token(chunk * TB + tid), fc = cursors[fct];
     };
@@ -361,6 +383,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
         const uint32_t i = i0 + CPT * (tid / L);
         const bool live = i < SZ; // head sizes below 64 leave waves without a column
         const uint32_t chan = head * SZ + min(i, (uint32_t)(SZ - CPT));
+        float *const rows = state + view_elem(vs, slot, l * JL + 1, chan); // the lane's rows of S, one row of the state apart
         float s[JL][CPT];
         bool held = false;
         for (base = 0; base < A; base += kSlotScan) {
@@ -369,7 +392,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
             fetch(0);
             if (!held) {
 #pragma unroll
-                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], state + view_elem(vs, slot, l * JL + jj + 1, chan));
+                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], rows + (uint64_t)jj * vs.stride[0]);
                 held = true;
             }
             const uint32_t nchunk = (n + TB - 1) / TB;
@@ -377,11 +400,14 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
             stage(0);
             for (uint32_t chunk = 0; chunk < nchunk; chunk++) {
                 const int buf = chunk & 1;
-                const uint2 cg = fg, cx = fx;
+                const uint2 cg = fg;
+                const IV cx = fx;
                 const uint32_t ct = ft;
                 if (chunk + 1 < nchunk) fetch(chunk + 1);
                 __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
                 const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
+                if (!GATE && first_pass && lt < tend && keeps_input(tsh[buf], csh[buf], lt, tend))
+                    *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                 if (live) {
                     float yo[CPT] = {}; // y of token u of a group of L in lane u of the L that share the columns
                     auto token = [&](uint32_t tt, int u) {
@@ -422,18 +448,18 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
                             yo[c] = l == (uint32_t)u ? y : yo[c];
                         }
                     };
-                    walk_tokens<L>(tend, token, [&](uint32_t from, uint32_t count) {
+                    walk_tokens<L, JL>(tend, token, [&](uint32_t from, uint32_t count) {
                         if constexpr (GATE) {
                             if (l < count) store_cols(&ysh[(from + l) * SZ + i], yo);
                         } else {
-                            store_tokens(count, l, tsh[buf] + from, csh[buf] + from, yo, x, state, vs, slot, C, chan);
+                            store_tokens(count, l, tsh[buf] + from, yo, x, C, chan);
                         }
                     });
                 }
                 if constexpr (GATE) {
                     __syncthreads(); // the chunk's y are in LDS
                     if (lt < tend) {
-                        if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const uint16_t *>(&cx));
+                        if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
                         const float4 k4 = *reinterpret_cast<const float4 *>(&ks[buf][4 * tid]), r4 = *reinterpret_cast<const float4 *>(&rs[buf][4 * tid]);
                         const float b = lanes_sum<16>((u4.x * k4.x * r4.x + u4.y * k4.y * r4.y) + (u4.z * k4.z * r4.z + u4.w * k4.w * r4.w));
@@ -449,8 +475,9 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
         }
         if (live && held) {
 #pragma unroll
-            for (int jj = 0; jj < JL; jj++) store_cols(state + view_elem(vs, slot, l * JL + jj + 1, chan), s[jj]);
+            for (int jj = 0; jj < JL; jj++) store_cols(rows + (uint64_t)jj * vs.stride[0], s[jj]);
         }
+        first_pass = false;
     }
 }
 
