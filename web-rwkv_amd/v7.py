@@ -62,10 +62,12 @@ class Runtime:
 
     def __init__(self, torch, C, hidden, A):
         z = lambda *s: torch.zeros(s, dtype=torch.float16, device="cuda")
-        for name in ("x", "att_x", "att_v0", "att_rx", "att_wx", "att_kx", "att_vx", "att_ax", "att_gx", "att_r", "att_w", "att_k", "att_v", "att_a",
-                     "att_g", "att_o", "att_kk", "att_vv", "ffn_x", "ffn_kx", "ffn_v"):
+        for name in ("x", "att_x", "att_v0", "att_rx", "att_wx", "att_kx", "att_vx", "att_ax", "att_gx", "att_r", "att_w", "att_g", "att_o", "att_vv",
+                     "ffn_x", "ffn_kx", "ffn_v"):
             setattr(self, name, z(1, A, C))
         self.att_n = z(4, A, C)
+        # the planes of att_n and what the op list copies into them are one: the fused form then stores each value once
+        self.att_k, self.att_v, self.att_a, self.att_kk = (self.att_n[i:i + 1] for i in range(4))
         self.aux_w, self.aux_a, self.aux_g, self.aux_v = z(1, A, RANK_W), z(1, A, RANK_A), z(1, A, RANK_G), z(1, A, RANK_V)
         self.ffn_k = z(1, A, hidden)
         self.x2 = z(1, A, C)  # the residual between the two halves of a layer on the fused path
@@ -139,7 +141,7 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now
     FusedV7.adapters_in(C, A, adapters[:3] if index == 0 else adapters)
     FusedV7.mid(S, H, A, index == 0, [buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v], [w["w2"], w["a2"], w["g2"], w["v2"]],
                 [t["w0"], t["a0"], t["v0"], t["k_k"], t["k_a"]], L2_EPS, buf.att_k, buf.att_v, buf.att_v0, buf.att_w, buf.att_g, buf.att_n,
-                [buf.att_k, buf.att_v, buf.att_a, buf.att_kk, buf.att_vv])
+                [None if b.data_ptr() == plane.data_ptr() else b for b, plane in zip((buf.att_k, buf.att_v, buf.att_a, buf.att_kk), buf.att_n)] + [buf.att_vv])
     FusedV7.wkv_gate(S, H, A, cursors, state, att_state, buf.att_r, buf.att_w, buf.att_n, t["r_k"], buf.att_g, t["gn_w"], t["gn_b"], GN_EPS, buf.att_x)
     m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)
     FusedV7.pre(C, A, cursors, buf.x, buf.att_o, buf.x2, t["ffn_ln_w"], t["ffn_ln_b"], LN_EPS, state, ffn_state, [t["ffn_x_k"]], buf.ffn_x, [buf.ffn_kx])
