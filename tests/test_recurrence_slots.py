@@ -150,3 +150,44 @@ def test_gpu_more_slots_than_tokens(gpu, form, B, runs):
     want = state.clone()
     want[named] = outs[1][1]
     assert torch.equal(outs[0][1], want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("version", [6, 7])
+@pytest.mark.parametrize("B,runs", [(6, [(4, 15), (1, 241), (4, 17), (0, 3), (5, 1)]), (2, [(0, 250), (1, 2), (0, 20), (1, 255), (0, 9)]), (1, [(0, 255), (0, 255), (0, 3)])])
+def test_gpu_fused_beyond_one_scan_of_the_cursors(gpu, version, B, runs):
+    """The gate forms over more tokens than one scan of the cursors (256), a slot that comes again behind the edge and a
+    single one: output and whole state against the op list (recurrence, group norm, gate) on the same operands."""
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("gate forms beyond one scan", version, B, runs, flush=True)
+    H, S = 2, 64
+    C, cur = H * S, lop.pack_cursors(runs)
+    A = len(cur)
+    g = torch.Generator().manual_seed(0x575B + A)
+    f32 = lambda *s: (torch.randn(s, generator=g) * 0.3).cuda()
+    f16 = lambda *s: f32(*s).half()
+    curd, view = torch.from_numpy(cur.view(np.int32)).cuda(), ((C, S + 1, B), (C, S + 2, B), (0, 0, 0))
+    state, x, gate, gw, gb = f32(B, S + 2, C), f16(A, H, S), f16(A, H, S), f16(H, S), f16(H, S)
+    want, y = state.clone(), None
+    if version == 6:
+        k, v, r, u, w = f32(A, H, S), f32(A, H, S), f32(A, H, S), f32(H, S), torch.sigmoid(f32(A, H, S))
+        y = x.float()
+        gpu.LayerOp.time_mix_v6(curd, w, u, want, k, v, r, y, state_view=view)
+        gpu.LayerOp.group_norm(gw, gb, y, 64e-5)
+        y = y.half()
+        gpu.LayerOp.mul_activate(gate, y, gpu.ACT_SILU)
+        gpu.FusedV6.wkv_gate(S, H, A, curd, w, u, state, view, k, v, r, gate, gw, gb, 64e-5, x)
+    else:
+        r, w, n, u = f16(A, H, S), f16(A, H, S), f16(4, A, H, S), f16(H, S)
+        y = x.clone()
+        gpu.LayerOp.time_mix_v7(curd, want, r, w, n, y, state_view=view)
+        gpu.LayerOp.group_norm(gw, gb, y, 64e-5)
+        gpu.LayerOp.time_first_v7(u, r, n, y)
+        gpu.LayerOp.mul(gate, y)
+        gpu.FusedV7.wkv_gate(S, H, A, curd, state, view, r, w, n, u, gate, gw, gb, 64e-5, x)
+    # the same roundings to f16 on both sides; f32 sums in another order flip one here and there: an ulp (2^-10) of values up to 4
+    assert_close(x.cpu().numpy(), y.cpu().numpy(), 4e-3, "gated output")
+    assert_close(state.cpu().numpy(), want.cpu().numpy(), 1e-6, "state")

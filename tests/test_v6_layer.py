@@ -95,7 +95,8 @@ def test_v6_layer_against_numpy(gpu, oracle, quant, runs):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant", ["int8", "nf4"])
-@pytest.mark.parametrize("runs", [[(2, 3), (0, 1), (5, 4)], [(1, 20), (3, 12)], [(4, 1)]], ids=["8 tokens", "32 tokens (chunk kernels)", "1 token"])
+@pytest.mark.parametrize("runs", [[(2, 3), (0, 1), (5, 4)], [(1, 20), (3, 12)], [(4, 1)], [(1, 9), (0, 230), (4, 14), (2, 41), (5, 2)]],
+                         ids=["8 tokens", "32 tokens (chunk kernels)", "1 token", "296 tokens"])
 def test_v6_layer_fused_equals_op_list(gpu, oracle, quant, runs):
     # the 12-launch form of the layer against the op list: same buffers, same roundings
     import torch

@@ -1,5 +1,5 @@
 """Two consecutive RWKV-v7 layers (the first keeps its values as `v0`, the second mixes its own with
-them), dispatched op by op like the reference (src/runtime/v7.rs:704-1006), on the GPU through the
+them), fused and op by op like the reference (src/runtime/v7.rs:704-1006), on the GPU through the
 library against a numpy composition of the oracle's restatements."""
 import importlib
 import os
@@ -59,7 +59,8 @@ def layer_numpy(lop, w, x, v0, state, cursors, H, S, index):
 @pytest.mark.gpu
 @pytest.mark.parametrize("quant", ["int8", "nf4"])
 @pytest.mark.parametrize("runs", [[(2, 3), (0, 1), (5, 4)], [(1, 20), (3, 12)], [(4, 1)]], ids=["8 tokens", "32 tokens (chunk kernels)", "1 token"])
-def test_v7_layers_against_numpy(gpu, oracle, quant, runs):
+@pytest.mark.parametrize("form", ["dispatch_layer", "dispatch_layer_ops"])
+def test_v7_layers_against_numpy(gpu, oracle, quant, runs, form):
     import torch
 
     sys.path.insert(0, ROOT)
@@ -90,7 +91,8 @@ def test_v7_layers_against_numpy(gpu, oracle, quant, runs):
         want_state = state.copy()
         want, v0 = layer_numpy(lop, wq, want, v0, want_state, cursors, H, S, index)
         sd = torch.from_numpy(state.copy()).cuda()
-        v7.dispatch_layer(layer, buf, sd, curd, A, H, S, index)
+        assert v7.fused_is_built(layer, H, S, buf, curd, A)  # which dispatch_layer then takes
+        getattr(v7, form)(layer, buf, sd, curd, A, H, S, index)
         torch.cuda.synchronize()
         got = buf.x.cpu().numpy()[0]
         # f16 buffers between 50 ops: a few f16 ulps of the O(1) activations
@@ -126,7 +128,7 @@ def test_v7_layer_packed_token_shifts_equal_the_op_list(gpu, runs):
         buf.x.copy_(torch.from_numpy(x).cuda().reshape(1, A, C))
         buf.att_v0.copy_(torch.from_numpy(x[::-1].copy()).cuda().reshape(1, A, C))
         sd = torch.from_numpy(state.copy()).cuda()
-        v7.dispatch_layer(layer, buf, sd, curd, A, H, S, 1, shifts=v7.PackedShifts(torch, layer, A) if packed else None)
+        v7.dispatch_layer_ops(layer, buf, sd, curd, A, H, S, 1, shifts=v7.PackedShifts(torch, layer, A) if packed else None)
         torch.cuda.synchronize()
         outs.append((buf.x.cpu().numpy(), sd.cpu().numpy()))
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
@@ -261,3 +263,40 @@ def test_v7_mid_of_the_first_layer_needs_no_adapter_v(gpu):
     for a, b in zip(*outs):
         assert torch.equal(a, b)
     assert torch.equal(outs[0][0], v) and torch.equal(outs[0][3][1], v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 17, 65], ids=lambda h: f"{64 * h} channels")
+@pytest.mark.parametrize("B,runs", [(6, [(1, 9), (0, 230), (4, 14), (2, 41), (5, 2)]), (1, [(0, 255), (0, 45)])], ids=["slots", "one slot"])
+def test_v7_layer_fused_beyond_one_scan_of_the_cursors(gpu, B, runs, H):
+    # runs of more than 256 tokens, the fused layer against the op list.  Either side is 7e-4 of the norm away from 64 bits
+    # (roundings of the f16 buffers), so they differ by up to 1e-3 of it; of 1.2 million values of rms 1.2 the largest
+    # difference is then 4.9 sigma = 6e-3
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    v7 = importlib.import_module(gpu.__name__ + ".v7")
+    print("v7 layer beyond 256 tokens", runs, H, flush=True)
+    S, hidden = 64, 256
+    C = H * S
+    rng = np.random.default_rng(SEED + 160 + H)
+    cursors = lop.pack_cursors(runs)
+    A = len(cursors)
+    curd = torch.from_numpy(cursors.view(np.int32)).cuda()
+    layer = v7.Layer(torch, v7.random_layer_weights(rng, C, H, S, hidden), "int8")
+    x, v0 = (rng.standard_normal((1, A, C)).astype(np.float16) for _ in range(2))
+    state = (0.1 * rng.standard_normal((B, S + 2, C))).astype(np.float32)
+    outs = []
+    for dispatch in (v7.dispatch_layer_ops, v7.dispatch_layer):
+        buf = v7.Runtime(torch, C, hidden, A)
+        assert v7.fused_is_built(layer, H, S, buf, curd, A)
+        buf.x.copy_(torch.from_numpy(x).cuda())
+        buf.att_v0.copy_(torch.from_numpy(v0).cuda())
+        sd = torch.from_numpy(state.copy()).cuda()
+        dispatch(layer, buf, sd, curd, A, H, S, 1)
+        torch.cuda.synchronize()
+        outs.append((buf.x.cpu().numpy().astype(np.float64), sd.cpu().numpy().astype(np.float64)))
+    for i, what in enumerate(("layer output", "state")):
+        assert_close(outs[1][i], outs[0][i], 8e-3, what)
+        assert np.linalg.norm(outs[1][i] - outs[0][i]) < 1.5e-3 * np.linalg.norm(outs[0][i]), what
