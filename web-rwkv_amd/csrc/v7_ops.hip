@@ -397,10 +397,12 @@ int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void
         aa.rank[i] = ranks[i], aa.act[i] = acts[i];
         tiles += ranks[i] / 16;
     }
-    // Ten steps in flight where eight waves then take K in one go (2560 channels, 160 rows, 100 tokens: 9.7 -> 7.1 us), and
-    // sixteen waves of ten beyond 4096 channels (5120: 13.1 -> 11.5 us; at 4096 sixteen waves of eight steps gained nothing: 9.7 us).
+    // Steps of 32 channels that the waves of a workgroup have in flight at once: eight waves of eight take K in one go up to 64
+    // steps, of ten up to 80 (2560 channels, 160 rows, 100 tokens: 9.7 -> 7.1 us); up to 128 (4096 channels) eight of eight go
+    // round twice (9.7 us; sixteen of eight gained nothing), beyond sixteen of ten (5120 channels: 13.1 -> 11.8 us).
+    const uint32_t steps = C / 32;
     auto go = [&](auto kern, int waves) { hipLaunchKernelGGL(kern, dim3(tiles, (A + 15) / 16), dim3(64 * waves), 0, static_cast<hipStream_t>(stream), C, A, aa); };
-    C > 4096 ? go(adapters_in_kernel<16, 10>, 16) : C > 2048 && C <= 2560 ? go(adapters_in_kernel<8, 10>, 8) : go(adapters_in_kernel<8, 8>, 8);
+    steps > 128 ? go(adapters_in_kernel<16, 10>, 16) : steps > 64 && steps <= 80 ? go(adapters_in_kernel<8, 10>, 8) : go(adapters_in_kernel<8, 8>, 8);
     return check_launch(what);
 }
 

@@ -130,10 +130,13 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
     ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
     slice_of = lambda i: ((C, A, 1), (C, A, 5), (0, 0, i))
 
-    # First half of an adapter: the launch of small tiles where it beats the f16 product, which is a one-shot kernel up to 4
-    # tokens and splits K beyond (160 rows: 2048 channels 5.2 against 6.9 us at 5 tokens, 6.2 against 8.3 at 100; 768 channels
-    # 6.1 against 5.0 at 16, 6.2 against 8.5 at 32; 5120 channels 9.8 against 7.9 at 8, 11.4 against 10.5 at 100).
-    tiles = C <= 2560 and A > (16 if C <= 1024 else 4)
+    # First half of an adapter: the launch of small tiles where it beats the f16 product, which is a one-shot kernel up to 4 tokens
+    # (below 1024 channels up to 16) and splits K beyond.  us, tiles against product, 160 and 64 rows: 768 channels 6.4 / 5.2 and
+    # 6.4 / 5.1 at 16 tokens, 6.4 / 9.3 and 6.4 / 9.0 at 17, 13.6 / 12.8 and 6.7 / 12.7 at 1024 (both adapters together still
+    # tiles); 1024 channels 5.5 / 7.3 and 5.4 / 7.0 at 5; 2560 channels 6.2 / 8.1 and 6.1 / 7.1 at 5, 7.4 / 10.1 and 7.4 / 9.9 at
+    # 100; 3072 channels 8.7 / 8.0 and 8.7 / 7.2 at 8, 10.1 / 10.3 and 10.0 / 10.2 at 100, 17.2 / 13.8 and 10.2 / 13.4 at 512;
+    # 5120 channels 10.1 / 8.2 and 10.1 / 7.7 at 8, 11.8 / 10.9 and 11.7 / 10.7 at 100.
+    tiles = C <= 2560 and A > (4 if C >= 1024 else 16)
 
     def adapter_in(name, x, out):
         if tiles:
@@ -158,7 +161,9 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
     FusedV6.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_r, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now)
 
 
-FUSED_MAX_TOKENS = 65535  # what the fused ops take
+# What the fused ops take.  Measured up to 2048 tokens (32 requests; 0.14 of the op list's time at 768 channels, 0.55 at 5120) and
+# 255 of one request (0.53 to 0.72); nowhere is the op list faster.
+FUSED_MAX_TOKENS = 65535
 VECTORS = ("att_ln_w", "att_ln_b", "ffn_ln_w", "ffn_ln_b", "time_mix_x", "time_decay", "gn_w", "gn_b", "ffn_time_mix_k", "ffn_time_mix_r")
 FUSED_ROWS = ("x", "x2", "att_x", "att_xx", "att_g", "att_o", "ffn_x", "ffn_kx", "ffn_rx", "ffn_v", "ffn_r")
 
