@@ -694,10 +694,16 @@ def v7_layers(wrq, torch, args):
     cursors = torch.from_numpy(np.full(A, (min(A, 255) << 24), dtype=np.uint32).view(np.int32)).cuda()
     shifts = [v7.PackedShifts(torch, layer, A) for layer in layers] if args.packed_shifts else None
 
+    dispatch = v7.dispatch_layer_ops if args.op_list else v7.dispatch_layer
+    if args.op_list or not v7.fused_is_built(layers[0], heads, S, buf, cursors, A, shifts[0] if shifts else None):
+        form = "37 calls per layer (the six token shifts in one)" if shifts else "42 calls per layer (39 in the first)"
+    else:
+        form = "11 launches per layer (fused small ops, the six token shifts in one)" if shifts else "10 launches per layer (fused small ops)"
+
     def step():
         buf.x.copy_(x0)  # the embedding of the next token would land here
         for i, (layer, st) in enumerate(zip(layers, states)):
-            v7.dispatch_layer(layer, buf, st, cursors, A, heads, S, i, shifts=shifts[i] if shifts else None)
+            dispatch(layer, buf, st, cursors, A, heads, S, i, shifts=shifts[i] if shifts else None)
 
     step()
     torch.cuda.synchronize()
@@ -713,7 +719,7 @@ def v7_layers(wrq, torch, args):
     print(json.dumps({"metric": "RWKV-v7 7B-shape layers, every op (no embedding, no head), tokens/s", "value": round(A * 1e3 / wall_ms, 2), "unit": "tok/s",
                       "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(wall_ms, 4), "gpu_ms_per_step": round(ms, 4),
                       "config": {"workload": f"{args.layers} v7 layers ({C} x {hidden}, {heads} heads), {args.quant}, {A} token(s) of one request per step, "
-                                             + ("46 ops per layer (the six token shifts in one launch)" if args.packed_shifts else "51 ops per layer (47 in the first)") + ", the three independent projections in one launch", "hip_graph": not args.no_graph}, "data": "synthetic"}))
+                                             + form + ", the three independent projections in one launch", "hip_graph": not args.no_graph}, "data": "synthetic"}))
 
 
 def ops_table(wrq, torch, args, C):
@@ -805,6 +811,7 @@ def main():
     ap.add_argument("--full-model", action="store_true", help="--full-layers plus embedding, head and softmax: a whole model step")
     ap.add_argument("--v7-layers", action="store_true",
                     help="every op of RWKV-v7 layers at the 7B shape (4096 channels, 64 heads, FFN 16384): --layers of them, --tokens per step")
+    ap.add_argument("--op-list", action="store_true", help="with --v7-layers: the ops one by one instead of the fused form")
     ap.add_argument("--packed-shifts", action="store_true", help="with --v5-model / --v7-layers: the token shifts of each half of a layer in one launch")
     ap.add_argument("--loader", action="store_true",
                     help="the C++ loader: the f16 matrices of --layers 7B-shape layers from a safetensors file into Int8 matrices (file -> device -> pack)")

@@ -13,7 +13,7 @@
 //
 // Fused forms of the layer's small ops (src/runtime/v7.rs:704-1006), which are bound by their launches at the run
 // lengths of a serving schedule: wrq_adapters_in, wrq_v7_mid, wrq_v7_wkv_gate, wrq_v7_post_ffn (with wrq_fused_pre of
-// fused_ops.hip).  A layer takes 10 launches beside the second ones of split products instead of 45.
+// fused_ops.hip).  A layer takes 10 launches beside the second ones of split products instead of 42.
 #include "recurrence.h"
 
 namespace wrq {
@@ -90,7 +90,7 @@ struct MidArgs {
 // one token and finishes them in registers with the roundings to f16 the op list has:
 //   w = w0 + w2 aux_w;   a = sigmoid(a0 + a2 aux_a);   g = g2 aux_g;   v <- mix(v, v0, sigmoid(v_0 + v2 aux_v)) (FIRST: v0 <- v);
 //   kk = l2_norm(k k_k) over the head;   k <- k (1 + (a - 1) k_a);   n = (k, v, a, kk)
-// (src/runtime/v7.rs:780-880).  2048 channels, 32 tokens: 5.8 us against about 60 us for the 17 launches of the list; bound by one
+// (src/runtime/v7.rs:780-880).  2048 channels, 32 tokens: 5.0 us (5.6 with the list's buffers) against about 60 us for the 16 launches of the list; bound by one
 // round trip to memory, which is why every operand is requested before the first use.
 template <int RW, int RA, int RG, int RV, bool FIRST>
 __global__ __launch_bounds__(256) void v7_mid_kernel(uint32_t C, uint32_t T, float eps, MidArgs m) {

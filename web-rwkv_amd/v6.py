@@ -122,7 +122,9 @@ def dispatch_layer(layer, buf, state, cursors, A, H, S, rescale_now=False):
 def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False):
     """The same layer in 12 launches: the 8 quantized products (3 launches for the independent ones, 2
     alone), the first halves of the two adapters, and 5 fused launches for the 27 small ops
-    (`wrq_v6_*`).  Same buffers and results as `dispatch_layer` up to f32 summation order."""
+    (`wrq_v6_*`).  The layer's output and state are those of `dispatch_layer` up to f32 summation order;
+    of the buffers between the ops `aux_x`, `time_mix` and `time_mix_t` stay unwritten and `ffn_x` keeps the
+    normalised row."""
     t, m, C = layer.t, layer.m, H * S
     B = state.shape[0]
     fast = turbo(A)
