@@ -118,7 +118,7 @@ def test_fused_form_takes_the_adapters_of_the_matrices(wrq, monkeypatch, version
     seen = []
     for cls in ("FusedV6", "FusedV7"):
         if hasattr(mod, cls):
-            recorder = type("R", (), {n: staticmethod(lambda *a: seen.append(a)) for n in ("pre", "time_mix", "decay", "wkv_gate", "post_ffn", "adapters_in", "mid")})
+            recorder = type("R", (), {n: staticmethod(lambda *a, **k: seen.append(a)) for n in ("pre", "time_mix", "decay", "wkv_gate", "post_ffn", "adapters_in", "mid")})
             monkeypatch.setattr(mod, cls, recorder)
     monkeypatch.setattr(mod, "matmul_vec_group", lambda ops: None)
     monkeypatch.setattr(wrq.Matrix, "matmul_op", lambda self, *a, **k: seen.append((self.w, a)))

@@ -485,18 +485,24 @@ def _operands(what, A, cursors, f16=(), f32=()):
                 raise TensorError(ERR_SHAPE, f"{what}: an operand of {t.numel()} elements, {n} are needed")
 
 
-def fused_operands(f16, f32=(), adapters=()):
-    """Whether a layer's operands have the types and sizes its fused form is built for: lists of `(tensor, elements)` and of
-    `(matrix, rows, columns)` of low-rank adapters.  The op list takes more (f32 vectors and buffers, packed adapters) and
-    refuses the rest op by op, so what is not built goes there."""
-    import torch
+def fused_operands(tensors, dtype, elements):
+    """Whether tensors have the element type and the number of elements the fused form of a layer is built for, and lie in one
+    piece.  The op list takes more (f32 vectors and buffers, packed adapters) and refuses the rest op by op, so what is not
+    built goes there."""
+    for t in tensors:
+        if t.dtype is not dtype or t.numel() != elements or not t.is_contiguous():
+            return False
+    return True
 
-    for dtype, operands in ((torch.float16, f16), (torch.float32, f32)):
-        for t, n in operands:
-            if t is None or t.dtype != dtype or t.numel() != n or not t.is_contiguous():
-                return False
-    return all(m.kind == "Fp16" and m.w.dtype == torch.float16 and m.w.numel() == rows * columns and m.w.shape[-1] == columns and m.w.is_contiguous()
-               for m, rows, columns in adapters)
+
+def fused_adapters(matrices, shapes, dtype):
+    """The same of f16 low-rank adapters: `shapes` are `(name, rows, columns)`."""
+    for name, rows, columns in shapes:
+        m = matrices[name]
+        w = m.w
+        if m.kind != "Fp16" or w.dtype is not dtype or w.numel() != rows * columns or w.shape[-1] != columns or not w.is_contiguous():
+            return False
+    return True
 
 
 def fused_run(cursors, A):
@@ -506,11 +512,11 @@ def fused_run(cursors, A):
 
 class FusedV6:
     """The fused forms of a v6 layer's small ops (`wrq_v6_*`); arguments are contiguous torch tensors of the types and
-    sizes in `include/wrq.h`."""
+    sizes in `include/wrq.h`, looked at here unless the caller has (`checked`)."""
 
     @staticmethod
     def _p(t):
-        return None if t is None else C.c_void_p(t.data_ptr())
+        return None if t is None else t.data_ptr()  # the argument types are pointers already
 
     @staticmethod
     def _check_pre(what, Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts):
@@ -518,88 +524,98 @@ class FusedV6:
         _operands(what, A, cursors, [(t, A * Cn) for t in rows] + [(t, Cn) for t in (ln_w, ln_b, *factors)])
 
     @staticmethod
-    def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts):
+    def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts, checked=False):
         p = FusedV6._p
-        FusedV6._check_pre("v6_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
+        if not checked:
+            FusedV6._check_pre("v6_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
         _check(lib().wrq_v6_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
                                 p(factors[0]), p(factors[1] if len(factors) > 1 else None), p(ln_out), p(shifts[0]), p(shifts[1] if len(shifts) > 1 else None)))
 
     @staticmethod
-    def time_mix(Cn, A, lora_size, cursors, lora, w2, time_mix, state, state_view, att_x, att_sx):
+    def time_mix(Cn, A, lora_size, cursors, lora, w2, time_mix, state, state_view, att_x, att_sx, checked=False):
         p, r, n = FusedV6._p, lora_size, A * Cn
-        _operands("v6_time_mix", A, cursors, ((lora, 5 * A * r), (w2, 5 * Cn * r), (time_mix, 5 * Cn), (att_x, n), (att_sx, 5 * n)))
+        if not checked:
+            _operands("v6_time_mix", A, cursors, ((lora, 5 * A * r), (w2, 5 * Cn * r), (time_mix, 5 * Cn), (att_x, n), (att_sx, 5 * n)))
         _check(lib().wrq_v6_time_mix(_stream(), Cn, A, lora_size, p(cursors), p(lora), p(w2), p(time_mix), C.byref(as_view(state, state_view)), p(att_x), p(att_sx)))
 
     @staticmethod
-    def decay(Cn, A, lora_size, lora, w2, time_decay, out):
+    def decay(Cn, A, lora_size, lora, w2, time_decay, out, checked=False):
         p, r = FusedV6._p, lora_size
-        _operands("v6_decay", A, None, ((lora, A * r), (w2, Cn * r), (time_decay, Cn)), ((out, A * Cn),))
+        if not checked:
+            _operands("v6_decay", A, None, ((lora, A * r), (w2, Cn * r), (time_decay, Cn)), ((out, A * Cn),))
         _check(lib().wrq_v6_decay(_stream(), Cn, A, lora_size, p(lora), p(w2), p(time_decay), p(out)))
 
     @staticmethod
-    def wkv_gate(S, H, A, cursors, time_decay, time_first, state, state_view, k, v, r, g, gn_w, gn_b, eps, att_x):
+    def wkv_gate(S, H, A, cursors, time_decay, time_first, state, state_view, k, v, r, g, gn_w, gn_b, eps, att_x, checked=False):
         p, n = FusedV6._p, A * S * H
-        _operands("v6_wkv_gate", A, cursors, ((g, n), (gn_w, S * H), (gn_b, S * H), (att_x, n)), ((time_decay, n), (time_first, S * H), (k, n), (v, n), (r, n)))
+        if not checked:
+            _operands("v6_wkv_gate", A, cursors, ((g, n), (gn_w, S * H), (gn_b, S * H), (att_x, n)), ((time_decay, n), (time_first, S * H), (k, n), (v, n), (r, n)))
         _check(lib().wrq_v6_wkv_gate(_stream(), S, H, A, p(cursors), p(time_decay), p(time_first), C.byref(as_view(state, state_view)), p(k), p(v), p(r), p(g),
                                      p(gn_w), p(gn_b), eps, p(att_x)))
 
     @staticmethod
-    def post_ffn(Cn, A, cursors, state, state_view, r, v, ffn_x, x_in, x_out, rescale):
+    def post_ffn(Cn, A, cursors, state, state_view, r, v, ffn_x, x_in, x_out, rescale, checked=False):
         p, n = FusedV6._p, A * Cn
-        _operands("v6_post_ffn", A, cursors, ((r, n), (v, n), (ffn_x, n), (x_in, n), (x_out, n)))
+        if not checked:
+            _operands("v6_post_ffn", A, cursors, ((r, n), (v, n), (ffn_x, n), (x_in, n), (x_out, n)))
         _check(lib().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
 
 
 class FusedV7:
     """The fused forms of a v7 layer's small ops (`wrq_fused_pre`, `wrq_adapters_in`, `wrq_v7_*`); arguments are contiguous
-    torch tensors of the types and sizes in `include/wrq.h`.  `adapters_in` serves any layer with low-rank adapters."""
+    torch tensors of the types and sizes in `include/wrq.h`, looked at here unless the caller has (`checked`).  `adapters_in`
+    serves any layer with low-rank adapters."""
 
     @staticmethod
     def _a(ts):
         return (C.c_void_p * len(ts))(*(None if t is None else t.data_ptr() for t in ts))
 
     @staticmethod
-    def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts):
+    def pre(Cn, A, cursors, x, add, x_out, ln_w, ln_b, eps, state, state_view, factors, ln_out, shifts, checked=False):
         p, a = FusedV6._p, FusedV7._a
-        FusedV6._check_pre("fused_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
+        if not checked:
+            FusedV6._check_pre("fused_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
         if len(shifts) < len(factors):
             raise TensorError(ERR_SHAPE, f"fused_pre: {len(shifts)} outputs for {len(factors)} token shifts")
         _check(lib().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
                                    a(factors), p(ln_out), a(shifts)))
 
     @staticmethod
-    def adapters_in(Cn, A, ops):
+    def adapters_in(Cn, A, ops, checked=False):
         """`ops`: list of `(w, x, out, act)`, w [rank, C]."""
         a, n = FusedV7._a, len(ops)
         w, x, out, act = zip(*ops)
-        _operands("adapters_in", A, None, [(t, A * Cn) for t in x] + [(t, t.shape[0] * Cn) for t in w] + [(o, A * t.shape[0]) for o, t in zip(out, w)])
+        if not checked:
+            _operands("adapters_in", A, None, [(t, A * Cn) for t in x] + [(t, t.shape[0] * Cn) for t in w] + [(o, A * t.shape[0]) for o, t in zip(out, w)])
         _check(lib().wrq_adapters_in(_stream(), Cn, A, n, a(w), (C.c_uint32 * n)(*(t.shape[0] for t in w)), (C.c_int * n)(*act), a(x), a(out)))
 
     @staticmethod
-    def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n, buffers=(None,) * 5):
+    def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n, buffers=(None,) * 5, checked=False):
         p, a, Cn = FusedV6._p, FusedV7._a, S * H
         if len(aux) != 4 or len(w2) != 4 or len(vectors) != 5 or len(buffers) != 5:
             raise TensorError(ERR_SHAPE, f"v7_mid: {len(aux)}, {len(w2)}, {len(vectors)} and {len(buffers)} operands, 4, 4, 5 and 5 are needed")
         if first:  # without the adapter v
             aux, w2, vectors = [*aux[:3], None], [*w2[:3], None], [*vectors[:2], None, *vectors[3:]]
-        _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2) if w is not None] + [(w, Cn * w.shape[1]) for w in w2 if w is not None]
-                  + [(t, Cn) for t in vectors]
-                  + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g, *buffers)] + [(n, 4 * A * Cn)])
+        if not checked:
+            _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2) if w is not None] + [(w, Cn * w.shape[1]) for w in w2 if w is not None]
+                      + [(t, Cn) for t in vectors] + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g, *buffers)] + [(n, 4 * A * Cn)])
         ranks = (C.c_uint32 * 4)(*(0 if t is None else t.shape[1] for t in w2))
         _check(lib().wrq_v7_mid_buffers(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n),
                                         a(buffers)))
 
     @staticmethod
-    def wkv_gate(S, H, A, cursors, state, state_view, r, w, n, r_k, g, gn_w, gn_b, eps, att_x):
+    def wkv_gate(S, H, A, cursors, state, state_view, r, w, n, r_k, g, gn_w, gn_b, eps, att_x, checked=False):
         p, m = FusedV6._p, A * S * H
-        _operands("v7_wkv_gate", A, cursors, ((r, m), (w, m), (n, 4 * m), (r_k, S * H), (g, m), (gn_w, S * H), (gn_b, S * H), (att_x, m)))
+        if not checked:
+            _operands("v7_wkv_gate", A, cursors, ((r, m), (w, m), (n, 4 * m), (r_k, S * H), (g, m), (gn_w, S * H), (gn_b, S * H), (att_x, m)))
         _check(lib().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
                                      p(att_x)))
 
     @staticmethod
-    def post_ffn(Cn, A, cursors, state, state_view, v, ffn_x, x_in, x_out, rescale, ffn_out=None):
+    def post_ffn(Cn, A, cursors, state, state_view, v, ffn_x, x_in, x_out, rescale, ffn_out=None, checked=False):
         p, n = FusedV6._p, A * Cn
-        _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n), (ffn_out, n)))
+        if not checked:
+            _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n), (ffn_out, n)))
         _check(lib().wrq_v7_post_ffn_buffers(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale),
                                              p(ffn_out)))
 

@@ -3,11 +3,13 @@ the same ops in the same order on the same buffers, every op one library call on
 stream.  Weights are random-init tensors of the reference's shapes (src/runtime/v6.rs:76-108,
 :1040-1132); nothing here loads a checkpoint."""
 import importlib
+from operator import attrgetter, itemgetter
 
 import numpy as np
 
 _pkg = importlib.import_module(__name__.rsplit(".", 1)[0])
-LayerOp, Matrix, turbo, matmul_vec_group, FusedV6, FusedV7, fused_operands, fused_run = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group, _pkg.FusedV6, _pkg.FusedV7, _pkg.fused_operands, _pkg.fused_run
+LayerOp, Matrix, turbo, matmul_vec_group, FusedV6, FusedV7 = _pkg.LayerOp, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group, _pkg.FusedV6, _pkg.FusedV7
+fused_operands, fused_adapters, fused_run = _pkg.fused_operands, _pkg.fused_adapters, _pkg.fused_run
 ACT_NONE, ACT_SQUARED_RELU, ACT_TANH, ACT_STABLE_EXP, ACT_SILU = _pkg.ACT_NONE, _pkg.ACT_SQUARED_RELU, _pkg.ACT_TANH, _pkg.ACT_STABLE_EXP, _pkg.ACT_SILU
 
 LN_EPS = 1.0e-5   # Model::LN_EPS, src/runtime/v6.rs:46
@@ -119,7 +121,7 @@ def dispatch_layer(layer, buf, state, cursors, A, H, S, rescale_now=False):
         LayerOp.affine(buf.x, 0.5, 0.0)
 
 
-def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False):
+def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False, checked=False):
     """The same layer in 12 launches: the 8 quantized products (3 launches for the independent ones, 2
     alone), the first halves of the two adapters, and 5 fused launches for the 27 small ops
     (`wrq_v6_*`).  The layer's output and state are those of `dispatch_layer` up to f32 summation order;
@@ -142,25 +144,26 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
 
     def adapter_in(name, x, out):
         if tiles:
-            FusedV7.adapters_in(C, A, [(m[name].w, x, out, ACT_TANH)])
+            FusedV7.adapters_in(C, A, [(m[name].w, x, out, ACT_TANH)], checked=checked)
         else:
             m[name].matmul_op(x, out, ACT_TANH, fast)
 
-    FusedV6.pre(C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state, [t["time_mix_x"]], buf.att_x, [buf.att_xx])
+    FusedV6.pre(C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state, [t["time_mix_x"]], buf.att_x, [buf.att_xx],
+                checked=checked)
     adapter_in("time_mix_w1", buf.att_xx, buf.time_mix_x.view(1, A, 5 * TIME_MIX_LORA))
-    FusedV6.time_mix(C, A, TIME_MIX_LORA, cursors, buf.time_mix_x, m["time_mix_w2"].w, t["time_mix"], state, att_state, buf.att_x, buf.att_sx)
+    FusedV6.time_mix(C, A, TIME_MIX_LORA, cursors, buf.time_mix_x, m["time_mix_w2"].w, t["time_mix"], state, att_state, buf.att_x, buf.att_sx, checked=checked)
     matmul_vec_group([(m[n], buf.att_sx, out, ACT_NONE, False, dict(input_view=slice_of(i)))
                       for n, out, i in (("att_w_k", buf.att_k, 1), ("att_w_v", buf.att_v, 2), ("att_w_r", buf.att_r, 3), ("att_w_g", buf.att_g, 4))])
     adapter_in("time_decay_w1", buf.att_sx[:1], buf.att_w)
-    FusedV6.decay(C, A, TIME_DECAY_LORA, buf.att_w, m["time_decay_w2"].w, t["time_decay"], buf.time_decay)
+    FusedV6.decay(C, A, TIME_DECAY_LORA, buf.att_w, m["time_decay_w2"].w, t["time_decay"], buf.time_decay, checked=checked)
     FusedV6.wkv_gate(S, H, A, cursors, buf.time_decay, t["time_first"], state, att_state, buf.att_k, buf.att_v, buf.att_r, buf.att_g, t["gn_w"], t["gn_b"],
-                     GN_EPS, buf.att_x)
+                     GN_EPS, buf.att_x, checked=checked)
     m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)
     FusedV6.pre(C, A, cursors, buf.x, buf.att_o, buf.x2, t["ffn_ln_w"], t["ffn_ln_b"], LN_EPS, state, ffn_state, [t["ffn_time_mix_k"], t["ffn_time_mix_r"]],
-                buf.ffn_x, [buf.ffn_kx, buf.ffn_rx])
+                buf.ffn_x, [buf.ffn_kx, buf.ffn_rx], checked=checked)
     matmul_vec_group([(m["ffn_w_k"], buf.ffn_kx, buf.ffn_k, ACT_SQUARED_RELU, False, {}), (m["ffn_w_r"], buf.ffn_rx, buf.ffn_r, ACT_NONE, False, {})])
     m["ffn_w_v"].matmul_op_sparse(buf.ffn_k, buf.ffn_v, ACT_NONE, fast)
-    FusedV6.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_r, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now)
+    FusedV6.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_r, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now, checked=checked)
 
 
 # What the fused ops take.  Measured up to 2048 tokens (32 requests; 0.14 of the op list's time at 768 channels, 0.55 at 5120) and
@@ -168,26 +171,31 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False)
 FUSED_MAX_TOKENS = 65535
 VECTORS = ("att_ln_w", "att_ln_b", "ffn_ln_w", "ffn_ln_b", "time_mix_x", "time_decay", "gn_w", "gn_b", "ffn_time_mix_k", "ffn_time_mix_r")
 FUSED_ROWS = ("x", "x2", "att_x", "att_xx", "att_g", "att_o", "ffn_x", "ffn_kx", "ffn_rx", "ffn_v", "ffn_r")
+vectors_of, rows_of = itemgetter(*VECTORS), attrgetter(*FUSED_ROWS)
 
 
 def fused_is_built(layer, buf, cursors, A, H, S):
     """Whether the fused form takes this run of this layer: heads of 64, up to 8192 channels, adapters of the sizes above,
     vectors and buffers of the types `Layer` and `Runtime` give them."""
-    t, m, C = layer.t, layer.m, H * S
+    import torch
+
+    t, C, f16, f32 = layer.t, H * S, torch.float16, torch.float32
     if S != 64 or C > 8192 or not fused_run(cursors, A):
         return False
     n, mix, decay = A * C, TIME_MIX_LORA, TIME_DECAY_LORA
-    rows = lambda names, size: [(getattr(buf, name, None), size) for name in names]  # None: buffers made for the op list alone have no x2
-    f16 = [(t[name], C) for name in VECTORS] + [(t["time_mix"], 5 * C)]
-    f16 += rows(FUSED_ROWS, n) + rows(("att_sx",), 5 * n) + rows(("time_mix_x",), 5 * mix * A) + rows(("att_w",), decay * A)
-    f32 = [(t["time_first"], C)] + rows(("att_k", "att_v", "att_r", "time_decay"), n)
-    return fused_operands(f16, f32, [(m["time_mix_w1"], 5 * mix, C), (m["time_mix_w2"], 5 * C, mix), (m["time_decay_w1"], decay, C), (m["time_decay_w2"], C, decay)])
+    try:
+        return (fused_operands(vectors_of(t), f16, C) and fused_operands((t["time_mix"],), f16, 5 * C) and fused_operands((t["time_first"],), f32, C)
+                and fused_operands(rows_of(buf), f16, n) and fused_operands((buf.att_k, buf.att_v, buf.att_r, buf.time_decay), f32, n)
+                and fused_operands((buf.att_sx,), f16, 5 * n) and fused_operands((buf.time_mix_x,), f16, 5 * mix * A) and fused_operands((buf.att_w,), f16, decay * A)
+                and fused_adapters(layer.m, (("time_mix_w1", 5 * mix, C), ("time_mix_w2", 5 * C, mix), ("time_decay_w1", decay, C), ("time_decay_w2", C, decay)), f16))
+    except AttributeError:  # buffers made for the op list alone have no x2
+        return False
 
 
 def dispatch_layer_auto(layer, buf, state, cursors, A, H, S, rescale_now=False):
     """The fused form where it is built (`fused_is_built`), the op list otherwise."""
     if A <= FUSED_MAX_TOKENS and fused_is_built(layer, buf, cursors, A, H, S):
-        dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now)
+        dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now, checked=True)
     else:
         dispatch_layer(layer, buf, state, cursors, A, H, S, rescale_now)
 

@@ -4,17 +4,20 @@ every op one library call; `dispatch_layer` leaves the same buffers behind fused
 built.  Weights are random-init tensors of the reference's shapes (src/runtime/v7.rs:77-128);
 nothing here loads a checkpoint."""
 import importlib
+from operator import attrgetter, itemgetter
 
 import numpy as np
 
 _pkg = importlib.import_module(__name__.rsplit(".", 1)[0])
-LayerOp, FusedV7, fused_operands, fused_run, Matrix, turbo, matmul_vec_group = _pkg.LayerOp, _pkg.FusedV7, _pkg.fused_operands, _pkg.fused_run, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group
+LayerOp, FusedV7, Matrix, turbo, matmul_vec_group = _pkg.LayerOp, _pkg.FusedV7, _pkg.Matrix, _pkg.turbo, _pkg.matmul_vec_group
+fused_operands, fused_adapters, fused_run = _pkg.fused_operands, _pkg.fused_adapters, _pkg.fused_run
 ACT_NONE, ACT_SQUARED_RELU, ACT_TANH, ACT_SIGMOID = _pkg.ACT_NONE, _pkg.ACT_SQUARED_RELU, _pkg.ACT_TANH, _pkg.ACT_SIGMOID
 
 L2_EPS = 1.0e-12  # Model::L2_EPS, src/runtime/v7.rs:46
 LN_EPS = 1.0e-5   # Model::LN_EPS, src/runtime/v7.rs:47
 GN_EPS = 64.0e-5  # Model::GN_EPS, src/runtime/v7.rs:48
 RANK_W, RANK_A, RANK_G, RANK_V = 64, 64, 128, 32  # inner sizes of the four adapters (read from the tensors by the reference)
+RANKS = (("w", RANK_W), ("a", RANK_A), ("g", RANK_G), ("v", RANK_V))
 
 QUANTIZED = ("att_w_r", "att_w_k", "att_w_v", "att_w_o", "ffn_w_k", "ffn_w_v")
 ADAPTERS = ("w1", "w2", "a1", "a2", "g1", "g2", "v1", "v2")
@@ -22,6 +25,7 @@ VECTORS = ("att_ln_w", "att_ln_b", "ffn_ln_w", "ffn_ln_b", "x_r", "x_w", "x_k", 
 SHIFTED = ("att_rx", "att_wx", "att_kx", "att_vx", "att_ax", "att_gx")
 FUSED_ROWS = ("x", "x2", "att_x", "att_v0", "att_r", "att_w", "att_k", "att_v", "att_a", "att_g", "att_kk", "att_vv", "att_o", "ffn_x", "ffn_kx",
               "ffn_v")
+vectors_of, rows_of, shifted_of = itemgetter(*VECTORS), attrgetter(*FUSED_ROWS), attrgetter(*SHIFTED)
 
 
 def random_layer_weights(rng, C, H, S, hidden):
@@ -94,30 +98,34 @@ def dispatch_layer(layer, buf, state, cursors, A, H, S, index, rescale_now=False
     values as `att_v0`, the later ones mix theirs with it).  The fused form where it is built (`fused_is_built`:
     heads of 64, up to 8192 channels, adapters of the sizes above, f16 vectors and buffers), the op list otherwise."""
     if fused_is_built(layer, H, S, buf, cursors, A, shifts):
-        dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts)
+        dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts, checked=True)
     else:
         dispatch_layer_ops(layer, buf, state, cursors, A, H, S, index, rescale_now, shifts)
 
 
 def fused_is_built(layer, H, S, buf=None, cursors=None, A=None, shifts=None):
     """Whether the fused form takes this layer, and with `buf`, `cursors` and `A` whether it takes this run."""
-    t, m, C = layer.t, layer.m, H * S
+    import torch
+
+    C, f16 = H * S, torch.float16
     if S != 64 or C > 8192:
         return False
-    ranks = (("w", RANK_W), ("a", RANK_A), ("g", RANK_G), ("v", RANK_V))
-    adapters = [(m[n + "1"], r, C) for n, r in ranks] + [(m[n + "2"], C, r) for n, r in ranks]
-    vectors = [(t.get(n), C) for n in VECTORS]
-    if buf is None:
-        return fused_operands(vectors, adapters=adapters)
-    n = A * C
-    rows = [(name, n) for name in FUSED_ROWS + (SHIFTED if shifts is None else ())] + [("aux_" + name, A * r) for name, r in ranks] + [("att_n", 4 * n)]
-    rows = [(getattr(buf, name, None), size) for name, size in rows]  # None: buffers made for the op list alone have no x2
-    if shifts is not None:
-        rows += [(shifts.mix, 6 * n), (shifts.sx, 6 * n)]
-    return fused_operands(vectors + rows, adapters=adapters) and fused_run(cursors, A)
+    try:
+        if not fused_operands(vectors_of(layer.t), f16, C) or not fused_adapters(layer.m, [(n + "1", r, C) for n, r in RANKS] + [(n + "2", C, r) for n, r in RANKS], f16):
+            return False
+        if buf is None:
+            return True
+        n = A * C
+        if not fused_run(cursors, A) or not fused_operands(rows_of(buf), f16, n) or not fused_operands((buf.att_n,), f16, 4 * n):
+            return False
+        if not all(fused_operands((t,), f16, A * r) for t, (_, r) in zip((buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v), RANKS)):
+            return False
+        return fused_operands(shifted_of(buf), f16, n) if shifts is None else fused_operands((shifts.mix, shifts.sx), f16, 6 * n)
+    except (KeyError, AttributeError):  # a first layer without v0, buffers made for the op list alone (no x2)
+        return False
 
 
-def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
+def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None, checked=False):
     """The layer in 10 launches (beside the second ones of split products): the six quantized products in four and six
     fused launches for the 38 small ops of `dispatch_layer_ops`; with `shifts` 11, the six token shifts being one over its
     factors.  Same results as the op list up to f32 summation order, in `buf`'s buffers too.
@@ -129,27 +137,30 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, index, rescale_now
     ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
     att_ln = (C, A, cursors, buf.x, None, None, t["att_ln_w"], t["att_ln_b"], LN_EPS, state, att_state)
     if shifts is None:
-        rx, wx, kx, vx, ax, gx = shifted = [getattr(buf, name) for name in SHIFTED]
-        FusedV7.pre(*att_ln, [t[n] for n in PackedShifts.NAMES], buf.att_x, shifted)
+        rx, wx, kx, vx, ax, gx = shifted = list(shifted_of(buf))
+        FusedV7.pre(*att_ln, [t[n] for n in PackedShifts.NAMES], buf.att_x, shifted, checked=checked)
     else:
         # the caller's factors may differ from token to token: the first shift is a layer norm's companion, the six are token_shift's
         rx, wx, kx, vx, ax, gx = shifted = [shifts.sx[i].view(1, A, C) for i in range(6)]
-        FusedV7.pre(*att_ln, [t[PackedShifts.NAMES[0]]], buf.att_x, shifted[:1])
+        FusedV7.pre(*att_ln, [t[PackedShifts.NAMES[0]]], buf.att_x, shifted[:1], checked=checked)
         LayerOp.token_shift(cursors, shifts.mix, state, buf.att_x, shifts.sx, True, state_view=att_state)
     matmul_vec_group([(m["att_w_r"], rx, buf.att_r, ACT_NONE, False, {}), (m["att_w_k"], kx, buf.att_k, ACT_NONE, False, {}),
                       (m["att_w_v"], vx, buf.att_v, ACT_NONE, False, {})])
     w = {n: m[n].w for n in ADAPTERS}
     adapters = [(w["w1"], wx, buf.aux_w, ACT_TANH), (w["a1"], ax, buf.aux_a, ACT_NONE), (w["g1"], gx, buf.aux_g, ACT_SIGMOID), (w["v1"], vx, buf.aux_v, ACT_NONE)]
-    FusedV7.adapters_in(C, A, adapters[:3] if index == 0 else adapters)
+    FusedV7.adapters_in(C, A, adapters[:3] if index == 0 else adapters, checked=checked)
     FusedV7.mid(S, H, A, index == 0, [buf.aux_w, buf.aux_a, buf.aux_g, buf.aux_v], [w["w2"], w["a2"], w["g2"], w["v2"]],
                 [t["w0"], t["a0"], t["v0"], t["k_k"], t["k_a"]], L2_EPS, buf.att_k, buf.att_v, buf.att_v0, buf.att_w, buf.att_g, buf.att_n,
-                [None if b.data_ptr() == plane.data_ptr() else b for b, plane in zip((buf.att_k, buf.att_v, buf.att_a, buf.att_kk), buf.att_n)] + [buf.att_vv])
-    FusedV7.wkv_gate(S, H, A, cursors, state, att_state, buf.att_r, buf.att_w, buf.att_n, t["r_k"], buf.att_g, t["gn_w"], t["gn_b"], GN_EPS, buf.att_x)
+                [None if b.data_ptr() == plane.data_ptr() else b for b, plane in zip((buf.att_k, buf.att_v, buf.att_a, buf.att_kk), buf.att_n)] + [buf.att_vv],
+                checked=checked)
+    FusedV7.wkv_gate(S, H, A, cursors, state, att_state, buf.att_r, buf.att_w, buf.att_n, t["r_k"], buf.att_g, t["gn_w"], t["gn_b"], GN_EPS, buf.att_x,
+                     checked=checked)
     m["att_w_o"].matmul_op(buf.att_x, buf.att_o, ACT_NONE, fast)
-    FusedV7.pre(C, A, cursors, buf.x, buf.att_o, buf.x2, t["ffn_ln_w"], t["ffn_ln_b"], LN_EPS, state, ffn_state, [t["ffn_x_k"]], buf.ffn_x, [buf.ffn_kx])
+    FusedV7.pre(C, A, cursors, buf.x, buf.att_o, buf.x2, t["ffn_ln_w"], t["ffn_ln_b"], LN_EPS, state, ffn_state, [t["ffn_x_k"]], buf.ffn_x, [buf.ffn_kx],
+                checked=checked)
     m["ffn_w_k"].matmul_op(buf.ffn_kx, buf.ffn_k, ACT_SQUARED_RELU, fast)
     m["ffn_w_v"].matmul_op_sparse(buf.ffn_k, buf.ffn_v, ACT_NONE, fast)
-    FusedV7.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now, buf.ffn_x)
+    FusedV7.post_ffn(C, A, cursors, state, ffn_state, buf.ffn_v, buf.ffn_x, buf.x2, buf.x, rescale_now, buf.ffn_x, checked=checked)
 
 
 def dispatch_layer_ops(layer, buf, state, cursors, A, H, S, index, rescale_now=False, shifts=None):
