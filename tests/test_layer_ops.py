@@ -828,6 +828,31 @@ def test_gpu_lerp_activate_affine(gpu, lop):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("C", [8192, 8196, 16384, 20000, 65532, 65536, 65540])
+def test_gpu_softmax_vocabulary_rows(gpu, dtype, C):
+    # both sides of the lengths at which a row moves into the registers of 1024 threads (beyond 8192) and out of them (65536);
+    # a row with masked entries, one where all but one are masked, one of equal values
+    import torch
+
+    print("softmax of long rows on the GPU", dtype.__name__, C, flush=True)
+    rng = np.random.default_rng(SEED + 77 + C)
+    x = (rng.standard_normal((1, 4, C)) * 4.0).astype(dtype)
+    x[0, 1, ::3] = -np.inf
+    x[0, 2] = -np.inf
+    x[0, 2, C - 1] = 1.0
+    x[0, 3] = 5.0
+    xd = torch.from_numpy(x.copy()).cuda()
+    gpu.LayerOp.softmax(xd)
+    got, want = xd.cpu().numpy(), softmax64(x.astype(np.float64))
+    # f32: expf within 2 ulp, a sum of C terms through 1024 partial ones; f16: half an ulp of the largest value it stores
+    assert_close(got, want, 1e-3 if dtype == np.float16 else 1e-6, "softmax vs float64")
+    assert (got[0, 1, ::3] == 0).all() and got[0, 2, C - 1] == 1 and (got[0, 2, :-1] == 0).all()
+    if dtype == np.float32:
+        assert np.allclose(got.sum(-1), 1.0, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("C,T,B", [(1000, 3, 2), (4096, 1, 1), (4096, 128, 1), (65536, 2, 1), (64, 5, 1), (4, 1, 3)])
 def test_gpu_softmax_layer_norm(gpu, lop, dtype, C, T, B):
     import torch

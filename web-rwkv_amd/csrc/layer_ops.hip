@@ -16,26 +16,30 @@ namespace wrq {
 namespace {
 
 constexpr int kRowThreads = 256;
-constexpr int kRowCache = 8; // vectors of 4 elements a thread keeps: rows up to 8192 elements stay in registers
+constexpr int kRowCache = 8;   // vectors of 4 elements a thread keeps: rows up to 8192 elements stay in registers
+constexpr int kVocabCache = 16; // the same for softmax rows of a vocabulary on 1024 threads: up to 65536 elements
 
 // One workgroup per row of `n` elements (n % 4 == 0).  MODE 0: softmax; 1: layer norm (w, b of the
 // row's length); 2: group norm (w, b indexed by head * n, the row index modulo `heads`).
-template <typename XT, int MODE, int THREADS>
+// A softmax keeps the exponentials of a cached row: one workgroup's time on a row of 65536 logits is reading it (256 KB at what
+// one CU takes from L2, 2 us a pass) and expf (about 8 us of its vector units a pass).  Read once and exponentiated once the
+// row takes 11.9 us (32 rows 13.2); in three passes over memory and two of expf it took 18.1 (19.6).
+template <typename XT, int MODE, int THREADS, int CACHE = kRowCache>
 __global__ __launch_bounds__(THREADS) void row_kernel(XT *x, const uint16_t *w, const uint16_t *b, uint32_t n, uint32_t heads, float eps) {
     __shared__ float red[THREADS / 64];
     XT *row = x + (uint64_t)blockIdx.x * n;
     const uint32_t nv = n / 4;
-    float4 cache[kRowCache];
-    const bool cached = nv <= (uint32_t)(THREADS * kRowCache);
+    float4 cache[CACHE];
+    const bool cached = nv <= (uint32_t)(THREADS * CACHE);
     // a cached row asks for its weights together with the row: they are needed only after both reductions, and
     // fetched then they would add a memory round trip to a kernel that is little more than round trips
-    uint2 wq[MODE == 0 ? 1 : kRowCache], bq[MODE == 0 ? 1 : kRowCache];
+    uint2 wq[MODE == 0 ? 1 : CACHE], bq[MODE == 0 ? 1 : CACHE];
     const uint16_t *wr = MODE == 2 ? w + (uint64_t)(blockIdx.x % heads) * n : w;
     const uint16_t *br = MODE == 2 ? b + (uint64_t)(blockIdx.x % heads) * n : b;
     if constexpr (MODE != 0) {
         if (cached) {
 #pragma unroll
-            for (int c = 0; c < kRowCache; c++) {
+            for (int c = 0; c < CACHE; c++) {
                 const uint32_t i = threadIdx.x + c * THREADS;
                 if (i < nv) wq[c] = *reinterpret_cast<const uint2 *>(wr + 4 * i), bq[c] = *reinterpret_cast<const uint2 *>(br + 4 * i);
             }
@@ -45,7 +49,7 @@ __global__ __launch_bounds__(THREADS) void row_kernel(XT *x, const uint16_t *w, 
     float part = MODE == 0 ? -1.0e30f : 0.0f;
     if (cached) {
 #pragma unroll
-        for (int c = 0; c < kRowCache; c++) {
+        for (int c = 0; c < CACHE; c++) {
             const uint32_t i = threadIdx.x + c * THREADS;
             if (i < nv) {
                 cache[c] = load_vec4(row + 4 * i);
@@ -67,8 +71,12 @@ __global__ __launch_bounds__(THREADS) void row_kernel(XT *x, const uint16_t *w, 
     auto term = [&](float v) { return MODE == 0 ? expf(v - centre) : (v - centre) * (v - centre); };
     if (cached) {
 #pragma unroll
-        for (int c = 0; c < kRowCache; c++)
-            if (threadIdx.x + c * THREADS < nv) acc += (term(cache[c].x) + term(cache[c].y)) + (term(cache[c].z) + term(cache[c].w));
+        for (int c = 0; c < CACHE; c++)
+            if (threadIdx.x + c * THREADS < nv) {
+                const float4 e = make_float4(term(cache[c].x), term(cache[c].y), term(cache[c].z), term(cache[c].w));
+                if (MODE == 0) cache[c] = e;
+                acc += (e.x + e.y) + (e.z + e.w);
+            }
     } else {
         for (uint32_t i = threadIdx.x; i < nv; i += THREADS) {
             const float4 v = load_vec4(row + 4 * i);
@@ -83,7 +91,8 @@ __global__ __launch_bounds__(THREADS) void row_kernel(XT *x, const uint16_t *w, 
     auto finish = [&](uint32_t i, float4 v, int c) { // c: the vector's place in the cache, or -1
         float4 o;
         if (MODE == 0) {
-            o = make_float4(expf(v.x - centre) * scale, expf(v.y - centre) * scale, expf(v.z - centre) * scale, expf(v.w - centre) * scale);
+            const float4 e = c >= 0 ? v : make_float4(term(v.x), term(v.y), term(v.z), term(v.w)); // a cached row holds its terms
+            o = make_float4(e.x * scale, e.y * scale, e.z * scale, e.w * scale);
         } else {
             const float4 wv = c >= 0 ? unpack(wq[MODE == 0 ? 0 : c]) : load_vec4(wr + 4 * i), bv = c >= 0 ? unpack(bq[MODE == 0 ? 0 : c]) : load_vec4(br + 4 * i);
             o = make_float4(fmaf((v.x - centre) * scale, wv.x, bv.x), fmaf((v.y - centre) * scale, wv.y, bv.y),
@@ -93,7 +102,7 @@ __global__ __launch_bounds__(THREADS) void row_kernel(XT *x, const uint16_t *w, 
     };
     if (cached) {
 #pragma unroll
-        for (int c = 0; c < kRowCache; c++) {
+        for (int c = 0; c < CACHE; c++) {
             const uint32_t i = threadIdx.x + c * THREADS;
             if (i < nv) finish(i, cache[c], c);
         }
@@ -177,8 +186,13 @@ int launch_rows(hipStream_t stream, void *x, int dtype, const void *w, const voi
     if (rows > 0x7fffffffull) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
     const uint16_t *wp = static_cast<const uint16_t *>(w), *bp = static_cast<const uint16_t *>(b);
     // short rows (a head of a group norm) take one wave, no LDS exchange
-    if (n > 16384) {
-        // a vocabulary-sized row (softmax over the logits): 1024 threads
+    if (MODE == 0 && n > 4 * kRowThreads * kRowCache && n <= 4 * 1024 * kVocabCache) {
+        // a vocabulary-sized softmax row (more than 256 threads keep): 1024 threads, the row in registers
+        // (16384 elements 12.2 us on 256 threads that read it three times, 5.6 us on 1024)
+        if (dtype == WRQ_F16) hipLaunchKernelGGL((row_kernel<uint16_t, 0, 1024, kVocabCache>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
+        else hipLaunchKernelGGL((row_kernel<float, 0, 1024, kVocabCache>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
+    } else if (n > 16384) {
+        // longer rows: 1024 threads, what does not fit the registers is read again
         if (dtype == WRQ_F16) hipLaunchKernelGGL((row_kernel<uint16_t, MODE, 1024>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
         else hipLaunchKernelGGL((row_kernel<float, MODE, 1024>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
     } else if (n <= 1024) {
