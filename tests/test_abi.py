@@ -35,6 +35,34 @@ def test_struct_layouts_match_the_header(wrq):
     assert wrq.ACTIVATIONS[1] == "squared_relu" and len(wrq.ACTIVATIONS) == 8
 
 
+@pytest.mark.parametrize("shape", [(64,), (3, 64), (2, 3, 64), (5, 2, 3, 64), (0, 64)], ids=str)
+def test_packed_descriptors_equal_the_structures(wrq, shape):
+    import torch
+
+    for dtype in (torch.float16, torch.float32, torch.uint8):
+        t = torch.zeros(shape, dtype=dtype)
+        assert wrq._tensor(t) == bytes(wrq.as_tensor(t))
+        assert wrq._view(t) == bytes(wrq.as_view(t)) and wrq._view(t, dtype=wrq.F16) == bytes(wrq.as_view(t, dtype=wrq.F16))
+    for view in (((64, 1, 1), (64, 3, 2), (0, 2, 1)), ([32, 2], [64, 3], [16, 1]), ((4, 1, 1, 1), (64, 3, 2, 5), (0, 0, 0, 4)), ((), (), ())):
+        assert wrq._view(t, view) == bytes(wrq.as_view(t, view))
+
+
+def test_packed_descriptors_leave_odd_values_to_the_structures(wrq):
+    import torch
+
+    t = torch.zeros((2, 64))
+    for view in (((64, 2 ** 32 + 1), (64, 2), (0, 0)), ((64, 2), (64, 2), (-4, 0))):  # wrapped to 32 bits, for the library to judge
+        assert bytes(wrq._view(t, view)._obj) == bytes(wrq.as_view(t, view))
+    for bad in (((64.5, 2), (64, 2), (0, 0)), ((1,) * 5, (64, 2), (0, 0))):
+        with pytest.raises((TypeError, IndexError, ValueError, RuntimeError)):
+            wrq.as_view(t, bad)
+        with pytest.raises((TypeError, IndexError, ValueError, RuntimeError)):
+            wrq._view(t, bad)
+    for make in (wrq._tensor, wrq._view):
+        with pytest.raises(AssertionError):
+            make(t.t())
+
+
 FAKE = 0x10000  # never dereferenced: every call below fails its checks first
 
 

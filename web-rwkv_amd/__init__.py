@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -175,7 +176,9 @@ def lib():
                 "(hipcc --offload-arch=gfx950); this package has no CPU or eager fallback"
             )
         L = C.CDLL(LIB_PATH)
-        T, V, vp, i = C.POINTER(CTensor), C.POINTER(CTensorView), C.c_void_p, C.c_int
+        # descriptors go as pointers to a struct of ctypes or to the packed bytes of one (see _tensor, _view)
+        vp, i = C.c_void_p, C.c_int
+        T = V = vp
         L.wrq_init.restype = i
         L.wrq_abi_version.restype = i
         L.wrq_status_string.restype = C.c_char_p
@@ -252,9 +255,14 @@ def _check(status):
 
 
 def _stream():
+    """Handle of torch's current stream.  ``torch.cuda.current_stream()`` builds a Stream object (1.5 us); the raw handle is what
+    a launch needs."""
     import torch
 
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
 
 
 def shape_of(t):
@@ -273,9 +281,10 @@ def as_tensor(t, shape=None):
 def _dtype(t):
     import torch
 
-    if t.dtype == torch.float16:
+    dt = t.dtype
+    if dt is torch.float16:
         return F16
-    if t.dtype == torch.float32:
+    if dt is torch.float32:
         return F32
     return 2  # rejected by the library with ERR_TYPE
 
@@ -291,6 +300,47 @@ def as_view(t, view=None, dtype=None):
     return CTensorView(t.data_ptr(), cv, _dtype(t) if dtype is None else dtype)
 
 
+# The descriptors of a call as packed bytes: a ctypes structure with its arrays costs 1 - 3 us to build, a packed one 0.4 us, and a
+# small product's whole call is host time (one token, 2048 x 2048: 13.8 us with structures and a Stream object, 7.5 us now).
+_PACK_TENSOR = struct.Struct("@Q4I").pack
+_PACK_VIEW = struct.Struct("@Q12Ii4x").pack
+assert struct.calcsize("@Q4I") == C.sizeof(CTensor) and struct.calcsize("@Q12Ii4x") == C.sizeof(CTensorView)
+
+
+def _shape4(t):
+    s = t.shape
+    n = len(s)
+    if n == 2:
+        return s[1], s[0], 1, 1
+    if n == 3:
+        return s[2], s[1], s[0], 1
+    return tuple(shape_of(t))
+
+
+def _tensor(t):
+    """``as_tensor`` as packed bytes."""
+    assert t.is_contiguous()
+    try:
+        return _PACK_TENSOR(t.data_ptr(), *_shape4(t))
+    except struct.error:  # extents that a field does not hold are for the structure to take or refuse
+        return C.byref(as_tensor(t))
+
+
+def _view(t, view=None, dtype=None):
+    """``as_view`` as packed bytes."""
+    assert t.is_contiguous()
+    if dtype is None:
+        dtype = _dtype(t)
+    try:
+        if view is None:
+            s = _shape4(t)
+            return _PACK_VIEW(t.data_ptr(), *s, *s, 0, 0, 0, 0, dtype)
+        shape, stride, offset = tuple(view[0]), tuple(view[1]), tuple(view[2])
+        return _PACK_VIEW(t.data_ptr(), *shape, *(1,) * (4 - len(shape)), *stride, *(1,) * (4 - len(stride)), *offset, *(0,) * (4 - len(offset)), dtype)
+    except struct.error:
+        return C.byref(as_view(t, view, dtype))
+
+
 class TensorOp:
     """The six constructors of the path; each enqueues on torch's current stream."""
 
@@ -299,46 +349,46 @@ class TensorOp:
 
     @staticmethod
     def quantize_mat_int8(input, minmax, output):
-        _check(lib().wrq_quantize_mat_int8(_stream(), C.byref(as_tensor(input)), C.byref(as_tensor(minmax)), C.byref(as_tensor(output))))
+        _check(lib().wrq_quantize_mat_int8(_stream(), _tensor(input), _tensor(minmax), _tensor(output)))
 
     @staticmethod
     def quantize_mat_nf4(input, quant, absmax, output):
-        _check(lib().wrq_quantize_mat_nf4(_stream(), C.byref(as_tensor(input)), C.byref(as_tensor(quant)), C.byref(as_tensor(absmax)), C.byref(as_tensor(output))))
+        _check(lib().wrq_quantize_mat_nf4(_stream(), _tensor(input), _tensor(quant), _tensor(absmax), _tensor(output)))
 
     @staticmethod
     def matmul_vec_int8(matrix, minmax, input, output, act=ACT_NONE, sparse=False, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_vec_int8(_stream(), C.byref(as_tensor(matrix)), C.byref(as_tensor(minmax)),
-                                         C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act, int(sparse)))
+        _check(lib().wrq_matmul_vec_int8(_stream(), _tensor(matrix), _tensor(minmax),
+                                         _view(input, input_view), _view(output, output_view), act, int(sparse)))
 
     @staticmethod
     def matmul_vec_nf4(matrix, quant, absmax, input, output, act=ACT_NONE, sparse=False, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_vec_nf4(_stream(), C.byref(as_tensor(matrix)), C.byref(as_tensor(quant)), C.byref(as_tensor(absmax)),
-                                        C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act, int(sparse)))
+        _check(lib().wrq_matmul_vec_nf4(_stream(), _tensor(matrix), _tensor(quant), _tensor(absmax),
+                                        _view(input, input_view), _view(output, output_view), act, int(sparse)))
 
     @staticmethod
     def matmul_mat_int8(matrix, minmax, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_int8(_stream(), C.byref(as_view(matrix, matrix_view, dtype=F16)), C.byref(as_tensor(minmax)),
-                                         C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act))
+        _check(lib().wrq_matmul_mat_int8(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(minmax),
+                                         _view(input, input_view), _view(output, output_view), act))
 
     @staticmethod
     def matmul_mat_int8_noalloc(matrix, minmax, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_int8_noalloc(_stream(), C.byref(as_view(matrix, matrix_view, dtype=F16)), C.byref(as_tensor(minmax)),
-                                                 C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act))
+        _check(lib().wrq_matmul_mat_int8_noalloc(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(minmax),
+                                                 _view(input, input_view), _view(output, output_view), act))
 
     @staticmethod
     def matmul_mat_nf4(matrix, quant, absmax, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_nf4(_stream(), C.byref(as_view(matrix, matrix_view, dtype=F16)), C.byref(as_tensor(quant)), C.byref(as_tensor(absmax)),
-                                        C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act))
+        _check(lib().wrq_matmul_mat_nf4(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(quant), _tensor(absmax),
+                                        _view(input, input_view), _view(output, output_view), act))
 
     @staticmethod
     def matmul_vec_fp16(matrix, input, output, act=ACT_NONE, sparse=False, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_vec_fp16(_stream(), C.byref(as_tensor(matrix)), C.byref(as_view(input, input_view)),
-                                         C.byref(as_view(output, output_view)), act, int(sparse)))
+        _check(lib().wrq_matmul_vec_fp16(_stream(), _tensor(matrix), _view(input, input_view),
+                                         _view(output, output_view), act, int(sparse)))
 
     @staticmethod
     def matmul_mat_fp16(matrix, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_fp16(_stream(), C.byref(as_view(matrix, matrix_view)), C.byref(as_view(input, input_view)),
-                                         C.byref(as_view(output, output_view)), act))
+        _check(lib().wrq_matmul_mat_fp16(_stream(), _view(matrix, matrix_view), _view(input, input_view),
+                                         _view(output, output_view), act))
 
 
 class LayerOp:
@@ -347,122 +397,122 @@ class LayerOp:
 
     @staticmethod
     def softmax(x):
-        _check(lib().wrq_softmax(_stream(), C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_softmax(_stream(), _tensor(x), _dtype(x)))
 
     @staticmethod
     def layer_norm(w, b, x, eps):
-        _check(lib().wrq_layer_norm(_stream(), C.byref(as_tensor(w)), C.byref(as_tensor(b)), C.byref(as_tensor(x)), _dtype(x), eps))
+        _check(lib().wrq_layer_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def group_norm(w, b, x, eps):
-        _check(lib().wrq_group_norm(_stream(), C.byref(as_tensor(w)), C.byref(as_tensor(b)), C.byref(as_tensor(x)), _dtype(x), eps))
+        _check(lib().wrq_group_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def add_activate(input, output, act_x=ACT_NONE, act_y=ACT_NONE, act_out=ACT_NONE, input_view=None, output_view=None):
-        _check(lib().wrq_add_activate(_stream(), C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act_x, act_y, act_out))
+        _check(lib().wrq_add_activate(_stream(), _view(input, input_view), _view(output, output_view), act_x, act_y, act_out))
 
     @staticmethod
     def mul_activate(input, output, act_x=ACT_NONE, act_y=ACT_NONE, act_out=ACT_NONE, input_view=None, output_view=None):
-        _check(lib().wrq_mul_activate(_stream(), C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)), act_x, act_y, act_out))
+        _check(lib().wrq_mul_activate(_stream(), _view(input, input_view), _view(output, output_view), act_x, act_y, act_out))
 
     add = add_activate
     mul = mul_activate
 
     @staticmethod
     def embed(tokens, input, output):
-        _check(lib().wrq_embed(_stream(), C.byref(as_tensor(tokens)), C.byref(as_tensor(input)), C.byref(as_tensor(output)), _dtype(output)))
+        _check(lib().wrq_embed(_stream(), _tensor(tokens), _tensor(input), _tensor(output), _dtype(output)))
 
     @staticmethod
     def blit(input, output, input_view=None, output_view=None):
-        _check(lib().wrq_blit(_stream(), C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view))))
+        _check(lib().wrq_blit(_stream(), _view(input, input_view), _view(output, output_view)))
 
     @staticmethod
     def transpose(input, output, input_view=None, output_view=None):
-        _check(lib().wrq_transpose(_stream(), C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view))))
+        _check(lib().wrq_transpose(_stream(), _view(input, input_view), _view(output, output_view)))
 
     @staticmethod
     def activate(x, act, view=None):
-        _check(lib().wrq_activate(_stream(), C.byref(as_view(x, view)), act))
+        _check(lib().wrq_activate(_stream(), _view(x, view), act))
 
     @staticmethod
     def affine(x, scale, bias):
-        _check(lib().wrq_affine(_stream(), C.byref(as_tensor(x)), _dtype(x), scale, bias))
+        _check(lib().wrq_affine(_stream(), _tensor(x), _dtype(x), scale, bias))
 
     @staticmethod
     def token_shift(cursors, time_mix, state, input, output, reversed=False, time_mix_view=None, state_view=None):
-        _check(lib().wrq_token_shift(_stream(), C.byref(as_tensor(cursors)), C.byref(as_view(time_mix, time_mix_view)), C.byref(as_view(state, state_view)),
-                                     C.byref(as_tensor(input)), _dtype(input), C.byref(as_tensor(output)), _dtype(output), int(reversed)))
+        _check(lib().wrq_token_shift(_stream(), _tensor(cursors), _view(time_mix, time_mix_view), _view(state, state_view),
+                                     _tensor(input), _dtype(input), _tensor(output), _dtype(output), int(reversed)))
 
     @staticmethod
     def channel_mix(cursors, state, r, v, x, state_view=None):
-        _check(lib().wrq_channel_mix(_stream(), C.byref(as_tensor(cursors)), C.byref(as_view(state, state_view)), C.byref(as_tensor(r)),
-                                     C.byref(as_tensor(v)), C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_channel_mix(_stream(), _tensor(cursors), _view(state, state_view), _tensor(r),
+                                     _tensor(v), _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_mix_v4(cursors, time_decay, time_first, state, k, v, r, x, state_view=None):
-        _check(lib().wrq_time_mix_v4(_stream(), C.byref(as_tensor(cursors)), C.byref(as_tensor(time_decay)), C.byref(as_tensor(time_first)),
-                                     C.byref(as_view(state, state_view)), C.byref(as_tensor(k)), C.byref(as_tensor(v)), C.byref(as_tensor(r)),
-                                     C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_time_mix_v4(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
+                                     _view(state, state_view), _tensor(k), _tensor(v), _tensor(r),
+                                     _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_mix_v5(cursors, time_decay, time_first, state, k, v, r, x, state_view=None):
-        _check(lib().wrq_time_mix_v5(_stream(), C.byref(as_tensor(cursors)), C.byref(as_tensor(time_decay)), C.byref(as_tensor(time_first)),
-                                     C.byref(as_view(state, state_view)), C.byref(as_tensor(k)), C.byref(as_tensor(v)), C.byref(as_tensor(r)),
-                                     C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_time_mix_v5(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
+                                     _view(state, state_view), _tensor(k), _tensor(v), _tensor(r),
+                                     _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_mix_v6(cursors, time_decay, time_first, state, k, v, r, x, state_view=None):
-        _check(lib().wrq_time_mix_v6(_stream(), C.byref(as_tensor(cursors)), C.byref(as_tensor(time_decay)), C.byref(as_tensor(time_first)),
-                                     C.byref(as_view(state, state_view)), C.byref(as_tensor(k)), C.byref(as_tensor(v)), C.byref(as_tensor(r)),
-                                     C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_time_mix_v6(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
+                                     _view(state, state_view), _tensor(k), _tensor(v), _tensor(r),
+                                     _tensor(x), _dtype(x)))
 
     @staticmethod
     def recenter(x):
-        _check(lib().wrq_recenter(_stream(), C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_recenter(_stream(), _tensor(x), _dtype(x)))
 
     @staticmethod
     def rms_norm(w, b, x, eps):
-        _check(lib().wrq_rms_norm(_stream(), C.byref(as_tensor(w)), C.byref(as_tensor(b)), C.byref(as_tensor(x)), _dtype(x), eps))
+        _check(lib().wrq_rms_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def broadcast(input, output, input_view=None, output_view=None):
-        _check(lib().wrq_broadcast(_stream(), C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view))))
+        _check(lib().wrq_broadcast(_stream(), _view(input, input_view), _view(output, output_view)))
 
     @staticmethod
     def blend(factor, input, output):
-        _check(lib().wrq_blend(_stream(), C.byref(as_tensor(factor)), C.byref(as_tensor(input)), _dtype(input), C.byref(as_tensor(output)), _dtype(output)))
+        _check(lib().wrq_blend(_stream(), _tensor(factor), _tensor(input), _dtype(input), _tensor(output), _dtype(output)))
 
     @staticmethod
     def blend_lora(factor, xa, xb, output, xa_view=None, xb_view=None, output_view=None):
-        _check(lib().wrq_blend_lora(_stream(), C.byref(as_tensor(factor)), C.byref(as_view(xa, xa_view)), C.byref(as_view(xb, xb_view)),
-                                    C.byref(as_view(output, output_view))))
+        _check(lib().wrq_blend_lora(_stream(), _tensor(factor), _view(xa, xa_view), _view(xb, xb_view),
+                                    _view(output, output_view)))
 
     @staticmethod
     def l2_norm(x, eps):
-        _check(lib().wrq_l2_norm(_stream(), C.byref(as_tensor(x)), _dtype(x), eps))
+        _check(lib().wrq_l2_norm(_stream(), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def control_k_v7(p, a, k, a_view=None, k_view=None):
-        _check(lib().wrq_control_k_v7(_stream(), C.byref(as_tensor(p)), C.byref(as_view(a, a_view)), C.byref(as_view(k, k_view))))
+        _check(lib().wrq_control_k_v7(_stream(), _tensor(p), _view(a, a_view), _view(k, k_view)))
 
     @staticmethod
     def time_mix_v7(cursors, state, r, w, n, x, state_view=None):
-        _check(lib().wrq_time_mix_v7(_stream(), C.byref(as_tensor(cursors)), C.byref(as_view(state, state_view)), C.byref(as_tensor(r)),
-                                     C.byref(as_tensor(w)), C.byref(as_tensor(n)), C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_time_mix_v7(_stream(), _tensor(cursors), _view(state, state_view), _tensor(r),
+                                     _tensor(w), _tensor(n), _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_first_v7(u, r, n, x):
-        _check(lib().wrq_time_first_v7(_stream(), C.byref(as_tensor(u)), C.byref(as_tensor(r)), C.byref(as_tensor(n)), C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_time_first_v7(_stream(), _tensor(u), _tensor(r), _tensor(n), _tensor(x), _dtype(x)))
 
     @staticmethod
     def channel_mix_v7(cursors, state, v, x, state_view=None):
-        _check(lib().wrq_channel_mix_v7(_stream(), C.byref(as_tensor(cursors)), C.byref(as_view(state, state_view)), C.byref(as_tensor(v)),
-                                        C.byref(as_tensor(x)), _dtype(x)))
+        _check(lib().wrq_channel_mix_v7(_stream(), _tensor(cursors), _view(state, state_view), _tensor(v),
+                                        _tensor(x), _dtype(x)))
 
     @staticmethod
     def lerp(input, output, factor, reversed=False, input_view=None, output_view=None, factor_view=None):
-        _check(lib().wrq_lerp(_stream(), C.byref(as_view(input, input_view)), C.byref(as_view(output, output_view)),
-                              C.byref(as_view(factor, factor_view)), int(reversed)))
+        _check(lib().wrq_lerp(_stream(), _view(input, input_view), _view(output, output_view),
+                              _view(factor, factor_view), int(reversed)))
 
 
 def _operands(what, A, cursors, f16=(), f32=()):
@@ -528,7 +578,7 @@ class FusedV6:
         p = FusedV6._p
         if not checked:
             FusedV6._check_pre("v6_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
-        _check(lib().wrq_v6_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
+        _check(lib().wrq_v6_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, _view(state, state_view), len(factors),
                                 p(factors[0]), p(factors[1] if len(factors) > 1 else None), p(ln_out), p(shifts[0]), p(shifts[1] if len(shifts) > 1 else None)))
 
     @staticmethod
@@ -536,7 +586,7 @@ class FusedV6:
         p, r, n = FusedV6._p, lora_size, A * Cn
         if not checked:
             _operands("v6_time_mix", A, cursors, ((lora, 5 * A * r), (w2, 5 * Cn * r), (time_mix, 5 * Cn), (att_x, n), (att_sx, 5 * n)))
-        _check(lib().wrq_v6_time_mix(_stream(), Cn, A, lora_size, p(cursors), p(lora), p(w2), p(time_mix), C.byref(as_view(state, state_view)), p(att_x), p(att_sx)))
+        _check(lib().wrq_v6_time_mix(_stream(), Cn, A, lora_size, p(cursors), p(lora), p(w2), p(time_mix), _view(state, state_view), p(att_x), p(att_sx)))
 
     @staticmethod
     def decay(Cn, A, lora_size, lora, w2, time_decay, out, checked=False):
@@ -550,7 +600,7 @@ class FusedV6:
         p, n = FusedV6._p, A * S * H
         if not checked:
             _operands("v6_wkv_gate", A, cursors, ((g, n), (gn_w, S * H), (gn_b, S * H), (att_x, n)), ((time_decay, n), (time_first, S * H), (k, n), (v, n), (r, n)))
-        _check(lib().wrq_v6_wkv_gate(_stream(), S, H, A, p(cursors), p(time_decay), p(time_first), C.byref(as_view(state, state_view)), p(k), p(v), p(r), p(g),
+        _check(lib().wrq_v6_wkv_gate(_stream(), S, H, A, p(cursors), p(time_decay), p(time_first), _view(state, state_view), p(k), p(v), p(r), p(g),
                                      p(gn_w), p(gn_b), eps, p(att_x)))
 
     @staticmethod
@@ -558,7 +608,7 @@ class FusedV6:
         p, n = FusedV6._p, A * Cn
         if not checked:
             _operands("v6_post_ffn", A, cursors, ((r, n), (v, n), (ffn_x, n), (x_in, n), (x_out, n)))
-        _check(lib().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
+        _check(lib().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), _view(state, state_view), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
 
 
 class FusedV7:
@@ -577,7 +627,7 @@ class FusedV7:
             FusedV6._check_pre("fused_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
         if len(shifts) < len(factors):
             raise TensorError(ERR_SHAPE, f"fused_pre: {len(shifts)} outputs for {len(factors)} token shifts")
-        _check(lib().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, C.byref(as_view(state, state_view)), len(factors),
+        _check(lib().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, _view(state, state_view), len(factors),
                                    a(factors), p(ln_out), a(shifts)))
 
     @staticmethod
@@ -608,7 +658,7 @@ class FusedV7:
         p, m = FusedV6._p, A * S * H
         if not checked:
             _operands("v7_wkv_gate", A, cursors, ((r, m), (w, m), (n, 4 * m), (r_k, S * H), (g, m), (gn_w, S * H), (gn_b, S * H), (att_x, m)))
-        _check(lib().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), C.byref(as_view(state, state_view)), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
+        _check(lib().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), _view(state, state_view), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
                                      p(att_x)))
 
     @staticmethod
@@ -616,7 +666,7 @@ class FusedV7:
         p, n = FusedV6._p, A * Cn
         if not checked:
             _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n), (ffn_out, n)))
-        _check(lib().wrq_v7_post_ffn_buffers(_stream(), Cn, A, p(cursors), C.byref(as_view(state, state_view)), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale),
+        _check(lib().wrq_v7_post_ffn_buffers(_stream(), Cn, A, p(cursors), _view(state, state_view), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale),
                                              p(ffn_out)))
 
 
