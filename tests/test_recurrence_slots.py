@@ -76,6 +76,50 @@ def test_gpu_fused_keeps_the_last_input(gpu, version, runs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("runs", [[(0, 15)], [(0, 16)], [(0, 17)], [(0, 33), (0, 7), (0, 255)], [(0, 40), (1, 1), (0, 3), (1, 20)]], ids=str)
+@pytest.mark.parametrize("form", ["time_mix_v5", "time_mix_v6", "time_mix_v7", "v6 gate", "v7 gate"])
+def test_gpu_wide_walk(gpu, form, runs):
+    """Sixteen lanes per pair of columns where the stack has 16 tokens and more per slot: the bits that eight lanes give for
+    the same stack on a state of many slots, outputs and state."""
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("wide walk of the recurrence", form, runs, flush=True)
+    H, S = 3, 64
+    C = H * S
+    cur = lop.pack_cursors(runs)
+    A, named = len(cur), 1 + max(slot for slot, _ in runs)
+    curd = torch.from_numpy(cur.view(np.int32)).cuda()
+    results = []
+    for B in (named, 40):
+        g = torch.Generator().manual_seed(0x5760 + A)
+        f32 = lambda *s: (torch.randn(s, generator=g) * 0.3).cuda()
+        f16 = lambda *s: f32(*s).half()
+        first = f32(named, S + 1, C)
+        state = torch.zeros((B, S + 1, C), device="cuda")
+        state[:named] = first
+        view = ((C, S + 1, B), (C, S + 1, B), (0, 0, 0))
+        decay = torch.sigmoid(f32(A, H, S))
+        if form == "v6 gate":
+            x = f16(A, C)
+            gpu.FusedV6.wkv_gate(S, H, A, curd, decay.view(A, C), f32(H, S), state, view, f32(A, C), f32(A, C), f32(A, C), f16(A, C), f16(H, S), f16(H, S), 64e-5, x)
+        elif form == "v7 gate":
+            x = f16(A, C)
+            gpu.FusedV7.wkv_gate(S, H, A, curd, state, view, f16(A, C), f16(A, C), f16(4, A, C), f16(H, S), f16(A, C), f16(H, S), f16(H, S), 64e-5, x)
+        elif form == "time_mix_v7":
+            x = f16(A, H, S)
+            gpu.LayerOp.time_mix_v7(curd, state, f16(A, H, S), f16(A, H, S), f16(4, A, H, S), x)
+        else:
+            x = f32(A, H, S)
+            getattr(gpu.LayerOp, form)(curd, decay[0].contiguous() if form == "time_mix_v5" else decay, f32(H, S), state, f32(A, H, S), f32(A, H, S), f32(A, H, S), x)
+        assert not state[named:].any()
+        results.append((x, state[:named].clone()))
+    for a, b in zip(*results):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("op", ["channel_mix", "channel_mix_v7", "v6_post_ffn", "v7_post_ffn"])
 @pytest.mark.parametrize("C", [64, 1028, 4096])
 @pytest.mark.parametrize("runs", [[(0, 1)], [(0, 1), (1, 2), (0, 1), (0, 3), (1, 1)], [(1, 1)] + [(0, 1)] * 63 + [(1, 1)], [(1, 1)] * 70 + [(0, 2), (3, 1)], [(2, 255), (2, 9), (7, 3)]],

@@ -36,9 +36,9 @@ __device__ __forceinline__ bool own_slot(const uint32_t *cursors, uint32_t A, ui
 __device__ __forceinline__ uint32_t slot_tokens(const uint32_t *cursors, uint32_t base, uint32_t A, uint32_t slot, uint32_t slots, bool every, uint8_t *list, uint32_t *count) {
     if (every) return min(kSlotScan, A - base);
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool mine = base + tid < A && min(cursors[min(base + tid, A - 1)] & 0xffu, slots - 1) == slot;
+    const bool mine = tid < kSlotScan && base + tid < A && min(cursors[min(base + tid, A - 1)] & 0xffu, slots - 1) == slot;
     const uint64_t mask = __ballot(mine);
-    if (lane == 0) count[wave] = (uint32_t)__popcll(mask);
+    if (lane == 0 && wave < kSlotScan / 64) count[wave] = (uint32_t)__popcll(mask);
     __syncthreads();
     uint32_t before = 0, total = 0;
 #pragma unroll
@@ -65,13 +65,15 @@ __device__ __forceinline__ float lanes_sum(float v) {
 
 __device__ __forceinline__ float round_h(float v) { return h2f(f2h(v)); }
 
-template <int SZ>
+template <int SZ, bool WIDE = false>
 struct RecurrenceTile {
-    static constexpr int L = SZ >= 32 ? 8 : 4;  // lanes that share CPT columns of S
-    static constexpr int CPT = L / 4;           // columns of a lane
+    static_assert(!WIDE || SZ == 64, "the wide form: head size 64");
+    static constexpr int THREADS = WIDE ? 512 : 256;
+    static constexpr int L = WIDE ? 16 : SZ >= 32 ? 8 : 4; // lanes that share CPT columns of S
+    static constexpr int CPT = SZ >= 32 ? 2 : 1;           // columns of a lane
     static constexpr int JL = SZ / L;           // rows of S a lane holds
     static constexpr int TB = 1024 / SZ;        // tokens per chunk: a 4-element vector of each operand per thread
-    static constexpr int TL = SZ / 4;           // threads per token of a chunk
+    static constexpr int TL = SZ / 4;           // threads per token of a chunk, the first 256 of the workgroup
 };
 
 template <int N>
@@ -126,6 +128,23 @@ __device__ __forceinline__ void walk_tokens(uint32_t tend, Token token, Flush fl
     flush(tt, tend - tt);
 }
 
+// The wide form: 512 threads, sixteen lanes share two columns and hold four rows each.  The same LDS bytes and half the vector work
+// per wave and token, by eight waves instead of four: one wave per SIMD issues a vector instruction every 2.3 ns whatever its
+// dependences allow, two reach one per 1.15 ns.  Both forms add a column's rows in the same order (rows_sum, then the lanes in
+// pairs, fours, ...), so they give the same bits.  The wide one is taken for head size 64 where the stack has 16 tokens and more per
+// slot of the state and the workgroups have a CU each: 32 heads, one request, v6 gate form / v7 / v5 (f32): 16 tokens 7.3 / 9.4 / 6.8 ->
+// 6.6 / 8.4 / 6.2 us, 100 tokens 25.6 / 38.8 / 21.7 -> 23.4 / 34.9 / 21.2, 512 tokens 111 / 177 / 91.6 -> 100 / 159 / 90.0; 64 heads,
+// 4 requests of 16 tokens 8.3 / 10.6 / 7.7 -> 7.9 / 9.8 / 7.4.  Not so beyond: 8 requests of 16 tokens 11.0 / 13.8 -> 11.1 / 17.7, 32
+// requests of one token (32 heads) 12.8 / 15.0 -> 15.3 / 18.7, their time being the state's way in and out.
+inline bool wide_walk(const ViewArgs &vs, uint32_t H, uint32_t A) { return A >= 16ull * vs.shape[2] && (uint64_t)H * vs.shape[2] <= 256; }
+
+// Sum of the partial sums of a lane's rows: [rows of an even or odd group of four][even or odd row].
+template <int JL>
+__device__ __forceinline__ float rows_sum(const float (&v)[2][2]) {
+    if constexpr (JL >= 8) return (v[0][0] + v[0][1]) + (v[1][0] + v[1][1]);
+    else return v[0][0] + v[0][1];
+}
+
 // Outputs of a group of tokens of one slot, token l in lane l.
 template <int N, typename XT>
 __device__ __forceinline__ void store_tokens(uint32_t count, uint32_t l, const uint32_t *tokens, const float (&y)[N], XT *x, uint32_t C, uint32_t chan) {
@@ -161,10 +180,10 @@ __device__ __forceinline__ float4 head_norm(float4 y, uint2 wq, uint2 bq, float 
 // GATE: the fused form, y then goes through the group norm (rounded to f16) and silu(g) into att_x; otherwise into x.
 // grid (heads, slot_grid).  The operands come in chunks of TB tokens of the slot: every thread fetches one 4-element
 // vector of each while the previous chunk is worked on and passes it round through LDS (two buffers).
-template <typename XT, int SZ, bool TOKEN_DECAY, bool GATE>
-__global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
+template <typename XT, int SZ, bool TOKEN_DECAY, bool GATE, bool WIDE = false>
+__global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
                                                        const XT *v, const XT *r, XT *x, ViewArgs vs, uint32_t H, uint32_t A, GateArgs ga) {
-    using G = RecurrenceTile<SZ>;
+    using G = RecurrenceTile<SZ, WIDE>;
     constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL;
     static_assert(!GATE || (SZ == 64 && sizeof(XT) == 4), "the fused form: head size 64, f32 operands");
     __shared__ __align__(16) float ks[2][1024], rs[2][1024], ws[TOKEN_DECAY ? 2 : 1][TOKEN_DECAY ? 1024 : 4], vsh[2][1024], ysh[GATE ? 1024 : 4];
@@ -179,7 +198,8 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
     const uint32_t l = tid % L;
     const uint32_t C = SZ * H;
     // this thread's vector of a chunk: token tid / TL of the chunk, elements 4 (tid % TL) ..
-    const uint32_t lt = tid / TL, le = 4 * (tid % TL);
+    const uint32_t lt = (tid % 256) / TL, le = 4 * (tid % TL);
+    const bool staging = !WIDE || tid < 256;
     const float4 u4 = *reinterpret_cast<const float4 *>(time_first + head * SZ + le);
     uint2 gw = make_uint2(0, 0), gb = make_uint2(0, 0);
     if constexpr (GATE) gw = *reinterpret_cast<const uint2 *>(ga.gn_w + head * SZ + le), gb = *reinterpret_cast<const uint2 *>(ga.gn_b + head * SZ + le);
@@ -197,6 +217,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
     uint32_t fc = 0, ft = 0, fct = 0;
     uint32_t base = 0, n = 0;
     auto fetch = [&](uint32_t chunk) {
+        if (!staging) return;
         auto token = [&](uint32_t j) { return base + (every ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
         ft = token(chunk * TB + lt);
         const uint64_t g = (uint64_t)ft * C + head * SZ + le;
@@ -208,6 +229,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
         else if (tid < (uint32_t)TB) fct = token(chunk * TB + tid), fc = cursors[fct];
     };
     auto stage = [&](int buf) {
+        if (!staging) return;
         *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
         *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
         if constexpr (TOKEN_DECAY) *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = fw;
@@ -248,7 +270,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
                 if (chunk + 1 < nchunk) fetch(chunk + 1);
                 __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
                 const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
-                if (!GATE && first_pass && lt < tend && keeps_input(tsh[buf], csh[buf], lt, tend))
+                if (!GATE && first_pass && staging && lt < tend && keeps_input(tsh[buf], csh[buf], lt, tend))
                     *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                 if (live) {
                     float yo[CPT] = {}; // y of token u of a group of L in lane u of the L that share the columns
@@ -256,9 +278,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
                         float vv[CPT], y[CPT];
                         load_cols(vv, &vsh[buf][tt * SZ + i]);
                         const float *kp = &ks[buf][tt * SZ + l * JL], *rp = &rs[buf][tt * SZ + l * JL], *wp = &ws[TOKEN_DECAY ? buf : 0][TOKEN_DECAY ? tt * SZ + l * JL : 0];
-                        float y2[CPT][2];
-#pragma unroll
-                        for (int c = 0; c < CPT; c++) y2[c][0] = y2[c][1] = 0.0f;
+                        float y2[CPT][2][2] = {};
 #pragma unroll
                         for (int q = 0; q < JL / 4; q++) {
                             const float4 k4 = *reinterpret_cast<const float4 *>(kp + 4 * q), r4 = *reinterpret_cast<const float4 *>(rp + 4 * q);
@@ -276,13 +296,13 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
 #pragma unroll
                                 for (int c = 0; c < CPT; c++) {
                                     float &sv = s[4 * q + e][c];
-                                    y2[c][e & 1] = fmaf(rr[e], sv, y2[c][e & 1]);
+                                    y2[c][q & 1][e & 1] = fmaf(rr[e], sv, y2[c][q & 1][e & 1]);
                                     sv = fmaf(ww[e], sv, kk[e] * vv[c]);
                                 }
                         }
 #pragma unroll
                         for (int c = 0; c < CPT; c++) {
-                            y[c] = lanes_sum<L>(y2[c][0] + y2[c][1]);
+                            y[c] = lanes_sum<L>(rows_sum<JL>(y2[c]));
                             if (!GATE) y[c] = fmaf(bonus[buf][tt], vv[c], y[c]);
                             yo[c] = l == (uint32_t)u ? y[c] : yo[c];
                         }
@@ -297,7 +317,7 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
                 }
                 if constexpr (GATE) {
                     __syncthreads(); // the chunk's y are in LDS
-                    if (lt < tend) {
+                    if (staging && lt < tend) {
                         if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
                         const float b = bonus[buf][lt];
@@ -322,10 +342,10 @@ __global__ __launch_bounds__(256) void time_mix_kernel(const uint32_t *cursors, 
 //   sa[i] = sum_j S[j][i] a[j];   S[j][i] <- S[j][i] w[j] + k[j] v[i] + sa[i] b[j];   y[i] = sum_j r[j] S[j][i]
 // GATE: the fused form; y (rounded to f16) then goes through the group norm, the bonus (sum_j u[j] k[j] r[j]) v[i]
 // (u = `first`) and the gate g into att_x, rounded to f16 after each as the op list stores it.
-template <typename XT, int SZ, bool GATE>
-__global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursors, float *state, const XT *r, const XT *w, const XT *n_, XT *x, ViewArgs vs,
+template <typename XT, int SZ, bool GATE, bool WIDE = false>
+__global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uint32_t *cursors, float *state, const XT *r, const XT *w, const XT *n_, XT *x, ViewArgs vs,
                                                           uint32_t H, uint32_t A, const uint16_t *first, GateArgs ga) {
-    using G = RecurrenceTile<SZ>;
+    using G = RecurrenceTile<SZ, WIDE>;
     constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL;
     static_assert(!GATE || (SZ == 64 && sizeof(XT) == 2), "the fused form: head size 64, f16 operands");
     __shared__ __align__(16) float rs[2][1024], ws[2][1024], ks[2][1024], as[2][1024], bs[2][1024], vsh[2][1024], ysh[GATE ? 1024 : 4];
@@ -339,7 +359,8 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
     const uint32_t l = tid % L;
     const uint32_t C = SZ * H;
     const uint64_t plane = (uint64_t)A * C; // n_ holds k, v, a, kk one after the other
-    const uint32_t lt = tid / TL, le = 4 * (tid % TL);
+    const uint32_t lt = (tid % 256) / TL, le = 4 * (tid % TL);
+    const bool staging = !WIDE || tid < 256;
     uint2 gw = make_uint2(0, 0), gb = make_uint2(0, 0);
     float4 u4 = make_float4(0.f, 0.f, 0.f, 0.f);
     if constexpr (GATE) {
@@ -358,6 +379,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
     uint32_t fc = 0, ft = 0, fct = 0;
     uint32_t base = 0, n = 0;
     auto fetch = [&](uint32_t chunk) {
+        if (!staging) return;
         auto token = [&](uint32_t j) { return base + (every ? min(j, n - 1) : (uint32_t)list[min(j, n - 1)]); }; // clamped: past the slot's tokens, never used
         ft = token(chunk * TB + lt);
         const uint64_t g = (uint64_t)ft * C + head * SZ + le;
@@ -370,6 +392,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
     };
     auto decay = [](float v) { return expf(-0.606531f / (1.0f + expf(-v))); }; // exp(-exp(-0.5) sigmoid(w))
     auto stage = [&](int buf) {
+        if (!staging) return;
         *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
         *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = make_float4(decay(fw.x), decay(fw.y), decay(fw.z), decay(fw.w));
         *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
@@ -406,16 +429,14 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
                 if (chunk + 1 < nchunk) fetch(chunk + 1);
                 __syncthreads(); // chunk `chunk` is in LDS; buffer buf ^ 1 is free
                 const uint32_t tend = min((uint32_t)TB, n - chunk * TB);
-                if (!GATE && first_pass && lt < tend && keeps_input(tsh[buf], csh[buf], lt, tend))
+                if (!GATE && first_pass && staging && lt < tend && keeps_input(tsh[buf], csh[buf], lt, tend))
                     *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                 if (live) {
                     float yo[CPT] = {}; // y of token u of a group of L in lane u of the L that share the columns
                     auto token = [&](uint32_t tt, int u) {
-                        float vv[CPT], sa[CPT], acc[CPT][2];
+                        float vv[CPT], sa[CPT], za[CPT][2][2] = {}, acc[CPT][2][2] = {};
                         load_cols(vv, &vsh[buf][tt * SZ + i]);
                         const uint32_t at = tt * SZ + l * JL;
-#pragma unroll
-                        for (int c = 0; c < CPT; c++) acc[c][0] = acc[c][1] = 0.0f;
 #pragma unroll
                         for (int q = 0; q < JL / 4; q++) {
                             const float4 a4 = *reinterpret_cast<const float4 *>(&as[buf][at + 4 * q]);
@@ -423,10 +444,10 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
 #pragma unroll
                             for (int e = 0; e < 4; e++)
 #pragma unroll
-                                for (int c = 0; c < CPT; c++) acc[c][e & 1] = fmaf(s[4 * q + e][c], aa[e], acc[c][e & 1]);
+                                for (int c = 0; c < CPT; c++) za[c][q & 1][e & 1] = fmaf(s[4 * q + e][c], aa[e], za[c][q & 1][e & 1]);
                         }
 #pragma unroll
-                        for (int c = 0; c < CPT; c++) sa[c] = lanes_sum<L>(acc[c][0] + acc[c][1]), acc[c][0] = acc[c][1] = 0.0f;
+                        for (int c = 0; c < CPT; c++) sa[c] = lanes_sum<L>(rows_sum<JL>(za[c]));
 #pragma unroll
                         for (int q = 0; q < JL / 4; q++) {
                             const float4 w4 = *reinterpret_cast<const float4 *>(&ws[buf][at + 4 * q]), k4 = *reinterpret_cast<const float4 *>(&ks[buf][at + 4 * q]),
@@ -439,12 +460,12 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
                                 for (int c = 0; c < CPT; c++) {
                                     float &sv = s[4 * q + e][c];
                                     sv = fmaf(sa[c], bb[e], fmaf(sv, ww[e], kk[e] * vv[c]));
-                                    acc[c][e & 1] = fmaf(rr[e], sv, acc[c][e & 1]);
+                                    acc[c][q & 1][e & 1] = fmaf(rr[e], sv, acc[c][q & 1][e & 1]);
                                 }
                         }
 #pragma unroll
                         for (int c = 0; c < CPT; c++) {
-                            const float y = lanes_sum<L>(acc[c][0] + acc[c][1]);
+                            const float y = lanes_sum<L>(rows_sum<JL>(acc[c]));
                             yo[c] = l == (uint32_t)u ? y : yo[c];
                         }
                     };
@@ -458,7 +479,7 @@ __global__ __launch_bounds__(256) void time_mix_v7_kernel(const uint32_t *cursor
                 }
                 if constexpr (GATE) {
                     __syncthreads(); // the chunk's y are in LDS
-                    if (lt < tend) {
+                    if (staging && lt < tend) {
                         if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
                         const float4 k4 = *reinterpret_cast<const float4 *>(&ks[buf][4 * tid]), r4 = *reinterpret_cast<const float4 *>(&rs[buf][4 * tid]);

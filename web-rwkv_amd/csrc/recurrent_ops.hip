@@ -208,23 +208,29 @@ int time_mix(const char *name, bool token_decay, wrq_stream stream, const wrq_te
     const float *td = static_cast<const float *>(time_decay->data), *tfp = static_cast<const float *>(time_first->data);
     float *sp = static_cast<float *>(state->data);
     const dim3 grid(H, slot_grid(vs, A));
+    const bool wide = S == 64 && wide_walk(vs, H, A);
+#define WRQ_TM_FORM(XT, SZ, TD, WIDE)                                                                                                            \
+    hipLaunchKernelGGL((time_mix_kernel<XT, SZ, TD, false, WIDE>), grid, dim3(WIDE ? 512 : 256), 0, hs, cur, td, tfp, sp,                         \
+                       static_cast<const XT *>(k->data), static_cast<const XT *>(v->data), static_cast<const XT *>(r->data),                    \
+                       static_cast<XT *>(x->data), vs, H, A, GateArgs{})
 #define WRQ_TM_LAUNCH(XT, SZ, TD)                                                                                                                \
-    hipLaunchKernelGGL((time_mix_kernel<XT, SZ, TD, false>), grid, dim3(256), 0, hs, cur, td, tfp, sp, static_cast<const XT *>(k->data),           \
-                       static_cast<const XT *>(v->data), static_cast<const XT *>(r->data), static_cast<XT *>(x->data), vs, H, A, GateArgs{})
+    if (wide) WRQ_TM_FORM(XT, SZ, TD, (SZ == 64));                                                                                               \
+    else WRQ_TM_FORM(XT, SZ, TD, false)
 #define WRQ_TM(SZ)                                                                                                                               \
     if (S == SZ) {                                                                                                                               \
         if (dtype == WRQ_F16) {                                                                                                                  \
-            if (token_decay) WRQ_TM_LAUNCH(uint16_t, SZ, true);                                                                                  \
-            else WRQ_TM_LAUNCH(uint16_t, SZ, false);                                                                                             \
+            if (token_decay) { WRQ_TM_LAUNCH(uint16_t, SZ, true); }                                                                              \
+            else { WRQ_TM_LAUNCH(uint16_t, SZ, false); }                                                                                         \
         } else {                                                                                                                                 \
-            if (token_decay) WRQ_TM_LAUNCH(float, SZ, true);                                                                                     \
-            else WRQ_TM_LAUNCH(float, SZ, false);                                                                                                \
+            if (token_decay) { WRQ_TM_LAUNCH(float, SZ, true); }                                                                                 \
+            else { WRQ_TM_LAUNCH(float, SZ, false); }                                                                                            \
         }                                                                                                                                        \
         return check_launch(name);                                                                                                               \
     }
     WRQ_TM(16) WRQ_TM(32) WRQ_TM(64) WRQ_TM(128) WRQ_TM(256)
 #undef WRQ_TM
 #undef WRQ_TM_LAUNCH
+#undef WRQ_TM_FORM
     return fail(WRQ_ERR_UNSUPPORTED, "%s: head size %u (16, 32, 64, 128 or 256 is built)", name, S);
 }
 

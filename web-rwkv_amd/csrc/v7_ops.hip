@@ -305,18 +305,24 @@ int wrq_time_mix_v7(wrq_stream stream, const wrq_tensor *cursors, const wrq_tens
     hipStream_t hs = static_cast<hipStream_t>(stream);
     const uint32_t *cur = static_cast<const uint32_t *>(cursors->data);
     float *sp = static_cast<float *>(state->data);
+    const bool wide = S == 64 && wide_walk(vs, H, A);
+#define WRQ_TM7_FORM(XT, SZ, WIDE)                                                                                                                   \
+    hipLaunchKernelGGL((time_mix_v7_kernel<XT, SZ, false, WIDE>), dim3(H, slot_grid(vs, A)), dim3(WIDE ? 512 : 256), 0, hs, cur, sp,                     \
+                       static_cast<const XT *>(r->data), static_cast<const XT *>(w->data), static_cast<const XT *>(n->data), static_cast<XT *>(x->data), \
+                       vs, H, A, nullptr, GateArgs{})
+#define WRQ_TM7_LAUNCH(XT, SZ)                                                                                                                       \
+    if (wide) WRQ_TM7_FORM(XT, SZ, (SZ == 64));                                                                                                      \
+    else WRQ_TM7_FORM(XT, SZ, false)
 #define WRQ_TM7(SZ)                                                                                                                                  \
     if (S == SZ) {                                                                                                                                   \
-        if (dtype == WRQ_F16)                                                                                                                        \
-            hipLaunchKernelGGL((time_mix_v7_kernel<uint16_t, SZ, false>), dim3(H, slot_grid(vs, A)), dim3(256), 0, hs, cur, sp, static_cast<const uint16_t *>(r->data),        \
-                               static_cast<const uint16_t *>(w->data), static_cast<const uint16_t *>(n->data), static_cast<uint16_t *>(x->data), vs, H, A, nullptr, GateArgs{}); \
-        else                                                                                                                                         \
-            hipLaunchKernelGGL((time_mix_v7_kernel<float, SZ, false>), dim3(H, slot_grid(vs, A)), dim3(256), 0, hs, cur, sp, static_cast<const float *>(r->data),              \
-                               static_cast<const float *>(w->data), static_cast<const float *>(n->data), static_cast<float *>(x->data), vs, H, A, nullptr, GateArgs{});   \
+        if (dtype == WRQ_F16) { WRQ_TM7_LAUNCH(uint16_t, SZ); }                                                                                      \
+        else { WRQ_TM7_LAUNCH(float, SZ); }                                                                                                          \
         return check_launch("time_mix_v7");                                                                                                          \
     }
     WRQ_TM7(32) WRQ_TM7(64) WRQ_TM7(128)
 #undef WRQ_TM7
+#undef WRQ_TM7_LAUNCH
+#undef WRQ_TM7_FORM
     return fail(WRQ_ERR_UNSUPPORTED, "time_mix_v7: head size %u (32, 64 or 128 is built)", S);
 }
 
@@ -457,7 +463,9 @@ int wrq_v7_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const
     if (s != WRQ_OK) return s;
     const ViewArgs vs = view_args(state->view);
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
-    hipLaunchKernelGGL((time_mix_v7_kernel<uint16_t, 64, true>), dim3(H, slot_grid(vs, A)), dim3(256), 0, static_cast<hipStream_t>(stream),
+    const bool wide = wide_walk(vs, H, A);
+    auto *kern = wide ? &time_mix_v7_kernel<uint16_t, 64, true, true> : &time_mix_v7_kernel<uint16_t, 64, true, false>;
+    hipLaunchKernelGGL(kern, dim3(H, slot_grid(vs, A)), dim3(wide ? 512 : 256), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint32_t *>(cursors), static_cast<float *>(state->data), u16(r), u16(w), u16(n), static_cast<uint16_t *>(nullptr), vs, H, A,
                        u16(r_k), GateArgs{u16(g), u16(gn_w), u16(gn_b), static_cast<uint16_t *>(att_x), eps});
     return check_launch(what);
