@@ -4,7 +4,7 @@
 // SZ x SZ).  Requests do not depend on each other, so a workgroup takes one head of ONE state slot and walks that
 // slot's tokens only: 32 requests of one token each are 32 workgroups per head instead of a chain of 32 state
 // reloads in one.  S stays in registers over the slot's tokens: L = 8 lanes share two columns of S and hold SZ / 8
-// of their rows each (SZ = 16: four lanes, one column).  What bounds a long run is the vector ALU of the one CU a
+// of their rows each (SZ = 16: four lanes, one column; long runs of SZ = 64: sixteen lanes, see wide_walk).  What bounds a long run is the vector ALU of the one CU a
 // head's state lives on: per element of S three fmas in v5 / v6 (k v, the decay, y) and five in v7; the bonus term
 // of v5 / v6, sum_j r[j] u[j] k[j] v[i], does not depend on S and is one number per token, formed while the operands
 // are staged.  Sharing two columns halves the LDS reads per token against one column per quad, which came out as
