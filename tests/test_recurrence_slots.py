@@ -75,6 +75,61 @@ def test_gpu_fused_keeps_the_last_input(gpu, version, runs):
         assert torch.equal(state[slot, 0], before[last].float()), slot
 
 
+def column_sums(S, a, s):
+    """sum_j a[j] s[j][i] in f32 as the recurrences add it: the even and the odd rows of S / 8 adjacent ones (S / 4 for S = 16) by
+    fused multiply-adds, these two, then the groups in pairs, fours, ..."""
+    fma = lambda x, y, z: (np.float64(x) * np.float64(y) + np.float64(z)).astype(np.float32)  # the product is exact
+    groups = 8 if S >= 32 else 4
+    part = np.zeros((groups, 2) + s.shape[1:], np.float32)
+    for j in range(S // groups):
+        rows = np.arange(groups) * (S // groups) + j
+        part[:, j & 1] = fma(a[rows, None], s[rows], part[:, j & 1])
+    v = part[:, 0] + part[:, 1]
+    while len(v) > 1:
+        v = v[0::2] + v[1::2]
+    return v[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A", [3, 17])  # 17: sixteen lanes per pair of columns for S = 64
+@pytest.mark.parametrize("version,S", [(5, 16), (5, 64), (6, 32), (6, 64), (6, 128), (6, 256), (7, 32), (7, 64), (7, 128)])
+def test_gpu_order_of_sums(gpu, version, S, A):
+    """One order of the f32 sums for every form of a head size, so that results are the same bits whichever is taken."""
+    import torch
+
+    sys.path.insert(0, ROOT)
+    lop = importlib.import_module("oracle.layer_ops")
+    print("order of the recurrence's sums", version, S, A, flush=True)
+    H, rng, f32 = 2, np.random.default_rng(0x57525C00 + S + A), np.float32
+    fma = lambda x, y, z: (np.float64(x) * np.float64(y) + np.float64(z)).astype(f32)
+    gen = lambda *s: (rng.standard_normal(s) * 0.3).astype(f32)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    k, v, r, a, kk, x, state = gen(A, H, S), gen(A, H, S), gen(A, H, S), gen(A, H, S), gen(A, H, S), gen(A, H, S), gen(1, S + 1, H * S)
+    cur, sd, xd = dev(lop.pack_cursors([(0, A)]).view(np.int32)), dev(state), dev(x)
+    if version == 7:
+        w = np.ones((A, H, S), f32)  # the decay of an input of -200 is exp(-0)
+        gpu.LayerOp.time_mix_v7(cur, sd, dev(r), dev(np.full((A, H, S), -200.0, f32)), dev(np.stack([k, v, a, kk])), xd)
+    else:
+        w = (1 / (1 + np.exp(-gen(A, H, S)))).astype(f32)
+        w = np.broadcast_to(w[0], w.shape) if version == 5 else w
+        op = gpu.LayerOp.time_mix_v5 if version == 5 else gpu.LayerOp.time_mix_v6
+        op(cur, dev(w[0] if version == 5 else w), dev(np.zeros((H, S), f32)), sd, dev(k), dev(v), dev(r), xd)
+    want, rows = np.empty_like(x), state[0, 1:].reshape(S, H, S).copy()
+    for t in range(A):
+        for h in range(H):
+            s = rows[:, h]
+            if version == 7:
+                sa = column_sums(S, -kk[t, h], s)
+                s = fma(sa, (kk[t, h] * a[t, h])[:, None], fma(s, w[t, h][:, None], k[t, h][:, None] * v[t, h]))
+                want[t, h] = column_sums(S, r[t, h], s)
+            else:
+                want[t, h] = column_sums(S, r[t, h], s)
+                s = fma(w[t, h][:, None], s, k[t, h][:, None] * v[t, h])
+            rows[:, h] = s
+    assert np.array_equal(xd.cpu().numpy(), want), "y"
+    assert np.array_equal(sd.cpu().numpy()[0, 1:].reshape(S, H, S), rows), "state"
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("runs", [[(0, 15)], [(0, 16)], [(0, 17)], [(0, 33), (0, 7), (0, 255)], [(0, 40), (1, 1), (0, 3), (1, 20)]], ids=str)
 @pytest.mark.parametrize("form", ["time_mix_v5", "time_mix_v6", "time_mix_v7", "v6 gate", "v7 gate"])

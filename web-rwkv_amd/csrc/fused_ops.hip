@@ -413,7 +413,7 @@ int wrq_v6_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     const bool wide = wide_walk(vs, H, A);
     auto *kern = wide ? &time_mix_kernel<float, 64, true, true, true> : &time_mix_kernel<float, 64, true, true, false>;
-    hipLaunchKernelGGL(kern, dim3(H, slot_grid(vs, A)), dim3(wide ? 512 : 256), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(kern, dim3(H, slot_grid(vs, A)), dim3(wide ? RecurrenceTile<64, true>::THREADS : RecurrenceTile<64>::THREADS), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint32_t *>(cursors), f32(time_decay), f32(time_first), static_cast<float *>(state->data), f32(k), f32(v), f32(r),
                        static_cast<float *>(nullptr), vs, H, A, GateArgs{u16(g), u16(gn_w), u16(gn_b), static_cast<uint16_t *>(att_x), eps});
     return check_launch(what);

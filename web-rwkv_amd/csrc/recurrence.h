@@ -4,11 +4,11 @@
 // SZ x SZ).  Requests do not depend on each other, so a workgroup takes one head of ONE state slot and walks that
 // slot's tokens only: 32 requests of one token each are 32 workgroups per head instead of a chain of 32 state
 // reloads in one.  S stays in registers over the slot's tokens: L = 8 lanes share two columns of S and hold SZ / 8
-// of their rows each (SZ = 16: four lanes, one column; long runs of SZ = 64: sixteen lanes, see wide_walk).  What bounds a long run is the vector ALU of the one CU a
-// head's state lives on: per element of S three fmas in v5 / v6 (k v, the decay, y) and five in v7; the bonus term
-// of v5 / v6, sum_j r[j] u[j] k[j] v[i], does not depend on S and is one number per token, formed while the operands
-// are staged.  Sharing two columns halves the LDS reads per token against one column per quad, which came out as
-// the second bound.
+// of their rows each (SZ = 16: four lanes, one column; long runs of SZ = 64: sixteen lanes, see wide_walk).  What bounds
+// a long run is the vector ALU of the one CU a head's state lives on: per element of S three fmas in v5 / v6 (k v, the
+// decay, y) and five in v7; the bonus term of v5 / v6, sum_j r[j] u[j] k[j] v[i], does not depend on S and is one number
+// per token, formed while the operands are staged.  Sharing two columns halves the LDS reads per token against one
+// column per quad, which came out as the second bound.
 #pragma once
 
 #include "layer_device.h"
@@ -33,12 +33,14 @@ __device__ __forceinline__ bool own_slot(const uint32_t *cursors, uint32_t A, ui
 
 // The tokens of `slot` among cursors[base .. base + 256): their offsets from `base` in stack order, and their number.
 // With a single slot (a slot beyond the view counts as the last one) or a single token, `every` token is its own and `list` stays unused.
+template <int THREADS>
 __device__ __forceinline__ uint32_t slot_tokens(const uint32_t *cursors, uint32_t base, uint32_t A, uint32_t slot, uint32_t slots, bool every, uint8_t *list, uint32_t *count) {
     if (every) return min(kSlotScan, A - base);
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool mine = tid < kSlotScan && base + tid < A && min(cursors[min(base + tid, A - 1)] & 0xffu, slots - 1) == slot;
+    const bool scans = THREADS == kSlotScan || tid < kSlotScan;
+    const bool mine = scans && base + tid < A && min(cursors[min(base + tid, A - 1)] & 0xffu, slots - 1) == slot;
     const uint64_t mask = __ballot(mine);
-    if (lane == 0 && wave < kSlotScan / 64) count[wave] = (uint32_t)__popcll(mask);
+    if (scans && lane == 0) count[wave] = (uint32_t)__popcll(mask);
     __syncthreads();
     uint32_t before = 0, total = 0;
 #pragma unroll
@@ -74,6 +76,29 @@ struct RecurrenceTile {
     static constexpr int JL = SZ / L;           // rows of S a lane holds
     static constexpr int TB = 1024 / SZ;        // tokens per chunk: a 4-element vector of each operand per thread
     static constexpr int TL = SZ / 4;           // threads per token of a chunk, the first 256 of the workgroup
+    static constexpr int PARTS = WIDE ? 1 : 2;  // partial sums of a lane's rows: the even and the odd ones, or all of its own
+    // Rows first_row(l), first_row(l) + ROW_STEP, .. are lane l's.  In the wide form a pair of lanes has eight adjacent rows, the
+    // even lane the even ones: the pair's two sums are then the two partial sums of the narrow form's lane.
+    static constexpr int ROW_STEP = WIDE ? 2 : 1;
+    static __device__ __forceinline__ uint32_t first_row(uint32_t l) { return WIDE ? 8 * (l >> 1) + (l & 1) : l * JL; }
+    // Vector `tid` of a chunk's operand that is indexed by rows; in LDS the rows of a lane lie side by side.
+    static __device__ __forceinline__ void put_rows(float *buf, uint32_t tid, float4 v) {
+        if constexpr (WIDE) {
+            float *p = buf + 4 * (tid & ~1u) + 2 * (tid & 1);
+            *reinterpret_cast<float2 *>(p) = make_float2(v.x, v.z), *reinterpret_cast<float2 *>(p + 4) = make_float2(v.y, v.w);
+        } else {
+            *reinterpret_cast<float4 *>(buf + 4 * tid) = v;
+        }
+    }
+    static __device__ __forceinline__ float4 get_rows(const float *buf, uint32_t tid) {
+        if constexpr (WIDE) {
+            const float *p = buf + 4 * (tid & ~1u) + 2 * (tid & 1);
+            const float2 even = *reinterpret_cast<const float2 *>(p), odd = *reinterpret_cast<const float2 *>(p + 4);
+            return make_float4(even.x, odd.x, even.y, odd.y);
+        } else {
+            return *reinterpret_cast<const float4 *>(buf + 4 * tid);
+        }
+    }
 };
 
 template <int N>
@@ -104,7 +129,7 @@ __device__ __forceinline__ bool keeps_input(const uint32_t *tokens, const uint32
     return true;
 }
 
-// The tokens of a chunk in groups of L.  A whole group is one piece of straight code: the operands of its later tokens are
+// The tokens of a chunk in groups of L (eight; sixteen, a whole chunk, in the wide form).  A whole group is one piece of straight code: the operands of its later tokens are
 // read from LDS while the earlier ones are worked on, where a loop over tokens waits out one LDS round trip, the
 // reduction over the lanes and a branch for the store at each of them.  `token(tt, u)` leaves its result in lane u of the L
 // that share the columns, `flush(from, count)` then stores the group at once.
@@ -130,19 +155,26 @@ __device__ __forceinline__ void walk_tokens(uint32_t tend, Token token, Flush fl
 
 // The wide form: 512 threads, sixteen lanes share two columns and hold four rows each.  The same LDS bytes and half the vector work
 // per wave and token, by eight waves instead of four: one wave per SIMD issues a vector instruction every 2.3 ns whatever its
-// dependences allow, two reach one per 1.15 ns.  Both forms add a column's rows in the same order (rows_sum, then the lanes in
-// pairs, fours, ...), so they give the same bits.  The wide one is taken for head size 64 where the stack has 16 tokens and more per
-// slot of the state and the workgroups have a CU each: 32 heads, one request, v6 gate form / v7 / v5 (f32): 16 tokens 7.3 / 9.4 / 6.8 ->
-// 6.6 / 8.4 / 6.2 us, 100 tokens 25.6 / 38.8 / 21.7 -> 23.4 / 34.9 / 21.2, 512 tokens 111 / 177 / 91.6 -> 100 / 159 / 90.0; 64 heads,
-// 4 requests of 16 tokens 8.3 / 10.6 / 7.7 -> 7.9 / 9.8 / 7.4.  Not so beyond: 8 requests of 16 tokens 11.0 / 13.8 -> 11.1 / 17.7, 32
-// requests of one token (32 heads) 12.8 / 15.0 -> 15.3 / 18.7, their time being the state's way in and out.
+// dependences allow, two reach one per 1.15 ns.  Both forms add a column's rows in the same order (of eight rows the even and the odd
+// ones, these two, then the eights in pairs, fours, ...), so they give the same bits.  The wide one is taken for head size 64 where
+// the stack has 16 tokens and more per slot of the state and the workgroups have a CU each; narrow -> wide in us, v6 gate form / v7
+// gate form / v5 (f32):
+//   32 heads, one request of 16 tokens  7.4 /  9.4 /  6.7 ->  6.7 /  8.1 /  6.3     64 heads, 4 x 16  8.5 / 10.7 / 7.9 -> 7.8 / 9.5 / 7.5
+//                            24 tokens  9.1 / 12.4 /  8.3 ->  8.8 / 11.5 /  8.3               4 x 31  11.9 / 15.8 / 10.9 -> 11.2 / 14.8 / 10.7
+//                            31 tokens 10.8 / 14.6 /  9.6 ->  9.9 / 13.3 /  9.3
+//                           100 tokens 25.6 / 39.0 / 21.7 -> 23.7 / 34.1 / 20.5
+//                           512 tokens  111 /  179 / 91.4 ->  102 /  155 / 85.5
+// Not so beyond: 64 heads, 8 x 16 10.9 / 13.4 / 10.3 -> 10.9 / 16.4 / 10.3; 32 heads, 32 x 1 12.7 / 15.0 / 12.2 -> 14.7 / 18.5 / 14.3
+// and 32 x 16 20.5 / 25.6 / 16.2 -> 21.8 / 32.6 / 20.4, their time being the state's way in and out.  The launch knows the state's
+// slots and not how many of them the stack names: one request of 100 tokens on a state of 32 slots keeps the narrow form (32 heads
+// 25.9 / 39.2 / 21.9, where the wide one takes 24.4 / 34.5 / 21.3).
 inline bool wide_walk(const ViewArgs &vs, uint32_t H, uint32_t A) { return A >= 16ull * vs.shape[2] && (uint64_t)H * vs.shape[2] <= 256; }
 
-// Sum of the partial sums of a lane's rows: [rows of an even or odd group of four][even or odd row].
-template <int JL>
-__device__ __forceinline__ float rows_sum(const float (&v)[2][2]) {
-    if constexpr (JL >= 8) return (v[0][0] + v[0][1]) + (v[1][0] + v[1][1]);
-    else return v[0][0] + v[0][1];
+// Sum of the partial sums of a lane's rows.
+template <int N>
+__device__ __forceinline__ float parts_sum(const float (&v)[N]) {
+    if constexpr (N == 2) return v[0] + v[1];
+    else return v[0];
 }
 
 // Outputs of a group of tokens of one slot, token l in lane l.
@@ -181,10 +213,10 @@ __device__ __forceinline__ float4 head_norm(float4 y, uint2 wq, uint2 bq, float 
 // grid (heads, slot_grid).  The operands come in chunks of TB tokens of the slot: every thread fetches one 4-element
 // vector of each while the previous chunk is worked on and passes it round through LDS (two buffers).
 template <typename XT, int SZ, bool TOKEN_DECAY, bool GATE, bool WIDE = false>
-__global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
+__global__ __launch_bounds__((RecurrenceTile<SZ, WIDE>::THREADS)) void time_mix_kernel(const uint32_t *cursors, const float *time_decay, const float *time_first, float *state, const XT *k,
                                                        const XT *v, const XT *r, XT *x, ViewArgs vs, uint32_t H, uint32_t A, GateArgs ga) {
     using G = RecurrenceTile<SZ, WIDE>;
-    constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL;
+    constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL, PARTS = G::PARTS;
     static_assert(!GATE || (SZ == 64 && sizeof(XT) == 4), "the fused form: head size 64, f32 operands");
     __shared__ __align__(16) float ks[2][1024], rs[2][1024], ws[TOKEN_DECAY ? 2 : 1][TOKEN_DECAY ? 1024 : 4], vsh[2][1024], ysh[GATE ? 1024 : 4];
     __shared__ float bonus[2][TB];
@@ -230,9 +262,9 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32
     };
     auto stage = [&](int buf) {
         if (!staging) return;
-        *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
-        *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
-        if constexpr (TOKEN_DECAY) *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = fw;
+        G::put_rows(ks[buf], tid, fk);
+        G::put_rows(rs[buf], tid, fr);
+        if constexpr (TOKEN_DECAY) G::put_rows(ws[buf], tid, fw);
         *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
         const float b = lanes_sum<TL>(fmaf(fr.x, u4.x * fk.x, fr.y * (u4.y * fk.y)) + fmaf(fr.z, u4.z * fk.z, fr.w * (u4.w * fk.w)));
         if (tid % TL == 0) bonus[buf][lt] = b;
@@ -243,20 +275,20 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32
         const uint32_t i = i0 + CPT * (tid / L);
         const bool live = i < SZ; // head sizes below 64 leave waves without a column
         const uint32_t chan = head * SZ + min(i, (uint32_t)(SZ - CPT));
-        float *const rows = state + view_elem(vs, slot, l * JL + 1, chan); // the lane's rows of S, one row of the state apart
+        float *const rows = state + view_elem(vs, slot, G::first_row(l) + 1, chan); // the lane's rows of S, ROW_STEP rows of the state apart
         float s[JL][CPT], wc[TOKEN_DECAY ? 1 : JL]; // wc: the constant decay of this lane's rows
         if constexpr (!TOKEN_DECAY) {
 #pragma unroll
-            for (int jj = 0; jj < JL; jj++) wc[jj] = time_decay[head * SZ + l * JL + jj];
+            for (int jj = 0; jj < JL; jj++) wc[jj] = time_decay[head * SZ + G::first_row(l) + G::ROW_STEP * jj];
         }
         bool held = false;
         for (base = 0; base < A; base += kSlotScan) {
-            n = slot_tokens(cursors, base, A, slot, slots, every, list, count);
+            n = slot_tokens<G::THREADS>(cursors, base, A, slot, slots, every, list, count);
             if (n == 0) continue;
             fetch(0);
             if (!held) {
 #pragma unroll
-                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], rows + (uint64_t)jj * vs.stride[0]);
+                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], rows + (uint64_t)(G::ROW_STEP * jj) * vs.stride[0]);
                 held = true;
             }
             const uint32_t nchunk = (n + TB - 1) / TB;
@@ -278,7 +310,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32
                         float vv[CPT], y[CPT];
                         load_cols(vv, &vsh[buf][tt * SZ + i]);
                         const float *kp = &ks[buf][tt * SZ + l * JL], *rp = &rs[buf][tt * SZ + l * JL], *wp = &ws[TOKEN_DECAY ? buf : 0][TOKEN_DECAY ? tt * SZ + l * JL : 0];
-                        float y2[CPT][2][2] = {};
+                        float y2[CPT][PARTS] = {};
 #pragma unroll
                         for (int q = 0; q < JL / 4; q++) {
                             const float4 k4 = *reinterpret_cast<const float4 *>(kp + 4 * q), r4 = *reinterpret_cast<const float4 *>(rp + 4 * q);
@@ -296,13 +328,13 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32
 #pragma unroll
                                 for (int c = 0; c < CPT; c++) {
                                     float &sv = s[4 * q + e][c];
-                                    y2[c][q & 1][e & 1] = fmaf(rr[e], sv, y2[c][q & 1][e & 1]);
+                                    y2[c][e % PARTS] = fmaf(rr[e], sv, y2[c][e % PARTS]);
                                     sv = fmaf(ww[e], sv, kk[e] * vv[c]);
                                 }
                         }
 #pragma unroll
                         for (int c = 0; c < CPT; c++) {
-                            y[c] = lanes_sum<L>(rows_sum<JL>(y2[c]));
+                            y[c] = lanes_sum<L>(parts_sum(y2[c]));
                             if (!GATE) y[c] = fmaf(bonus[buf][tt], vv[c], y[c]);
                             yo[c] = l == (uint32_t)u ? y[c] : yo[c];
                         }
@@ -332,7 +364,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32
         }
         if (live && held) {
 #pragma unroll
-            for (int jj = 0; jj < JL; jj++) store_cols(rows + (uint64_t)jj * vs.stride[0], s[jj]);
+            for (int jj = 0; jj < JL; jj++) store_cols(rows + (uint64_t)(G::ROW_STEP * jj) * vs.stride[0], s[jj]);
         }
         first_pass = false;
     }
@@ -343,10 +375,10 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_kernel(const uint32
 // GATE: the fused form; y (rounded to f16) then goes through the group norm, the bonus (sum_j u[j] k[j] r[j]) v[i]
 // (u = `first`) and the gate g into att_x, rounded to f16 after each as the op list stores it.
 template <typename XT, int SZ, bool GATE, bool WIDE = false>
-__global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uint32_t *cursors, float *state, const XT *r, const XT *w, const XT *n_, XT *x, ViewArgs vs,
+__global__ __launch_bounds__((RecurrenceTile<SZ, WIDE>::THREADS)) void time_mix_v7_kernel(const uint32_t *cursors, float *state, const XT *r, const XT *w, const XT *n_, XT *x, ViewArgs vs,
                                                           uint32_t H, uint32_t A, const uint16_t *first, GateArgs ga) {
     using G = RecurrenceTile<SZ, WIDE>;
-    constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL;
+    constexpr int L = G::L, CPT = G::CPT, JL = G::JL, TB = G::TB, TL = G::TL, PARTS = G::PARTS;
     static_assert(!GATE || (SZ == 64 && sizeof(XT) == 2), "the fused form: head size 64, f16 operands");
     __shared__ __align__(16) float rs[2][1024], ws[2][1024], ks[2][1024], as[2][1024], bs[2][1024], vsh[2][1024], ysh[GATE ? 1024 : 4];
     __shared__ uint32_t csh[2][TB], tsh[2][TB]; // cursors and numbers of the chunk's tokens
@@ -393,11 +425,11 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
     auto decay = [](float v) { return expf(-0.606531f / (1.0f + expf(-v))); }; // exp(-exp(-0.5) sigmoid(w))
     auto stage = [&](int buf) {
         if (!staging) return;
-        *reinterpret_cast<float4 *>(&rs[buf][4 * tid]) = fr;
-        *reinterpret_cast<float4 *>(&ws[buf][4 * tid]) = make_float4(decay(fw.x), decay(fw.y), decay(fw.z), decay(fw.w));
-        *reinterpret_cast<float4 *>(&ks[buf][4 * tid]) = fk;
-        *reinterpret_cast<float4 *>(&as[buf][4 * tid]) = make_float4(-fkk.x, -fkk.y, -fkk.z, -fkk.w);
-        *reinterpret_cast<float4 *>(&bs[buf][4 * tid]) = make_float4(fkk.x * fa.x, fkk.y * fa.y, fkk.z * fa.z, fkk.w * fa.w);
+        G::put_rows(rs[buf], tid, fr);
+        G::put_rows(ws[buf], tid, make_float4(decay(fw.x), decay(fw.y), decay(fw.z), decay(fw.w)));
+        G::put_rows(ks[buf], tid, fk);
+        G::put_rows(as[buf], tid, make_float4(-fkk.x, -fkk.y, -fkk.z, -fkk.w));
+        G::put_rows(bs[buf], tid, make_float4(fkk.x * fa.x, fkk.y * fa.y, fkk.z * fa.z, fkk.w * fa.w));
         *reinterpret_cast<float4 *>(&vsh[buf][4 * tid]) = fv;
         if (GATE && tid % TL == 0) csh[buf][lt] = fc, tsh[buf][lt] = ft;
         if (!GATE && tid < (uint32_t)TB) csh[buf][tid] = fc, tsh[buf][tid] = fct;
@@ -406,16 +438,16 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
         const uint32_t i = i0 + CPT * (tid / L);
         const bool live = i < SZ; // head sizes below 64 leave waves without a column
         const uint32_t chan = head * SZ + min(i, (uint32_t)(SZ - CPT));
-        float *const rows = state + view_elem(vs, slot, l * JL + 1, chan); // the lane's rows of S, one row of the state apart
+        float *const rows = state + view_elem(vs, slot, G::first_row(l) + 1, chan); // the lane's rows of S, ROW_STEP rows of the state apart
         float s[JL][CPT];
         bool held = false;
         for (base = 0; base < A; base += kSlotScan) {
-            n = slot_tokens(cursors, base, A, slot, slots, every, list, count);
+            n = slot_tokens<G::THREADS>(cursors, base, A, slot, slots, every, list, count);
             if (n == 0) continue;
             fetch(0);
             if (!held) {
 #pragma unroll
-                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], rows + (uint64_t)jj * vs.stride[0]);
+                for (int jj = 0; jj < JL; jj++) load_cols(s[jj], rows + (uint64_t)(G::ROW_STEP * jj) * vs.stride[0]);
                 held = true;
             }
             const uint32_t nchunk = (n + TB - 1) / TB;
@@ -434,7 +466,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
                 if (live) {
                     float yo[CPT] = {}; // y of token u of a group of L in lane u of the L that share the columns
                     auto token = [&](uint32_t tt, int u) {
-                        float vv[CPT], sa[CPT], za[CPT][2][2] = {}, acc[CPT][2][2] = {};
+                        float vv[CPT], sa[CPT], za[CPT][PARTS] = {}, acc[CPT][PARTS] = {};
                         load_cols(vv, &vsh[buf][tt * SZ + i]);
                         const uint32_t at = tt * SZ + l * JL;
 #pragma unroll
@@ -444,10 +476,10 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
 #pragma unroll
                             for (int e = 0; e < 4; e++)
 #pragma unroll
-                                for (int c = 0; c < CPT; c++) za[c][q & 1][e & 1] = fmaf(s[4 * q + e][c], aa[e], za[c][q & 1][e & 1]);
+                                for (int c = 0; c < CPT; c++) za[c][e % PARTS] = fmaf(s[4 * q + e][c], aa[e], za[c][e % PARTS]);
                         }
 #pragma unroll
-                        for (int c = 0; c < CPT; c++) sa[c] = lanes_sum<L>(rows_sum<JL>(za[c]));
+                        for (int c = 0; c < CPT; c++) sa[c] = lanes_sum<L>(parts_sum(za[c]));
 #pragma unroll
                         for (int q = 0; q < JL / 4; q++) {
                             const float4 w4 = *reinterpret_cast<const float4 *>(&ws[buf][at + 4 * q]), k4 = *reinterpret_cast<const float4 *>(&ks[buf][at + 4 * q]),
@@ -460,12 +492,12 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
                                 for (int c = 0; c < CPT; c++) {
                                     float &sv = s[4 * q + e][c];
                                     sv = fmaf(sa[c], bb[e], fmaf(sv, ww[e], kk[e] * vv[c]));
-                                    acc[c][q & 1][e & 1] = fmaf(rr[e], sv, acc[c][q & 1][e & 1]);
+                                    acc[c][e % PARTS] = fmaf(rr[e], sv, acc[c][e % PARTS]);
                                 }
                         }
 #pragma unroll
                         for (int c = 0; c < CPT; c++) {
-                            const float y = lanes_sum<L>(rows_sum<JL>(acc[c]));
+                            const float y = lanes_sum<L>(parts_sum(acc[c]));
                             yo[c] = l == (uint32_t)u ? y : yo[c];
                         }
                     };
@@ -482,7 +514,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
                     if (staging && lt < tend) {
                         if (keeps_input(tsh[buf], csh[buf], lt, tend)) *reinterpret_cast<float4 *>(state + view_elem(vs, slot, 0, head * SZ + le)) = load_vec4(reinterpret_cast<const IT *>(&cx));
                         const float4 y0 = *reinterpret_cast<const float4 *>(&ysh[4 * tid]), v4 = *reinterpret_cast<const float4 *>(&vsh[buf][4 * tid]);
-                        const float4 k4 = *reinterpret_cast<const float4 *>(&ks[buf][4 * tid]), r4 = *reinterpret_cast<const float4 *>(&rs[buf][4 * tid]);
+                        const float4 k4 = G::get_rows(ks[buf], tid), r4 = G::get_rows(rs[buf], tid);
                         const float b = lanes_sum<16>((u4.x * k4.x * r4.x + u4.y * k4.y * r4.y) + (u4.z * k4.z * r4.z + u4.w * k4.w * r4.w));
                         const float4 o = head_norm(make_float4(round_h(y0.x), round_h(y0.y), round_h(y0.z), round_h(y0.w)), gw, gb, ga.eps);
                         const float4 g4 = load_vec4(reinterpret_cast<const uint16_t *>(&cg));
@@ -496,7 +528,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256) void time_mix_v7_kernel(const uin
         }
         if (live && held) {
 #pragma unroll
-            for (int jj = 0; jj < JL; jj++) store_cols(rows + (uint64_t)jj * vs.stride[0], s[jj]);
+            for (int jj = 0; jj < JL; jj++) store_cols(rows + (uint64_t)(G::ROW_STEP * jj) * vs.stride[0], s[jj]);
         }
         first_pass = false;
     }

@@ -210,7 +210,7 @@ int time_mix(const char *name, bool token_decay, wrq_stream stream, const wrq_te
     const dim3 grid(H, slot_grid(vs, A));
     const bool wide = S == 64 && wide_walk(vs, H, A);
 #define WRQ_TM_FORM(XT, SZ, TD, WIDE)                                                                                                            \
-    hipLaunchKernelGGL((time_mix_kernel<XT, SZ, TD, false, WIDE>), grid, dim3(WIDE ? 512 : 256), 0, hs, cur, td, tfp, sp,                         \
+    hipLaunchKernelGGL((time_mix_kernel<XT, SZ, TD, false, WIDE>), grid, dim3(RecurrenceTile<SZ, WIDE>::THREADS), 0, hs, cur, td, tfp, sp,                         \
                        static_cast<const XT *>(k->data), static_cast<const XT *>(v->data), static_cast<const XT *>(r->data),                    \
                        static_cast<XT *>(x->data), vs, H, A, GateArgs{})
 #define WRQ_TM_LAUNCH(XT, SZ, TD)                                                                                                                \

@@ -307,7 +307,7 @@ int wrq_time_mix_v7(wrq_stream stream, const wrq_tensor *cursors, const wrq_tens
     float *sp = static_cast<float *>(state->data);
     const bool wide = S == 64 && wide_walk(vs, H, A);
 #define WRQ_TM7_FORM(XT, SZ, WIDE)                                                                                                                   \
-    hipLaunchKernelGGL((time_mix_v7_kernel<XT, SZ, false, WIDE>), dim3(H, slot_grid(vs, A)), dim3(WIDE ? 512 : 256), 0, hs, cur, sp,                     \
+    hipLaunchKernelGGL((time_mix_v7_kernel<XT, SZ, false, WIDE>), dim3(H, slot_grid(vs, A)), dim3(RecurrenceTile<SZ, WIDE>::THREADS), 0, hs, cur, sp,                     \
                        static_cast<const XT *>(r->data), static_cast<const XT *>(w->data), static_cast<const XT *>(n->data), static_cast<XT *>(x->data), \
                        vs, H, A, nullptr, GateArgs{})
 #define WRQ_TM7_LAUNCH(XT, SZ)                                                                                                                       \
@@ -465,7 +465,7 @@ int wrq_v7_wkv_gate(wrq_stream stream, uint32_t S, uint32_t H, uint32_t A, const
     auto u16 = [](const void *p) { return static_cast<const uint16_t *>(p); };
     const bool wide = wide_walk(vs, H, A);
     auto *kern = wide ? &time_mix_v7_kernel<uint16_t, 64, true, true> : &time_mix_v7_kernel<uint16_t, 64, true, false>;
-    hipLaunchKernelGGL(kern, dim3(H, slot_grid(vs, A)), dim3(wide ? 512 : 256), 0, static_cast<hipStream_t>(stream),
+    hipLaunchKernelGGL(kern, dim3(H, slot_grid(vs, A)), dim3(wide ? RecurrenceTile<64, true>::THREADS : RecurrenceTile<64>::THREADS), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint32_t *>(cursors), static_cast<float *>(state->data), u16(r), u16(w), u16(n), static_cast<uint16_t *>(nullptr), vs, H, A,
                        u16(r_k), GateArgs{u16(g), u16(gn_w), u16(gn_b), static_cast<uint16_t *>(att_x), eps});
     return check_launch(what);
