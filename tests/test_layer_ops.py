@@ -828,10 +828,10 @@ def test_gpu_lerp_activate_affine(gpu, lop):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
-@pytest.mark.parametrize("C", [8192, 8196, 16384, 20000, 65532, 65536, 65540])
+@pytest.mark.parametrize("C", [8192, 8196, 16384, 16388, 20000, 32768, 32772, 65532, 65536, 65540])
 def test_gpu_softmax_vocabulary_rows(gpu, dtype, C):
-    # both sides of the lengths at which a row moves into the registers of 1024 threads (beyond 8192) and out of them (65536);
-    # a row with masked entries, one where all but one are masked, one of equal values
+    # both sides of the lengths at which a row moves into the registers of 1024 threads (beyond 8192), of which it takes
+    # more (16384, 32768), and out of them (65536); a row with masked entries, one where all but one are masked, one of equal values
     import torch
 
     print("softmax of long rows on the GPU", dtype.__name__, C, flush=True)

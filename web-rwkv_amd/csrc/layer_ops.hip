@@ -16,21 +16,21 @@ namespace wrq {
 namespace {
 
 constexpr int kRowThreads = 256;
-constexpr int kRowCache = 8;   // vectors of 4 elements a thread keeps: rows up to 8192 elements stay in registers
-constexpr int kVocabCache = 16; // the same for softmax rows of a vocabulary on 1024 threads: up to 65536 elements
+constexpr int kRowCache = 8; // vectors of 4 elements a thread keeps: rows up to 8192 elements stay in registers
 
 // One workgroup per row of `n` elements (n % 4 == 0).  MODE 0: softmax; 1: layer norm (w, b of the
 // row's length); 2: group norm (w, b indexed by head * n, the row index modulo `heads`).
 // A softmax keeps the exponentials of a cached row: one workgroup's time on a row of 65536 logits is reading it (256 KB at what
 // one CU takes from L2, 2 us a pass) and expf (about 8 us of its vector units a pass).  Read once and exponentiated once the
 // row takes 11.9 us (32 rows 13.2); in three passes over memory and two of expf it took 18.1 (19.6).
+// CACHE: vectors of 4 elements a thread keeps; 0: the row is read at each use.
 template <typename XT, int MODE, int THREADS, int CACHE = kRowCache>
 __global__ __launch_bounds__(THREADS) void row_kernel(XT *x, const uint16_t *w, const uint16_t *b, uint32_t n, uint32_t heads, float eps) {
     __shared__ float red[THREADS / 64];
     XT *row = x + (uint64_t)blockIdx.x * n;
     const uint32_t nv = n / 4;
-    float4 cache[CACHE];
-    const bool cached = nv <= (uint32_t)(THREADS * CACHE);
+    float4 cache[CACHE ? CACHE : 1];
+    const bool cached = CACHE > 0 && nv <= (uint32_t)(THREADS * CACHE);
     // a cached row asks for its weights together with the row: they are needed only after both reductions, and
     // fetched then they would add a memory round trip to a kernel that is little more than round trips
     uint2 wq[MODE == 0 ? 1 : CACHE], bq[MODE == 0 ? 1 : CACHE];
@@ -186,21 +186,26 @@ int launch_rows(hipStream_t stream, void *x, int dtype, const void *w, const voi
     if (rows > 0x7fffffffull) return fail(WRQ_ERR_SIZE, "%s: data size not match", what);
     const uint16_t *wp = static_cast<const uint16_t *>(w), *bp = static_cast<const uint16_t *>(b);
     // short rows (a head of a group norm) take one wave, no LDS exchange
-    if (MODE == 0 && n > 4 * kRowThreads * kRowCache && n <= 4 * 1024 * kVocabCache) {
-        // a vocabulary-sized softmax row (more than 256 threads keep): 1024 threads, the row in registers
-        // (16384 elements 12.2 us on 256 threads that read it three times, 5.6 us on 1024)
-        if (dtype == WRQ_F16) hipLaunchKernelGGL((row_kernel<uint16_t, 0, 1024, kVocabCache>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
-        else hipLaunchKernelGGL((row_kernel<float, 0, 1024, kVocabCache>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
+    auto run = [&](auto *f16, auto *f32, uint32_t threads) {
+        if (dtype == WRQ_F16) hipLaunchKernelGGL(f16, dim3((uint32_t)rows), dim3(threads), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
+        else hipLaunchKernelGGL(f32, dim3((uint32_t)rows), dim3(threads), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
+    };
+    if (MODE == 0 && n > 4 * kRowThreads * kRowCache) {
+        // Softmax rows that 256 threads do not keep: 1024 threads and no more registers than the row's length needs, so that two
+        // workgroups share a CU where there are more rows than CUs.  f32, one row / 4096 rows: 12288 elements 10.0 / 117 us on 256
+        // threads that read the row three times, 4.4 / 60.4 with 4 vectors per thread, 5.4 / 88.5 with room for 16; 20000 elements
+        // 7.2 / 118 in the other modes' form, 5.7 / 117 with 8 vectors, 6.4 / 156 with room for 16.  Beyond 65536 elements no part is kept.
+        if (n <= 4 * 1024 * 4) run(&row_kernel<uint16_t, 0, 1024, 4>, &row_kernel<float, 0, 1024, 4>, 1024);
+        else if (n <= 4 * 1024 * 8) run(&row_kernel<uint16_t, 0, 1024, 8>, &row_kernel<float, 0, 1024, 8>, 1024);
+        else if (n <= 4 * 1024 * 16) run(&row_kernel<uint16_t, 0, 1024, 16>, &row_kernel<float, 0, 1024, 16>, 1024);
+        else run(&row_kernel<uint16_t, 0, 1024, 0>, &row_kernel<float, 0, 1024, 0>, 1024);
     } else if (n > 16384) {
-        // longer rows: 1024 threads, what does not fit the registers is read again
-        if (dtype == WRQ_F16) hipLaunchKernelGGL((row_kernel<uint16_t, MODE, 1024>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
-        else hipLaunchKernelGGL((row_kernel<float, MODE, 1024>), dim3((uint32_t)rows), dim3(1024), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
+        // 1024 threads; a row of more than 32768 elements does not fit their registers and is read again
+        run(&row_kernel<uint16_t, MODE, 1024>, &row_kernel<float, MODE, 1024>, 1024);
     } else if (n <= 1024) {
-        if (dtype == WRQ_F16) hipLaunchKernelGGL((row_kernel<uint16_t, MODE, 64>), dim3((uint32_t)rows), dim3(64), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
-        else hipLaunchKernelGGL((row_kernel<float, MODE, 64>), dim3((uint32_t)rows), dim3(64), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
+        run(&row_kernel<uint16_t, MODE, 64>, &row_kernel<float, MODE, 64>, 64);
     } else {
-        if (dtype == WRQ_F16) hipLaunchKernelGGL((row_kernel<uint16_t, MODE, kRowThreads>), dim3((uint32_t)rows), dim3(kRowThreads), 0, stream, static_cast<uint16_t *>(x), wp, bp, n, heads, eps);
-        else hipLaunchKernelGGL((row_kernel<float, MODE, kRowThreads>), dim3((uint32_t)rows), dim3(kRowThreads), 0, stream, static_cast<float *>(x), wp, bp, n, heads, eps);
+        run(&row_kernel<uint16_t, MODE, kRowThreads>, &row_kernel<float, MODE, kRowThreads>, kRowThreads);
     }
     return check_launch(what);
 }
