@@ -852,6 +852,31 @@ def test_gpu_softmax_vocabulary_rows(gpu, dtype, C):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C", [8196, 16384])
+def test_gpu_softmax_sums_in_pairs(gpu, C):
+    """The rounding of a row's sum in f32, alone: the outputs are the terms of that sum times its reciprocal, so their sum in 64
+    bits is off 1 by it.  Rows whose sum is just below a power of two, where one rounding is u = 1.76e-8 rms of it (half an ulp
+    evenly, over sqrt(3)) and the reciprocal's 2 u.  Partial sums added in pairs, each level in the last one's binade or in the one
+    above it: at most sqrt(1 + 4 (1/2 + 1/4 + ...) + 4) u = 5.3e-8 (measured 4.5e-8).  Sixteen waves' sums one after the other: half
+    of them are in the last one's binade, sqrt(9 + 4) u = 6.3e-8 (measured 6.7e-8)."""
+    import torch
+
+    print("rounding of softmax sums on the GPU", C, flush=True)
+    rng = np.random.default_rng(SEED + 78 + C)
+    x = rng.standard_normal((1, 512, C)).astype(np.float32)
+    x[..., 0] = 0
+    x[..., 1:] -= 12
+    rest = np.exp(x[..., 1:].astype(np.float64)).sum(-1)
+    x[..., 1:] += np.log((0.98 * 16 - 1) / rest)[..., None].astype(np.float32)  # sum of exp(x - 0): 0.98 x 2^4
+    assert x.max() == 0
+    xd = torch.from_numpy(x).cuda()
+    gpu.LayerOp.softmax(xd)
+    off = xd.double().sum(-1) - 1
+    print("rms", off.square().mean().sqrt().item(), flush=True)
+    assert off.square().mean().sqrt().item() < 5.3e-8
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("C,T,B", [(1000, 3, 2), (4096, 1, 1), (4096, 128, 1), (65536, 2, 1), (64, 5, 1), (4, 1, 3)])
 def test_gpu_softmax_layer_norm(gpu, lop, dtype, C, T, B):

@@ -101,8 +101,9 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// sum or maximum over the workgroup, the same value in every thread; `red` holds THREADS / 64 floats
-template <bool MAX, int THREADS>
+// sum or maximum over the workgroup, the same value in every thread; `red` holds THREADS / 64 floats.  PAIRS: the waves' sums are
+// added in pairs, fours, ... and not one after the other
+template <bool MAX, int THREADS, bool PAIRS = false>
 __device__ __forceinline__ float block_reduce(float v, float *red) {
     v = MAX ? wave_max(v) : wave_sum(v);
     if constexpr (THREADS == 64) return v;
@@ -110,6 +111,17 @@ __device__ __forceinline__ float block_reduce(float v, float *red) {
     __syncthreads(); // `red` may still be read from the previous reduction
     if ((threadIdx.x & 63) == 0) red[wave] = v;
     __syncthreads();
+    if constexpr (PAIRS) {
+        static_assert(!MAX, "the order matters to sums");
+        float r[THREADS / 64];
+#pragma unroll
+        for (int w = 0; w < THREADS / 64; w++) r[w] = red[w];
+#pragma unroll
+        for (int d = 1; d < THREADS / 64; d *= 2)
+#pragma unroll
+            for (int w = 0; w < THREADS / 64; w += 2 * d) r[w] += r[w + d];
+        return r[0];
+    }
     float r = red[0];
 #pragma unroll
     for (int w = 1; w < THREADS / 64; w++) r = MAX ? fmaxf(r, red[w]) : r + red[w];
