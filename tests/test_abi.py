@@ -78,6 +78,65 @@ def err(wrq):
     return wrq.lib().wrq_last_error().decode()
 
 
+def test_binding_tells_tensors_from_views(wrq):
+    L = wrq.lib()
+    t, v = T(wrq, (64, 1, 1, 1)), V(wrq, (64, 1, 1, 1))
+    for tensor in (t, C.byref(t), C.pointer(t)):  # a structure goes by itself, by reference or by pointer
+        assert L.wrq_softmax(None, tensor, 7) == wrq.ERR_TYPE
+    for view in (v, C.byref(v), C.pointer(v)):
+        assert L.wrq_activate(None, view, 99) == wrq.ERR_UNSUPPORTED
+    assert L.wrq_softmax(None, None, 0) == wrq.ERR_NULL
+    for other in (v, C.byref(v), C.pointer(v), FAKE, bytes(v), bytes(8)):
+        with pytest.raises(C.ArgumentError):
+            L.wrq_softmax(None, other, 7)
+    for other in (t, C.byref(t), C.pointer(t), FAKE, bytes(t), bytes(8)):
+        with pytest.raises(C.ArgumentError):
+            L.wrq_activate(None, other, 99)
+
+
+def test_wrappers_hand_over_the_descriptors_declared(wrq, monkeypatch):
+    """Every wrapper against the argument types of its entry point: a tensor's bytes where a tensor is read, a view's where a view is."""
+    import inspect
+
+    import torch
+
+    sizes = {C.POINTER(wrq.CTensor): C.sizeof(wrq.CTensor), C.POINTER(wrq.CTensorView): C.sizeof(wrq.CTensorView)}
+    typed, seen = wrq.lib(), {}
+
+    class Recorder:
+        def __getattr__(self, name):
+            def call(*args):
+                want = getattr(typed, name).argtypes
+                assert len(args) == len(want), name
+                for k, (arg, kind) in enumerate(zip(args, want)):
+                    if kind in sizes:
+                        assert type(arg) is bytes and len(arg) == sizes[kind], (name, k)
+                    else:
+                        assert type(arg) is not bytes, (name, k)
+                seen[name] = seen.get(name, 0) + 1
+                return wrq.OK
+
+            return call
+
+    monkeypatch.setattr(wrq, "_packed", Recorder)
+    monkeypatch.setattr(wrq, "_stream", lambda: 0)
+    t = torch.zeros((2, 64), dtype=torch.float16)
+    view = ((64, 2), (64, 2), (0, 0))
+    plain = dict(eps=1e-5, scale=1.0, bias=0.0, act=0, act_x=0, act_y=0, act_out=0, sparse=False, reversed=False, rescale=False, first=False, checked=True,
+                 Cn=64, S=64, H=1, A=2, lora_size=32, factors=[t], shifts=[t], aux=[t] * 4, vectors=[t] * 5, buffers=[None] * 5, ops=[(t, t, t, 0)])
+    for cls in (wrq.TensorOp, wrq.LayerOp, wrq.FusedV6, wrq.FusedV7):
+        for name, f in vars(cls).items():
+            if not isinstance(f, staticmethod) or name.startswith("_"):
+                continue
+            names = list(inspect.signature(f.__func__).parameters)
+            plain["w2"] = [t] * 4 if "aux" in names else t
+            for views in (None, view):
+                f.__func__(**{n: views if n == "view" or n.endswith("_view") else plain.get(n, t) for n in names})
+    described = {n for n in wrq.EXPORTS if any(a in sizes for a in getattr(typed, n).argtypes or ())}
+    older = {"wrq_v7_post_ffn"}  # the wrapper calls its _buffers form
+    assert described - older <= set(seen), described - older - set(seen)
+
+
 def test_shape_errors_read_like_the_reference(wrq):
     L = wrq.lib()
     K, R, Tn = 256, 8, 1

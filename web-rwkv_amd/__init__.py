@@ -176,9 +176,7 @@ def lib():
                 "(hipcc --offload-arch=gfx950); this package has no CPU or eager fallback"
             )
         L = C.CDLL(LIB_PATH)
-        # descriptors go as pointers to a struct of ctypes or to the packed bytes of one (see _tensor, _view)
-        vp, i = C.c_void_p, C.c_int
-        T = V = vp
+        T, V, vp, i = C.POINTER(CTensor), C.POINTER(CTensorView), C.c_void_p, C.c_int
         L.wrq_init.restype = i
         L.wrq_abi_version.restype = i
         L.wrq_status_string.restype = C.c_char_p
@@ -244,6 +242,25 @@ def lib():
     return _lib
 
 
+_packed_lib = None
+
+
+def _packed():
+    """The library as the wrappers below call it: a descriptor is an address, of packed bytes or of a structure (``_tensor``, ``_view``).
+    Looking at the kind of each in Python costs 0.08 us, 4 % of a small product's call; ``lib()`` tells them apart by its argument
+    types, and that each wrapper hands over the kinds its entry point declares is fixed by its text and tested."""
+    global _packed_lib
+    if _packed_lib is None:
+        typed, L = lib(), C.CDLL(LIB_PATH)
+        for name in EXPORTS:
+            f, g = getattr(typed, name), getattr(L, name)
+            g.restype = f.restype
+            if f.argtypes is not None:
+                g.argtypes = [C.c_void_p if t in (C.POINTER(CTensor), C.POINTER(CTensorView)) else t for t in f.argtypes]
+        _packed_lib = L
+    return _packed_lib
+
+
 def debug_override(key, value=-1):
     """``wrq_debug_override``: pin (value >= 0) or release (value < 0) one kernel / tile choice."""
     _check(lib().wrq_debug_override(key.encode(), int(value)))
@@ -302,6 +319,7 @@ def as_view(t, view=None, dtype=None):
 
 # The descriptors of a call as packed bytes: a ctypes structure with its arrays costs 1 - 3 us to build, a packed one 0.4 us, and a
 # small product's whole call is host time (one token, 2048 x 2048: 13.8 us with structures and a Stream object, 7.5 us now).
+# matmul_vec_group, whose products name their descriptors by pointer, builds structures.
 _PACK_TENSOR = struct.Struct("@Q4I").pack
 _PACK_VIEW = struct.Struct("@Q12Ii4x").pack
 assert struct.calcsize("@Q4I") == C.sizeof(CTensor) and struct.calcsize("@Q12Ii4x") == C.sizeof(CTensorView)
@@ -349,45 +367,45 @@ class TensorOp:
 
     @staticmethod
     def quantize_mat_int8(input, minmax, output):
-        _check(lib().wrq_quantize_mat_int8(_stream(), _tensor(input), _tensor(minmax), _tensor(output)))
+        _check(_packed().wrq_quantize_mat_int8(_stream(), _tensor(input), _tensor(minmax), _tensor(output)))
 
     @staticmethod
     def quantize_mat_nf4(input, quant, absmax, output):
-        _check(lib().wrq_quantize_mat_nf4(_stream(), _tensor(input), _tensor(quant), _tensor(absmax), _tensor(output)))
+        _check(_packed().wrq_quantize_mat_nf4(_stream(), _tensor(input), _tensor(quant), _tensor(absmax), _tensor(output)))
 
     @staticmethod
     def matmul_vec_int8(matrix, minmax, input, output, act=ACT_NONE, sparse=False, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_vec_int8(_stream(), _tensor(matrix), _tensor(minmax),
+        _check(_packed().wrq_matmul_vec_int8(_stream(), _tensor(matrix), _tensor(minmax),
                                          _view(input, input_view), _view(output, output_view), act, int(sparse)))
 
     @staticmethod
     def matmul_vec_nf4(matrix, quant, absmax, input, output, act=ACT_NONE, sparse=False, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_vec_nf4(_stream(), _tensor(matrix), _tensor(quant), _tensor(absmax),
+        _check(_packed().wrq_matmul_vec_nf4(_stream(), _tensor(matrix), _tensor(quant), _tensor(absmax),
                                         _view(input, input_view), _view(output, output_view), act, int(sparse)))
 
     @staticmethod
     def matmul_mat_int8(matrix, minmax, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_int8(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(minmax),
+        _check(_packed().wrq_matmul_mat_int8(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(minmax),
                                          _view(input, input_view), _view(output, output_view), act))
 
     @staticmethod
     def matmul_mat_int8_noalloc(matrix, minmax, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_int8_noalloc(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(minmax),
+        _check(_packed().wrq_matmul_mat_int8_noalloc(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(minmax),
                                                  _view(input, input_view), _view(output, output_view), act))
 
     @staticmethod
     def matmul_mat_nf4(matrix, quant, absmax, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_nf4(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(quant), _tensor(absmax),
+        _check(_packed().wrq_matmul_mat_nf4(_stream(), _view(matrix, matrix_view, dtype=F16), _tensor(quant), _tensor(absmax),
                                         _view(input, input_view), _view(output, output_view), act))
 
     @staticmethod
     def matmul_vec_fp16(matrix, input, output, act=ACT_NONE, sparse=False, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_vec_fp16(_stream(), _tensor(matrix), _view(input, input_view),
+        _check(_packed().wrq_matmul_vec_fp16(_stream(), _tensor(matrix), _view(input, input_view),
                                          _view(output, output_view), act, int(sparse)))
 
     @staticmethod
     def matmul_mat_fp16(matrix, input, output, act=ACT_NONE, matrix_view=None, input_view=None, output_view=None):
-        _check(lib().wrq_matmul_mat_fp16(_stream(), _view(matrix, matrix_view), _view(input, input_view),
+        _check(_packed().wrq_matmul_mat_fp16(_stream(), _view(matrix, matrix_view), _view(input, input_view),
                                          _view(output, output_view), act))
 
 
@@ -397,121 +415,121 @@ class LayerOp:
 
     @staticmethod
     def softmax(x):
-        _check(lib().wrq_softmax(_stream(), _tensor(x), _dtype(x)))
+        _check(_packed().wrq_softmax(_stream(), _tensor(x), _dtype(x)))
 
     @staticmethod
     def layer_norm(w, b, x, eps):
-        _check(lib().wrq_layer_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
+        _check(_packed().wrq_layer_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def group_norm(w, b, x, eps):
-        _check(lib().wrq_group_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
+        _check(_packed().wrq_group_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def add_activate(input, output, act_x=ACT_NONE, act_y=ACT_NONE, act_out=ACT_NONE, input_view=None, output_view=None):
-        _check(lib().wrq_add_activate(_stream(), _view(input, input_view), _view(output, output_view), act_x, act_y, act_out))
+        _check(_packed().wrq_add_activate(_stream(), _view(input, input_view), _view(output, output_view), act_x, act_y, act_out))
 
     @staticmethod
     def mul_activate(input, output, act_x=ACT_NONE, act_y=ACT_NONE, act_out=ACT_NONE, input_view=None, output_view=None):
-        _check(lib().wrq_mul_activate(_stream(), _view(input, input_view), _view(output, output_view), act_x, act_y, act_out))
+        _check(_packed().wrq_mul_activate(_stream(), _view(input, input_view), _view(output, output_view), act_x, act_y, act_out))
 
     add = add_activate
     mul = mul_activate
 
     @staticmethod
     def embed(tokens, input, output):
-        _check(lib().wrq_embed(_stream(), _tensor(tokens), _tensor(input), _tensor(output), _dtype(output)))
+        _check(_packed().wrq_embed(_stream(), _tensor(tokens), _tensor(input), _tensor(output), _dtype(output)))
 
     @staticmethod
     def blit(input, output, input_view=None, output_view=None):
-        _check(lib().wrq_blit(_stream(), _view(input, input_view), _view(output, output_view)))
+        _check(_packed().wrq_blit(_stream(), _view(input, input_view), _view(output, output_view)))
 
     @staticmethod
     def transpose(input, output, input_view=None, output_view=None):
-        _check(lib().wrq_transpose(_stream(), _view(input, input_view), _view(output, output_view)))
+        _check(_packed().wrq_transpose(_stream(), _view(input, input_view), _view(output, output_view)))
 
     @staticmethod
     def activate(x, act, view=None):
-        _check(lib().wrq_activate(_stream(), _view(x, view), act))
+        _check(_packed().wrq_activate(_stream(), _view(x, view), act))
 
     @staticmethod
     def affine(x, scale, bias):
-        _check(lib().wrq_affine(_stream(), _tensor(x), _dtype(x), scale, bias))
+        _check(_packed().wrq_affine(_stream(), _tensor(x), _dtype(x), scale, bias))
 
     @staticmethod
     def token_shift(cursors, time_mix, state, input, output, reversed=False, time_mix_view=None, state_view=None):
-        _check(lib().wrq_token_shift(_stream(), _tensor(cursors), _view(time_mix, time_mix_view), _view(state, state_view),
+        _check(_packed().wrq_token_shift(_stream(), _tensor(cursors), _view(time_mix, time_mix_view), _view(state, state_view),
                                      _tensor(input), _dtype(input), _tensor(output), _dtype(output), int(reversed)))
 
     @staticmethod
     def channel_mix(cursors, state, r, v, x, state_view=None):
-        _check(lib().wrq_channel_mix(_stream(), _tensor(cursors), _view(state, state_view), _tensor(r),
+        _check(_packed().wrq_channel_mix(_stream(), _tensor(cursors), _view(state, state_view), _tensor(r),
                                      _tensor(v), _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_mix_v4(cursors, time_decay, time_first, state, k, v, r, x, state_view=None):
-        _check(lib().wrq_time_mix_v4(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
+        _check(_packed().wrq_time_mix_v4(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
                                      _view(state, state_view), _tensor(k), _tensor(v), _tensor(r),
                                      _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_mix_v5(cursors, time_decay, time_first, state, k, v, r, x, state_view=None):
-        _check(lib().wrq_time_mix_v5(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
+        _check(_packed().wrq_time_mix_v5(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
                                      _view(state, state_view), _tensor(k), _tensor(v), _tensor(r),
                                      _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_mix_v6(cursors, time_decay, time_first, state, k, v, r, x, state_view=None):
-        _check(lib().wrq_time_mix_v6(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
+        _check(_packed().wrq_time_mix_v6(_stream(), _tensor(cursors), _tensor(time_decay), _tensor(time_first),
                                      _view(state, state_view), _tensor(k), _tensor(v), _tensor(r),
                                      _tensor(x), _dtype(x)))
 
     @staticmethod
     def recenter(x):
-        _check(lib().wrq_recenter(_stream(), _tensor(x), _dtype(x)))
+        _check(_packed().wrq_recenter(_stream(), _tensor(x), _dtype(x)))
 
     @staticmethod
     def rms_norm(w, b, x, eps):
-        _check(lib().wrq_rms_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
+        _check(_packed().wrq_rms_norm(_stream(), _tensor(w), _tensor(b), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def broadcast(input, output, input_view=None, output_view=None):
-        _check(lib().wrq_broadcast(_stream(), _view(input, input_view), _view(output, output_view)))
+        _check(_packed().wrq_broadcast(_stream(), _view(input, input_view), _view(output, output_view)))
 
     @staticmethod
     def blend(factor, input, output):
-        _check(lib().wrq_blend(_stream(), _tensor(factor), _tensor(input), _dtype(input), _tensor(output), _dtype(output)))
+        _check(_packed().wrq_blend(_stream(), _tensor(factor), _tensor(input), _dtype(input), _tensor(output), _dtype(output)))
 
     @staticmethod
     def blend_lora(factor, xa, xb, output, xa_view=None, xb_view=None, output_view=None):
-        _check(lib().wrq_blend_lora(_stream(), _tensor(factor), _view(xa, xa_view), _view(xb, xb_view),
+        _check(_packed().wrq_blend_lora(_stream(), _tensor(factor), _view(xa, xa_view), _view(xb, xb_view),
                                     _view(output, output_view)))
 
     @staticmethod
     def l2_norm(x, eps):
-        _check(lib().wrq_l2_norm(_stream(), _tensor(x), _dtype(x), eps))
+        _check(_packed().wrq_l2_norm(_stream(), _tensor(x), _dtype(x), eps))
 
     @staticmethod
     def control_k_v7(p, a, k, a_view=None, k_view=None):
-        _check(lib().wrq_control_k_v7(_stream(), _tensor(p), _view(a, a_view), _view(k, k_view)))
+        _check(_packed().wrq_control_k_v7(_stream(), _tensor(p), _view(a, a_view), _view(k, k_view)))
 
     @staticmethod
     def time_mix_v7(cursors, state, r, w, n, x, state_view=None):
-        _check(lib().wrq_time_mix_v7(_stream(), _tensor(cursors), _view(state, state_view), _tensor(r),
+        _check(_packed().wrq_time_mix_v7(_stream(), _tensor(cursors), _view(state, state_view), _tensor(r),
                                      _tensor(w), _tensor(n), _tensor(x), _dtype(x)))
 
     @staticmethod
     def time_first_v7(u, r, n, x):
-        _check(lib().wrq_time_first_v7(_stream(), _tensor(u), _tensor(r), _tensor(n), _tensor(x), _dtype(x)))
+        _check(_packed().wrq_time_first_v7(_stream(), _tensor(u), _tensor(r), _tensor(n), _tensor(x), _dtype(x)))
 
     @staticmethod
     def channel_mix_v7(cursors, state, v, x, state_view=None):
-        _check(lib().wrq_channel_mix_v7(_stream(), _tensor(cursors), _view(state, state_view), _tensor(v),
+        _check(_packed().wrq_channel_mix_v7(_stream(), _tensor(cursors), _view(state, state_view), _tensor(v),
                                         _tensor(x), _dtype(x)))
 
     @staticmethod
     def lerp(input, output, factor, reversed=False, input_view=None, output_view=None, factor_view=None):
-        _check(lib().wrq_lerp(_stream(), _view(input, input_view), _view(output, output_view),
+        _check(_packed().wrq_lerp(_stream(), _view(input, input_view), _view(output, output_view),
                               _view(factor, factor_view), int(reversed)))
 
 
@@ -578,7 +596,7 @@ class FusedV6:
         p = FusedV6._p
         if not checked:
             FusedV6._check_pre("v6_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
-        _check(lib().wrq_v6_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, _view(state, state_view), len(factors),
+        _check(_packed().wrq_v6_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, _view(state, state_view), len(factors),
                                 p(factors[0]), p(factors[1] if len(factors) > 1 else None), p(ln_out), p(shifts[0]), p(shifts[1] if len(shifts) > 1 else None)))
 
     @staticmethod
@@ -586,21 +604,21 @@ class FusedV6:
         p, r, n = FusedV6._p, lora_size, A * Cn
         if not checked:
             _operands("v6_time_mix", A, cursors, ((lora, 5 * A * r), (w2, 5 * Cn * r), (time_mix, 5 * Cn), (att_x, n), (att_sx, 5 * n)))
-        _check(lib().wrq_v6_time_mix(_stream(), Cn, A, lora_size, p(cursors), p(lora), p(w2), p(time_mix), _view(state, state_view), p(att_x), p(att_sx)))
+        _check(_packed().wrq_v6_time_mix(_stream(), Cn, A, lora_size, p(cursors), p(lora), p(w2), p(time_mix), _view(state, state_view), p(att_x), p(att_sx)))
 
     @staticmethod
     def decay(Cn, A, lora_size, lora, w2, time_decay, out, checked=False):
         p, r = FusedV6._p, lora_size
         if not checked:
             _operands("v6_decay", A, None, ((lora, A * r), (w2, Cn * r), (time_decay, Cn)), ((out, A * Cn),))
-        _check(lib().wrq_v6_decay(_stream(), Cn, A, lora_size, p(lora), p(w2), p(time_decay), p(out)))
+        _check(_packed().wrq_v6_decay(_stream(), Cn, A, lora_size, p(lora), p(w2), p(time_decay), p(out)))
 
     @staticmethod
     def wkv_gate(S, H, A, cursors, time_decay, time_first, state, state_view, k, v, r, g, gn_w, gn_b, eps, att_x, checked=False):
         p, n = FusedV6._p, A * S * H
         if not checked:
             _operands("v6_wkv_gate", A, cursors, ((g, n), (gn_w, S * H), (gn_b, S * H), (att_x, n)), ((time_decay, n), (time_first, S * H), (k, n), (v, n), (r, n)))
-        _check(lib().wrq_v6_wkv_gate(_stream(), S, H, A, p(cursors), p(time_decay), p(time_first), _view(state, state_view), p(k), p(v), p(r), p(g),
+        _check(_packed().wrq_v6_wkv_gate(_stream(), S, H, A, p(cursors), p(time_decay), p(time_first), _view(state, state_view), p(k), p(v), p(r), p(g),
                                      p(gn_w), p(gn_b), eps, p(att_x)))
 
     @staticmethod
@@ -608,7 +626,7 @@ class FusedV6:
         p, n = FusedV6._p, A * Cn
         if not checked:
             _operands("v6_post_ffn", A, cursors, ((r, n), (v, n), (ffn_x, n), (x_in, n), (x_out, n)))
-        _check(lib().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), _view(state, state_view), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
+        _check(_packed().wrq_v6_post_ffn(_stream(), Cn, A, p(cursors), _view(state, state_view), p(r), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale)))
 
 
 class FusedV7:
@@ -627,7 +645,7 @@ class FusedV7:
             FusedV6._check_pre("fused_pre", Cn, A, cursors, x, add, x_out, ln_w, ln_b, factors, ln_out, shifts)
         if len(shifts) < len(factors):
             raise TensorError(ERR_SHAPE, f"fused_pre: {len(shifts)} outputs for {len(factors)} token shifts")
-        _check(lib().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, _view(state, state_view), len(factors),
+        _check(_packed().wrq_fused_pre(_stream(), Cn, A, p(cursors), p(x), p(add), p(x_out), p(ln_w), p(ln_b), eps, _view(state, state_view), len(factors),
                                    a(factors), p(ln_out), a(shifts)))
 
     @staticmethod
@@ -637,7 +655,7 @@ class FusedV7:
         w, x, out, act = zip(*ops)
         if not checked:
             _operands("adapters_in", A, None, [(t, A * Cn) for t in x] + [(t, t.shape[0] * Cn) for t in w] + [(o, A * t.shape[0]) for o, t in zip(out, w)])
-        _check(lib().wrq_adapters_in(_stream(), Cn, A, n, a(w), (C.c_uint32 * n)(*(t.shape[0] for t in w)), (C.c_int * n)(*act), a(x), a(out)))
+        _check(_packed().wrq_adapters_in(_stream(), Cn, A, n, a(w), (C.c_uint32 * n)(*(t.shape[0] for t in w)), (C.c_int * n)(*act), a(x), a(out)))
 
     @staticmethod
     def mid(S, H, A, first, aux, w2, vectors, eps, k, v, att_v0, att_w, att_g, n, buffers=(None,) * 5, checked=False):
@@ -650,7 +668,7 @@ class FusedV7:
             _operands("v7_mid", A, None, [(t, A * w.shape[1]) for t, w in zip(aux, w2) if w is not None] + [(w, Cn * w.shape[1]) for w in w2 if w is not None]
                       + [(t, Cn) for t in vectors] + [(t, A * Cn) for t in (k, v, att_v0, att_w, att_g, *buffers)] + [(n, 4 * A * Cn)])
         ranks = (C.c_uint32 * 4)(*(0 if t is None else t.shape[1] for t in w2))
-        _check(lib().wrq_v7_mid_buffers(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n),
+        _check(_packed().wrq_v7_mid_buffers(_stream(), S, H, A, int(first), ranks, a(aux), a(w2), a(vectors), eps, p(k), p(v), p(att_v0), p(att_w), p(att_g), p(n),
                                         a(buffers)))
 
     @staticmethod
@@ -658,7 +676,7 @@ class FusedV7:
         p, m = FusedV6._p, A * S * H
         if not checked:
             _operands("v7_wkv_gate", A, cursors, ((r, m), (w, m), (n, 4 * m), (r_k, S * H), (g, m), (gn_w, S * H), (gn_b, S * H), (att_x, m)))
-        _check(lib().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), _view(state, state_view), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
+        _check(_packed().wrq_v7_wkv_gate(_stream(), S, H, A, p(cursors), _view(state, state_view), p(r), p(w), p(n), p(r_k), p(g), p(gn_w), p(gn_b), eps,
                                      p(att_x)))
 
     @staticmethod
@@ -666,7 +684,7 @@ class FusedV7:
         p, n = FusedV6._p, A * Cn
         if not checked:
             _operands("v7_post_ffn", A, cursors, ((v, n), (ffn_x, n), (x_in, n), (x_out, n), (ffn_out, n)))
-        _check(lib().wrq_v7_post_ffn_buffers(_stream(), Cn, A, p(cursors), _view(state, state_view), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale),
+        _check(_packed().wrq_v7_post_ffn_buffers(_stream(), Cn, A, p(cursors), _view(state, state_view), p(v), p(ffn_x), p(x_in), p(x_out), int(rescale),
                                              p(ffn_out)))
 
 
