@@ -129,10 +129,11 @@ __device__ __forceinline__ bool keeps_input(const uint32_t *tokens, const uint32
     return true;
 }
 
-// The tokens of a chunk in groups of L (eight; sixteen, a whole chunk, in the wide form).  A whole group is one piece of straight code: the operands of its later tokens are
-// read from LDS while the earlier ones are worked on, where a loop over tokens waits out one LDS round trip, the
-// reduction over the lanes and a branch for the store at each of them.  `token(tt, u)` leaves its result in lane u of the L
-// that share the columns, `flush(from, count)` then stores the group at once.
+// The tokens of a chunk in groups of L (eight; sixteen, a whole chunk, in the wide form).  A whole group is one piece of straight code:
+// the operands of its later tokens are read from LDS while the earlier ones are worked on, where a loop over tokens waits out one LDS
+// round trip, the reduction over the lanes and a branch for the store at each of them.  The tokens past the last whole group take
+// that loop.  `token(tt, u)` leaves its result in lane u of the L that share the columns, `flush(from, count)` then stores the group
+// at once.
 // 32 heads of 64, one request: v6 gate form 100 tokens 31.0 -> 27.2 us, 255 tokens 72.5 -> 62.1; v7, whose tokens are a chain through
 // sa, 45.4 -> 44.4 and 109.0 -> 106.1.  Reads ahead stop at every second token where a lane holds up to eight rows: over the
 // whole group they took up to 250 registers, two waves per SIMD instead of three, and were slower in the end (v6 gate form 27.7 -> 25.6 us, v7
