@@ -739,6 +739,42 @@ def test_chunk_tiles_from_the_measured_table(gpu, oracle, kind, C, H, overrides)
 
 
 @pytest.mark.parametrize("kind", ["int8", "nf4"])
+@pytest.mark.parametrize("T", [4, 8, 9, 16, 17, 24, 25, 32, 33, 48], ids=str)
+def test_short_run_kernel(gpu, oracle, kind, T, overrides):
+    # the kernel of short runs (csrc/gemm_short.hip) at the edges of its token tiles: rows that fill no tile, fewer K
+    # steps than waves, rows of 4 KiB (every workgroup starts at another step), one to four row tiles per workgroup, steps
+    # of 256 elements and several rounds of workgroups; strided activations, groups of products of different size, every
+    # activation.  f32 outputs against float64: operands are exact, so a sum of K products of |w x| < 0.1 * 4 in f32
+    # stays below 2^-23 * K * 0.4 < 1e-3, and far below it for random signs.
+    import torch
+
+    announce("short run", kind, T)
+    rng = np.random.default_rng(SEED + 91 + T)
+    groups = [[(128, 4)], [(384, 20), (384, 132)], [(4096 if kind == "int8" else 8192, 68)], [(2048, 2048), (2048, 2052)], [(256, 4100), (256, 4)],
+              [(256, 8196), (256, 36)], [(256, 12304)], [(256, 16388), (256, 400)], [(7168, 64)]]
+    for i, shapes in enumerate(groups):
+        K, ops, want = shapes[0][0], [], []
+        for j, (_, R) in enumerate(shapes):
+            wp, scale, wdeq = pack(oracle, kind, gen_f16(rng, (R, K), 0.02))
+            parent = gen_f16(rng, (2, T + 1, K + 64), 1.0)  # the activations are a slice of it
+            view = ((K, T, 1), (K + 64, T + 1, 2), (64, 1, 1))
+            out = torch.full((T, R), float("nan"), dtype=torch.float32 if (i + j) % 3 else torch.float16, device="cuda")
+            act = (i + j) % 2 * 6
+            ops.append((gpu_matrix(gpu, kind, wp, scale), dev(parent), out, act, False, dict(input_view=view)))
+            truth = truth_matmul(wdeq, parent[1, 1:, 64:])
+            want.append(1.0 / (1.0 + np.exp(-truth)) if act else truth)
+        results = []
+        for short in (1, 0):
+            overrides(gemm_short=short, vec_chunk_min_t=2)
+            gpu.matmul_vec_group(ops)
+            results.append([host(op[2]) for op in ops])
+        for j, op in enumerate(ops):
+            eps = 3e-4 if op[2].dtype == torch.float32 else EPS
+            assert_close(results[0][j], want[j], eps, f"{kind} T={T} {shapes}[{j}] vs float64")
+            assert_close(results[0][j], results[1][j], EPS, f"{kind} T={T} {shapes}[{j}] vs the chunk kernel")
+
+
+@pytest.mark.parametrize("kind", ["int8", "nf4"])
 @pytest.mark.parametrize("T,ksplit", [(128, 2), (256, 1), (252, 1)], ids=str)
 def test_chunk_grid_a_little_above_two_workgroups_per_cu(gpu, oracle, kind, T, ksplit, overrides):
     # 576 workgroups (288 tiles of 128 rows x 64 tokens split in two, or 576 tiles) run as two launches:

@@ -47,22 +47,13 @@
 // so the only per-block work outside the matrix cores is one or two fmas per output.
 // Plain f16 weights (matmul_mat_fp16, src/shaders/matmul_mat_fp16.wgsl:57-140) take the same
 // kernel: they are A operands as loaded and accumulate in the matrix cores over the whole K.
-#include "wrq_device.h"
+#include "gemm_device.h"
 #include "wrq_host.h"
 
 #include <algorithm>
 #include <atomic>
 
 namespace wrq {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-
-union HalfPack {
-    uint32_t u[4];
-    half8 h;
-};
 
 constexpr int kStep = 128; // K elements per step
 #ifndef WRQ_UNROLL_STAGES
@@ -85,26 +76,6 @@ __device__ __align__(256) float g_splitk_scratch[kScratchSlices * kScratchFloats
 // device (static_scratch_ptr), and only that pointer is ever handed to a kernel.
 constexpr size_t kStaticScratchFloats = 4u << 20;
 static __device__ __align__(256) float scratch[kStaticScratchFloats];
-
-__device__ __forceinline__ uint32_t pack_h2(float a, float b) {
-    return (uint32_t)f2h(a) | ((uint32_t)f2h(b) << 16);
-}
-
-__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
-__device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
-
-__device__ __forceinline__ float dot2_ones(uint32_t v, float acc) {
-    // acc + lo(v) + hi(v) with f32 accumulation: v_dot2_f32_f16 against (1.0, 1.0)
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, v), half2v{(_Float16)1.0f, (_Float16)1.0f}, acc, false);
-}
-
-__device__ __forceinline__ float row16_sum(float v) {
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xf, 0xf, true));
-    return v;
-}
 
 // Tile geometry of one instantiation.  The 4 waves of a workgroup are RW row groups times KG
 // "k groups": the k groups share the rows and the staged activations and take alternate K
@@ -1185,7 +1156,9 @@ int launch_gemm_group(hipStream_t stream, Quant quant, int in_f16, const MatmulA
                    args[i + m].T == args[i].T)
                 m++;
         int s;
-        if (quant == kInt8)
+        if (in_f16 && launch_gemm_short(stream, quant, args + i, m, s))
+            ; // short runs have a kernel of their own
+        else if (quant == kInt8)
             s = in_f16 ? launch_shape<kInt8, __half>(stream, args + i, m, sp) : launch_shape<kInt8, float>(stream, args + i, m, sp);
         else if (quant == kFp16)
             s = in_f16 ? launch_shape<kFp16, __half>(stream, args + i, m, sp) : launch_shape<kFp16, float>(stream, args + i, m, sp);

@@ -1,0 +1,436 @@
+// Products on packed weights for short runs (a few tokens up to 48) for gfx950, on the f16 matrix cores:
+// the same sums as gemm.hip (src/shaders/matmul_vec_int8.wgsl, matmul_vec_nf4.wgsl, matmul_mat_int8.wgsl,
+// matmul_mat_nf4.wgsl), split over the machine in another way.
+//
+// A short run reads every weight once and has little to do with it, so a launch is a few microseconds long and what counts
+// is how soon all its loads are under way and how few times a wave has to wait for another one.  The chunk kernel of gemm.hip
+// shares one activation tile between the waves of a workgroup: a barrier per K step or four, narrow grids, and a split of K
+// over the grid with a second launch (4.5 us) where rows are few.  Here
+//   * a workgroup owns 16 * MRT rows and the whole K; its NW waves take the K steps (128 * SUB elements) in turn and each
+//     keeps everything it needs to itself: weights and activations go line-wise from memory into registers (a row's bytes of
+//     a step in adjacent lanes) and through a slot of LDS that belongs to the wave into operand layout, while the next step is
+//     on its way.  No barrier between the first load and the sum of the waves' partial tiles at the end, no second launch;
+//   * activations come first in a step's loads and in the order of their use, so that staging starts on the first of them;
+//     buffer loads keep addresses in scalar registers and return zeros for rows and tokens past the end;
+//   * the first product's operands are leading scalar arguments (preloaded); what only the end of the kernel needs is
+//     fetched before the first step, behind the loads.
+// Bound: at 5 .. 16 tokens the stream of weights (with the latency of one launch), from 17 tokens on the activations
+// that every workgroup fetches and stages again (2 K T bytes against 16 MRT K or half of that) and, for nf4, the table lookups.
+// Scales are applied per block in f32 as in gemm.hip: the f16 operands stay exact.
+//
+// Measured (us per launch in a graph over cold copies, chunk kernel -> here; attention group / att.output / {ffn.key,
+// ffn.receptance} / ffn.value): 1.6B nf4 at 5 tokens 8.2 / 5.8 / 10.4 / 10.6 -> 6.2 / 4.1 / 7.5 / 7.8; 3B int8 at 19
+// tokens 14.3 / 8.4 / 14.4 / 16.5 -> 9.9 / 5.7 / 10.1 / 13.0; 7B int8 at 8 tokens 18.7 / 10.3 / 23.3 / 19.7 ->
+// 14.4 / 6.1 / 18.5 / 14.2; 7B nf4 at 32 tokens 25.7 / 12.7 / 33.0 / 24.0 -> 20.5 / 8.7 / 26.8 / 22.9.
+#include "gemm_device.h"
+#include "wrq_host.h"
+
+namespace wrq {
+
+// Geometry of one instantiation: 16 * MRT rows, up to TOK tokens, NW waves that split K in steps of 128 * SUB elements.
+template <int QUANT, int MRT, int TOK, int NW, int SUB>
+struct ShortGeometry {
+    static constexpr bool N4 = QUANT == kNf4;
+    static constexpr int KST = 128 * SUB;
+    static constexpr int WB = N4 ? KST / 2 : KST;  // weight bytes per row and step
+    static constexpr int NT = (TOK + 15) / 16;     // token tiles; the last may be half full (TOK = 8, 24)
+    static constexpr int XL = TOK * KST * 2 / 1024; // 1 KiB activation loads per wave and step
+    static constexpr int WL = 16 * MRT * WB / 1024; // 1 KiB weight loads per wave and step
+    static constexpr int XPITCH = KST * 2 + 16;     // bytes per staged token: +16 B rotates the banks
+    static constexpr int WPITCH = WB + 16;
+    // a wave's slot: weights | activations | scales [2 * SUB][16 * MRT] f32 | token sums [SUB][TOK] f32 (int8);
+    // the wave's partial tile takes its place at the end
+    static constexpr int W_BYTES = MRT * 16 * WPITCH, X_BYTES = TOK * XPITCH, S_BYTES = MRT * 16 * 4 * 2 * SUB;
+    static constexpr int STAGED = W_BYTES + X_BYTES + S_BYTES + (N4 ? 0 : TOK * 4 * SUB), PARTIAL = MRT * NT * 1024;
+    static constexpr int SLOT = STAGED > PARTIAL ? STAGED : PARTIAL;
+    static constexpr int TABLE = N4 ? 256 * 8 : 0;
+    static constexpr int LDS = TABLE + SLOT * NW;
+    static_assert(LDS <= 160 * 1024 && SLOT % 16 == 0, "a workgroup's slots fit the LDS of a CU");
+};
+
+struct ShortArgs {
+    uint32_t begin[kMaxGroup]; // first workgroup of every product, unused entries 0xffffffff
+    MatmulArgs m[kMaxGroup];
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00027000);
+}
+
+template <int AUX>
+__device__ __forceinline__ uint4 buffer_load128(__amdgpu_buffer_rsrc_t r, uint32_t offset) {
+    const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, AUX));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+constexpr int kStream = 2; // nt: weights are read once (7B int8 at 8 tokens 15.9 against 16.9 us without)
+
+template <int QUANT, int MRT, int TOK, int NW, int SUB>
+__global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, const uint16_t *scale0, const void *x0, const float *quant0,
+                                                             const uint32_t begin1, const uint32_t R0, const uint32_t x_stride0, const uint32_t K,
+                                                             const uint32_t T, const ShortArgs a) {
+    using G = ShortGeometry<QUANT, MRT, TOK, NW, SUB>;
+    constexpr bool N4 = G::N4;
+    constexpr int NT = G::NT, XL = G::XL, WL = G::WL, KST = G::KST, WB = G::WB;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r16 = lane & 15, g = lane >> 4;
+    const uint8_t *w = w0;
+    const uint16_t *scale = scale0;
+    const void *x = x0;
+    const float *quant = quant0;
+    uint32_t R = R0, x_stride = x_stride0, pi = 0, wg = blockIdx.x;
+    if (blockIdx.x >= begin1) {
+        pi = 1;
+#pragma unroll
+        for (uint32_t i = 2; i < (uint32_t)kMaxGroup; i++)
+            if (blockIdx.x >= a.begin[i]) pi = i;
+        const MatmulArgs &m = a.m[pi];
+        w = m.w, scale = m.scale, x = m.x, quant = m.quant, R = m.R, x_stride = (uint32_t)m.x_token_stride;
+        wg -= a.begin[pi];
+    }
+    const uint32_t row0 = wg * (16 * MRT);
+    uint2 *pair = reinterpret_cast<uint2 *>(smem);
+    uint8_t *const slot = smem + G::TABLE + wv * G::SLOT;
+    uint8_t *const ws = slot, *const xs = slot + G::W_BYTES;
+    float *const scl = reinterpret_cast<float *>(xs + G::X_BYTES); // nf4: absmax of block b at [b][row]; int8: (s, min - 1024 s) of step u at [2 u][row], [2 u + 1][row]
+    float *const sxs = scl + MRT * 16 * 2 * SUB;                   // int8: token sums at [u][token]
+    // nf4: requested before everything else, so that the table is written while the weights are on their way
+    float tq0 = 0.0f, tq1 = 0.0f;
+    if (N4) tq0 = quant[tid & 15], tq1 = quant[(tid >> 4) & 15];
+
+    const uint32_t rows = min((uint32_t)(16 * MRT), R - row0);
+    const uint32_t row_bytes = N4 ? K / 2 : K, scale_bytes = K / 128 * 4; // one 32-bit scale word per row and 128 elements in both formats
+    const auto rw = buffer_of(w + (size_t)row0 * row_bytes, rows * row_bytes);
+    const auto rs = buffer_of(reinterpret_cast<const uint8_t *>(scale) + (size_t)row0 * scale_bytes, rows * scale_bytes);
+    const auto rx = buffer_of(x, ((T - 1) * x_stride + K) * 2);
+    constexpr int LPR = WB / 16, RPL = 64 / LPR; // lanes per row and rows per weight load
+    constexpr int LPT = KST / 8, TPL = 64 / LPT; // lanes per token and tokens per activation load
+    const uint32_t w_lane = (lane / LPR) * row_bytes + 16 * (lane % LPR), x_lane = (lane / LPT) * (x_stride * 2) + 16 * (lane % LPT);
+    const uint32_t s_lane = lane * scale_bytes; // lane = row of the workgroup; rows past the end read zeros
+
+    // The waves take the steps in turn.  Rows a multiple of 4 KiB apart lie on the same memory channels: there every workgroup
+    // starts at another step (7B int8 at 8 tokens, attention group: 15.6 -> 14.6 us; other row lengths lose 1 % from it).
+    const uint32_t nsteps = K / KST, count = (nsteps + NW - 1 - wv) / NW;
+    const uint32_t turn = row_bytes % 4096 == 0 ? (wg * 5) % nsteps : 0;
+
+    struct Step {
+        uint4 x[XL], w[WL];
+        uint32_t s[SUB];
+    } st;
+    auto load = [&](uint32_t m) {
+        uint32_t s = min(wv + m * NW, nsteps - 1) + turn;
+        s = s >= nsteps ? s - nsteps : s;
+#pragma unroll
+        for (int i = 0; i < XL; i++) st.x[i] = buffer_load128<0>(rx, x_lane + (i * TPL * x_stride * 2 + s * (KST * 2)));
+        if constexpr (SUB == 2) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, s_lane + s * 8, 0, 0);
+            st.s[0] = v[0], st.s[SUB - 1] = v[1];
+        } else {
+            st.s[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, s_lane + s * 4, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < WL; i++) st.w[i] = buffer_load128<kStream>(rw, w_lane + (i * RPL * row_bytes + s * WB));
+    };
+    // nf4 rows as long as a single row tile may have them: even and odd blocks are summed apart, which halves the longest chain
+    // of f32 additions (14336 x 4096, f32 outputs against 64 bits: 1.33e-7 in one chain, the chunk kernel's K split 1.20e-7)
+    constexpr int CHAINS = N4 && MRT == 1 ? 2 : 1;
+    float4v out[CHAINS][MRT][NT];
+    const float4v zero4 = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < CHAINS; c++)
+#pragma unroll
+        for (int i = 0; i < MRT; i++)
+#pragma unroll
+            for (int n = 0; n < NT; n++) out[c][i][n] = zero4;
+
+    load(0);
+    __builtin_amdgcn_sched_barrier(0); // the order of these loads is the order of the loop's
+    if (N4) {
+        // entry for byte v: (hi(q[v & 15]), hi(q[v >> 4])), (lo(..), lo(..)); lo scaled by 2^11
+        const float h0 = h2f(f2h(tq0)), h1 = h2f(f2h(tq1));
+        if (tid < 256) pair[tid] = make_uint2(pack_h2(tq0, tq1), pack_h2((tq0 - h0) * 2048.0f, (tq1 - h1) * 2048.0f));
+        lds_barrier();
+    }
+    // scalar loads of cold argument memory, waited for here rather than in front of the stores (0.1 us per launch)
+    void *const o_ptr = a.m[pi].out;
+    const uint64_t o_stride = a.m[pi].out_token_stride;
+    const int o_f16 = a.m[pi].out_f16, o_act = a.m[pi].act;
+    asm volatile("" ::"s"(o_ptr), "s"(o_stride), "s"(o_f16), "s"(o_act));
+
+    uint32_t token[NT]; // staged token of this lane's column; of a half tile the upper columns repeat the lower ones and are not stored
+    const uint8_t *xb[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        token[n] = 16 * n + (TOK - 16 * n < 16 ? (r16 & 7) : r16);
+        xb[n] = xs + token[n] * G::XPITCH + 32 * g;
+    }
+    // B operands of 64 elements: lane (token, g) holds elements 16 g .. + 8 and 16 g + 8 .. + 16
+    auto read_b = [&](int half, HalfPack (&b)[NT][2]) {
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const uint4 v = *reinterpret_cast<const uint4 *>(xb[n] + 128 * half + 16 * j);
+                b[n][j].u[0] = v.x, b[n][j].u[1] = v.y, b[n][j].u[2] = v.z, b[n][j].u[3] = v.w;
+            }
+    };
+#pragma unroll 1
+    for (uint32_t m = 0; m < count; m++) {
+        // registers -> the wave's slot (one wave writes and reads it, in program order: no barrier)
+#pragma unroll
+        for (int i = 0; i < XL; i++) {
+            *reinterpret_cast<uint4 *>(xs + (i * TPL + lane / LPT) * G::XPITCH + 16 * (lane % LPT)) = st.x[i];
+            if (!N4) { // the 16 pieces of a token and 128 elements sit in one DPP row
+                float q = dot2_ones(st.x[i].x, 0.0f);
+                q = dot2_ones(st.x[i].y, q);
+                q = dot2_ones(st.x[i].z, q);
+                q = dot2_ones(st.x[i].w, q);
+                q = row16_sum(q);
+                if ((lane & 15) == 0) sxs[((lane % LPT) / 16) * TOK + i * TPL + lane / LPT] = q;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < WL; i++) *reinterpret_cast<uint4 *>(ws + (RPL * i + lane / LPR) * G::WPITCH + 16 * (lane % LPR)) = st.w[i];
+        if (lane < 16 * MRT) {
+#pragma unroll
+            for (int u = 0; u < SUB; u++) {
+                const float lo = h2f((uint16_t)st.s[u]), hi = h2f((uint16_t)(st.s[u] >> 16));
+                const float s = (hi - lo) * (1.0f / 255.0f); // (min, max) -> (s, min - 1024 s)
+                scl[(2 * u) * 16 * MRT + lane] = N4 ? lo : s;
+                scl[(2 * u + 1) * 16 * MRT + lane] = N4 ? hi : fmaf(-1024.0f, s, lo);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (m + 1 < count) load(m + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // Work items of a step: (64 elements, row tile), row tiles first.  Weights are read two items ahead, an item's table
+        // lookups are issued in front of the matrix work of the item before it, whose sums are taken in behind the next one's.
+        constexpr int ITEMS = 2 * SUB * MRT;
+        HalfPack B[2][NT][2];
+        auto scale_of = [&](int word, int i) { return *reinterpret_cast<const float4 *>(scl + word * 16 * MRT + 16 * i + 4 * g); };
+        if constexpr (N4) {
+            uint2 wq[2];
+            HalfPack Ah[2][2], Al[2][2];
+            float4 am[2];
+            float4v Dh[2][NT], Dl[2][NT];
+            auto read_w = [&](int it) { return *reinterpret_cast<const uint2 *>(ws + (16 * (it % MRT) + r16) * G::WPITCH + 32 * (it / MRT) + 8 * g); };
+            auto lookup = [&](int it) {
+                const int q = it & 1, blk = it / MRT;
+                if (it % MRT == 0) read_b(blk, B[blk & 1]);
+                const uint32_t ww[2] = {wq[q].x, wq[q].y};
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const uint2 e = pair[(ww[j] >> (8 * c)) & 0xffu];
+                        Ah[q][j].u[c] = e.x;
+                        Al[q][j].u[c] = e.y;
+                    }
+                am[q] = scale_of(blk, it % MRT);
+                if (it + 2 < ITEMS) wq[q] = read_w(it + 2);
+            };
+            auto take_in = [&](int it) { // out += absmax * (D_hi + 2^-11 D_lo)
+                const int q = it & 1, i = it % MRT, c = it / MRT % CHAINS;
+                const float s[4] = {am[q].x, am[q].y, am[q].z, am[q].w};
+#pragma unroll
+                for (int n = 0; n < NT; n++)
+#pragma unroll
+                    for (int d = 0; d < 4; d++) out[c][i][n][d] = fmaf(s[d], fmaf(Dl[q][n][d], 1.0f / 2048.0f, Dh[q][n][d]), out[c][i][n][d]);
+            };
+            wq[0] = read_w(0);
+            wq[1] = read_w(1);
+            lookup(0);
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const int q = it & 1, blk = it / MRT;
+                __builtin_amdgcn_sched_barrier(0);
+                if (it > 0) take_in(it - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (it + 1 < ITEMS) lookup(it + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    Dh[q][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[q][0].h, B[blk & 1][n][0].h, zero4, 0, 0, 0);
+                    Dl[q][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[q][0].h, B[blk & 1][n][0].h, zero4, 0, 0, 0);
+                }
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    Dh[q][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[q][1].h, B[blk & 1][n][1].h, Dh[q][n], 0, 0, 0);
+                    Dl[q][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[q][1].h, B[blk & 1][n][1].h, Dl[q][n], 0, 0, 0);
+                }
+            }
+            take_in(ITEMS - 1);
+        } else {
+            uint4 wq[2];
+            float4v D[MRT][NT];
+            auto read_w = [&](int it) { return *reinterpret_cast<const uint4 *>(ws + (16 * (it % MRT) + r16) * G::WPITCH + 64 * (it / MRT) + 16 * g); };
+            read_b(0, B[0]);
+            wq[0] = read_w(0);
+            wq[1] = read_w(1);
+#pragma unroll
+            for (int it = 0; it < ITEMS; it++) {
+                const int q = it & 1, half = it / MRT, i = it % MRT;
+                __builtin_amdgcn_sched_barrier(0);
+                const uint32_t ww[4] = {wq[q].x, wq[q].y, wq[q].z, wq[q].w};
+                HalfPack A[2];
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int c = 0; c < 2; c++) { // 4 codes of one dword -> f16 pairs 1024 + u
+                        A[j].u[2 * c] = __builtin_amdgcn_perm(0x64646464u, ww[2 * j + c], 0x04010400u);
+                        A[j].u[2 * c + 1] = __builtin_amdgcn_perm(0x64646464u, ww[2 * j + c], 0x04030402u);
+                    }
+                if (it + 2 < ITEMS) wq[q] = read_w(it + 2);
+                if (i == 0 && half + 1 < 2 * SUB) read_b(half + 1, B[(half + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int n = 0; n < NT; n++)
+                    D[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[0].h, B[half & 1][n][0].h, (half & 1) == 0 ? zero4 : D[i][n], 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n < NT; n++) D[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[1].h, B[half & 1][n][1].h, D[i][n], 0, 0, 0);
+                if ((half & 1) && i == MRT - 1) { // a 128-block is complete: out += s * D + (min - 1024 s) * sum_k x
+                    const int u = half >> 1;
+#pragma unroll
+                    for (int k = 0; k < MRT; k++) {
+                        const float4 sv = scale_of(2 * u, k), cv = scale_of(2 * u + 1, k);
+                        const float s[4] = {sv.x, sv.y, sv.z, sv.w}, c[4] = {cv.x, cv.y, cv.z, cv.w};
+#pragma unroll
+                        for (int n = 0; n < NT; n++) {
+                            const float sx = sxs[u * TOK + token[n]];
+#pragma unroll
+                            for (int d = 0; d < 4; d++) out[0][k][n][d] = fmaf(s[d], D[k][n][d], fmaf(c[d], sx, out[0][k][n][d]));
+                        }
+                    }
+                }
+            }
+        }
+    }
+
+    // The partial tiles of the waves, each in the wave's own slot, summed pairwise.  D layout of a 16 x 16 tile: lane holds
+    // token column (lane & 15), rows 4 g .. 4 g + 3.
+    float4 *const part = reinterpret_cast<float4 *>(slot);
+#pragma unroll
+    for (int i = 0; i < MRT; i++)
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            float4v o = out[0][i][n];
+            if constexpr (CHAINS == 2) o += out[CHAINS - 1][i][n];
+            part[(i * NT + n) * 64 + lane] = make_float4(o[0], o[1], o[2], o[3]);
+        }
+    lds_barrier();
+    for (uint32_t q = tid; q < MRT * NT * 64; q += 64 * NW) {
+        float4 e[NW];
+#pragma unroll
+        for (int u = 0; u < NW; u++) e[u] = *reinterpret_cast<const float4 *>(smem + G::TABLE + u * G::SLOT + 16 * q);
+#pragma unroll
+        for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+            for (int u = 0; u < NW; u += 2 * d) e[u].x += e[u + d].x, e[u].y += e[u + d].y, e[u].z += e[u + d].z, e[u].w += e[u + d].w;
+        const float4 v = e[0];
+        const uint32_t tile = q >> 6, l = q & 63, i = tile / NT, n = tile % NT;
+        const uint32_t row = row0 + 16 * i + 4 * (l >> 4), t = 16 * n + (l & 15);
+        if (t >= T || row >= R) continue;
+        const float o[4] = {act_apply(o_act, v.x), act_apply(o_act, v.y), act_apply(o_act, v.z), act_apply(o_act, v.w)};
+        const uint64_t idx = (uint64_t)t * o_stride + row;
+        if (o_f16)
+            *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(o_ptr) + idx) = make_uint2(pack_h2(o[0], o[1]), pack_h2(o[2], o[3]));
+        else
+            *reinterpret_cast<float4 *>(reinterpret_cast<float *>(o_ptr) + idx) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+namespace {
+
+template <int QUANT, int MRT, int TOK, int NW, int SUB>
+int launch_one(hipStream_t stream, const MatmulArgs *args, int n) {
+    using G = ShortGeometry<QUANT, MRT, TOK, NW, SUB>;
+    auto *kern = &gemm_short_kernel<QUANT, MRT, TOK, NW, SUB>;
+    if (G::LDS > 48 * 1024) {
+        // one-time opt-in to more than the default dynamic LDS limit
+        static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
+        (void)once;
+    }
+    ShortArgs a;
+    uint32_t total = 0;
+    for (int i = 0; i < kMaxGroup; i++) {
+        a.begin[i] = 0xffffffffu;
+        if (i >= n) continue;
+        a.m[i] = args[i];
+        a.begin[i] = total;
+        total += (args[i].R + 16 * MRT - 1) / (16 * MRT);
+    }
+    const MatmulArgs &m = args[0];
+    hipLaunchKernelGGL(kern, dim3(total), dim3(64 * NW), G::LDS, stream, m.w, m.scale, m.x, m.quant, a.begin[1], m.R, (uint32_t)m.x_token_stride,
+                       m.K, m.T, a);
+    return check_launch("matmul (short run)");
+}
+
+// Row tiles per workgroup: one up to 4096 rows (256 workgroups), then the fewest that leave one workgroup per CU; beyond
+// 16384 rows no number does, and three keep the last round short (18432 x 4096 at 8 tokens: int8 18.5 us with 3, 20.5 with 4).
+// Workgroups have eight waves, two per SIMD.  Where two rounds of workgroups with three row tiles run, and where the
+// activations of 33 tokens and more leave no room for eight slots, they have four (18432 x 4096 nf4 at 32 tokens 26.8 against 29.0 us).
+template <int QUANT, int TOK>
+int launch_tok(hipStream_t stream, const MatmulArgs *args, int n, uint64_t rows) {
+    const uint64_t tiles = (rows + 15) / 16;
+    const bool rounds = tiles > 1024;
+    if constexpr (TOK == 8) {
+        // up to 8 tokens activations are cheap: steps of 256 elements keep twice the bytes in flight.  One row tile of long
+        // int8 rows (4096 x 14336: 14.2 against 14.8 us), and every grid of several rounds (nf4 18432 x 4096 17.8 against 19.2 us,
+        // 20480 x 5120 22.0 against 24.7; int8 20480 x 5120 24.2 against 25.4)
+        if (args[0].K % 256 == 0 && (rounds || (QUANT == kInt8 && tiles <= 256 && args[0].K >= 7168)))
+            return launch_one<QUANT, 1, TOK, 8, 2>(stream, args, n);
+    }
+    if (tiles <= 256) return launch_one<QUANT, 1, TOK, 8, 1>(stream, args, n);
+    if (tiles <= 512) return launch_one<QUANT, 2, TOK, 8, 1>(stream, args, n);
+    if constexpr (TOK <= 32) {
+        if (tiles <= 768) return launch_one<QUANT, 3, TOK, 8, 1>(stream, args, n);
+        if (!rounds) return launch_one<QUANT, 4, TOK, 8, 1>(stream, args, n);
+    } else {
+        if (tiles > 768 && !rounds) return launch_one<QUANT, 4, TOK, 4, 1>(stream, args, n);
+    }
+    return launch_one<QUANT, 3, TOK, TOK <= 16 ? 8 : 4, 1>(stream, args, n);
+}
+
+template <int QUANT>
+int launch_quant(hipStream_t stream, const MatmulArgs *args, int n, uint64_t rows) {
+    const uint32_t T = args[0].T;
+    if (T <= 8) return launch_tok<QUANT, 8>(stream, args, n, rows);
+    if (T <= 16) return launch_tok<QUANT, 16>(stream, args, n, rows);
+    if (T <= 24) return launch_tok<QUANT, 24>(stream, args, n, rows);
+    if (T <= 32) return launch_tok<QUANT, 32>(stream, args, n, rows);
+    return launch_tok<QUANT, 48>(stream, args, n, rows);
+}
+
+// Where a workgroup per 16 rows over the whole K is the faster split than the chunk kernel's (measured over the layer shapes of the
+// 0.1B .. 14B models and 128 .. 6144 rows x 896 .. 14336, 5 .. 64 tokens).  With few rows most CUs have no workgroup and a
+// long K is a long chain: there the chunk kernel's split of K over the grid wins, the sooner the more activations a
+// workgroup has to fetch for its rows.
+bool faster(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
+    if (T <= 8) return quant == kNf4 || rows >= 2048 || K <= 10240;              // int8 1024 rows: K 8192 0.89 of the chunk kernel's time, 14336 1.01
+    if (T <= 16) return rows >= 2048 || K <= (quant == kNf4 ? 10240u : 5120u);    // int8 1024 rows: 4096 0.81, 8192 1.07; nf4 0.78, 0.95
+    if (T <= 24) return quant == kNf4 || K <= 10240 || (T <= 20 && rows >= 2048); // int8 4096 x 14336 at 19 / 24 tokens 0.92 / 1.04; nf4 0.85
+    if (T <= 32) return rows >= 2560 ? quant == kNf4 || K <= 8192 : K <= 4096;    // 2048 x 7168 1.04 (nf4), 1.13 (int8); 4096 x 14336 0.96, 1.18
+    return rows >= 2560 && K <= 8192;                                             // up to 48 tokens: 1.6B / 3B / 7B groups 0.7 .. 0.9, 2048 x 7168 1.02 .. 1.14
+}
+
+} // namespace
+
+// Takes the `n` products of a launch (one K and token count, f16 activations, one batch, K % 128 == 0 and the
+// alignments of the chunk kernel) if this kernel is the faster one for them; false leaves them to the caller.
+bool launch_gemm_short(hipStream_t stream, Quant quant, const MatmulArgs *args, int n, int &status) {
+    const uint32_t K = args[0].K, T = args[0].T;
+    if (quant == kFp16 || T > 48 || K < 128 || !tune(kTuneGemmShort, 1)) return false;
+    // a pinned tile of the chunk kernel means that kernel
+    if (tune_is_set(kTuneGemmNtile) || tune_is_set(kTuneGemmMrt) || tune_is_set(kTuneGemmKg) || tune_is_set(kTuneGemmKsplit)) return false;
+    uint64_t rows = 0;
+    for (int i = 0; i < n; i++) {
+        // 32-bit byte offsets into a workgroup's rows and into the activations
+        if (args[i].B != 1 || K > (1u << 24) || ((uint64_t)(T - 1) * args[i].x_token_stride + K) * 2 > 0x7fffffffull) return false;
+        rows += args[i].R;
+    }
+    if (!faster(quant, rows, K, T)) return false;
+    status = quant == kNf4 ? launch_quant<kNf4>(stream, args, n, rows) : launch_quant<kInt8>(stream, args, n, rows);
+    return true;
+}
+
+} // namespace wrq

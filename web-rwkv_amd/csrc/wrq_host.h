@@ -45,6 +45,9 @@ int launch_gemm_noalloc(hipStream_t stream, Quant quant, int in_f16, const Matmu
 // The same for `n` independent products of one quantisation and input type: those with one K
 // and token count share a launch (and then rarely need a split of K).
 int launch_gemm_group(hipStream_t stream, Quant quant, int in_f16, const MatmulArgs *args, int n, const ScratchPolicy *sp = nullptr);
+// Short runs (gemm_short.hip): launches `n` products that share K, token count and f16 activations if that kernel is the
+// faster one for them, with the launch's result in `status`; false: nothing was launched.
+bool launch_gemm_short(hipStream_t stream, Quant quant, const MatmulArgs *args, int n, int &status);
 // Overrides of the kernel and tile choice, for tests and sweeps that must reach one particular
 // instantiation.  Every key is unset (-1) unless the environment variable of the same name (WRQ_ +
 // upper-case key) was set when the library first looked, or wrq_debug_override() set it since; the
@@ -66,6 +69,7 @@ enum TuneKey {
     kTuneGemvRowsTokens, // gemv_rows_tokens: 0 keeps int8 runs of 2 .. 4 tokens off the wave-owns-rows and K-split kernels
     kTuneGemmTable,    // gemm_table: 0 leaves the measured tile table (gemm_tuned.inc) out and picks chunk tiles by the rules alone
     kTuneGemvTable,    // gemv_table: 0 leaves the measured table of the one-shot decode kernels (gemv_tuned.inc) out
+    kTuneGemmShort,    // gemm_short: 0 keeps short runs on the chunk kernel
     kTuneCount
 };
 // The override of `key`, or `fallback` when it is unset.
