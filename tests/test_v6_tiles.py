@@ -69,6 +69,25 @@ def test_gpu_adapters_in_long_rows(gpu, C, A):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C", [128, 768, 1152, 2048, 2176, 4224])
+@pytest.mark.parametrize("A", [1, 15, 16, 33])
+def test_gpu_adapters_in_lines(gpu, C, A):
+    """First halves of adapters over channels in whole steps of 128: fewer steps than waves, one round of two steps per wave, more."""
+    import torch
+
+    print("adapters_in in lines on the GPU", C, A, flush=True)
+    g = torch.Generator().manual_seed(0x575A + C + A)
+    h = lambda *s: (torch.randn(s, generator=g) * 0.05).half()
+    ops = [(h(r, C), h(A, C), torch.empty((A, r), dtype=torch.float16, device="cuda"), act) for r, act in ((32, gpu.ACT_NONE), (16, gpu.ACT_SIGMOID), (80, gpu.ACT_NONE))]
+    gpu.FusedV7.adapters_in(C, A, [(w.cuda(), x.cuda(), out, act) for w, x, out, act in ops])
+    for w, x, out, act in ops:
+        want = x.double() @ w.double().t()
+        want = torch.sigmoid(want) if act == gpu.ACT_SIGMOID else want
+        # f32 sums of up to 4224 products of 2.5e-3 each, one rounding to f16 (2^-11) of values below 1
+        assert_close(out.cpu().numpy(), want.numpy(), 1e-3, "adapters_in vs float64")
+
+
+@pytest.mark.gpu
 def test_gpu_pre_of_one_token_in_place(gpu):
     """A single token has no neighbour that reads its row: normalised in place as into a buffer of its own."""
     import torch

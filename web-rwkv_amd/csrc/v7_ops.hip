@@ -33,11 +33,14 @@ struct AdapterArgs {
 
 // First halves of a layer's low-rank adapters, out[t][r] = f16(act(sum_k w[r][k] x[t][k])): a few dozen rows over K = C
 // per adapter, so the product is one short pass over weights that fit in the caches and its time is latency.  One workgroup
-// per 16 rows x 16 tokens of any adapter of the layer; its WAVES waves take every WAVES-th 32-element step of K, straight from
-// memory in the operand layout of the 16x16x32 MFMA, Q steps in flight, and add up through LDS.  2048 channels, 32 tokens, four adapters: 7 us
-// in one launch, against 4 x (5 + 3) us for products split over K and summed by a second launch each.
-template <int WAVES, int Q>
+// per 16 rows x 16 tokens of any adapter of the layer; its WAVES waves take the steps of 128 elements of K in turn, Q steps in flight,
+// and add up through LDS.  LINES: a step comes line-wise from memory (the 256 bytes of a row in 16 adjacent lanes) and gets
+// into the operand layout of the 16x16x32 MFMA through LDS of the wave's own; gathered straight into that layout a load touches 16 rows and costs
+// the address units three times as much.  Without LINES (K no multiple of 128) steps are 32 elements, gathered.
+template <int WAVES, int Q, bool LINES>
 __global__ __launch_bounds__(64 * WAVES) void adapters_in_kernel(uint32_t K, uint32_t T, AdapterArgs aa) {
+    constexpr int PITCH = 256 + 16; // bytes per staged row: +16 B rotates the banks
+    __shared__ __align__(16) uint8_t slots[LINES ? WAVES : 1][LINES ? 32 * PITCH : 16];
     __shared__ float4 red[WAVES - 1][64];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
     uint32_t p = 0;
@@ -45,20 +48,51 @@ __global__ __launch_bounds__(64 * WAVES) void adapters_in_kernel(uint32_t K, uin
     for (uint32_t i = 1; i < kMaxAdapters; i++)
         if (blockIdx.x >= aa.tile_begin[i]) p = i;
     const uint32_t row0 = 16 * (blockIdx.x - aa.tile_begin[p]), t0 = 16 * blockIdx.y;
-    const uint32_t steps = K / 32;
-    const uint16_t *wp = aa.w[p] + (uint64_t)(row0 + r16) * K + 8 * g;
-    const uint16_t *xp = aa.x[p] + (uint64_t)min(t0 + r16, T - 1) * K + 8 * g; // columns past the run repeat its last token, never stored
+    // columns past the run repeat its last token, never stored
     float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s0 = wave; s0 < steps; s0 += Q * WAVES) {
-        uint4 a[Q], b[Q];
+    if constexpr (LINES) {
+        const uint32_t steps = K / 128, at = lane / 16, piece = 8 * (lane % 16);
+        const uint16_t *wp = aa.w[p] + (uint64_t)(row0 + at) * K + piece, *xp[4];
 #pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const uint32_t at = 32 * min(s0 + q * WAVES, steps - 1);
-            a[q] = load128(wp + at), b[q] = load128(xp + at);
+        for (int i = 0; i < 4; i++) xp[i] = aa.x[p] + (uint64_t)min(t0 + 4 * i + at, T - 1) * K + piece;
+        uint8_t *const put = slots[wave] + at * PITCH + 2 * piece;
+        const uint8_t *const get = slots[wave] + r16 * PITCH + 16 * g;
+        for (uint32_t s0 = wave; s0 < steps; s0 += Q * WAVES) {
+            uint4 a[Q][4], b[Q][4];
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t k = 128 * min(s0 + q * WAVES, steps - 1);
+                    a[q][i] = load128(wp + (uint64_t)(4 * i) * K + k), b[q][i] = load128(xp[i] + k);
+                }
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                if (s0 + q * WAVES >= steps) break;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    *reinterpret_cast<uint4 *>(put + 4 * i * PITCH) = a[q][i];
+                    *reinterpret_cast<uint4 *>(put + (16 + 4 * i) * PITCH) = b[q][i];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8 *>(get + 64 * j), *reinterpret_cast<const half8 *>(get + 16 * PITCH + 64 * j), acc, 0, 0, 0);
+            }
         }
+    } else {
+        const uint32_t steps = K / 32;
+        const uint16_t *wp = aa.w[p] + (uint64_t)(row0 + r16) * K + 8 * g, *xp = aa.x[p] + (uint64_t)min(t0 + r16, T - 1) * K + 8 * g;
+        for (uint32_t s0 = wave; s0 < steps; s0 += Q * WAVES) {
+            uint4 a[Q], b[Q];
 #pragma unroll
-        for (int q = 0; q < Q; q++)
-            if (s0 + q * WAVES < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[q]), __builtin_bit_cast(half8, b[q]), acc, 0, 0, 0);
+            for (int q = 0; q < Q; q++) {
+                const uint32_t at = 32 * min(s0 + q * WAVES, steps - 1);
+                a[q] = load128(wp + at), b[q] = load128(xp + at);
+            }
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                if (s0 + q * WAVES < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[q]), __builtin_bit_cast(half8, b[q]), acc, 0, 0, 0);
+        }
     }
     if (wave) red[wave - 1][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
     __syncthreads();
@@ -403,12 +437,12 @@ int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void
         aa.rank[i] = ranks[i], aa.act[i] = acts[i];
         tiles += ranks[i] / 16;
     }
-    // Steps of 32 channels that the waves of a workgroup have in flight at once: eight waves of eight take K in one go up to 64
-    // steps, of ten up to 80 (2560 channels, 160 rows, 100 tokens: 9.7 -> 7.1 us); up to 128 (4096 channels) eight of eight go
-    // round twice (9.7 us; sixteen of eight gained nothing), beyond sixteen of ten (5120 channels: 13.1 -> 11.8 us).
-    const uint32_t steps = C / 32;
     auto go = [&](auto kern, int waves) { hipLaunchKernelGGL(kern, dim3(tiles, (A + 15) / 16), dim3(64 * waves), 0, static_cast<hipStream_t>(stream), C, A, aa); };
-    steps > 128 ? go(adapters_in_kernel<16, 10>, 16) : steps > 64 && steps <= 80 ? go(adapters_in_kernel<8, 10>, 8) : go(adapters_in_kernel<8, 8>, 8);
+    // Eight waves, two steps each in flight: 2048 channels in one go.  us, gathered -> line-wise: 160 rows x 100 tokens over 768 / 2048 / 4096 / 5120
+    // channels 6.5 / 6.5 / 10.3 / 12.0 -> 3.7 / 4.5 / 6.0 / 6.9; four adapters of a v7 layer, 32 tokens, 6.3 / 6.5 / 10.2 / 12.0 -> 3.5 / 4.5 /
+    // 5.8 / 6.8.  Sixteen waves of one step 3.7 / 4.5 / 6.1 / 7.3, four of four 4.0 / 5.3 / 7.7 / 8.8.
+    if (C % 128 == 0) go(adapters_in_kernel<8, 2, true>, 8);
+    else go(adapters_in_kernel<8, 8, false>, 8);
     return check_launch(what);
 }
 

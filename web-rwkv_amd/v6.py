@@ -134,13 +134,11 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False,
     ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
     slice_of = lambda i: ((C, A, 1), (C, A, 5), (0, 0, i))
 
-    # First half of an adapter: the launch of small tiles where it beats the f16 product, which is a one-shot kernel up to 4 tokens
-    # (below 1024 channels up to 16) and splits K beyond.  us, tiles against product, 160 and 64 rows: 768 channels 6.4 / 5.2 and
-    # 6.4 / 5.1 at 16 tokens, 6.4 / 9.3 and 6.4 / 9.0 at 17, 13.6 / 12.8 and 6.7 / 12.7 at 1024 (both adapters together still
-    # tiles); 1024 channels 5.5 / 7.3 and 5.4 / 7.0 at 5; 2560 channels 6.2 / 8.1 and 6.1 / 7.1 at 5, 7.4 / 10.1 and 7.4 / 9.9 at
-    # 100; 3072 channels 8.7 / 8.0 and 8.7 / 7.2 at 8, 10.1 / 10.3 and 10.0 / 10.2 at 100, 17.2 / 13.8 and 10.2 / 13.4 at 512;
-    # 5120 channels 10.1 / 8.2 and 10.1 / 7.7 at 8, 11.8 / 10.9 and 11.7 / 10.7 at 100.
-    tiles = C <= 2560 and A > (4 if C >= 1024 else 16)
+    # First half of an adapter: the launch of small tiles, or the f16 product up to 4 tokens, where that is a one-shot kernel (2.5 us
+    # at 2048 and 4096 channels, one token).  us, tiles / product, 160 rows: 768 channels 3.6 / 6.0 at 16 tokens; 1024 channels 3.7 / 8.1 at 5;
+    # 3072 channels 5.2 / 8.9 at 5, 5.7 / 10.8 at 100; 4096 channels 5.9 / 8.5 at 5, 6.4 / 10.0 at 100; 5120 channels 6.7 / 9.2 at 5,
+    # 7.4 / 11.6 at 100, 7.8 / 13.6 at 255.  Channels in no whole steps of 128 are gathered: below 1024 the product keeps runs up to 16 tokens.
+    tiles = A > (4 if C % 128 == 0 or C >= 1024 else 16)
 
     def adapter_in(name, x, out):
         if tiles:
