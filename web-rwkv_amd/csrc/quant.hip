@@ -6,8 +6,8 @@
 // DPP inside the lane group, and every lane packs its own eight elements.  The
 // reference's two/three dispatches per matrix (statistics, quantise, f32->f16 blit;
 // src/tensor/ops.rs:2393-2486, :2488-2589) collapse into one launch with no
-// temporary.  Workgroups are resident and walk the matrix with a grid stride, the next
-// 16 bytes of a lane already in flight while it packs the current ones.
+// temporary.  Workgroups walk the matrix with a grid stride, the next
+// 16-byte loads of a lane already in flight while it packs the current ones.
 //
 // The results are the reference shaders' results bit for bit
 // (src/shaders/quant_mat_int8.wgsl:24-59, quant_mat_nf4.wgsl:24-81): IEEE f32
@@ -44,16 +44,21 @@ __device__ __forceinline__ float dpp_f(float v, int ctrl) {
     }
 }
 
-// Large workgroups, few of them: workgroups are handed out at a limited rate, and a packer's
-// whole run is a handful of microseconds.
-constexpr uint32_t kPackThreads = 1024;
-
-// Resident grid: two workgroups of 16 waves per CU, never more than the work.
-static uint32_t resident_grid(uint64_t ngroup) {
-    const uint64_t need = (ngroup + kPackThreads - 1) / kPackThreads;
-    const uint64_t cap = 256 * 2;
-    return (uint32_t)(need < cap ? need : cap);
-}
+// Workgroup size, most workgroups of a launch and 16-byte groups a thread has in flight per pass, of each packer; the current pass
+// is packed while the next one's loads are on their way (four groups, 68 - 82 registers, are slower on every shape).  A packer's whole run is a handful of microseconds.  int8 is bound by memory
+// and takes many small workgroups with two groups each; against the 1024 threads, 512 workgroups and one group that nf4 keeps, us
+// cold: 768^2 2.99 -> 2.64, 2048^2 5.10 -> 4.49, 7168 x 2048 12.4 -> 10.5, 4096^2 13.9 -> 11.5, 14336 x 4096 38.5 -> 35.4, 65536 x 2048 77.2 ->
+// 74.5.  nf4 searches its thresholds in every workgroup before it starts: more of them cost more than they bring (4096^2 12.7 -> 16.1).
+template <int THREADS_, int GRID, int GROUPS_>
+struct PackForm {
+    static constexpr int THREADS = THREADS_, GROUPS = GROUPS_;
+    static uint32_t grid(uint64_t ngroup) { // never more than the work
+        const uint64_t need = (ngroup + THREADS - 1) / THREADS;
+        return (uint32_t)(need < GRID ? need : GRID);
+    }
+};
+using Int8Form = PackForm<512, 3072, 2>;
+using Nf4Form = PackForm<1024, 512, 1>;
 
 // ---------------------------------------------------------------------------------- int8
 
@@ -78,35 +83,29 @@ __device__ __forceinline__ float div_shared(float a, float b, float r) {
     return fmaf(e, r, q);
 }
 
-// Groups of 8 elements a lane packs per pass over its loop; the loads of the next pass are
-// issued before the current one is packed, so a wave keeps 2 * kPassGroups KiB in flight.
-// Measured: 4 groups per pass (68 - 82 registers, 5 - 7 waves per SIMD) are 5 - 15 % slower than 1
-// (26 - 41 registers, 8 waves) on every shape.
-constexpr int kPassGroups = 1;
-
 // One lane per 8 elements; 16 lanes (one DPP row) per 128-element block.  ngroup is a
 // multiple of 16, so a row of lanes is live or idle as a whole.
-__global__ __launch_bounds__(kPackThreads) void quant_int8_kernel(const uint16_t *__restrict__ in,
+__global__ __launch_bounds__(Int8Form::THREADS) void quant_int8_kernel(const uint16_t *__restrict__ in,
                                                          uint32_t *__restrict__ minmax,
                                                          uint8_t *__restrict__ out, uint64_t ngroup) {
-    const uint64_t stride = (uint64_t)gridDim.x * kPackThreads;
-    uint64_t gid = (uint64_t)blockIdx.x * kPackThreads + threadIdx.x;
-    uint4 raw[kPassGroups];
+    const uint64_t stride = (uint64_t)gridDim.x * Int8Form::THREADS;
+    uint64_t gid = (uint64_t)blockIdx.x * Int8Form::THREADS + threadIdx.x;
+    uint4 raw[Int8Form::GROUPS];
 #pragma unroll
-    for (int u = 0; u < kPassGroups; u++) {
+    for (int u = 0; u < Int8Form::GROUPS; u++) {
         raw[u] = make_uint4(0, 0, 0, 0);
         if (gid + u * stride < ngroup) raw[u] = load128_stream(in + (gid + u * stride) * 8);
     }
     while (gid < ngroup) {
-        const uint64_t next = gid + kPassGroups * stride;
-        uint4 raw_next[kPassGroups];
+        const uint64_t next = gid + Int8Form::GROUPS * stride;
+        uint4 raw_next[Int8Form::GROUPS];
 #pragma unroll
-        for (int u = 0; u < kPassGroups; u++) {
+        for (int u = 0; u < Int8Form::GROUPS; u++) {
             raw_next[u] = make_uint4(0, 0, 0, 0);
             if (next + u * stride < ngroup) raw_next[u] = load128_stream(in + (next + u * stride) * 8);
         }
 #pragma unroll
-        for (int u = 0; u < kPassGroups; u++) {
+        for (int u = 0; u < Int8Form::GROUPS; u++) {
             const uint64_t g = gid + u * stride;
             if (g >= ngroup) break;
             float v[8];
@@ -145,7 +144,7 @@ __global__ __launch_bounds__(kPackThreads) void quant_int8_kernel(const uint16_t
         }
         gid = next;
 #pragma unroll
-        for (int u = 0; u < kPassGroups; u++) raw[u] = raw_next[u];
+        for (int u = 0; u < Int8Form::GROUPS; u++) raw[u] = raw_next[u];
     }
 }
 
@@ -193,18 +192,18 @@ __device__ __forceinline__ uint32_t nf4_cell(float x) {
 
 // One lane per 8 elements (one output u32); 8 lanes per 64-element block.  ngroup is a
 // multiple of 8, so a lane group is live or idle as a whole.
-__global__ __launch_bounds__(kPackThreads) void quant_nf4_kernel(const uint16_t *__restrict__ in,
+__global__ __launch_bounds__(Nf4Form::THREADS) void quant_nf4_kernel(const uint16_t *__restrict__ in,
                                                         const float *__restrict__ quant,
                                                         uint16_t *__restrict__ absmax,
                                                         uint32_t *__restrict__ out, uint64_t ngroup) {
     __shared__ uint2 lut[256]; // per cell: (threshold inside the cell or +inf, thresholds below the cell)
     __shared__ float thr_value[15];
     __shared__ uint32_t thr_cell[16]; // [15]: whether the table qualifies for the search path
-    const uint64_t stride = (uint64_t)gridDim.x * kPackThreads;
-    uint64_t gid = (uint64_t)blockIdx.x * kPackThreads + threadIdx.x;
-    uint4 raw[kPassGroups]; // in flight during the threshold search
+    const uint64_t stride = (uint64_t)gridDim.x * Nf4Form::THREADS;
+    uint64_t gid = (uint64_t)blockIdx.x * Nf4Form::THREADS + threadIdx.x;
+    uint4 raw[Nf4Form::GROUPS]; // in flight during the threshold search
 #pragma unroll
-    for (int u = 0; u < kPassGroups; u++) {
+    for (int u = 0; u < Nf4Form::GROUPS; u++) {
         raw[u] = make_uint4(0, 0, 0, 0);
         if (gid + u * stride < ngroup) raw[u] = load128_stream(in + (gid + u * stride) * 8);
     }
@@ -254,15 +253,15 @@ __global__ __launch_bounds__(kPackThreads) void quant_nf4_kernel(const uint16_t 
         }
         lds_barrier();
         while (gid < ngroup) {
-            const uint64_t next = gid + kPassGroups * stride;
-            uint4 raw_next[kPassGroups];
+            const uint64_t next = gid + Nf4Form::GROUPS * stride;
+            uint4 raw_next[Nf4Form::GROUPS];
 #pragma unroll
-            for (int u = 0; u < kPassGroups; u++) {
+            for (int u = 0; u < Nf4Form::GROUPS; u++) {
                 raw_next[u] = make_uint4(0, 0, 0, 0);
                 if (next + u * stride < ngroup) raw_next[u] = load128_stream(in + (next + u * stride) * 8);
             }
 #pragma unroll
-            for (int u = 0; u < kPassGroups; u++) {
+            for (int u = 0; u < Nf4Form::GROUPS; u++) {
                 const uint64_t g = gid + u * stride;
                 if (g >= ngroup) break;
                 float v[8];
@@ -286,7 +285,7 @@ __global__ __launch_bounds__(kPackThreads) void quant_nf4_kernel(const uint16_t 
             }
             gid = next;
 #pragma unroll
-            for (int u = 0; u < kPassGroups; u++) raw[u] = raw_next[u];
+            for (int u = 0; u < Nf4Form::GROUPS; u++) raw[u] = raw_next[u];
         }
         return;
     }
@@ -333,7 +332,7 @@ __global__ __launch_bounds__(kPackThreads) void quant_nf4_kernel(const uint16_t 
 int launch_quant_int8(hipStream_t stream, const void *in, void *minmax, void *out, uint64_t len) {
     const uint64_t ngroup = len / 8;
     if (ngroup == 0) return WRQ_OK;
-    hipLaunchKernelGGL(quant_int8_kernel, dim3(resident_grid(ngroup)), dim3(kPackThreads), 0, stream,
+    hipLaunchKernelGGL(quant_int8_kernel, dim3(Int8Form::grid(ngroup)), dim3(Int8Form::THREADS), 0, stream,
                        (const uint16_t *)in, (uint32_t *)minmax, (uint8_t *)out, ngroup);
     return check_launch("quant_mat_int8");
 }
@@ -342,7 +341,7 @@ int launch_quant_nf4(hipStream_t stream, const void *in, const void *quant, void
                      uint64_t len) {
     const uint64_t ngroup = len / 8;
     if (ngroup == 0) return WRQ_OK;
-    hipLaunchKernelGGL(quant_nf4_kernel, dim3(resident_grid(ngroup)), dim3(kPackThreads), 0, stream,
+    hipLaunchKernelGGL(quant_nf4_kernel, dim3(Nf4Form::grid(ngroup)), dim3(Nf4Form::THREADS), 0, stream,
                        (const uint16_t *)in, (const float *)quant, (uint16_t *)absmax, (uint32_t *)out,
                        ngroup);
     return check_launch("quant_mat_nf4");
