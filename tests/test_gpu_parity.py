@@ -775,6 +775,34 @@ def test_short_run_kernel(gpu, oracle, kind, T, overrides):
 
 
 @pytest.mark.parametrize("kind", ["int8", "nf4"])
+@pytest.mark.parametrize("T", [33, 49, 64, 65, 97, 192, 255, 256], ids=str)
+def test_short_run_kernel_in_token_blocks(gpu, oracle, kind, T, overrides):
+    # the same kernel over several blocks of 32, 48 or 64 tokens, the last one partly filled: tiles of one to four times 16 rows, row
+    # tiles that are padded to eight per product (workgroups without rows), groups, strided activations.  Tolerance as above.
+    import torch
+
+    announce("short run in token blocks", kind, T)
+    rng = np.random.default_rng(SEED + 92 + T)
+    for i, shapes in enumerate([[(256, 4)], [(640, 516), (640, 20)], [(1024, 1024)], [(256, 2052), (256, 1000), (256, 68)], [(2176, 4100)], [(4096, 264)]]):
+        K, ops, want = shapes[0][0], [], []
+        for j, (_, R) in enumerate(shapes):
+            wp, scale, wdeq = pack(oracle, kind, gen_f16(rng, (R, K), 0.02))
+            parent = gen_f16(rng, (T + 2, K + 8), 1.0)
+            out = torch.full((T, R), float("nan"), dtype=torch.float32 if (i + j) % 3 else torch.float16, device="cuda")
+            ops.append((gpu_matrix(gpu, kind, wp, scale), dev(parent), out, (i + j) % 2 * 6, False, dict(input_view=((K, T, 1), (K + 8, T + 2, 1), (8, 2, 0)))))
+            truth = truth_matmul(wdeq, parent[2:, 8:])
+            want.append(1.0 / (1.0 + np.exp(-truth)) if ops[-1][3] else truth)
+        results = []
+        for short in (1, 0):
+            overrides(gemm_short=short)
+            gpu.matmul_vec_group(ops)
+            results.append([host(op[2]) for op in ops])
+        for j, op in enumerate(ops):
+            assert_close(results[0][j], want[j], 3e-4 if op[2].dtype == torch.float32 else EPS, f"{kind} T={T} {shapes}[{j}] vs float64")
+            assert_close(results[0][j], results[1][j], EPS, f"{kind} T={T} {shapes}[{j}] vs the chunk kernel")
+
+
+@pytest.mark.parametrize("kind", ["int8", "nf4"])
 @pytest.mark.parametrize("T,ksplit", [(128, 2), (256, 1), (252, 1)], ids=str)
 def test_chunk_grid_a_little_above_two_workgroups_per_cu(gpu, oracle, kind, T, ksplit, overrides):
     # 576 workgroups (288 tiles of 128 rows x 64 tokens split in two, or 576 tiles) run as two launches:

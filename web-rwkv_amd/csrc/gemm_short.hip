@@ -1,4 +1,4 @@
-// Products on packed weights for short runs (a few tokens up to 48) for gfx950, on the f16 matrix cores:
+// Products on packed weights for short runs (a few tokens up to 48, small products up to 256) for gfx950, on the f16 matrix cores:
 // the same sums as gemm.hip (src/shaders/matmul_vec_int8.wgsl, matmul_vec_nf4.wgsl, matmul_mat_int8.wgsl,
 // matmul_mat_nf4.wgsl), split over the machine in another way.
 //
@@ -24,6 +24,8 @@
 // 14.4 / 6.1 / 18.5 / 14.2; 7B nf4 at 32 tokens 25.7 / 12.7 / 33.0 / 24.0 -> 20.5 / 8.7 / 26.8 / 22.9.
 #include "gemm_device.h"
 #include "wrq_host.h"
+
+#include <iterator>
 
 namespace wrq {
 
@@ -67,7 +69,7 @@ constexpr int kStream = 2; // nt: weights are read once (7B int8 at 8 tokens 15.
 template <int QUANT, int MRT, int TOK, int NW, int SUB>
 __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, const uint16_t *scale0, const void *x0, const float *quant0,
                                                              const uint32_t begin1, const uint32_t R0, const uint32_t x_stride0, const uint32_t K,
-                                                             const uint32_t T, const ShortArgs a) {
+                                                             const uint32_t T_all, const uint32_t tblocks, const ShortArgs a) {
     using G = ShortGeometry<QUANT, MRT, TOK, NW, SUB>;
     constexpr bool N4 = G::N4;
     constexpr int NT = G::NT, XL = G::XL, WL = G::WL, KST = G::KST, WB = G::WB;
@@ -88,6 +90,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, 
         w = m.w, scale = m.scale, x = m.x, quant = m.quant, R = m.R, x_stride = (uint32_t)m.x_token_stride;
         wg -= a.begin[pi];
     }
+    uint32_t t0 = 0;
+    if (tblocks > 1) { // the token blocks of one row tile run on one XCD one after the other: its L2 serves their weights
+        const uint32_t slot = wg >> 3;
+        t0 = slot % tblocks * TOK;
+        wg = slot / tblocks * 8 + (wg & 7);
+        if (wg * (16 * MRT) >= R) return; // padding to eight row tiles
+        x = static_cast<const uint16_t *>(x) + (uint64_t)t0 * x_stride;
+    }
+    const uint32_t T = min(T_all - t0, (uint32_t)TOK); // of this workgroup
     const uint32_t row0 = wg * (16 * MRT);
     uint2 *pair = reinterpret_cast<uint2 *>(smem);
     uint8_t *const slot = smem + G::TABLE + wv * G::SLOT;
@@ -331,7 +342,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, 
         const uint32_t row = row0 + 16 * i + 4 * (l >> 4), t = 16 * n + (l & 15);
         if (t >= T || row >= R) continue;
         const float o[4] = {act_apply(o_act, v.x), act_apply(o_act, v.y), act_apply(o_act, v.z), act_apply(o_act, v.w)};
-        const uint64_t idx = (uint64_t)t * o_stride + row;
+        const uint64_t idx = (uint64_t)(t0 + t) * o_stride + row;
         if (o_f16)
             *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(o_ptr) + idx) = make_uint2(pack_h2(o[0], o[1]), pack_h2(o[2], o[3]));
         else
@@ -352,65 +363,105 @@ int launch_one(hipStream_t stream, const MatmulArgs *args, int n) {
     }
     ShortArgs a;
     uint32_t total = 0;
+    const uint32_t tblocks = (args[0].T + TOK - 1) / TOK;
     for (int i = 0; i < kMaxGroup; i++) {
         a.begin[i] = 0xffffffffu;
         if (i >= n) continue;
         a.m[i] = args[i];
         a.begin[i] = total;
-        total += (args[i].R + 16 * MRT - 1) / (16 * MRT);
+        const uint32_t tiles = (args[i].R + 16 * MRT - 1) / (16 * MRT);
+        total += tblocks > 1 ? (tiles + 7) / 8 * 8 * tblocks : tiles;
     }
     const MatmulArgs &m = args[0];
     hipLaunchKernelGGL(kern, dim3(total), dim3(64 * NW), G::LDS, stream, m.w, m.scale, m.x, m.quant, a.begin[1], m.R, (uint32_t)m.x_token_stride,
-                       m.K, m.T, a);
+                       m.K, m.T, tblocks, a);
     return check_launch("matmul (short run)");
 }
 
-// Row tiles per workgroup: one up to 4096 rows (256 workgroups), then the fewest that leave one workgroup per CU; beyond
-// 16384 rows no number does, and three keep the last round short (18432 x 4096 at 8 tokens: int8 18.5 us with 3, 20.5 with 4).
-// Workgroups have eight waves, two per SIMD.  Where two rounds of workgroups with three row tiles run, and where the
-// activations of 33 tokens and more leave no room for eight slots, they have four (18432 x 4096 nf4 at 32 tokens 26.8 against 29.0 us).
-template <int QUANT, int TOK>
-int launch_tok(hipStream_t stream, const MatmulArgs *args, int n, uint64_t rows) {
+// Tile of a launch: row tiles, tokens, waves and 128-element pieces of a step; mrt 0: the chunk kernel is the faster one.
+struct ShortTile {
+    int mrt, tok, nw, sub;
+};
+constexpr ShortTile kNoTile{0, 0, 0, 0};
+
+// Runs of up to 48 tokens in one token block.  Row tiles per workgroup: one up to 4096 rows (256 workgroups), then the fewest that
+// leave one workgroup per CU; beyond 16384 rows no number does, and three keep the last round short (18432 x 4096 at 8 tokens: int8
+// 18.5 us with 3, 20.5 with 4).  Workgroups have eight waves, two per SIMD.  Where two rounds of workgroups with three row tiles run, and
+// where the activations of 33 tokens and more leave no room for eight slots, they have four (18432 x 4096 nf4 at 32 tokens 26.8
+// against 29.0 us).
+ShortTile one_block(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     const uint64_t tiles = (rows + 15) / 16;
     const bool rounds = tiles > 1024;
-    if constexpr (TOK == 8) {
-        // up to 8 tokens activations are cheap: steps of 256 elements keep twice the bytes in flight.  One row tile of long
-        // int8 rows (4096 x 14336: 14.2 against 14.8 us), and every grid of several rounds (nf4 18432 x 4096 17.8 against 19.2 us,
-        // 20480 x 5120 22.0 against 24.7; int8 20480 x 5120 24.2 against 25.4)
-        if (args[0].K % 256 == 0 && (rounds || (QUANT == kInt8 && tiles <= 256 && args[0].K >= 7168)))
-            return launch_one<QUANT, 1, TOK, 8, 2>(stream, args, n);
-    }
-    if (tiles <= 256) return launch_one<QUANT, 1, TOK, 8, 1>(stream, args, n);
-    if (tiles <= 512) return launch_one<QUANT, 2, TOK, 8, 1>(stream, args, n);
-    if constexpr (TOK <= 32) {
-        if (tiles <= 768) return launch_one<QUANT, 3, TOK, 8, 1>(stream, args, n);
-        if (!rounds) return launch_one<QUANT, 4, TOK, 8, 1>(stream, args, n);
-    } else {
-        if (tiles > 768 && !rounds) return launch_one<QUANT, 4, TOK, 4, 1>(stream, args, n);
-    }
-    return launch_one<QUANT, 3, TOK, TOK <= 16 ? 8 : 4, 1>(stream, args, n);
+    const int tok = T <= 8 ? 8 : T <= 16 ? 16 : T <= 24 ? 24 : T <= 32 ? 32 : 48;
+    // up to 8 tokens activations are cheap: steps of 256 elements keep twice the bytes in flight.  One row tile of long
+    // int8 rows (4096 x 14336: 14.2 against 14.8 us), and every grid of several rounds (nf4 18432 x 4096 17.8 against 19.2 us,
+    // 20480 x 5120 22.0 against 24.7; int8 20480 x 5120 24.2 against 25.4)
+    if (tok == 8 && K % 256 == 0 && (rounds || (quant == kInt8 && tiles <= 256 && K >= 7168))) return {1, tok, 8, 2};
+    if (tiles <= 256) return {1, tok, 8, 1};
+    if (tiles <= 512) return {2, tok, 8, 1};
+    if (tok <= 32 && tiles <= 768) return {3, tok, 8, 1};
+    if (tiles > 768 && !rounds) return {4, tok, tok <= 32 ? 8 : 4, 1};
+    return {3, tok, tok <= 16 ? 8 : 4, 1};
 }
 
-template <int QUANT>
-int launch_quant(hipStream_t stream, const MatmulArgs *args, int n, uint64_t rows) {
-    const uint32_t T = args[0].T;
-    if (T <= 8) return launch_tok<QUANT, 8>(stream, args, n, rows);
-    if (T <= 16) return launch_tok<QUANT, 16>(stream, args, n, rows);
-    if (T <= 24) return launch_tok<QUANT, 24>(stream, args, n, rows);
-    if (T <= 32) return launch_tok<QUANT, 32>(stream, args, n, rows);
-    return launch_tok<QUANT, 48>(stream, args, n, rows);
-}
-
-// Where a workgroup per 16 rows over the whole K is the faster split than the chunk kernel's (measured over the layer shapes of the
+// Where one block is the faster split than the chunk kernel's (measured over the layer shapes of the
 // 0.1B .. 14B models and 128 .. 6144 rows x 896 .. 14336, 5 .. 64 tokens).  With few rows most CUs have no workgroup and a
 // long K is a long chain: there the chunk kernel's split of K over the grid wins, the sooner the more activations a
 // workgroup has to fetch for its rows.
-bool faster(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
+bool one_block_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     if (T <= 8) return quant == kNf4 || rows >= 2048 || K <= 10240;              // int8 1024 rows: K 8192 0.89 of the chunk kernel's time, 14336 1.01
     if (T <= 16) return rows >= 2048 || K <= (quant == kNf4 ? 10240u : 5120u);    // int8 1024 rows: 4096 0.81, 8192 1.07; nf4 0.78, 0.95
     if (T <= 24) return quant == kNf4 || K <= 10240 || (T <= 20 && rows >= 2048); // int8 4096 x 14336 at 19 / 24 tokens 0.92 / 1.04; nf4 0.85
     if (T <= 32) return rows >= 2560 ? quant == kNf4 || K <= 8192 : K <= 4096;    // 2048 x 7168 1.04 (nf4), 1.13 (int8); 4096 x 14336 0.96, 1.18
-    return rows >= 2560 && K <= 8192;                                             // up to 48 tokens: 1.6B / 3B / 7B groups 0.7 .. 0.9, 2048 x 7168 1.02 .. 1.14
+    return T <= 48 && rows >= 2560 && K <= 8192;                                  // 1.6B / 3B / 7B groups 0.7 .. 0.9, 2048 x 7168 1.02 .. 1.14
+}
+
+// Runs of 33 .. 256 tokens in several token blocks: where the smallest tile that gives every workgroup a CU of its own is the chunk
+// kernel's better.  That is single products with few rows (att.output, ffn.value) and the groups of small models; as a share of the chunk
+// kernel's time, int8 / nf4: att.output 1.6B 64 tokens 0.78 / 0.80, 128 0.70 / 0.78, 256 0.79 / 0.81, 7B 64 0.72 / 0.70, 128 0.79 / 0.72, 192 0.81 / 0.85;
+// ffn.value 1.6B 128 tokens 0.90 / 0.74, 3B 128 0.90 / 0.83; attention group 0.4B 128 tokens 0.82 / 0.90, 1.6B 96 0.81 / 0.82.  In two rounds the
+// chunk kernel is the faster one (1.6B attention group int8 192 tokens 1.05, 7B 128 1.14).
+ShortTile several_blocks(Quant quant, const MatmulArgs *args, int n, uint64_t rows, uint32_t K, uint32_t T) {
+    // long K: the chunk kernel splits it over the grid.  2560 x 8960 int8 64 tokens 1.04, 96 0.92; 4096 x 14336 int8 1.07 .. 1.28,
+    // nf4 64 / 96 / 128 tokens 0.96 / 0.85 / 1.04
+    if (T > 256 || K > (quant == kInt8 ? (T > 64 ? 10240u : 8192u) : T <= 96 ? 17920u : 10240u) || (K > 4096 && rows < 2048)) return kNoTile;
+    // padding included: a launch is dealt to the XCDs round-robin, and 256 live workgroups among more are not 32 on each of them
+    // (588 + 548 + 2804 + 1040 rows, 148 tokens, counted without: 1.42 of the chunk kernel's time)
+    auto workgroups = [&](int mrt, int tok) {
+        uint64_t w = 0;
+        for (int i = 0; i < n; i++) w += ((args[i].R + 16 * mrt - 1) / (16 * mrt) + 7) / 8 * 8;
+        return w * ((T + tok - 1) / tok);
+    };
+    constexpr uint64_t kOneRound = 256;
+    constexpr ShortTile int8_tiles[] = {{1, 32, 8, 1}, {2, 32, 8, 1}, {3, 32, 8, 1}, {2, 48, 8, 1}, {4, 32, 8, 1}, {3, 48, 4, 1}, {4, 48, 4, 1}};
+    constexpr ShortTile nf4_tiles[] = {{1, 32, 8, 1}, {1, 48, 8, 1}, {2, 32, 8, 1}, {2, 48, 8, 1}, {3, 32, 8, 1}, {4, 32, 8, 1}, {3, 48, 4, 1}, {4, 48, 4, 1}};
+    const ShortTile *tile = quant == kInt8 ? std::begin(int8_tiles) : std::begin(nf4_tiles), *const end = quant == kInt8 ? std::end(int8_tiles) : std::end(nf4_tiles);
+    for (; tile != end; tile++) // in the order of their size, near ties as measured
+        if (workgroups(tile->mrt, tile->tok) <= kOneRound) break;
+    // four waves instead of eight: long K loses what the wide tile saves (nf4 3036 x 7936, 214 tokens 1.06; 16296 x 9344, 34 tokens 1.16)
+    if (tile != end) return tile->nw == 8 || K <= 5120 ? *tile : kNoTile;
+    // int8, 64 x 64: from 2048 channels on (1.6B group 128 tokens 0.93, 3B and 7B 64 tokens 0.87 .. 0.90; 0.1B 256 tokens 1.08, 8040 x 7936,
+    // 57 tokens 1.20)
+    if (quant == kInt8 && K >= 2048 && K <= 5120 && workgroups(4, 64) <= kOneRound) return {4, 64, 4, 1};
+    // nf4, 64 x 48: two workgroups fit a CU.  Where they fill most of them and the last block is nearly full (3B 96 and 128 tokens 0.73,
+    // 1.6B group 192 tokens 0.79, 7B 96 tokens 0.77; 288 .. 384 workgroups 0.95 .. 1.12, 64 tokens in two blocks 1.05 .. 1.20, K of 256 1.14)
+    const uint64_t w = workgroups(4, 48);
+    if (quant == kNf4 && K >= 1024 && K <= 5120 && w >= 400 && w <= 2 * kOneRound && T * 8 >= (T + 47) / 48 * 48 * 7) return {4, 48, 4, 1};
+    return kNoTile;
+}
+
+template <int QUANT>
+int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTile &t) {
+#define WRQ_SHORT(M, TOK, NW, SUB) \
+    if (t.mrt == M && t.tok == TOK && t.nw == NW && t.sub == SUB) return launch_one<QUANT, M, TOK, NW, SUB>(stream, args, n);
+#define WRQ_SHORT_TOK(TOK) WRQ_SHORT(1, TOK, 8, 1) WRQ_SHORT(2, TOK, 8, 1) WRQ_SHORT(3, TOK, 8, 1) WRQ_SHORT(4, TOK, 8, 1)
+    WRQ_SHORT(1, 8, 8, 2) WRQ_SHORT_TOK(8) WRQ_SHORT_TOK(16) WRQ_SHORT_TOK(24) WRQ_SHORT_TOK(32)
+    WRQ_SHORT(3, 24, 4, 1) WRQ_SHORT(3, 32, 4, 1)
+    WRQ_SHORT(1, 48, 8, 1) WRQ_SHORT(2, 48, 8, 1) WRQ_SHORT(3, 48, 4, 1) WRQ_SHORT(4, 48, 4, 1)
+    if constexpr (QUANT == kInt8) { WRQ_SHORT(4, 64, 4, 1) }
+#undef WRQ_SHORT_TOK
+#undef WRQ_SHORT
+    return fail(WRQ_ERR_UNSUPPORTED, "no short-run kernel for tile (%d, %d, %d, %d)", t.mrt, t.tok, t.nw, t.sub);
 }
 
 } // namespace
@@ -419,17 +470,18 @@ bool faster(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
 // alignments of the chunk kernel) if this kernel is the faster one for them; false leaves them to the caller.
 bool launch_gemm_short(hipStream_t stream, Quant quant, const MatmulArgs *args, int n, int &status) {
     const uint32_t K = args[0].K, T = args[0].T;
-    if (quant == kFp16 || T > 48 || K < 128 || !tune(kTuneGemmShort, 1)) return false;
+    if (quant == kFp16 || T > 256 || K < 128 || !tune(kTuneGemmShort, 1)) return false;
     // a pinned tile of the chunk kernel means that kernel
     if (tune_is_set(kTuneGemmNtile) || tune_is_set(kTuneGemmMrt) || tune_is_set(kTuneGemmKg) || tune_is_set(kTuneGemmKsplit)) return false;
     uint64_t rows = 0;
     for (int i = 0; i < n; i++) {
-        // 32-bit byte offsets into a workgroup's rows and into the activations
-        if (args[i].B != 1 || K > (1u << 24) || ((uint64_t)(T - 1) * args[i].x_token_stride + K) * 2 > 0x7fffffffull) return false;
+        // 32-bit byte offsets into a workgroup's rows and into the activations of its tokens
+        if (args[i].B != 1 || K > (1u << 24) || ((uint64_t)((T < 64 ? T : 64) - 1) * args[i].x_token_stride + K) * 2 > 0x7fffffffull) return false;
         rows += args[i].R;
     }
-    if (!faster(quant, rows, K, T)) return false;
-    status = quant == kNf4 ? launch_quant<kNf4>(stream, args, n, rows) : launch_quant<kInt8>(stream, args, n, rows);
+    const ShortTile t = one_block_pays(quant, rows, K, T) ? one_block(quant, rows, K, T) : T > 32 ? several_blocks(quant, args, n, rows, K, T) : kNoTile;
+    if (!t.mrt) return false;
+    status = quant == kNf4 ? launch_tile<kNf4>(stream, args, n, t) : launch_tile<kInt8>(stream, args, n, t);
     return true;
 }
 
