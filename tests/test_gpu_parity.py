@@ -775,6 +775,27 @@ def test_short_run_kernel(gpu, oracle, kind, T, overrides):
 
 
 @pytest.mark.parametrize("kind", ["int8", "nf4"])
+@pytest.mark.parametrize("T", [2, 3, 4], ids=str)
+def test_decode_runs_on_the_short_run_kernel(gpu, oracle, kind, T):
+    # runs of 2 .. 4 tokens either side of the rule that sends them to the matrix cores: few and many rows, short and long K, whole
+    # steps of 1024, and a group of products whose K differ (which stays on the decode kernels as a whole)
+    import torch
+
+    announce("decode runs", kind, T)
+    rng = np.random.default_rng(SEED + 93 + T)
+    for shapes in ([(128, 4)], [(896, 1028)], [(1024, 4096)], [(1152, 1000), (1152, 24)], [(2560, 132)], [(2560, 1024)], [(2688, 2560)], [(768, 516), (1024, 4096)]):
+        ops, want = [], []
+        for K, R in shapes:
+            wp, scale, wdeq = pack(oracle, kind, gen_f16(rng, (R, K), 0.02))
+            x = gen_f16(rng, (T, K), 1.0)
+            ops.append((gpu_matrix(gpu, kind, wp, scale), dev(x), torch.full((T, R), float("nan"), dtype=torch.float32, device="cuda"), 0, False, {}))
+            want.append(truth_matmul(wdeq, x))
+        gpu.matmul_vec_group(ops)
+        for op, truth in zip(ops, want):
+            assert_close(host(op[2]), truth, 3e-4, f"{kind} T={T} {shapes} vs float64")
+
+
+@pytest.mark.parametrize("kind", ["int8", "nf4"])
 @pytest.mark.parametrize("T", [33, 49, 64, 65, 97, 192, 255, 256], ids=str)
 def test_short_run_kernel_in_token_blocks(gpu, oracle, kind, T, overrides):
     # the same kernel over several blocks of 32, 48 or 64 tokens, the last one partly filled: tiles of one to four times 16 rows, row

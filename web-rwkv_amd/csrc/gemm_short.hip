@@ -466,6 +466,24 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 
 } // namespace
 
+// Decode runs of 2 .. 4 tokens: where this kernel is faster than the decode kernels, which share a pass of the vector ALU between the
+// tokens.  Those are at their best for int8 where whole waves own rows (K a multiple of 1024) and anywhere with long K and few rows.  Their
+// time against this kernel's as 1, 600 drawn launches and the model shapes: int8, K < 1024: 2 tokens 0.84 .. 0.99, 3 and 4 0.59 .. 0.75;
+// K up to 2560 from 1024 rows on, up to 10240 from 2560 rows on, 3 and 4 tokens 0.49 .. 0.85 (fewer rows 0.83 .. 1.6, beyond 10240 0.78 .. 1.7); whole waves,
+// 4 tokens from 4096 rows on 0.75 .. 1.0, otherwise 0.95 .. 1.35.  nf4, K up to 1024: 2 tokens 0.66 .. 0.99, 3 0.52 .. 0.71; K up to 2560 0.67 .. 1.0
+// (2 tokens: 9216 x 2048 1.06); K up to 5120 from 1024 rows on, 3 tokens, 0.69 .. 0.98, 2 tokens 0.84 .. 1.07; longer K 0.9 .. 1.8.
+bool short_run_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
+    if (T < 2 || T > 4 || K % 128 || !tune(kTuneGemmShort, 1)) return false;
+    if (quant == kInt8) {
+        if (K % 1024 == 0) return T == 4 && rows >= 4096;
+        if (T == 2) return K < 1024 && rows <= 8192; // 16428 x 512 1.39
+        return K < 1024 || (K <= 2560 ? rows >= 1024 : K <= 10240 && rows >= 2560);
+    }
+    if (quant != kNf4) return false;
+    if (T == 2) return K <= 1024 || (K <= 2560 && rows >= 1024 && rows <= 8192);
+    return K <= 2560 || (K <= 5120 && rows >= 1024);
+}
+
 // Takes the `n` products of a launch (one K and token count, f16 activations, one batch, K % 128 == 0 and the
 // alignments of the chunk kernel) if this kernel is the faster one for them; false leaves them to the caller.
 bool launch_gemm_short(hipStream_t stream, Quant quant, const MatmulArgs *args, int n, int &status) {

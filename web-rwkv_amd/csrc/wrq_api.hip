@@ -173,6 +173,7 @@ struct Prepared {
     MatmulArgs a;
     int in_f16;
     bool mfma; // route to the matrix-core kernel
+    bool decode_mfma; // a decode run that could take it: `decode_run` decides over all products of its launch
 };
 
 int prepare(Entry entry, Quant quant, const void *w, const Shape4 &mshape, const wrq_tensor *scale,
@@ -252,7 +253,18 @@ int prepare(Entry entry, Quant quant, const void *w, const Shape4 &mshape, const
     const bool chunk = entry == kMat ? true : n >= (in_f16 ? chunk_min_t : (uint64_t)16);
     out.in_f16 = in_f16;
     out.mfma = chunk && mfma_ok;
+    out.decode_mfma = !chunk && mfma_ok && in_f16 && b == 1 && !tune_is_set(kTuneVecChunkMinT);
     return WRQ_OK;
+}
+
+// Whether `n` decode products that share a launch go to the matrix cores after all.
+bool decode_run(Quant quant, const Prepared *ops, int n) {
+    uint64_t rows = 0;
+    for (int i = 0; i < n; i++) {
+        if (!ops[i].decode_mfma || ops[i].a.K != ops[0].a.K) return false;
+        rows += ops[i].a.R;
+    }
+    return short_run_pays(quant, rows, ops[0].a.K, ops[0].a.T);
 }
 
 int launch_vec(hipStream_t stream, Quant quant, const Prepared &p) {
@@ -269,7 +281,7 @@ int matmul(hipStream_t stream, Entry entry, Quant quant, const void *w, const Sh
            const wrq_tensor_view *output, int act, bool noalloc = false) {
     Prepared p;
     WRQ_TRY(prepare(entry, quant, w, mshape, scale, table, input, output, act, p));
-    if (p.mfma) return launch_chunk(stream, quant, p, noalloc);
+    if (p.mfma || decode_run(quant, &p, 1)) return launch_chunk(stream, quant, p, noalloc);
     return launch_vec(stream, quant, p);
 }
 
@@ -286,7 +298,7 @@ int dispatch_group(hipStream_t stream, Quant quant, const Prepared *ops, int n) 
             run[m] = ops[i + m].a;
             m++;
         }
-        if (ops[i].mfma && ops[i].a.K != 0)
+        if ((ops[i].mfma && ops[i].a.K != 0) || decode_run(quant, ops + i, m))
             WRQ_TRY(launch_gemm_group(stream, quant, ops[i].in_f16, run, m));
         else
             WRQ_TRY(launch_gemv_group(stream, quant, ops[i].in_f16, run, m));
