@@ -472,6 +472,9 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 // K up to 2560 from 1024 rows on, up to 10240 from 2560 rows on, 3 and 4 tokens 0.49 .. 0.85 (fewer rows 0.83 .. 1.6, beyond 10240 0.78 .. 1.7); whole waves,
 // 4 tokens from 4096 rows on 0.75 .. 1.0, otherwise 0.95 .. 1.35.  nf4, K up to 1024: 2 tokens 0.66 .. 0.99, 3 0.52 .. 0.71; K up to 2560 0.67 .. 1.0
 // (2 tokens: 9216 x 2048 1.06); K up to 5120 from 1024 rows on, 3 tokens, 0.69 .. 0.98, 2 tokens 0.84 .. 1.07; longer K 0.9 .. 1.8.
+// nf4 runs of 4 tokens through these entries are on the matrix cores anyway, so their launches were compared with the chunk kernel.
+// Four products of K x K in one launch, before and now, us: int8 K 2560 3 tokens 10.7 -> 7.6, 4 tokens 10.7 -> 7.7; K 4096 4 tokens
+// 15.9 -> 13.8; nf4 K 2048 2 tokens 6.5 -> 6.2, 3 tokens 7.7 -> 6.1; K 2560 3 tokens 11.8 -> 8.5; K 4096 3 tokens 17.0 -> 14.6.
 bool short_run_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     if (T < 2 || T > 4 || K % 128 || !tune(kTuneGemmShort, 1)) return false;
     if (quant == kInt8) {
