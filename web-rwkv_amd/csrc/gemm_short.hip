@@ -404,11 +404,25 @@ ShortTile one_block(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     return {3, tok, tok <= 16 ? 8 : 4, 1};
 }
 
+// Most rows for which one block was measured the faster one: with more, its workgroups come in rounds that each begin with the
+// latency of a whole K, while the chunk kernel's wide tiles read the activations less often.  Share of the chunk kernel's time, single
+// products of 16384 .. 65536 rows, K of 768 .. 5120: int8 up to 8 tokens, K 1024: 20480 rows 0.97, 24576 1.06, 65536 1.45; K 2560 and more: 49152 rows
+// 0.73 .. 0.88, 65536 up to 1.08; 9 .. 48 tokens, K from 2048: 24576 rows 0.79 .. 0.97, 32768 0.90 .. 1.26, 65536 up to 1.7.  nf4 up to 8 tokens, K below
+// 2048: 16384 rows 0.83 .. 0.86, 20480 1.02 .. 1.10; up to 16 tokens otherwise: 49152 rows 0.61 .. 0.87, 65536 up to 1.04; up to 48 tokens: 24576 rows
+// 0.58 .. 0.88, 32768 0.82 .. 1.19, 65536 1.06 .. 1.35.
+uint64_t one_block_rows(Quant quant, uint32_t K, uint32_t T) {
+    if (K < 512) return 16384; // K 256: int8 16620 rows, 5 tokens 1.05; nf4 29128 rows, 11 tokens 1.21
+    if (quant == kNf4) return T > 16 ? 24576 : K < (T <= 8 ? 2048 : 768) ? 16384 : 49152;
+    if (K < 2048) return T > 32 && K < 1024 ? 16384 : 20480; // 18664 x 512, 39 tokens 1.07
+    return T <= 8 && K >= 2560 ? 49152 : 24576;
+}
+
 // Where one block is the faster split than the chunk kernel's (measured over the layer shapes of the
 // 0.1B .. 14B models and 128 .. 6144 rows x 896 .. 14336, 5 .. 64 tokens).  With few rows most CUs have no workgroup and a
 // long K is a long chain: there the chunk kernel's split of K over the grid wins, the sooner the more activations a
 // workgroup has to fetch for its rows.
 bool one_block_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
+    if (rows > one_block_rows(quant, K, T)) return false;
     if (T <= 8) return quant == kNf4 || rows >= 2048 || K <= 10240;              // int8 1024 rows: K 8192 0.89 of the chunk kernel's time, 14336 1.01
     if (T <= 16) return rows >= 2048 || K <= (quant == kNf4 ? 10240u : 5120u);    // int8 1024 rows: 4096 0.81, 8192 1.07; nf4 0.78, 0.95
     if (T <= 24) return quant == kNf4 || K <= 10240 || (T <= 20 && rows >= 2048); // int8 4096 x 14336 at 19 / 24 tokens 0.92 / 1.04; nf4 0.85
@@ -444,9 +458,9 @@ ShortTile several_blocks(Quant quant, const MatmulArgs *args, int n, uint64_t ro
     // 57 tokens 1.20)
     if (quant == kInt8 && K >= 2048 && K <= 5120 && workgroups(4, 64) <= kOneRound) return {4, 64, 4, 1};
     // nf4, 64 x 48: two workgroups fit a CU.  Where they fill most of them and the last block is nearly full (3B 96 and 128 tokens 0.73,
-    // 1.6B group 192 tokens 0.79, 7B 96 tokens 0.77; 288 .. 384 workgroups 0.95 .. 1.12, 64 tokens in two blocks 1.05 .. 1.20, K of 256 1.14)
+    // 1.6B group 192 tokens 0.79, 7B 96 tokens 0.77; one block, 32768 rows, 0.82 .. 0.99, K of 5120 1.03; 288 .. 384 workgroups 0.95 .. 1.12, 64 tokens in two blocks 1.05 .. 1.20, K of 256 1.14)
     const uint64_t w = workgroups(4, 48);
-    if (quant == kNf4 && K >= 1024 && K <= 5120 && w >= 400 && w <= 2 * kOneRound && T * 8 >= (T + 47) / 48 * 48 * 7) return {4, 48, 4, 1};
+    if (quant == kNf4 && K >= 1024 && K <= (T > 48 ? 5120 : 4096) && w >= 400 && w <= 2 * kOneRound && T * 8 >= (T + 47) / 48 * 48 * 7) return {4, 48, 4, 1};
     return kNoTile;
 }
 
@@ -472,15 +486,19 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 // K up to 2560 from 1024 rows on, up to 10240 from 2560 rows on, 3 and 4 tokens 0.49 .. 0.85 (fewer rows 0.83 .. 1.6, beyond 10240 0.78 .. 1.7); whole waves,
 // 4 tokens from 4096 rows on 0.75 .. 1.0, otherwise 0.95 .. 1.35.  nf4, K up to 1024: 2 tokens 0.66 .. 0.99, 3 0.52 .. 0.71; K up to 2560 0.67 .. 1.0
 // (2 tokens: 9216 x 2048 1.06); K up to 5120 from 1024 rows on, 3 tokens, 0.69 .. 0.98, 2 tokens 0.84 .. 1.07; longer K 0.9 .. 1.8.
+// Many rows, single products: int8, 4 tokens, K 1024: 16384 rows 0.88, 20480 1.12, 65536 1.23; K 2048: 20480 1.01, 32768 1.07; K 4096 and 5120 up to 65536 rows
+// 0.83 .. 0.98; K 768, 3 and 4 tokens: 20480 rows 0.87, 65536 1.00; K 2560 up to 65536 rows 0.64 .. 0.76.  nf4, K 1024, 2 tokens: 16384 rows 0.83, 20480 1.03,
+// 65536 1.11; 3 tokens, K of 768 .. 5120, up to 65536 rows 0.58 .. 0.97, but K 1792 19092 rows 1.08, 24876 1.16.
 // nf4 runs of 4 tokens through these entries are on the matrix cores anyway, so their launches were compared with the chunk kernel.
 // Four products of K x K in one launch, before and now, us: int8 K 2560 3 tokens 10.7 -> 7.6, 4 tokens 10.7 -> 7.7; K 4096 4 tokens
 // 15.9 -> 13.8; nf4 K 2048 2 tokens 6.5 -> 6.2, 3 tokens 7.7 -> 6.1; K 2560 3 tokens 11.8 -> 8.5; K 4096 3 tokens 17.0 -> 14.6.
 bool short_run_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
-    if (T < 2 || T > 4 || K % 128 || !tune(kTuneGemmShort, 1)) return false;
+    // what `launch_gemm_short` would hand on to the chunk kernel stays on the decode kernels
+    if (T < 2 || T > 4 || K % 128 || rows > one_block_rows(quant, K, T) || !tune(kTuneGemmShort, 1)) return false;
     if (quant == kInt8) {
-        if (K % 1024 == 0) return T == 4 && rows >= 4096;
-        if (T == 2) return K < 1024 && rows <= 8192; // 16428 x 512 1.39
-        return K < 1024 || (K <= 2560 ? rows >= 1024 : K <= 10240 && rows >= 2560);
+        if (K % 1024 == 0) return T == 4 && rows >= 4096 && rows <= (K < 2048 ? 16384 : K < 4096 ? 20480 : 49152);
+        if (K < 1024) return T > 2 || rows <= 8192; // 2 tokens, 16428 x 512 1.39
+        return T > 2 && (K <= 2560 ? rows >= 1024 : K <= 10240 && rows >= 2560);
     }
     if (quant != kNf4) return false;
     if (T == 2) return K <= 1024 || (K <= 2560 && rows >= 1024 && rows <= 8192);
