@@ -4,6 +4,8 @@
 // out[t, r] = ACT( sum_k deq(W[r, k]) * x[t, k] )      (src/shaders/matmul_mat_int8.wgsl:62-153,
 //                                                        src/shaders/matmul_mat_nf4.wgsl:94-220)
 //
+// Runs of up to 48 tokens and small products up to 256 mostly take the kernel of gemm_short.hip; its rules are there.
+//
 // The shapes of this path are skinny: 16..256 tokens against thousands of weight rows, so
 // even the chunk products are bound by streaming the packed weights once (below ~100
 // tokens) or sit close to that point.  The decomposition follows from it:
