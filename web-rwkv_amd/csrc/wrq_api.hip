@@ -236,9 +236,10 @@ int prepare(Entry entry, Quant quant, const void *w, const Shape4 &mshape, const
 
     // Matrix cores need K in whole 128-steps, 16-byte activation rows and output quads on
     // their natural alignment; everything else runs on the VALU kernels, which accept
-    // every shape the reference accepts.
+    // every shape the reference accepts.  A product over no elements at all is the VALU kernels' too: the chunk kernel
+    // divides by its K steps.
     const size_t xs = in_f16 ? 2 : 4, osz = a.out_f16 ? 2 : 4;
-    const bool mfma_ok = (k % 128 == 0) && ((uintptr_t)a.w % 16 == 0) && ((uintptr_t)a.x % 16 == 0) &&
+    const bool mfma_ok = (k > 0) && (k % 128 == 0) && ((uintptr_t)a.w % 16 == 0) && ((uintptr_t)a.x % 16 == 0) &&
                          ((a.x_token_stride * xs) % 16 == 0) && ((a.x_batch_stride * xs) % 16 == 0) &&
                          ((uintptr_t)a.out % (4 * osz) == 0) && ((a.out_token_stride * osz) % (4 * osz) == 0) &&
                          ((a.out_batch_stride * osz) % (4 * osz) == 0);
@@ -272,7 +273,6 @@ int launch_vec(hipStream_t stream, Quant quant, const Prepared &p) {
 }
 
 int launch_chunk(hipStream_t stream, Quant quant, const Prepared &p, bool noalloc) {
-    if (p.a.K == 0) return launch_vec(stream, quant, p); // nothing to stream: plain zeros through the generic kernel
     return noalloc ? launch_gemm_noalloc(stream, quant, p.in_f16, p.a) : launch_gemm(stream, quant, p.in_f16, p.a);
 }
 
@@ -298,7 +298,7 @@ int dispatch_group(hipStream_t stream, Quant quant, const Prepared *ops, int n) 
             run[m] = ops[i + m].a;
             m++;
         }
-        if ((ops[i].mfma && ops[i].a.K != 0) || decode_run(quant, ops + i, m))
+        if (ops[i].mfma || decode_run(quant, ops + i, m))
             WRQ_TRY(launch_gemm_group(stream, quant, ops[i].in_f16, run, m));
         else
             WRQ_TRY(launch_gemv_group(stream, quant, ops[i].in_f16, run, m));
