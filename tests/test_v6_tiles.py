@@ -88,6 +88,26 @@ def test_gpu_adapters_in_lines(gpu, C, A):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C", [2112, 2144, 2528, 2592, 4256, 4320, 5088, 5184, 5216])
+@pytest.mark.parametrize("A", [1, 33])
+def test_gpu_adapters_in_gathered(gpu, C, A):
+    """First halves of adapters over channels in no whole steps of 128, either side of the lines between their three forms: one round of
+    eight or ten steps per wave, more, sixteen waves."""
+    import torch
+
+    print("adapters_in gathered on the GPU", C, A, flush=True)
+    g = torch.Generator().manual_seed(0x575B + C + A)
+    h = lambda *s: (torch.randn(s, generator=g) * 0.05).half()
+    ops = [(h(r, C), h(A, C), torch.empty((A, r), dtype=torch.float16, device="cuda"), act) for r, act in ((48, gpu.ACT_NONE), (16, gpu.ACT_SIGMOID))]
+    gpu.FusedV7.adapters_in(C, A, [(w.cuda(), x.cuda(), out, act) for w, x, out, act in ops])
+    for w, x, out, act in ops:
+        want = x.double() @ w.double().t()
+        want = torch.sigmoid(want) if act == gpu.ACT_SIGMOID else want
+        # f32 sums of up to 5216 products of 2.5e-3 each, one rounding to f16 (2^-11) of values below 1
+        assert_close(out.cpu().numpy(), want.numpy(), 1e-3, "adapters_in vs float64")
+
+
+@pytest.mark.gpu
 def test_gpu_pre_of_one_token_in_place(gpu):
     """A single token has no neighbour that reads its row: normalised in place as into a buffer of its own."""
     import torch

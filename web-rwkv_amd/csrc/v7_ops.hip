@@ -441,7 +441,13 @@ int wrq_adapters_in(wrq_stream stream, uint32_t C, uint32_t A, int n, const void
     // Eight waves, two steps each in flight: 2048 channels in one go.  us, gathered -> line-wise: 160 rows x 100 tokens over 768 / 2048 / 4096 / 5120
     // channels 6.5 / 6.5 / 10.3 / 12.0 -> 3.7 / 4.5 / 6.0 / 6.9; four adapters of a v7 layer, 32 tokens, 6.3 / 6.5 / 10.2 / 12.0 -> 3.5 / 4.5 /
     // 5.8 / 6.8.  Sixteen waves of one step 3.7 / 4.5 / 6.1 / 7.3, four of four 4.0 / 5.3 / 7.7 / 8.8.
+    // Gathered, steps of 32: eight waves of eight steps, where their rounds are full.  A second round that would hold less than a quarter of the steps goes into
+    // the first one with ten steps, a third one with sixteen waves of ten.  160 rows x 100 tokens, us, eight of eight / the other: 2112 channels 7.2 / 7.4,
+    // 2144 6.4 / 6.3, 2240 8.8 / 7.4, 2496 10.1 / 7.4; 4256 9.3 / 9.4, 4320 9.7 / 9.4, 4672 13.5 / 11.7, 5184 13.4 / 12.7, 6112 10.8 / 16.0, 8160 13.2 / 15.8.
+    const uint32_t steps = C / 32;
     if (C % 128 == 0) go(adapters_in_kernel<8, 2, true>, 8);
+    else if (steps >= 67 && steps <= 80) go(adapters_in_kernel<8, 10, false>, 8);
+    else if (steps >= 135 && steps <= 162) go(adapters_in_kernel<16, 10, false>, 16);
     else go(adapters_in_kernel<8, 8, false>, 8);
     return check_launch(what);
 }
