@@ -121,6 +121,19 @@ def dispatch_layer(layer, buf, state, cursors, A, H, S, rescale_now=False):
         LayerOp.affine(buf.x, 0.5, 0.0)
 
 
+def adapters_in_tiles(C, A):
+    """Whether the first half of an adapter over C channels and A tokens is a launch of small tiles (`wrq_adapters_in`) or the f16
+    product, which is a one-shot kernel up to 4 tokens (2.5 us at 2048 and 4096 channels, one token)."""
+    # us, tiles / product, 160 rows: 768 channels 3.6 / 6.0 at 16 tokens; 1024 channels 3.7 / 8.1 at 5; 3072 channels 5.2 / 8.9 at 5,
+    # 5.7 / 10.8 at 100; 4096 channels 5.9 / 8.5 at 5, 6.4 / 10.0 at 100; 5120 channels 6.7 / 9.2 at 5, 7.4 / 11.6 at 100, 7.8 / 13.6 at 255
+    if C % 128 == 0:
+        return A > 4
+    # Channels in no whole steps of 128 are gathered: 832 channels 5.4 / 3.6 at 8 tokens; 2112 channels 5.9 / 6.2 at 5, 7.3 / 9.8 at 256.  Beyond 2560 they
+    # take more rounds: 2624 channels 8.9 / 3.9 at 8, 10.2 / 6.0 at 100, 10.2 / 9.7 at 224, 10.3 / 14.2 at 255; 4672 channels 10.1 / 4.4, 11.8 / 7.8, 11.8 /
+    # 12.8, 11.8 / 18.2; at 512 tokens 17.2 / 17.4 and 21.9 / 24.6
+    return A > (224 if C > 2560 else 4 if C >= 1024 else 16)
+
+
 def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False, checked=False):
     """The same layer in 12 launches: the 8 quantized products (3 launches for the independent ones, 2
     alone), the first halves of the two adapters, and 5 fused launches for the 27 small ops
@@ -134,11 +147,7 @@ def dispatch_layer_fused(layer, buf, state, cursors, A, H, S, rescale_now=False,
     ffn_state = ((C, 1, B), (C, S + 2, B), (0, S + 1, 0))
     slice_of = lambda i: ((C, A, 1), (C, A, 5), (0, 0, i))
 
-    # First half of an adapter: the launch of small tiles, or the f16 product up to 4 tokens, where that is a one-shot kernel (2.5 us
-    # at 2048 and 4096 channels, one token).  us, tiles / product, 160 rows: 768 channels 3.6 / 6.0 at 16 tokens; 1024 channels 3.7 / 8.1 at 5;
-    # 3072 channels 5.2 / 8.9 at 5, 5.7 / 10.8 at 100; 4096 channels 5.9 / 8.5 at 5, 6.4 / 10.0 at 100; 5120 channels 6.7 / 9.2 at 5,
-    # 7.4 / 11.6 at 100, 7.8 / 13.6 at 255.  Channels in no whole steps of 128 are gathered: below 1024 the product keeps runs up to 16 tokens.
-    tiles = A > (4 if C % 128 == 0 or C >= 1024 else 16)
+    tiles = adapters_in_tiles(C, A)
 
     def adapter_in(name, x, out):
         if tiles:
