@@ -44,7 +44,7 @@ extern "C" {
 #define WRQ_ABI_VERSION 1
 /* Counts additions that leave every existing signature as it is (new entry points, new override keys);
  * a binding built against minor m runs on any library of the same WRQ_ABI_VERSION with minor >= m. */
-#define WRQ_ABI_MINOR 4
+#define WRQ_ABI_MINOR 5
 #define WRQ_INT8_BLOCK_SIZE 128u /* TensorOp::INT8_BLOCK_SIZE, src/tensor/ops.rs:292 */
 #define WRQ_NF4_BLOCK_SIZE 64u   /* TensorOp::NF4_BLOCK_SIZE, src/tensor/ops.rs:291 */
 
@@ -130,6 +130,15 @@ int wrq_debug_override(const char *key, int value);
  * product kernels carry no stamp code; `python3 bench.py --stamps` prints the timeline of a decode step.
  */
 int wrq_debug_stamps(void *buffer, uint64_t bytes);
+
+/*
+ * Test and sweep hook; no counterpart in the reference.  The kernel that `count` products of `rows[i]` rows over
+ * K elements and T tokens of f16 activations would share a launch of: 0 the decode kernels, 1 the chunk kernel, otherwise the
+ * short-run kernel with its tile, row tiles of 16 | tokens << 8 | waves << 16 | pieces of 128 elements per step << 24; -1 if
+ * the products are refused.  `nf4` 0: int8; `mat` 1: wrq_matmul_mat_* (one product), 0: wrq_matmul_vec_* and their groups;
+ * `x_token_stride` in elements.  Nothing is launched and no device is needed; overrides count as for a launch.
+ */
+int wrq_debug_route(int nf4, int mat, int count, const uint32_t *rows, uint32_t K, uint32_t T, uint32_t x_token_stride);
 
 int wrq_abi_version(void);
 int wrq_abi_minor(void); /* WRQ_ABI_MINOR of the loaded library */

@@ -1,0 +1,44 @@
+"""Which kernel a product runs on (no GPU needed): the rules that share launches out between the decode, short-run and chunk kernels
+have to agree with one another and with the overrides."""
+import random
+
+import pytest
+
+KINDS = ["int8", "nf4"]
+SHAPES = {"int8": ([4096] * 4, 4096, 4), "nf4": ([2048] * 4, 2048, 3)}  # products that the short-run kernel takes from the decode kernels
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_route_of_a_refused_product(wrq, kind):
+    with pytest.raises(ValueError, match="multiple of 4"):
+        wrq.debug_route(kind, 1022, 1024, 3)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_decode_runs_leave_for_the_short_run_kernel_only(wrq, kind):
+    # what that kernel does not take has to stay on the decode kernels, not to end on the chunk kernel
+    rows, K, T = SHAPES[kind]
+    assert isinstance(wrq.debug_route(kind, rows, K, T), tuple)
+    stride = (1 << 30) // (T - 1) + 8 & ~7  # a token's row more than 2 GiB behind the first one's: beyond its 32-bit offsets
+    assert wrq.debug_route(kind, rows, K, T, x_token_stride=stride) == "decode"
+    assert wrq.debug_route(kind, rows, K, T, x_token_stride=stride // 2 & ~7) != "decode"
+    for K in (1 << 24, (1 << 24) + 1024, 0):
+        for T in (1, 2, 3, 4):
+            for rows in (4, 4096):
+                assert wrq.debug_route(kind, rows, K, T) != "chunk" or (kind, T) == ("nf4", 4), (rows, K, T)
+    rng = random.Random(5)
+    for _ in range(2000):  # nf4 runs of 4 tokens are the matrix cores' in any case
+        rows, K, T = [4 * rng.randint(1, int(2 ** rng.uniform(0, 14))) for _ in range(rng.randint(1, 8))], 128 * rng.randint(1, int(2 ** rng.uniform(0, 8))), rng.randint(2, 4)
+        assert wrq.debug_route(kind, rows, K, T) != "chunk" or (kind, T) == ("nf4", 4), (rows, K, T)
+    assert wrq.debug_route("int8", 4096, (1 << 24) + 1024, 4) == "decode"
+    assert wrq.debug_route(kind, 4096, 0, 5) == "decode"
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("key,value", [("gemm_ntile", 1), ("gemm_mrt", 2), ("gemm_kg", 2), ("gemm_ksplit", 1), ("gemm_short", 0)])
+def test_pinned_chunk_tiles_leave_decode_runs_alone(wrq, overrides, kind, key, value):
+    rows, K, T = SHAPES[kind]
+    assert isinstance(wrq.debug_route(kind, rows, K, 16), tuple)
+    overrides(**{key: value})
+    assert wrq.debug_route(kind, rows, K, T) == "decode"
+    assert wrq.debug_route(kind, rows, K, 16) == "chunk"

@@ -40,6 +40,7 @@ EXPORTS = [
     "wrq_init", "wrq_abi_version", "wrq_abi_minor", "wrq_status_string", "wrq_last_error",
     "wrq_debug_override",
     "wrq_debug_stamps",
+    "wrq_debug_route",
     "wrq_quantize_mat_int8", "wrq_quantize_mat_nf4",
     "wrq_matmul_vec_int8", "wrq_matmul_vec_nf4", "wrq_matmul_mat_int8", "wrq_matmul_mat_nf4", "wrq_matmul_mat_int8_noalloc",
     "wrq_matmul_vec_int8_group", "wrq_matmul_vec_nf4_group",
@@ -184,6 +185,7 @@ def lib():
         L.wrq_last_error.restype = C.c_char_p
         L.wrq_debug_override.argtypes = [C.c_char_p, i]
         L.wrq_debug_stamps.argtypes = [vp, C.c_uint64]
+        L.wrq_debug_route.argtypes = [i, i, i, C.POINTER(C.c_uint32), C.c_uint32, C.c_uint32, C.c_uint32]
         L.wrq_quantize_mat_int8.argtypes = [vp, T, T, T]
         L.wrq_quantize_mat_nf4.argtypes = [vp, T, T, T, T]
         L.wrq_matmul_vec_int8.argtypes = [vp, T, T, V, V, i, i]
@@ -264,6 +266,16 @@ def _packed():
 def debug_override(key, value=-1):
     """``wrq_debug_override``: pin (value >= 0) or release (value < 0) one kernel / tile choice."""
     _check(lib().wrq_debug_override(key.encode(), int(value)))
+
+
+def debug_route(kind, rows, K, T, mat=False, x_token_stride=None):
+    """``wrq_debug_route``: the kernel that products of ``rows`` (one number, or one per product of a launch) would run on, ``"decode"``,
+    ``"chunk"`` or the short-run kernel's tile (row tiles of 16, tokens, waves, pieces of 128 elements per step).  ``kind``: "int8", "nf4"."""
+    rows = (rows,) if isinstance(rows, int) else tuple(rows)
+    r = lib().wrq_debug_route(int(kind == "nf4"), int(mat), len(rows), (C.c_uint32 * len(rows))(*rows), K, T, K if x_token_stride is None else x_token_stride)
+    if r < 0:
+        raise ValueError(lib().wrq_last_error().decode())
+    return ("decode", "chunk")[r] if r < 2 else (r & 255, r >> 8 & 255, r >> 16 & 255, r >> 24)
 
 
 def _check(status):

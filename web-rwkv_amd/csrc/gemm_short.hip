@@ -464,6 +464,25 @@ ShortTile several_blocks(Quant quant, const MatmulArgs *args, int n, uint64_t ro
     return kNoTile;
 }
 
+uint64_t rows_of(const MatmulArgs *args, int n) {
+    uint64_t rows = 0;
+    for (int i = 0; i < n; i++) rows += args[i].R;
+    return rows;
+}
+
+// The tile of a launch, kNoTile where the chunk kernel takes it: the one place that decides.
+ShortTile short_tile(Quant quant, const MatmulArgs *args, int n) {
+    const uint32_t K = args[0].K, T = args[0].T;
+    if (quant == kFp16 || T > 256 || K < 128 || !tune(kTuneGemmShort, 1)) return kNoTile;
+    // a pinned tile of the chunk kernel means that kernel
+    if (tune_is_set(kTuneGemmNtile) || tune_is_set(kTuneGemmMrt) || tune_is_set(kTuneGemmKg) || tune_is_set(kTuneGemmKsplit)) return kNoTile;
+    // 32-bit byte offsets into a workgroup's rows and into the activations of its tokens
+    for (int i = 0; i < n; i++)
+        if (args[i].B != 1 || K > (1u << 24) || ((uint64_t)((T < 64 ? T : 64) - 1) * args[i].x_token_stride + K) * 2 > 0x7fffffffull) return kNoTile;
+    const uint64_t rows = rows_of(args, n);
+    return one_block_pays(quant, rows, K, T) ? one_block(quant, rows, K, T) : T > 32 ? several_blocks(quant, args, n, rows, K, T) : kNoTile;
+}
+
 template <int QUANT>
 int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTile &t) {
 #define WRQ_SHORT(M, TOK, NW, SUB) \
@@ -492,33 +511,28 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 // nf4 runs of 4 tokens through these entries are on the matrix cores anyway, so their launches were compared with the chunk kernel.
 // Four products of K x K in one launch, before and now, us: int8 K 2560 3 tokens 10.7 -> 7.6, 4 tokens 10.7 -> 7.7; K 4096 4 tokens
 // 15.9 -> 13.8; nf4 K 2048 2 tokens 6.5 -> 6.2, 3 tokens 7.7 -> 6.1; K 2560 3 tokens 11.8 -> 8.5; K 4096 3 tokens 17.0 -> 14.6.
-bool short_run_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
-    // what `launch_gemm_short` would hand on to the chunk kernel stays on the decode kernels
-    if (T < 2 || T > 4 || K % 128 || rows > one_block_rows(quant, K, T) || !tune(kTuneGemmShort, 1)) return false;
+bool short_run_pays(Quant quant, const MatmulArgs *args, int n) {
+    const uint32_t K = args[0].K, T = args[0].T;
+    if (T < 2 || T > 4 || !short_tile(quant, args, n).mrt) return false; // what `launch_gemm_short` hands on stays on the decode kernels
+    const uint64_t rows = rows_of(args, n);
     if (quant == kInt8) {
         if (K % 1024 == 0) return T == 4 && rows >= 4096 && rows <= (K < 2048 ? 16384 : K < 4096 ? 20480 : 49152);
         if (K < 1024) return T > 2 || rows <= 8192; // 2 tokens, 16428 x 512 1.39
         return T > 2 && (K <= 2560 ? rows >= 1024 : K <= 10240 && rows >= 2560);
     }
-    if (quant != kNf4) return false;
     if (T == 2) return K <= 1024 || (K <= 2560 && rows >= 1024 && rows <= 8192);
     return K <= 2560 || (K <= 5120 && rows >= 1024);
+}
+
+uint32_t short_run_tile(Quant quant, const MatmulArgs *args, int n) {
+    const ShortTile t = short_tile(quant, args, n);
+    return (uint32_t)(t.mrt | t.tok << 8 | t.nw << 16 | t.sub << 24);
 }
 
 // Takes the `n` products of a launch (one K and token count, f16 activations, one batch, K % 128 == 0 and the
 // alignments of the chunk kernel) if this kernel is the faster one for them; false leaves them to the caller.
 bool launch_gemm_short(hipStream_t stream, Quant quant, const MatmulArgs *args, int n, int &status) {
-    const uint32_t K = args[0].K, T = args[0].T;
-    if (quant == kFp16 || T > 256 || K < 128 || !tune(kTuneGemmShort, 1)) return false;
-    // a pinned tile of the chunk kernel means that kernel
-    if (tune_is_set(kTuneGemmNtile) || tune_is_set(kTuneGemmMrt) || tune_is_set(kTuneGemmKg) || tune_is_set(kTuneGemmKsplit)) return false;
-    uint64_t rows = 0;
-    for (int i = 0; i < n; i++) {
-        // 32-bit byte offsets into a workgroup's rows and into the activations of its tokens
-        if (args[i].B != 1 || K > (1u << 24) || ((uint64_t)((T < 64 ? T : 64) - 1) * args[i].x_token_stride + K) * 2 > 0x7fffffffull) return false;
-        rows += args[i].R;
-    }
-    const ShortTile t = one_block_pays(quant, rows, K, T) ? one_block(quant, rows, K, T) : T > 32 ? several_blocks(quant, args, n, rows, K, T) : kNoTile;
+    const ShortTile t = short_tile(quant, args, n);
     if (!t.mrt) return false;
     status = quant == kNf4 ? launch_tile<kNf4>(stream, args, n, t) : launch_tile<kInt8>(stream, args, n, t);
     return true;

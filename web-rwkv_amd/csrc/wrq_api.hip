@@ -258,14 +258,11 @@ int prepare(Entry entry, Quant quant, const void *w, const Shape4 &mshape, const
     return WRQ_OK;
 }
 
-// Whether `n` decode products that share a launch go to the matrix cores after all.
-bool decode_run(Quant quant, const Prepared *ops, int n) {
-    uint64_t rows = 0;
-    for (int i = 0; i < n; i++) {
+// Whether `n` decode products that share a launch go to the matrix cores after all; `run`: their arguments.
+bool decode_run(Quant quant, const Prepared *ops, const MatmulArgs *run, int n) {
+    for (int i = 0; i < n; i++)
         if (!ops[i].decode_mfma || ops[i].a.K != ops[0].a.K) return false;
-        rows += ops[i].a.R;
-    }
-    return short_run_pays(quant, rows, ops[0].a.K, ops[0].a.T);
+    return short_run_pays(quant, run, n);
 }
 
 int launch_vec(hipStream_t stream, Quant quant, const Prepared &p) {
@@ -281,7 +278,7 @@ int matmul(hipStream_t stream, Entry entry, Quant quant, const void *w, const Sh
            const wrq_tensor_view *output, int act, bool noalloc = false) {
     Prepared p;
     WRQ_TRY(prepare(entry, quant, w, mshape, scale, table, input, output, act, p));
-    if (p.mfma || decode_run(quant, &p, 1)) return launch_chunk(stream, quant, p, noalloc);
+    if (p.mfma || decode_run(quant, &p, &p.a, 1)) return launch_chunk(stream, quant, p, noalloc);
     return launch_vec(stream, quant, p);
 }
 
@@ -298,7 +295,7 @@ int dispatch_group(hipStream_t stream, Quant quant, const Prepared *ops, int n) 
             run[m] = ops[i + m].a;
             m++;
         }
-        if (ops[i].mfma || decode_run(quant, ops + i, m))
+        if (ops[i].mfma || decode_run(quant, ops + i, run, m))
             WRQ_TRY(launch_gemm_group(stream, quant, ops[i].in_f16, run, m));
         else
             WRQ_TRY(launch_gemv_group(stream, quant, ops[i].in_f16, run, m));
@@ -343,6 +340,24 @@ int wrq_debug_stamps(void *buffer, uint64_t bytes) {
     if (!g_test_hooks.load(std::memory_order_relaxed))
         return fail(WRQ_ERR_UNSUPPORTED, "wrq_debug_stamps needs WRQ_TEST_HOOKS=1 in the environment");
     return stamps_set(buffer, bytes);
+}
+
+int wrq_debug_route(int nf4, int mat, int count, const uint32_t *rows, uint32_t K, uint32_t T, uint32_t x_token_stride) {
+    if (count < 1 || count > kMaxGroup || !rows || (mat && count > 1)) return fail(WRQ_ERR_SIZE, "data size not match: %d vs. %d", count, mat ? 1 : kMaxGroup), -1;
+    void *const at = reinterpret_cast<void *>((uintptr_t)4096); // an aligned address that nothing is read from
+    const Quant quant = nf4 ? kNf4 : kInt8;
+    Prepared ops[kMaxGroup];
+    MatmulArgs run[kMaxGroup];
+    for (int i = 0; i < count; i++) {
+        const uint64_t len = (uint64_t)K * rows[i];
+        const wrq_tensor scale{at, {(uint32_t)(nf4 ? len / WRQ_NF4_BLOCK_SIZE : 2 * (len / WRQ_INT8_BLOCK_SIZE)), 1, 1, 1}}, table{at, {16, 1, 1, 1}};
+        const wrq_tensor_view x{at, {{K, T, 1, 1}, {x_token_stride, T, 1, 1}, {0, 0, 0, 0}}, WRQ_F16}, out{at, {{rows[i], T, 1, 1}, {rows[i], T, 1, 1}, {0, 0, 0, 0}}, WRQ_F16};
+        if (prepare(mat ? kMat : kVec, quant, at, Shape4{{nf4 ? K / 2 : K, rows[i], 1, 1}}, &scale, nf4 ? &table : nullptr, &x, &out, WRQ_ACT_NONE, ops[i]) != WRQ_OK) return -1;
+        run[i] = ops[i].a;
+    }
+    if (!ops[0].mfma && !decode_run(quant, ops, run, count)) return 0;
+    const uint32_t tile = short_run_tile(quant, run, count);
+    return tile ? (int)tile : 1;
 }
 
 int wrq_init(void) {

@@ -45,10 +45,12 @@ int launch_gemm_noalloc(hipStream_t stream, Quant quant, int in_f16, const Matmu
 // The same for `n` independent products of one quantisation and input type: those with one K
 // and token count share a launch (and then rarely need a split of K).
 int launch_gemm_group(hipStream_t stream, Quant quant, int in_f16, const MatmulArgs *args, int n, const ScratchPolicy *sp = nullptr);
-// Short runs (gemm_short.hip): launches `n` products that share K, token count and f16 activations if that kernel is the
-// faster one for them, with the launch's result in `status`; false: nothing was launched.
-// Whether runs of 2 .. 4 tokens of f16 activations belong there rather than on the decode kernels.
-bool short_run_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T);
+// Short runs (gemm_short.hip), `n` products that share K, token count and f16 activations and meet the chunk kernel's alignments.
+// Whether runs of 2 .. 4 tokens belong there rather than on the decode kernels; implies that `launch_gemm_short` takes them.
+bool short_run_pays(Quant quant, const MatmulArgs *args, int n);
+// The tile that kernel takes them with, MRT | TOK << 8 | NW << 16 | SUB << 24; 0: the chunk kernel is the faster one.
+uint32_t short_run_tile(Quant quant, const MatmulArgs *args, int n);
+// Launches them if that kernel is the faster one, with the launch's result in `status`; false: nothing was launched.
 bool launch_gemm_short(hipStream_t stream, Quant quant, const MatmulArgs *args, int n, int &status);
 // Overrides of the kernel and tile choice, for tests and sweeps that must reach one particular
 // instantiation.  Every key is unset (-1) unless the environment variable of the same name (WRQ_ +
