@@ -42,3 +42,22 @@ def test_pinned_chunk_tiles_leave_decode_runs_alone(wrq, overrides, kind, key, v
     overrides(**{key: value})
     assert wrq.debug_route(kind, rows, K, T) == "decode"
     assert wrq.debug_route(kind, rows, K, 16) == "chunk"
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("key,value", [("gemv_oneshot", 1), ("gemv_rows", 8), ("gemv_nt", 128), ("gemv_sl", 1), ("gemv_grid", 256), ("gemv_waverows", 1), ("gemv_rows_tokens", 0)])
+def test_pinned_decode_kernels_keep_their_runs(wrq, overrides, kind, key, value):
+    rows, K, T = SHAPES[kind]
+    assert isinstance(wrq.debug_route(kind, rows, K, T), tuple)
+    overrides(**{key: value})
+    assert wrq.debug_route(kind, rows, K, T) == "decode"
+    assert isinstance(wrq.debug_route(kind, rows, K, 16), tuple)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("key", ["gemm_table", "gemv_table"])
+def test_leaving_a_table_out_moves_no_product(wrq, overrides, kind, key):
+    rows, K, T = SHAPES[kind]
+    want = [wrq.debug_route(kind, rows, K, t) for t in (T, 16)]
+    overrides(**{key: 0})
+    assert [wrq.debug_route(kind, rows, K, t) for t in (T, 16)] == want

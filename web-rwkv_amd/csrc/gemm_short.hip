@@ -514,6 +514,9 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 bool short_run_pays(Quant quant, const MatmulArgs *args, int n) {
     const uint32_t K = args[0].K, T = args[0].T;
     if (T < 2 || T > 4 || !short_tile(quant, args, n).mrt) return false; // what `launch_gemm_short` hands on stays on the decode kernels
+    // a pinned choice among the decode kernels means those
+    for (const TuneKey key : {kTuneGemvOneshot, kTuneGemvRows, kTuneGemvSl, kTuneGemvNt, kTuneGemvGrid, kTuneGemvWaveRows, kTuneGemvRowsTokens})
+        if (tune_is_set(key)) return false;
     const uint64_t rows = rows_of(args, n);
     if (quant == kInt8) {
         if (K % 1024 == 0) return T == 4 && rows >= 4096 && rows <= (K < 2048 ? 16384 : K < 4096 ? 20480 : 49152);

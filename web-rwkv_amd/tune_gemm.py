@@ -60,7 +60,8 @@ def sweep(args):
     f16 = torch.float16
     gen = torch.Generator(device="cuda").manual_seed(7)
     out = open(args.out, "a")
-    wrq.debug_override("gemm_table", 0)  # the "rule" rows: the library without its table
+    wrq.debug_override("gemm_table", 0)  # the "rule" rows: the chunk kernel without its table
+    wrq.debug_override("gemm_short", 0)
     last = [time.time()]
     shortlist = load(args.refine.split(",")) if args.refine else None
 
@@ -120,8 +121,10 @@ def sweep(args):
                     rec = {"quant": quant, "kind": kind, "C": C, "H": H, "rows": rows, "K": K, "n": len(prods), "T": T}
                     out.write(json.dumps(dict(rec, cfg="rule", us=round(rule, 3))) + "\n")
                     wrq.debug_override("gemm_table", -1)
+                    wrq.debug_override("gemm_short", -1)
                     tab = timed(fn, copies)  # what the library does by itself, with the table it was built with
                     wrq.debug_override("gemm_table", 0)
+                    wrq.debug_override("gemm_short", 0)
                     out.write(json.dumps(dict(rec, cfg="table", us=round(tab, 3))) + "\n")
                     best = (rule, "rule")
                     if shortlist is not None:
@@ -196,6 +199,7 @@ def sweep_decode(args):
     gen = torch.Generator(device="cuda").manual_seed(7)
     out = open(args.out, "a")
     wrq.debug_override("gemv_table", 0)
+    wrq.debug_override("gemm_short", 0)  # the "rule" rows: the decode kernels
 
     def timed(fn, launches, min_ms=20.0):
         fn()
