@@ -1,5 +1,6 @@
 """Which kernel a product runs on (no GPU needed): the rules that share launches out between the decode, short-run and chunk kernels
 have to agree with one another and with the overrides."""
+import importlib
 import random
 
 import pytest
@@ -61,3 +62,14 @@ def test_leaving_a_table_out_moves_no_product(wrq, overrides, kind, key):
     want = [wrq.debug_route(kind, rows, K, t) for t in (T, 16)]
     overrides(**{key: 0})
     assert [wrq.debug_route(kind, rows, K, t) for t in (T, 16)] == want
+
+
+@pytest.mark.parametrize("kind,rows,K,T", [("int8", 65536, 4096, 8), ("int8", 65536, 4096, 16)])
+def test_products_of_many_rows_keep_their_measured_tiles(wrq, kind, rows, K, T):
+    # beyond the rows that the short-run kernel takes short runs are the chunk kernel's; its measured tiles beat its rules there (55.2 against 61.6 us at 8 tokens)
+    from test_tuned_table import rows_of_table
+
+    tune = importlib.import_module("web-rwkv_amd.tune_gemm")
+    assert wrq.debug_route(kind, rows, K, T) == "chunk"
+    bucket = next(i for i, t in enumerate(tune.T_GRID) if t >= T)
+    assert any(cells[bucket] for q, r, k, cells in rows_of_table() if (q, r, k) == (KINDS.index(kind), rows, K))
