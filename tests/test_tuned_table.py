@@ -82,3 +82,14 @@ def test_table_generation_keeps_the_rules_where_they_are_close(tmp_path, capsys)
     cells = [int(c, 0) for c in re.search(r"\{([^{}]*)\}\},", row[0]).group(1).split(",")]
     assert cells[0] == 0 and cells[2] == 0
     assert cells[1] == (1 | 1 << 4 | 2 << 8 | 1 << 12)
+
+
+def test_every_bucket_is_reached_by_some_launch(wrq):
+    # a bucket whose launches all go to another kernel is dead data, and a sweep or test of it would look at that kernel
+    tune = importlib.import_module("web-rwkv_amd.tune_gemm")
+    cells = {(q, r, k): row for q, r, k, row in rows_of_table()}
+    dead = [(key, tune.T_GRID[b]) for key, row in cells.items() for b, c in enumerate(row) if c and not tune.reached(wrq, cells, key, b)]
+    assert not dead, dead
+    # ... and what the short-run kernel has at every size around is not
+    assert not tune.reached(wrq, {(0, 768, 768): [1] * len(tune.T_GRID)}, (0, 768, 768), 0)
+    assert tune.reached(wrq, {(1, 4096, 14336): [1] * len(tune.T_GRID)}, (1, 4096, 14336), 13)

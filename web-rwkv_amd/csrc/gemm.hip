@@ -940,7 +940,8 @@ int launch_one(hipStream_t stream, const MatmulArgs *args, int n, uint32_t kspli
 // Measured tile choices.  web-rwkv_amd/tune_gemm.py times every tile shape and split for the launches of the RWKV model sizes
 // (the four attention projections, att.output, {ffn.key, ffn.receptance}, ffn.key, ffn.value, the head; 8 .. 512 tokens) and
 // writes the fastest per (format, rows, K, run-length bucket) into gemm_tuned.inc.  A launch of f16 activations on one batch
-// whose rows and K lie within 7 % of a measured product takes that entry; everything else goes by the rules below.
+// whose rows and K lie within 7 % of a measured product takes that entry; everything else goes by the rules below.  Buckets whose launches
+// all go to the short-run kernel, which is asked first, are taken out (`tune_gemm.py prune`; a test holds the table to it).
 struct TunedRow {
     uint32_t quant, rows, K;
     uint16_t cfg[18]; // MRT | NTILE << 4 | KG << 8 | split << 12 per bucket; 0: the rules decide

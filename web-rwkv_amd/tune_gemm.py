@@ -10,6 +10,11 @@ sizes and writes the winners as a table:
   python3 web-rwkv_amd/tune_gemm.py sweep --out refined.jsonl --refine sweep.jsonl
   python3 web-rwkv_amd/tune_gemm.py table sweep.jsonl refined.jsonl > web-rwkv_amd/csrc/gemm_tuned.inc
 
+  python3 web-rwkv_amd/tune_gemm.py prune web-rwkv_amd/csrc/gemm_tuned.inc     (no GPU needed)
+
+`prune` takes out the buckets that no launch reaches because the short-run kernel (csrc/gemm_short.hip) has all of theirs: run it after
+every change of that kernel's rules, and `table` again where they get narrower.
+
 The one-shot decode kernels (csrc/gemv.hip, runs of 1 .. 4 tokens on products the wave-owns-rows and K-split
 kernels do not take) have two such choices, lanes per task and rows per task; `sweep --decode` and
 `table --decode` do the same for them (gemv_tuned.inc).
@@ -27,6 +32,7 @@ import collections
 import importlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -297,6 +303,59 @@ def table_decode(args):
     print(f"// {filled} cells filled")
 
 
+ROW = re.compile(r"^\{(\d+),\s*(\d+)u,\s*(\d+)u,\s*\{([^}]*)\}\},\s*$", re.M)
+
+
+def parse(text):
+    """The rows of a chunk table: (format, rows, K) -> cells."""
+    return {(int(q), int(r), int(k)): [int(c, 0) for c in cells.split(",")] for q, r, k, cells in ROW.findall(text)}
+
+
+def groups_of(rows):
+    """Ways to share `rows` rows out over the products of a launch: one product, equal ones, the two of a feed-forward layer, a large one among small ones."""
+    yield (rows,)
+    for n in range(2, 9):
+        if rows >= 4 * n:
+            part = rows // n // 4 * 4
+            yield (part,) * (n - 1) + (rows - part * (n - 1),)
+            yield (rows - 4 * (n - 1),) + (4,) * (n - 1)
+    if rows >= 12:
+        yield rows * 7 // 36 * 4, rows - rows * 7 // 36 * 4
+
+
+def reached(wrq, cells, key, bucket):
+    """Whether some launch takes this bucket's tile: its rows and K lie within 7 % of the product's and nearer to it than to any other
+    product with that bucket, and no rule sends it to another kernel.  Launches are looked at on a grid over that range."""
+    quant, rows, K = key
+    kind, others = ("int8", "nf4")[quant], [(r, k) for (q, r, k), c in cells.items() if q == quant and c[bucket]]
+    near = lambda r, k, at: abs(r - at[0]) * 100 <= 7 * at[0] and abs(k - at[1]) * 100 <= 7 * at[1]
+    off = lambda r, k, at: abs(r - at[0]) * 1000 // at[0] + abs(k - at[1]) * 1000 // at[1]
+    low, high = (T_GRID[bucket - 1] + 1 if bucket else 4), T_GRID[bucket]
+    tokens = sorted({high, low, (low + high) // 2, high // 4 * 4, -(-low // 4) * 4}, reverse=True)
+    around = lambda at, step: sorted(range(-(-at * 93 // 100 // step) * step, at * 107 // 100 + 1, step), key=lambda v: abs(v - at))
+    for k in around(K, 128):
+        for r in around(rows, max(4, rows // 256 // 4 * 4)):
+            here = [at for at in others if near(r, k, at)]
+            if not near(r, k, (rows, K)) or min(here, key=lambda at: off(r, k, at)) != (rows, K):
+                continue
+            for T in tokens:
+                if any(wrq.debug_route(kind, g, k, T) == "chunk" for g in groups_of(r)) or T % 4 == 0 and wrq.debug_route(kind, r, k, T, mat=True) == "chunk":
+                    return True
+    return False
+
+
+def prune(args):
+    sys.path.insert(0, ROOT)
+    wrq = importlib.import_module("web-rwkv_amd")
+    text = open(args.file).read()
+    cells = parse(text)
+    kept = {key: [c if c and reached(wrq, cells, key, b) else 0 for b, c in enumerate(row)] for key, row in cells.items()}
+    comments = [line for line in text.splitlines() if line.startswith("//")]
+    comments[-1] = f"// {sum(c != 0 for row in kept.values() for c in row)} buckets that launches reach; the rules or the short-run kernel have the others"
+    body = ["{%d, %6du, %6du, {%s}}," % (*key, ", ".join("0x%04x" % c if c else "0" for c in kept[key])) for key in sorted(kept) if any(kept[key])]
+    open(args.file, "w").write("\n".join(comments[:-1] + body + comments[-1:]) + "\n")
+
+
 def load(paths, decode=False):
     d = collections.defaultdict(dict)
     refined = set()
@@ -369,8 +428,12 @@ def main():
     t = sub.add_parser("table")
     t.add_argument("--decode", action="store_true", help="write gemv_tuned.inc from a sweep --decode")
     t.add_argument("files", nargs="+")
+    r = sub.add_parser("prune")
+    r.add_argument("file", help="a chunk table, rewritten in place")
     args = ap.parse_args()
-    if args.cmd == "sweep":
+    if args.cmd == "prune":
+        prune(args)
+    elif args.cmd == "sweep":
         (sweep_decode if args.decode else sweep)(args)
     else:
         (table_decode if args.decode else table)(args)
