@@ -675,7 +675,7 @@ def test_chunk_k_groups_by_default(gpu, oracle, kind, T):
 def test_decode_tasks_from_the_measured_table(gpu, oracle, kind, C, H, overrides):
     # runs of 1 .. 4 tokens on the launches of model sizes whose lanes and rows per task come from the measured
     # table of the one-shot kernels (csrc/gemv_tuned.inc), against float64 on sampled rows; once more with the
-    # table switched off (gemv_table = 0)
+    # table switched off (gemv_table = 0), both with the short-run kernel left out, and once as the library chooses
     import torch
 
     announce("decode tasks from the table", kind, C, H)
@@ -686,8 +686,8 @@ def test_decode_tasks_from_the_measured_table(gpu, oracle, kind, C, H, overrides
         wp, scale, wdeq = pack(oracle, kind, w)
         rows = np.sort(rng.choice(R, 64, replace=False))
         mats[(R, K)] = (gpu_matrix(gpu, kind, wp, scale), wdeq[rows], rows)
-    for table in (1, 0):
-        overrides(gemv_table=table)
+    for table, short in ((1, 0), (0, 0), (1, 1)):
+        overrides(gemv_table=table, gemm_short=short)
         for T in (1, 2, 3, 4):
             for group in ([(C, C)] * 4, [(C, C)], [(H, C), (C, C)], [(C, H)]):
                 xs = [gen_f16(rng, (T, K), 1.0) for _, K in group]
@@ -708,8 +708,8 @@ def test_decode_tasks_from_the_measured_table(gpu, oracle, kind, C, H, overrides
 def test_chunk_tiles_from_the_measured_table(gpu, oracle, kind, C, H, overrides):
     # the launches of the smaller model sizes take their tile shape and split from the measured table
     # (csrc/gemm_tuned.inc): {k, v, r, g}, att.output, {ffn.key, ffn.receptance} and ffn.value at run lengths
-    # in several buckets, against float64 on sampled rows -- and once more with the table switched off
-    # (gemm_table = 0), where the rules pick the tile.  2176 / 7296 is no model size: its rows and K lie within
+    # in several buckets, against float64 on sampled rows -- once more with the table switched off
+    # (gemm_table = 0), where the rules pick the tile, both with the short-run kernel left out, and once as the library chooses.  2176 / 7296 is no model size: its rows and K lie within
     # 7 % of the 2048 / 7168 entries and take them, with row and K counts that fill no tile evenly
     import torch
 
@@ -721,8 +721,8 @@ def test_chunk_tiles_from_the_measured_table(gpu, oracle, kind, C, H, overrides)
         wp, scale, wdeq = pack(oracle, kind, w)
         rows = np.sort(rng.choice(R, 64, replace=False))
         mats[(R, K)] = (gpu_matrix(gpu, kind, wp, scale), wdeq[rows], rows)
-    for table in (1, 0):
-        overrides(gemm_table=table)
+    for table, short in ((1, 0), (0, 0), (1, 1)):
+        overrides(gemm_table=table, gemm_short=short)
         for T in (6, 24, 40, 96, 130, 256, 300, 500):
             for group in ([(C, C)] * 4, [(C, C)], [(H, C), (C, C)], [(C, H)]):
                 xs = [gen_f16(rng, (T, K), 1.0) for _, K in group]
@@ -738,22 +738,34 @@ def test_chunk_tiles_from_the_measured_table(gpu, oracle, kind, C, H, overrides)
                     assert_close(got[:, rows], truth_matmul(wsub, x), EPS, f"{kind} {group} T={T} table={table} vs float64")
 
 
+# Launches of the tests of the short-run kernel, (K, rows) of every product: which tile each takes at which run length is the rules' choice,
+# and tests/test_product_routes.py holds the lists to every tile the kernel is built for.
+SHORT_T = (4, 8, 9, 16, 17, 24, 25, 32, 33, 48)
+SHORT_ROUNDS_T = (8, 16, 24, 32, 48)
+SHORT_BLOCKS_T = (33, 49, 64, 65, 97, 192, 255, 256)
+SHORT_GROUPS = {kind: [[(128, 4)], [(384, 20), (384, 132)], [(4096 if kind == "int8" else 8192, 68)], [(2048, 2048), (2048, 2052)], [(256, 4100), (256, 4)],
+                       [(256, 8196), (256, 36)], [(256, 12304)], [(256, 15980), (256, 400)], [(7168, 64)]] for kind in ("int8", "nf4")}
+SHORT_ROUNDS = [(2048, 16388), (2048, 400)]
+SHORT_BLOCKS = [[(256, 4)], [(640, 516), (640, 20)], [(1024, 1024)], [(256, 2052), (256, 1000), (256, 68)], [(2176, 4100)], [(4096, 264)]]
+
+
 @pytest.mark.parametrize("kind", ["int8", "nf4"])
-@pytest.mark.parametrize("T", [4, 8, 9, 16, 17, 24, 25, 32, 33, 48], ids=str)
+@pytest.mark.parametrize("T", SHORT_T, ids=str)
 def test_short_run_kernel(gpu, oracle, kind, T, overrides):
     # the kernel of short runs (csrc/gemm_short.hip) at the edges of its token tiles: rows that fill no tile, fewer K
     # steps than waves, rows of 4 KiB (every workgroup starts at another step), one to four row tiles per workgroup, steps
-    # of 256 elements and several rounds of workgroups; strided activations, groups of products of different size, every
+    # of 256 elements; strided activations, groups of products of different size, every
     # activation.  f32 outputs against float64: operands are exact, so a sum of K products of |w x| < 0.1 * 4 in f32
     # stays below 2^-23 * K * 0.4 < 1e-3, and far below it for random signs.
     import torch
 
     announce("short run", kind, T)
     rng = np.random.default_rng(SEED + 91 + T)
-    groups = [[(128, 4)], [(384, 20), (384, 132)], [(4096 if kind == "int8" else 8192, 68)], [(2048, 2048), (2048, 2052)], [(256, 4100), (256, 4)],
-              [(256, 8196), (256, 36)], [(256, 12304)], [(256, 16388), (256, 400)], [(7168, 64)]]
-    for i, shapes in enumerate(groups):
+    overrides(vec_chunk_min_t=2)
+    for i, shapes in enumerate(SHORT_GROUPS[kind]):
         K, ops, want = shapes[0][0], [], []
+        if gpu.debug_route(kind, [R for _, R in shapes], K, T) == "chunk":
+            continue  # few rows of long K: nothing of this kernel to look at
         for j, (_, R) in enumerate(shapes):
             wp, scale, wdeq = pack(oracle, kind, gen_f16(rng, (R, K), 0.02))
             parent = gen_f16(rng, (2, T + 1, K + 64), 1.0)  # the activations are a slice of it
@@ -765,7 +777,7 @@ def test_short_run_kernel(gpu, oracle, kind, T, overrides):
             want.append(1.0 / (1.0 + np.exp(-truth)) if act else truth)
         results = []
         for short in (1, 0):
-            overrides(gemm_short=short, vec_chunk_min_t=2)
+            overrides(gemm_short=short)
             gpu.matmul_vec_group(ops)
             results.append([host(op[2]) for op in ops])
         for j, op in enumerate(ops):
@@ -796,7 +808,33 @@ def test_decode_runs_on_the_short_run_kernel(gpu, oracle, kind, T):
 
 
 @pytest.mark.parametrize("kind", ["int8", "nf4"])
-@pytest.mark.parametrize("T", [33, 49, 64, 65, 97, 192, 255, 256], ids=str)
+@pytest.mark.parametrize("T", SHORT_ROUNDS_T, ids=str)
+def test_short_run_kernel_in_rounds(gpu, oracle, kind, T, overrides):
+    # several rounds of workgroups: more rows than one workgroup per CU holds, against float64 on sampled rows and the chunk kernel.  Tolerance as above.
+    import torch
+
+    announce("short run in rounds", kind, T)
+    rng = np.random.default_rng(SEED + 94)
+    K, ops, want = SHORT_ROUNDS[0][0], [], []
+    assert gpu.debug_route(kind, [R for _, R in SHORT_ROUNDS], K, T) != "chunk"
+    for _, R in SHORT_ROUNDS:
+        wp, scale, wdeq = pack(oracle, kind, gen_f16(rng, (R, K), 0.02))
+        x = gen_f16(rng, (T, K), 1.0)
+        rows = np.unique(np.append(rng.choice(R, 64, replace=False), [0, R - 1]))
+        ops.append((gpu_matrix(gpu, kind, wp, scale), dev(x), torch.full((T, R), float("nan"), dtype=torch.float32, device="cuda"), 0, False, {}))
+        want.append((rows, truth_matmul(wdeq[rows], x)))
+    results = []
+    for short in (1, 0):
+        overrides(gemm_short=short)
+        gpu.matmul_vec_group(ops)
+        results.append([host(op[2]) for op in ops])
+    for short, chunk, (rows, truth) in zip(*results, want):
+        assert_close(short[:, rows], truth, 3e-4, f"{kind} T={T} vs float64")
+        assert_close(short, chunk, EPS, f"{kind} T={T} vs the chunk kernel")
+
+
+@pytest.mark.parametrize("kind", ["int8", "nf4"])
+@pytest.mark.parametrize("T", SHORT_BLOCKS_T, ids=str)
 def test_short_run_kernel_in_token_blocks(gpu, oracle, kind, T, overrides):
     # the same kernel over several blocks of 32, 48 or 64 tokens, the last one partly filled: tiles of one to four times 16 rows, row
     # tiles that are padded to eight per product (workgroups without rows), groups, strided activations.  Tolerance as above.
@@ -804,8 +842,10 @@ def test_short_run_kernel_in_token_blocks(gpu, oracle, kind, T, overrides):
 
     announce("short run in token blocks", kind, T)
     rng = np.random.default_rng(SEED + 92 + T)
-    for i, shapes in enumerate([[(256, 4)], [(640, 516), (640, 20)], [(1024, 1024)], [(256, 2052), (256, 1000), (256, 68)], [(2176, 4100)], [(4096, 264)]]):
+    for i, shapes in enumerate(SHORT_BLOCKS):
         K, ops, want = shapes[0][0], [], []
+        if gpu.debug_route(kind, [R for _, R in shapes], K, T) == "chunk":
+            continue
         for j, (_, R) in enumerate(shapes):
             wp, scale, wdeq = pack(oracle, kind, gen_f16(rng, (R, K), 0.02))
             parent = gen_f16(rng, (T + 2, K + 8), 1.0)
@@ -995,20 +1035,23 @@ def test_full_size_properties(gpu, oracle, kind):
 @pytest.mark.parametrize("kind", ["int8", "nf4"])
 @pytest.mark.parametrize("T", [2, 3, 4])
 @pytest.mark.parametrize("K,R", [(14336, 516), (4096, 2060), (2048, 16388)], ids=str)
-def test_short_runs_on_decode_kernels(gpu, oracle, kind, K, R, T):
+def test_short_runs_on_decode_kernels(gpu, oracle, kind, K, R, T, overrides):
     # 2 - 4 tokens share one pass of the decode kernels: long rows (two chunks per lane), row
-    # counts that leave a partial task, enough rows for 8 per task, f16 output with an activation
+    # counts that leave a partial task, enough rows for 8 per task, f16 output with an activation; without the short-run
+    # kernel, and once more as the library chooses
     announce("short run", kind, K, R, T)
     rng = np.random.default_rng(SEED + 29 + T + K)
     w = gen_f16(rng, (R, K), 0.02)
     x = gen_f16(rng, (T, K), 1.0)
     wp, scale, wdeq = pack(oracle, kind, w)
     m = gpu_matrix(gpu, kind, wp, scale)
-    got = run(gpu, m, x, R, "vec", np.float16, act=gpu.ACT_SILU)
-    assert got.shape == (T, R)
-    assert_close(got, truth_matmul(wdeq, x, "silu"), EPS, "vs float64")
     one = np.concatenate([run(gpu, m, x[t:t + 1], R, "vec", np.float16, act=gpu.ACT_SILU) for t in range(T)])
-    assert_close(got, one, 1e-3, "vs one call per token")  # same arithmetic up to the last f16 ulp
+    for short in (0, 1):
+        overrides(gemm_short=short)
+        got = run(gpu, m, x, R, "vec", np.float16, act=gpu.ACT_SILU)
+        assert got.shape == (T, R)
+        assert_close(got, truth_matmul(wdeq, x, "silu"), EPS, f"short={short} vs float64")
+        assert_close(got, one, 1e-3, f"short={short} vs one call per token")  # same arithmetic up to the last f16 ulp
 
 
 @pytest.mark.parametrize("T,x_dtype", [(1, np.float16), (2, np.float16), (3, np.float32), (32, np.float16), (40, np.float16)])

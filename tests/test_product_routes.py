@@ -73,3 +73,17 @@ def test_products_of_many_rows_keep_their_measured_tiles(wrq, kind, rows, K, T):
     assert wrq.debug_route(kind, rows, K, T) == "chunk"
     bucket = next(i for i, t in enumerate(tune.T_GRID) if t >= T)
     assert any(cells[bucket] for q, r, k, cells in rows_of_table() if (q, r, k) == (KINDS.index(kind), rows, K))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_every_tile_of_the_short_run_kernel_has_a_test(wrq, overrides, kind):
+    # the GPU tests compare that kernel with the chunk kernel on launches whose tile the rules choose
+    import test_gpu_parity as gpu_tests
+
+    built = {(1, 8, 8, 2)} | {(m, t, 8, 1) for m in (1, 2, 3, 4) for t in (8, 16, 24, 32)} | {(3, 24, 4, 1), (3, 32, 4, 1), (1, 48, 8, 1), (2, 48, 8, 1), (3, 48, 4, 1), (4, 48, 4, 1)}
+    built |= {(4, 64, 4, 1)} if kind == "int8" else set()
+    overrides(vec_chunk_min_t=2)
+    launches = [(g, T) for g in gpu_tests.SHORT_GROUPS[kind] for T in gpu_tests.SHORT_T] + [(gpu_tests.SHORT_ROUNDS, T) for T in gpu_tests.SHORT_ROUNDS_T]
+    launches += [(g, T) for g in gpu_tests.SHORT_BLOCKS for T in gpu_tests.SHORT_BLOCKS_T]
+    seen = {wrq.debug_route(kind, [R for _, R in g], g[0][0], T) for g, T in launches} - {"chunk"}
+    assert seen == built, (built - seen, seen - built)

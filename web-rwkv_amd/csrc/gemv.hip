@@ -1648,7 +1648,7 @@ int launch_generic(hipStream_t stream, Quant quant, int in_f16, const MatmulArgs
 // Measured task shapes of the one-shot kernels.  web-rwkv_amd/tune_gemm.py (sweep --decode) times lanes per task x rows per
 // task for the launches of the RWKV model sizes at 1 .. 4 tokens and writes the fastest, where it beats the rules below by more
 // than 4 %, into gemv_tuned.inc; a launch of f16 activations on one batch whose rows and K lie within 7 % of a measured product
-// takes that entry.  Half of the entries for 2 .. 4 tokens were measured at a K whose runs the short-run kernel takes today: they serve products
+// takes that entry.  27 of the 44 entries for 2 .. 4 tokens were measured on launches that leave for the matrix cores today: they serve products
 // whose K is no multiple of 128 and groups that mix several K.
 namespace {
 struct TunedDecodeRow {
