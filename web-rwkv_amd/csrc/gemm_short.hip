@@ -423,11 +423,19 @@ uint64_t one_block_rows(Quant quant, uint32_t K, uint32_t T) {
 // workgroup has to fetch for its rows.
 bool one_block_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     if (rows > one_block_rows(quant, K, T)) return false;
-    if (T <= 8) return quant == kNf4 || rows >= 2048 || K <= 10240;              // int8 1024 rows: K 8192 0.89 of the chunk kernel's time, 14336 1.01
-    if (T <= 16) return rows >= 2048 || K <= (quant == kNf4 ? 10240u : 5120u);    // int8 1024 rows: 4096 0.81, 8192 1.07; nf4 0.78, 0.95
-    if (T <= 24) return quant == kNf4 || K <= 10240 || (T <= 20 && rows >= 2048); // int8 4096 x 14336 at 19 / 24 tokens 0.92 / 1.04; nf4 0.85
-    if (T <= 32) return rows >= 2560 ? quant == kNf4 || K <= 8192 : K <= 4096;    // 2048 x 7168 1.04 (nf4), 1.13 (int8); 4096 x 14336 0.96, 1.18
-    return T <= 48 && rows >= 2560 && K <= 8192;                                  // 1.6B / 3B / 7B groups 0.7 .. 0.9, 2048 x 7168 1.02 .. 1.14
+    const bool nf4 = quant == kNf4;
+    if (T <= 8) return nf4 || rows >= 2048 || K <= 10240; // int8 1024 rows: K 8192 0.89 of the chunk kernel's time, 14336 1.01
+    // int8 1024 rows: 4096 0.81, 8192 1.07; nf4 0.78, 0.95.  2048 rows, which the chunk kernel splits eight ways: int8 8960 0.97, 10240 1.08, 14336
+    // 1.26; nf4 12288 1.00, 14336 1.07; 2560 rows of 14336 0.95, 0.82
+    if (T <= 16) return rows > 2048 || K <= (nf4 ? (rows < 2048 ? 10240u : 12288u) : rows < 2048 ? 5120u : 8960u);
+    if (T <= 24) return nf4 || K <= 10240 || (T <= 20 && rows >= 2048 && (rows > 4096 || K <= 14336)); // int8 4096 x 14336 at 19 / 24 tokens 0.92 / 1.04, 17920 at 20 1.04, 11260 x 15488 0.78; nf4 0.85
+    if (T <= 32) {
+        if (rows >= 2560) return nf4 ? rows > 4096 || K <= 16384 : K <= 8192; // 4096 x 14336 0.96 .. 1.01 (nf4), 1.18 (int8), 17920 nf4 1.06, 5120 x 17920 1.02
+        // 2048 x 7168 1.04 (nf4), 1.13 (int8); 1024 x 4096 int8 1.10 (its measured chunk tile serves up to 7 % around), 768 and 1280 rows 0.84 and 0.77
+        return K <= 4096 && (nf4 || K < 3810 || rows < 953 || rows > 1095);
+    }
+    // 1.6B / 3B / 7B groups 0.7 .. 0.9, 2048 x 7168 1.02 .. 1.14; one K step: 16384 x 128 1.07 (int8), 1.20 (nf4)
+    return T <= 48 && rows >= 2560 && K <= 8192 && (K >= 256 || rows <= 8192);
 }
 
 // Runs of 33 .. 256 tokens in several token blocks: where the smallest tile that gives every workgroup a CU of its own is the chunk
@@ -439,6 +447,11 @@ ShortTile several_blocks(Quant quant, const MatmulArgs *args, int n, uint64_t ro
     // long K: the chunk kernel splits it over the grid.  2560 x 8960 int8 64 tokens 1.04, 96 0.92; 4096 x 14336 int8 1.07 .. 1.28,
     // nf4 64 / 96 / 128 tokens 0.96 / 0.85 / 1.04
     if (T > 256 || K > (quant == kInt8 ? (T > 64 ? 10240u : 8192u) : T <= 96 ? 17920u : 10240u) || (K > 4096 && rows < 2048)) return kNoTile;
+    // ... and where four row tiles are needed for one round: 4096 x 8960 at 112 and 128 tokens int8 1.12, nf4 1.00, 10240 1.27, 1.05; nf4 8192 x 8960 .. 17920 at 64
+    // tokens 1.04 .. 1.11 (two row tiles, 48 tokens: 0.81 .. 0.91)
+    if (K > 8192 && ((T > 96 && rows > 3072) || (T > 48 && T <= 64 && rows > 6144))) return kNoTile;
+    // int8 10240: 2560 .. 4096 rows at 80 .. 128 tokens 1.02 .. 1.08, 2048 from 160 tokens on 1.04 .. 1.16; 5120 rows 0.94, 3072 at 160 tokens 0.89
+    if (quant == kInt8 && K > 8960 && rows <= (T > 128 ? 2560 : 4096)) return kNoTile;
     // padding included: a launch is dealt to the XCDs round-robin, and 256 live workgroups among more are not 32 on each of them
     // (588 + 548 + 2804 + 1040 rows, 148 tokens, counted without: 1.42 of the chunk kernel's time)
     auto workgroups = [&](int mrt, int tok) {
@@ -453,10 +466,13 @@ ShortTile several_blocks(Quant quant, const MatmulArgs *args, int n, uint64_t ro
     for (; tile != end; tile++) // in the order of their size, near ties as measured
         if (workgroups(tile->mrt, tile->tok) <= kOneRound) break;
     // four waves instead of eight: long K loses what the wide tile saves (nf4 3036 x 7936, 214 tokens 1.06; 16296 x 9344, 34 tokens 1.16)
+    // one K step keeps one wave busy: there wide tiles lose as well (K of 128, int8 3 and 4 x 48 1.01 .. 1.16; nf4 4 x 32 1.02 .. 1.14, 3 and 4 x 48 1.09 .. 1.31;
+    // nf4 3 x 32 0.95 .. 1.07 from one run to another)
+    if (tile != end && K < 256 && (tile->nw == 4 || (quant == kNf4 && tile->mrt == 4))) return kNoTile;
     if (tile != end) return tile->nw == 8 || K <= 5120 ? *tile : kNoTile;
     // int8, 64 x 64: from 2048 channels on (1.6B group 128 tokens 0.93, 3B and 7B 64 tokens 0.87 .. 0.90; 0.1B 256 tokens 1.08, 8040 x 7936,
-    // 57 tokens 1.20)
-    if (quant == kInt8 && K >= 2048 && K <= 5120 && workgroups(4, 64) <= kOneRound) return {4, 64, 4, 1};
+    // 57 tokens 1.20; 3072 .. 5120 rows at 160 .. 256 tokens: K 4096 0.97 .. 1.04, 5120 1.04 .. 1.09)
+    if (quant == kInt8 && K >= 2048 && K <= (T > 128 ? 4096 : 5120) && workgroups(4, 64) <= kOneRound) return {4, 64, 4, 1};
     // nf4, 64 x 48: two workgroups fit a CU.  Where they fill most of them and the last block is nearly full (3B 96 and 128 tokens 0.73,
     // 1.6B group 192 tokens 0.79, 7B 96 tokens 0.77; one block, 32768 rows, 0.82 .. 0.99, K of 5120 1.03; 288 .. 384 workgroups 0.95 .. 1.12, 64 tokens in two blocks 1.05 .. 1.20, K of 256 1.14)
     const uint64_t w = workgroups(4, 48);
@@ -504,7 +520,8 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 // time against this kernel's as 1, 600 drawn launches and the model shapes: int8, K < 1024: 2 tokens 0.84 .. 0.99, 3 and 4 0.59 .. 0.75;
 // K up to 2560 from 1024 rows on, up to 10240 from 2560 rows on, 3 and 4 tokens 0.49 .. 0.85 (fewer rows 0.83 .. 1.6, beyond 10240 0.78 .. 1.7); whole waves,
 // 4 tokens from 4096 rows on 0.75 .. 1.0, otherwise 0.95 .. 1.35.  nf4, K up to 1024: 2 tokens 0.66 .. 0.99, 3 0.52 .. 0.71; K up to 2560 0.67 .. 1.0
-// (2 tokens: 9216 x 2048 1.06); K up to 5120 from 1024 rows on, 3 tokens, 0.69 .. 0.98, 2 tokens 0.84 .. 1.07; longer K 0.9 .. 1.8.
+// (2 tokens: 9216 x 2048 1.06); K up to 5120 beyond 1024 rows, 3 tokens, 0.69 .. 1.04 (1024 rows,
+// one task of the decode kernel per CU: K 4096 1.13, 5120 1.27), 2 tokens 0.84 .. 1.07; longer K 0.9 .. 1.8.
 // Many rows, single products: int8, 4 tokens, K 1024: 16384 rows 0.88, 20480 1.12, 65536 1.23; K 2048: 20480 1.01, 32768 1.07; K 4096 and 5120 up to 65536 rows
 // 0.83 .. 0.98; K 768, 3 and 4 tokens: 20480 rows 0.87, 65536 1.00; K 2560 up to 65536 rows 0.64 .. 0.76.  nf4, K 1024, 2 tokens: 16384 rows 0.83, 20480 1.03,
 // 65536 1.11; 3 tokens, K of 768 .. 5120, up to 65536 rows 0.58 .. 0.97, but K 1792 19092 rows 1.08, 24876 1.16.
@@ -524,7 +541,7 @@ bool short_run_pays(Quant quant, const MatmulArgs *args, int n) {
         return T > 2 && (K <= 2560 ? rows >= 1024 : K <= 10240 && rows >= 2560);
     }
     if (T == 2) return K <= 1024 || (K <= 2560 && rows >= 1024 && rows <= 8192);
-    return K <= 2560 || (K <= 5120 && rows >= 1024);
+    return K <= 2560 || (K <= 5120 && rows > 1024);
 }
 
 uint32_t short_run_tile(Quant quant, const MatmulArgs *args, int n) {
