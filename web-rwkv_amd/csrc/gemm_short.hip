@@ -66,7 +66,11 @@ __device__ __forceinline__ uint4 buffer_load128(__amdgpu_buffer_rsrc_t r, uint32
 }
 constexpr int kStream = 2; // nt: weights are read once (7B int8 at 8 tokens 15.9 against 16.9 us without)
 
-template <int QUANT, int MRT, int TOK, int NW, int SUB>
+// CENTRED (int8, runs of 2 .. 4 tokens, which the decode kernels took before): codes enter as u - 128 instead of 1024 + u and the step of a block
+// is rounded correctly.  The decode kernels cancel 1024 sum_k x over 16 elements, the sums below over 128, which loses more:
+// f32 outputs against 64 bits, decode kernels / 1024 + u / u - 128: 7680 x 2560, 3 tokens, normal inputs 1.4e-6 / 2.0e-6 / 1.0e-7, squared relu of them
+// 3.9e-6 / 8.5e-6 / 3.0e-7 (with 1 / 255 rounded once, as elsewhere, the last is 3.2e-6: an error of one sign).  Costs 2 % of a launch.
+template <int QUANT, int MRT, int TOK, int NW, int SUB, bool CENTRED>
 __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, const uint16_t *scale0, const void *x0, const float *quant0,
                                                              const uint32_t begin1, const uint32_t R0, const uint32_t x_stride0, const uint32_t K,
                                                              const uint32_t T_all, const uint32_t tblocks, const ShortArgs a) {
@@ -206,9 +210,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, 
 #pragma unroll
             for (int u = 0; u < SUB; u++) {
                 const float lo = h2f((uint16_t)st.s[u]), hi = h2f((uint16_t)(st.s[u] >> 16));
-                const float s = (hi - lo) * (1.0f / 255.0f); // (min, max) -> (s, min - 1024 s)
+                constexpr float kInv = 1.0f / 255.0f, kInvRest = (float)(1.0 / 255.0 - (double)kInv);
+                const float s = CENTRED ? fmaf(hi - lo, kInv, (hi - lo) * kInvRest) : (hi - lo) * kInv; // (min, max) -> (s, min - 1024 s)
                 scl[(2 * u) * 16 * MRT + lane] = N4 ? lo : s;
-                scl[(2 * u + 1) * 16 * MRT + lane] = N4 ? hi : fmaf(-1024.0f, s, lo);
+                scl[(2 * u + 1) * 16 * MRT + lane] = N4 ? hi : fmaf(CENTRED ? 128.0f : -1024.0f, s, lo);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -290,6 +295,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, 
                     for (int c = 0; c < 2; c++) { // 4 codes of one dword -> f16 pairs 1024 + u
                         A[j].u[2 * c] = __builtin_amdgcn_perm(0x64646464u, ww[2 * j + c], 0x04010400u);
                         A[j].u[2 * c + 1] = __builtin_amdgcn_perm(0x64646464u, ww[2 * j + c], 0x04030402u);
+                        if constexpr (CENTRED) {
+                            const half2v centre{(_Float16)1152.0f, (_Float16)1152.0f};
+                            A[j].u[2 * c] = as_u32(as_h2(A[j].u[2 * c]) - centre);
+                            A[j].u[2 * c + 1] = as_u32(as_h2(A[j].u[2 * c + 1]) - centre);
+                        }
                     }
                 if (it + 2 < ITEMS) wq[q] = read_w(it + 2);
                 if (i == 0 && half + 1 < 2 * SUB) read_b(half + 1, B[(half + 1) & 1]);
@@ -352,10 +362,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_short_kernel(const uint8_t *w0, 
 
 namespace {
 
-template <int QUANT, int MRT, int TOK, int NW, int SUB>
+template <int QUANT, int MRT, int TOK, int NW, int SUB, bool CENTRED = false>
 int launch_one(hipStream_t stream, const MatmulArgs *args, int n) {
     using G = ShortGeometry<QUANT, MRT, TOK, NW, SUB>;
-    auto *kern = &gemm_short_kernel<QUANT, MRT, TOK, NW, SUB>;
+    auto *kern = &gemm_short_kernel<QUANT, MRT, TOK, NW, SUB, CENTRED>;
     if (G::LDS > 48 * 1024) {
         // one-time opt-in to more than the default dynamic LDS limit
         static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
@@ -501,6 +511,14 @@ ShortTile short_tile(Quant quant, const MatmulArgs *args, int n) {
 
 template <int QUANT>
 int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTile &t) {
+    if constexpr (QUANT == kInt8) {
+        if (args[0].T <= 4 && t.tok == 8) {
+#define WRQ_SHORT(M, SUB) \
+    if (t.mrt == M && t.nw == 8 && t.sub == SUB) return launch_one<QUANT, M, 8, 8, SUB, true>(stream, args, n);
+            WRQ_SHORT(1, 2) WRQ_SHORT(1, 1) WRQ_SHORT(2, 1) WRQ_SHORT(3, 1) WRQ_SHORT(4, 1)
+#undef WRQ_SHORT
+        }
+    }
 #define WRQ_SHORT(M, TOK, NW, SUB) \
     if (t.mrt == M && t.tok == TOK && t.nw == NW && t.sub == SUB) return launch_one<QUANT, M, TOK, NW, SUB>(stream, args, n);
 #define WRQ_SHORT_TOK(TOK) WRQ_SHORT(1, TOK, 8, 1) WRQ_SHORT(2, TOK, 8, 1) WRQ_SHORT(3, TOK, 8, 1) WRQ_SHORT(4, TOK, 8, 1)
