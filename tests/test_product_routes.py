@@ -95,10 +95,10 @@ def test_every_tile_of_the_short_run_kernel_has_a_test(wrq, overrides, kind):
     ("int8", 2048, 10240, 16, "chunk"), ("int8", 2048, 14336, 12, "chunk"), ("int8", 2048, 8192, 16, "short"), ("int8", 2560, 14336, 16, "short"),
     ("nf4", 2048, 14336, 16, "chunk"), ("nf4", 2048, 12288, 16, "short"), ("int8", 4096, 17920, 20, "chunk"), ("int8", 4096, 14336, 20, "short"), ("int8", 11260, 15488, 18, "short"),
     ("int8", 1024, 4096, 32, "chunk"), ("int8", 1280, 4096, 32, "short"), ("int8", 768, 4096, 28, "short"), ("nf4", 1024, 4096, 32, "short"),
-    ("nf4", 4096, 17920, 32, "chunk"), ("nf4", 4096, 14336, 32, "short"), ("nf4", 5120, 17920, 32, "short"),
+    ("nf4", 4096, 16384, 32, "chunk"), ("nf4", 4096, 14336, 32, "short"), ("nf4", 5120, 17920, 32, "short"),
     ("nf4", 16384, 128, 48, "chunk"), ("int8", 16384, 128, 48, "chunk"), ("nf4", 5120, 128, 128, "chunk"), ("int8", 2560, 128, 256, "chunk"), ("nf4", 1024, 128, 128, "short"),
     ("int8", 4096, 8960, 128, "chunk"), ("int8", 4096, 10240, 112, "chunk"), ("int8", 2560, 10240, 128, "chunk"), ("int8", 2048, 10240, 224, "chunk"),
-    ("int8", 2560, 8960, 128, "short"), ("int8", 5120, 10240, 96, "short"), ("int8", 3072, 10240, 160, "short"), ("int8", 4096, 8192, 128, "short"),
+    ("int8", 2048, 8960, 256, "chunk"), ("int8", 2048, 8960, 192, "short"), ("int8", 2560, 8960, 128, "short"), ("int8", 5120, 10240, 96, "short"), ("int8", 3072, 10240, 160, "short"), ("int8", 4096, 8192, 128, "short"),
     ("nf4", 8192, 14336, 64, "chunk"), ("nf4", 4096, 10240, 128, "chunk"), ("nf4", 8192, 8192, 64, "short"), ("nf4", 8192, 14336, 48, "short"), ("nf4", 5120, 17920, 96, "short"),
     ("int8", 5120, 5120, 192, "chunk"), ("int8", 3072, 5120, 256, "chunk"), ("int8", 5120, 4096, 192, "short"), ("int8", 6144, 5120, 128, "short")])
 def test_short_run_rules_end_where_the_other_kernels_are_faster(wrq, kind, rows, K, T, route):

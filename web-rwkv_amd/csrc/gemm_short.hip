@@ -16,7 +16,8 @@
 //     fetched before the first step, behind the loads.
 // Bound: at 5 .. 16 tokens the stream of weights (with the latency of one launch), from 17 tokens on the activations
 // that every workgroup fetches and stages again (2 K T bytes against 16 MRT K or half of that) and, for nf4, the table lookups.
-// Scales are applied per block in f32 as in gemm.hip: the f16 operands stay exact.
+// Scales are applied per block in f32 as in gemm.hip: the f16 operands stay exact.  Lines of the rules below are where the time against the kernels that took these
+// launches before crosses 1, on a grid of 18 row counts x 21 K x 23 run lengths and drawn groups of products.
 //
 // Measured (us per launch in a graph over cold copies, chunk kernel -> here; attention group / att.output / {ffn.key,
 // ffn.receptance} / ffn.value): 1.6B nf4 at 5 tokens 8.2 / 5.8 / 10.4 / 10.6 -> 6.2 / 4.1 / 7.5 / 7.8; 3B int8 at 19
@@ -395,10 +396,10 @@ struct ShortTile {
 constexpr ShortTile kNoTile{0, 0, 0, 0};
 
 // Runs of up to 48 tokens in one token block.  Row tiles per workgroup: one up to 4096 rows (256 workgroups), then the fewest that
-// leave one workgroup per CU; beyond 16384 rows no number does, and three keep the last round short (18432 x 4096 at 8 tokens: int8
-// 18.5 us with 3, 20.5 with 4).  Workgroups have eight waves, two per SIMD.  Where two rounds of workgroups with three row tiles run, and
-// where the activations of 33 tokens and more leave no room for eight slots, they have four (18432 x 4096 nf4 at 32 tokens 26.8
-// against 29.0 us).
+// leave one workgroup per CU; beyond 16384 rows no number does, and three keep the last round short (18432 x 4096 at 16 tokens: int8
+// 21.0 us with 3, 24.8 with 4; nf4 20.1, 24.3).  Workgroups have eight waves, two per SIMD.  Where two rounds of workgroups with three row tiles run, and
+// where the activations of 33 tokens and more leave no room for eight slots, they have four (18432 x 4096 at 24 / 32 tokens, four waves / eight: int8 24.2 / 24.6 and
+// 26.1 / 27.0 us, nf4 25.3 / 27.1 and 26.3 / 28.6; 20480 x 5120 int8 31.9 / 31.2 and 34.5 / 33.6, nf4 31.6 / 33.6 and 33.5 / 35.3).
 ShortTile one_block(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     const uint64_t tiles = (rows + 15) / 16;
     const bool rounds = tiles > 1024;
@@ -440,7 +441,7 @@ bool one_block_pays(Quant quant, uint64_t rows, uint32_t K, uint32_t T) {
     if (T <= 16) return rows > 2048 || K <= (nf4 ? (rows < 2048 ? 10240u : 12288u) : rows < 2048 ? 5120u : 8960u);
     if (T <= 24) return nf4 || K <= 10240 || (T <= 20 && rows >= 2048 && (rows > 4096 || K <= 14336)); // int8 4096 x 14336 at 19 / 24 tokens 0.92 / 1.04, 17920 at 20 1.04, 11260 x 15488 0.78; nf4 0.85
     if (T <= 32) {
-        if (rows >= 2560) return nf4 ? rows > 4096 || K <= 16384 : K <= 8192; // 4096 x 14336 0.96 .. 1.01 (nf4), 1.18 (int8), 17920 nf4 1.06, 5120 x 17920 1.02
+        if (rows >= 2560) return nf4 ? rows > 4096 || K <= 15360 : K <= 8192; // 4096 x 14336 0.96 .. 1.02 (nf4), 1.18 (int8), 16384 nf4 1.03 .. 1.06, 5120 x 17920 1.02
         // 2048 x 7168 1.04 (nf4), 1.13 (int8); 1024 x 4096 int8 1.10 (its measured chunk tile serves up to 7 % around), 768 and 1280 rows 0.84 and 0.77
         return K <= 4096 && (nf4 || K < 3810 || rows < 953 || rows > 1095);
     }
@@ -461,7 +462,8 @@ ShortTile several_blocks(Quant quant, const MatmulArgs *args, int n, uint64_t ro
     // tokens 1.04 .. 1.11 (two row tiles, 48 tokens: 0.81 .. 0.91)
     if (K > 8192 && ((T > 96 && rows > 3072) || (T > 48 && T <= 64 && rows > 6144))) return kNoTile;
     // int8 10240: 2560 .. 4096 rows at 80 .. 128 tokens 1.02 .. 1.08, 2048 from 160 tokens on 1.04 .. 1.16; 5120 rows 0.94, 3072 at 160 tokens 0.89
-    if (quant == kInt8 && K > 8960 && rows <= (T > 128 ? 2560 : 4096)) return kNoTile;
+    // (8960: 2048 rows at 224 and 256 tokens 1.04)
+    if (quant == kInt8 && (K > 8960 ? rows <= (T > 128 ? 2560 : 4096) : K > 8192 && T > 192)) return kNoTile;
     // padding included: a launch is dealt to the XCDs round-robin, and 256 live workgroups among more are not 32 on each of them
     // (588 + 548 + 2804 + 1040 rows, 148 tokens, counted without: 1.42 of the chunk kernel's time)
     auto workgroups = [&](int mrt, int tok) {
@@ -543,6 +545,8 @@ int launch_tile(hipStream_t stream, const MatmulArgs *args, int n, const ShortTi
 // Many rows, single products: int8, 4 tokens, K 1024: 16384 rows 0.88, 20480 1.12, 65536 1.23; K 2048: 20480 1.01, 32768 1.07; K 4096 and 5120 up to 65536 rows
 // 0.83 .. 0.98; K 768, 3 and 4 tokens: 20480 rows 0.87, 65536 1.00; K 2560 up to 65536 rows 0.64 .. 0.76.  nf4, K 1024, 2 tokens: 16384 rows 0.83, 20480 1.03,
 // 65536 1.11; 3 tokens, K of 768 .. 5120, up to 65536 rows 0.58 .. 0.97, but K 1792 19092 rows 1.08, 24876 1.16.
+// nf4, f32 outputs against 64 bits: 0.85 .. 0.91 of the decode kernels' error for symmetric inputs, 1.00 .. 1.16 for inputs of one sign (of a layer's products ffn.value
+// alone has those, and its K keeps it on the decode kernels).
 // nf4 runs of 4 tokens through these entries are on the matrix cores anyway, so their launches were compared with the chunk kernel.
 // Four products of K x K in one launch, before and now, us: int8 K 2560 3 tokens 10.7 -> 7.6, 4 tokens 10.7 -> 7.7; K 4096 4 tokens
 // 15.9 -> 13.8; nf4 K 2048 2 tokens 6.5 -> 6.2, 3 tokens 7.7 -> 6.1; K 2560 3 tokens 11.8 -> 8.5; K 4096 3 tokens 17.0 -> 14.6.
